@@ -264,8 +264,7 @@ struct GatherParams {
   KeyGeom kg;
   int HY, HZ;
   int64_t cells;
-  int64_t ks;
-  int64_t max_items;  // entries of the item-to-tile table
+  TileList list;
   int64_t rowlen;
   double mass;
   FastDiv fhz, fhy;
@@ -274,13 +273,14 @@ struct GatherParams {
 
 // One workgroup per work item of the tile order: stage the halo'd tile of
 // G = dL/drho in LDS, then the gradients of the item's records, written at
-// the records' own (tile-order) positions as (dL/dx, dL/dy, dL/dz[, dL/dm]):
+// the records' own pool slots as (dL/dx, dL/dy, dL/dz[, dL/dm]):
 // coalesced.
 template <typename T, int NM, int GM>
 __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__restrict__ G, const float *__restrict__ rec,
-                                                                 const uint32_t *__restrict__ tile_start,
-                                                                 const uint32_t *__restrict__ item_start,
                                                                  const uint32_t *__restrict__ item_tile,
+                                                                 const uint32_t *__restrict__ item_start,
+                                                                 const uint32_t *__restrict__ start,
+                                                                 const uint32_t *__restrict__ blist,
                                                                  GatherParams P, float *__restrict__ out) {
   constexpr int RW = 3 + NM;
   constexpr int RWO = 3 + GM;
@@ -293,8 +293,8 @@ __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__rest
   const uint32_t xcd = blockIdx.x % NUM_XCD, slot = blockIdx.x / NUM_XCD;
   const uint32_t item = ((slot / GATHER_RUN) * NUM_XCD + xcd) * GATHER_RUN + slot % GATHER_RUN;
   ItemRange ir;
-  if (!item_range(item_tile, item_start, tile_start, P.ks, P.max_items, item, ir)) return;
-  if (ir.pb >= ir.pe) return;
+  if (!item_range(item_tile, item_start, start, P.list.ks, P.list.max_items, item, ir)) return;
+  if (ir.lb >= ir.le) return;
   const int64_t k = ir.k;
   const int ntz = P.kg.ntz, nty = P.kg.nty, d = P.kg.d;
   const uint32_t kxy = P.fntz.div((uint32_t)k), kx = P.fnty.div(kxy);
@@ -302,8 +302,45 @@ __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__rest
   const int ty = (int)(kxy - kx * (uint32_t)nty);
   const int tx = (int)kx;
   const int ox = tx << P.kg.sx, oy = ty << P.kg.sy, oz = tz << P.kg.sz;
-  // four loads in flight per thread while staging, and four records while gathering
+  // four loads in flight per thread while staging, and four records while
+  // gathering: the next batch's records, through the list entries loaded one
+  // batch earlier, load while this batch is worked on (the first ones during
+  // the staging)
   constexpr int UNR = 4;
+  const int lg = P.list.lg;
+  // a thread's place in the blocks is the same in every batch (blocks of at
+  // most 256 slots divide the 512 threads)
+  const uint32_t in = threadIdx.x & ((1u << lg) - 1), te = threadIdx.x >> lg, eu = (uint32_t)GATHER_THREADS >> lg;
+  const uint32_t ents = ir.le - ir.lb;
+  float rr[UNR][RW], nx[UNR][RW];
+  uint32_t ent[UNR], at_slot[UNR], nslot[UNR];
+  uint32_t em = 0, vm = 0, nvm = 0;
+  auto load_entries = [&](uint32_t rel) {
+    em = 0;
+#pragma unroll
+    for (int u = 0; u < UNR; u++) {
+      const uint32_t e = rel + u * eu + te;
+      if (e < ents) {
+        ent[u] = blist[ir.lb + e];
+        em |= 1u << u;
+      }
+    }
+  };
+  auto load_records = [&]() {
+    nvm = 0;
+#pragma unroll
+    for (int u = 0; u < UNR; u++) {
+      if (((em >> u) & 1u) && in < P.list.fill(ent[u])) {
+        nvm |= 1u << u;
+        nslot[u] = P.list.slot0(ent[u]) + in;
+#pragma unroll
+        for (int q = 0; q < RW; q++) nx[u][q] = rec[(int64_t)nslot[u] * RW + q];
+      }
+    }
+  };
+  load_entries(0);
+  load_records();
+  load_entries(UNR * eu);
   for (int c0 = threadIdx.x; c0 < (int)P.cells; c0 += GATHER_THREADS * UNR) {
     T t[UNR];
 #pragma unroll
@@ -330,20 +367,19 @@ __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__rest
   __syncthreads();
   const int sy = P.HZ, sx = P.HY * P.HZ;
   const double units = P.kg.units;
-  for (uint32_t i0 = ir.pb + threadIdx.x; i0 < ir.pe; i0 += GATHER_THREADS * UNR) {
-    float rr[UNR][RW];
+  for (uint32_t e0 = 0; e0 < ents; e0 += UNR * eu) {
+    vm = nvm;
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
-      const uint32_t i = i0 + u * GATHER_THREADS;
-      if (i < ir.pe) {
+      at_slot[u] = nslot[u];
 #pragma unroll
-        for (int q = 0; q < RW; q++) rr[u][q] = rec[(int64_t)i * RW + q];
-      }
+      for (int q = 0; q < RW; q++) rr[u][q] = nx[u][q];
     }
+    load_records();
+    load_entries(e0 + 2 * UNR * eu);
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
-      const uint32_t i = i0 + u * GATHER_THREADS;
-      if (i >= ir.pe) break;
+      if (!((vm >> u) & 1u)) continue;
       const float *r = rr[u];
       double fx, fy, fz;
       const int lx = cell_of(r[0], units, d, fx) - ox;
@@ -368,7 +404,7 @@ __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__rest
       const double gm = b00 * a00 + b10 * a10 + b01 * a01 + b11 * a11;
       const double m = NM ? (double)r[3] : P.mass;
       const double s = m * units;
-      float *o = out + (int64_t)i * RWO;
+      float *o = out + (int64_t)at_slot[u] * RWO;
       o[0] = (float)(dgx * s);
       o[1] = (float)(dgy * s);
       o[2] = (float)(dgz * s);
@@ -465,18 +501,17 @@ void gather_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass, fl
   P.HY = tg.HY;
   P.HZ = tg.HZ;
   P.cells = tg.cells;
-  P.ks = o.ks;
-  P.max_items = o.max_items;
+  P.list = o.list;
   P.rowlen = p.rowlen;
   P.mass = mass;
   P.fhz = FastDiv((uint32_t)tg.HZ);
   P.fhy = FastDiv((uint32_t)tg.HY);
   P.fntz = FastDiv((uint32_t)tg.ntz);
   P.fnty = FastDiv((uint32_t)tg.nty);
-  const int64_t grid = ceil_div(o.max_items, 8 * GATHER_RUN) * 8 * GATHER_RUN;
+  const int64_t grid = ceil_div(o.list.max_items, 8 * GATHER_RUN) * 8 * GATHER_RUN;
   hipLaunchKernelGGL((k_gather_tiles<T, NM, GM>), dim3((unsigned)grid), dim3(GATHER_THREADS),
-                     (size_t)tg.cells * sizeof(T), p.stream, p.field.as<const T>(), o.rec, o.tile_start, o.item_start,
-                     o.item_tile, P, out);
+                     (size_t)tg.cells * sizeof(T), p.stream, p.field.as<const T>(), o.rec, o.list.item_tile, o.list.item_start,
+                     o.list.start, o.list.blist, P, out);
   GENPK_LAUNCH_CHECK();
 }
 

@@ -72,7 +72,7 @@ void plan_set_tiles(Plan &p, int tx, int ty, int tz) {
   t.cm = (int64_t)t.HX * t.HY * t.TZ;
   t.cz = (int64_t)t.HX * t.HY;
   t.kbits = bits_for(t.K);
-  if (t.kbits <= 9) {
+  if (t.kbits <= ONE_PASS_BITS) {
     t.passes = 1;
     t.hi_bits = t.kbits;
     t.lo_bits = 0;

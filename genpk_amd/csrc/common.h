@@ -64,7 +64,10 @@ int guarded(F &&f) {
 constexpr int FIXED_FRAC_BITS = 36;
 constexpr double FIXED_ONE = 68719476736.0;            // 2^36
 constexpr double FIXED_INV = 1.0 / 68719476736.0;      // 2^-36
-constexpr int DEPOSIT_ITEM_MAX = 131072;
+constexpr int LG_ITEM_MAX = 17;
+constexpr int DEPOSIT_ITEM_MAX = 1 << LG_ITEM_MAX;
+// Tile keys of at most this many bits are partitioned in one pass.
+constexpr int ONE_PASS_BITS = 10;
 // Smallest item cap that deposit_item_max (tilesort.h) takes for few tiles.
 constexpr int DEPOSIT_ITEM_MIN = 16384;
 

@@ -54,8 +54,7 @@ struct DepParams {
   int HX, HY, HZ;
   int64_t cells;       // accumulator cells HX*HY*HZ
   int64_t cm, cz, zoff;  // tile store layout
-  int64_t ks;          // key space size (tile_start has ks+1 entries)
-  int64_t max_items;   // entries of the item-to-tile table
+  TileList list;       // the tiles' records and work items
   double mass;         // constant mass (u64 path)
   double bias;         // 2^52 (to_fixed)
   const uint32_t *mrange;  // per-particle masses: the sort's |mass| range (float bits)
@@ -78,14 +77,14 @@ struct DepParams {
 // offsets fold into the LDS instructions' immediate offsets.
 template <typename Real, int NM, int RW, bool STD>
 __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict__ rec,
-                                                         const uint32_t *__restrict__ tile_start,
-                                                         const uint32_t *__restrict__ item_start,
                                                          const uint32_t *__restrict__ item_tile,
+                                                         const uint32_t *__restrict__ item_start,
+                                                         const uint32_t *__restrict__ start,
+                                                         const uint32_t *__restrict__ blist,
                                                          const uint32_t *__restrict__ part_start, DepParams P,
                                                          Real *__restrict__ tiles, double *__restrict__ partials) {
   using Acc = unsigned long long;
   constexpr int UNR = 4;
-  constexpr int BATCH = DEP_THREADS * UNR;
   extern __shared__ unsigned long long lds_raw[];
   Acc *acc = reinterpret_cast<Acc *>(lds_raw);
   const int TX = STD ? 16 : P.kg.TX, TY = STD ? 32 : P.kg.TY, TZ = STD ? 32 : P.kg.TZ;
@@ -110,39 +109,92 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
     else
       return (double)a * scale;
   };
+  // The records reach the accumulation through two stages of loads that run
+  // ahead of it over the batches of this workgroup's items, in order (empty
+  // items have none): the block-list entries of batch b + 2 and the records
+  // of batch b + 1 are loading while batch b accumulates.
   float r[UNR][RW], nx[UNR][RW];
-  auto load_batch = [&](uint32_t i0, uint32_t pe) {
+  uint32_t ent[UNR];            // list entries of the batch whose records load next
+  uint32_t em = 0;              // bit u: ent[u] is an entry
+  uint32_t vm = 0, nvm = 0;     // bit u: r[u] / nx[u] holds a record
+  const TileList &T = P.list;
+  // a thread's place in the blocks is the same in every batch (blocks of at
+  // most 256 slots divide the 1024 threads)
+  const int lg = T.lg;
+  const uint32_t in = threadIdx.x & ((1u << lg) - 1), te = threadIdx.x >> lg, eu = (uint32_t)DEP_THREADS >> lg;
+  auto range_of = [&](uint32_t it, ItemRange &o) { return item_range(item_tile, item_start, start, T.ks, T.max_items, it, o); };
+  struct {
+    uint32_t item, lb, ents, rel;  // the batch: entries [rel, rel + UNR * eu) of the item's `ents`
+  } ld;
+  ItemRange ahead;  // the item after ld's
+  bool ahead_ok;
+  auto load_step = [&]() {  // to the next batch (past the last item: ents = 0)
+    ld.rel += UNR * eu;
+    while (ld.rel >= ld.ents) {
+      ld.item += gridDim.x;
+      ld.rel = 0;
+      ld.ents = 0;
+      if (!ahead_ok) break;
+      ld.lb = ahead.lb;
+      ld.ents = ahead.le - ahead.lb;
+      ahead_ok = range_of(ld.item + gridDim.x, ahead);
+    }
+  };
+  auto load_entries = [&]() {
+    em = 0;
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
-      const uint32_t i = i0 + u * DEP_THREADS + threadIdx.x;
-      if (i < pe) {
+      const uint32_t e = ld.rel + u * eu + te;
+      if (e < ld.ents) {
+        ent[u] = blist[ld.lb + e];
+        em |= 1u << u;
+      }
+    }
+  };
+  auto load_records = [&]() {
+    nvm = 0;
 #pragma unroll
-        for (int q = 0; q < RW; q++) nx[u][q] = rec[(int64_t)i * RW + q];
+    for (int u = 0; u < UNR; u++) {
+      if (((em >> u) & 1u) && in < T.fill(ent[u])) {
+        nvm |= 1u << u;
+        const float *src = rec + (int64_t)(T.slot0(ent[u]) + in) * RW;
+#pragma unroll
+        for (int q = 0; q < RW; q++) nx[u][q] = src[q];
       }
     }
   };
   auto take_batch = [&]() {
+    vm = nvm;
 #pragma unroll
     for (int u = 0; u < UNR; u++)
 #pragma unroll
       for (int q = 0; q < RW; q++) r[u][q] = nx[u][q];
   };
-  // Persistent over the items (item, item + gridDim.x, ...).  The next
-  // item's first records load during this item's last batch and are in
-  // registers before the flush: the flush's stores then drain while the next
-  // item accumulates (a wait for loads issued after them would wait for the
-  // stores too, the counter being in order).
+  // Persistent over the items (item, item + gridDim.x, ...).  Every load
+  // issued before an item's flush has arrived before it too: the flush's
+  // stores then drain while the next item accumulates (a wait for loads
+  // issued before them, the counter being in order and the stores' count not
+  // known, would wait for the stores as well).
   uint32_t item = blockIdx.x;
   ItemRange ir;
-  bool have = item_range(item_tile, item_start, tile_start, P.ks, P.max_items, item, ir);
-  if (have) load_batch(ir.pb, ir.pe);
+  bool have = range_of(item, ir);
+  ahead_ok = have && range_of(item + gridDim.x, ahead);
+  ld.item = item;
+  ld.lb = have ? ir.lb : 0u;
+  ld.ents = have ? ir.le - ir.lb : 0u;
+  ld.rel = 0;
+  if (ld.ents == 0) load_step();  // an empty first item
+  load_entries();
+  load_records();
+  load_step();
+  load_entries();
   // the tile starts cleared; each flush clears the cells it reads
   for (int64_t c = threadIdx.x; c < P.cells; c += DEP_THREADS) acc[c] = 0;
   take_batch();
   __syncthreads();
   while (have) {
     const int64_t k = ir.k;
-    const uint32_t m = ir.m, j = ir.j, pb = ir.pb, pe = ir.pe;
+    const uint32_t m = ir.m, j = ir.j, ents = ir.le - ir.lb;
     const int ntz = P.kg.ntz, nty = P.kg.nty;
     // 32-bit multiply-high, not 64-bit divisions (~130 scalar instructions each)
     const uint32_t kxy = P.fntz.div((uint32_t)k), kx = P.fnty.div(kxy);
@@ -154,21 +206,14 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
     // the next item (uniform over the workgroup)
     const uint32_t nitem = item + gridDim.x;
     ItemRange nir;
-    const bool next = item_range(item_tile, item_start, tile_start, P.ks, P.max_items, nitem, nir);
-    bool pre = false;  // the next item's first records are loading
-    for (uint32_t i0 = pb; i0 < pe; i0 += BATCH) {
-      // loads of the next batch (this item's, or the next item's first) are
-      // issued before this batch (in r) is accumulated; one load site (two
-      // would merge their registers with copies that wait for the loads)
-      const bool more = i0 + BATCH < pe;
-      if (more || next) {
-        load_batch(more ? i0 + BATCH : nir.pb, more ? pe : nir.pe);
-        pre = !more;
-      }
+    const bool next = range_of(nitem, nir);
+    for (uint32_t e0 = 0; e0 < ents; e0 += UNR * eu) {
+      load_records();
+      load_step();
+      load_entries();
 #pragma unroll
       for (int u = 0; u < UNR; u++) {
-        const uint32_t i = i0 + u * DEP_THREADS + threadIdx.x;
-        if (i >= pe) continue;
+        if (!((vm >> u) & 1u)) continue;
         // cell_of without its wrap: a floor cell inside the tile's own cells
         // [o, o + w) lies in [0, d), where cell_of does not wrap
         double fx, fy, fz;
@@ -223,12 +268,9 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
       }
       take_batch();
     }
-    // an item without records: the next item's first records load here
-    // (taken before the flush too, so that no load is left in flight across it)
-    if (next && !pre) {
-      load_batch(nir.pb, nir.pe);
-      take_batch();
-    }
+    // the entries too have arrived before the flush
+#pragma unroll
+    for (int u = 0; u < UNR; u++) asm volatile("" : "+v"(ent[u]));
     __syncthreads();
     if (m == 1) {
       // rows of TZ values (aligned), then the z-halo plane
@@ -287,7 +329,6 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
 template <typename Real, int NM>
 __global__ void __launch_bounds__(256) k_reduce_partials(const uint32_t *__restrict__ nheavy,
                                                          const uint32_t *__restrict__ heavy,
-                                                         const uint32_t *__restrict__ item_start,
                                                          const uint32_t *__restrict__ part_start,
                                                          const double *__restrict__ partials, DepParams P,
                                                          Real *__restrict__ tiles) {
@@ -308,7 +349,7 @@ __global__ void __launch_bounds__(256) k_reduce_partials(const uint32_t *__restr
     const uint32_t k = heavy[h];
     const int64_t c = (int64_t)((uint32_t)u - h * (uint32_t)nblk) * 256 + threadIdx.x;
     if (c >= cells) continue;
-    const uint32_t m = item_start[k + 1] - item_start[k];
+    const uint32_t m = P.list.item_start[k + 1] - P.list.item_start[k];
     const int64_t at = (int64_t)part_start[k] * cells + c;
     double s;
     if (fixed) {
@@ -364,12 +405,15 @@ __global__ void __launch_bounds__(256) k_reduce_partials(const uint32_t *__restr
 // own store location is written (never a halo), so the order against the
 // halo folds does not matter, and later deposits keep it NaN.
 template <typename Real>
-__global__ void __launch_bounds__(256) k_poison(const float *__restrict__ rec, int rw, int64_t n, KeyGeom kg,
+__global__ void __launch_bounds__(256) k_poison(const float *__restrict__ rec, int rw, TileList T, KeyGeom kg,
                                                 FoldGeom fg, const uint32_t *__restrict__ nonfinite,
                                                 Real *__restrict__ tiles) {
   if (*nonfinite == 0u) return;
+  const int64_t n = (int64_t)T.start[T.ks] << T.lg;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const float *r = rec + i * rw;
+    const uint32_t ent = T.blist[i >> T.lg], in = (uint32_t)i & ((1u << T.lg) - 1);
+    if (in >= T.fill(ent)) continue;
+    const float *r = rec + (int64_t)(T.slot0(ent) + in) * rw;
     double fx, fy, fz;
     const int cx = cell_of_x86(r[0], kg.units, kg.d, fx);
     const int cy = cell_of_x86(r[1], kg.units, kg.d, fy);
@@ -462,11 +506,9 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
   const TileGeom &tg = p.tg;
   const int store = p.tiles_live ? 0 : 1;
   const float *sorted = o.rec;
-  const uint32_t *tile_start = o.tile_start, *item_start = o.item_start, *part_start = o.part_start;
-  const uint32_t *nheavy = o.nheavy, *heavy = o.heavy;
-  const int64_t ks = o.ks, n = o.n, max_items = o.max_items;
-  const int64_t max_parts = 2 * ceil_div(n, (int64_t)o.item_max);
-  double *partials = static_cast<double *>(p.partials.ensure((size_t)max_parts * tg.cells * 8 + 64));
+  const uint32_t *part_start = o.part_start, *nheavy = o.nheavy, *heavy = o.heavy;
+  const int64_t n = o.n, max_items = o.list.max_items;
+  double *partials = static_cast<double *>(p.partials.ensure((size_t)o.max_parts * tg.cells * 8 + 64));
 
   DepParams P;
   P.kg = kg;
@@ -475,44 +517,42 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
   P.cm = tg.cm;
   P.cz = tg.cz;
   P.zoff = tg.K * tg.cm;
-  P.ks = ks;
-  P.max_items = max_items;
+  P.list = o.list;
   P.mass = mass;
   P.bias = 4503599627370496.0;
   P.mrange = o.mrange;
-  P.nonfinite = static_cast<uint32_t *>(p.nonfinite.ensure(64));
+  P.nonfinite = p.nonfinite.as<uint32_t>();  // cleared by the sort (a repeated deposit finds the same particles)
   P.store = store;
   P.fntz = FastDiv((uint32_t)tg.ntz);
   P.fnty = FastDiv((uint32_t)tg.nty);
   P.fnblk = FastDiv((uint32_t)ceil_div(tg.cells, 256));
-  fill_zero(P.nonfinite, 4, s);
   const size_t lds = (size_t)tg.cells * 8;
   {
     Stage st(p, "deposit_tiles");
     const bool std_tiles = tg.TX == 16 && tg.TY == 32 && tg.TZ == 32;
     const dim3 grid((unsigned)deposit_grid<NM, RW>(p, std_tiles, lds, max_items)), block(DEP_THREADS);
     if (p.prec == 4 && std_tiles)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, true>), grid, block, lds, s, sorted, tile_start, item_start,
-                         o.item_tile, part_start, P, p.tiles.as<float>(), partials);
+      hipLaunchKernelGGL((k_deposit<float, NM, RW, true>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
+                         o.list.start, o.list.blist, part_start, P, p.tiles.as<float>(), partials);
     else if (p.prec == 4)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, false>), grid, block, lds, s, sorted, tile_start, item_start,
-                         o.item_tile, part_start, P, p.tiles.as<float>(), partials);
+      hipLaunchKernelGGL((k_deposit<float, NM, RW, false>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
+                         o.list.start, o.list.blist, part_start, P, p.tiles.as<float>(), partials);
     else if (std_tiles)
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, true>), grid, block, lds, s, sorted, tile_start, item_start,
-                         o.item_tile, part_start, P, p.tiles.as<double>(), partials);
+      hipLaunchKernelGGL((k_deposit<double, NM, RW, true>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
+                         o.list.start, o.list.blist, part_start, P, p.tiles.as<double>(), partials);
     else
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, false>), grid, block, lds, s, sorted, tile_start, item_start,
-                         o.item_tile, part_start, P, p.tiles.as<double>(), partials);
+      hipLaunchKernelGGL((k_deposit<double, NM, RW, false>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
+                         o.list.start, o.list.blist, part_start, P, p.tiles.as<double>(), partials);
     GENPK_LAUNCH_CHECK();
   }
   {
     Stage st(p, "reduce_partials");
     if (p.prec == 4)
-      hipLaunchKernelGGL((k_reduce_partials<float, NM>), dim3(1024), dim3(256), 0, s, nheavy, heavy, item_start,
-                         part_start, partials, P, p.tiles.as<float>());
+      hipLaunchKernelGGL((k_reduce_partials<float, NM>), dim3(1024), dim3(256), 0, s, nheavy, heavy, part_start,
+                         partials, P, p.tiles.as<float>());
     else
-      hipLaunchKernelGGL((k_reduce_partials<double, NM>), dim3(1024), dim3(256), 0, s, nheavy, heavy, item_start,
-                         part_start, partials, P, p.tiles.as<double>());
+      hipLaunchKernelGGL((k_reduce_partials<double, NM>), dim3(1024), dim3(256), 0, s, nheavy, heavy, part_start,
+                         partials, P, p.tiles.as<double>());
     GENPK_LAUNCH_CHECK();
   }
   {
@@ -520,10 +560,10 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
     const FoldGeom fg = fold_geom(p);
     const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(n, 256), 2048);
     if (p.prec == 4)
-      hipLaunchKernelGGL(k_poison<float>, dim3(grid), dim3(256), 0, s, sorted, o.rw, n, kg, fg, P.nonfinite,
+      hipLaunchKernelGGL(k_poison<float>, dim3(grid), dim3(256), 0, s, sorted, o.rw, o.list, kg, fg, P.nonfinite,
                          p.tiles.as<float>());
     else
-      hipLaunchKernelGGL(k_poison<double>, dim3(grid), dim3(256), 0, s, sorted, o.rw, n, kg, fg, P.nonfinite,
+      hipLaunchKernelGGL(k_poison<double>, dim3(grid), dim3(256), 0, s, sorted, o.rw, o.list, kg, fg, P.nonfinite,
                          p.tiles.as<double>());
     GENPK_LAUNCH_CHECK();
   }

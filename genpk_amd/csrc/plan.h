@@ -84,22 +84,35 @@ struct BinTables {
 
 enum class FieldState { None, Real, Spectrum, YDone };
 
-// Particles partitioned by tile (plan scratch; see sort_by_tile): records
-// of rw floats (x, y, z[, mass]), tile starts, work items, and optionally
-// the permutations input -> sorted position.
+// The particles of a partition by tile, as the tile kernels read them: tile
+// k's records fill the listed blocks [start[k], start[k + 1]) of 2^lg record
+// slots (entry: the block in the low 32 - lg bits, its fill less one above);
+// its work items are [item_start[k], item_start[k + 1]).
+struct TileList {
+  const uint32_t *start = nullptr, *item_start = nullptr;
+  const uint32_t *item_tile = nullptr;  // tile of each work item (max_items entries)
+  const uint32_t *blist = nullptr;
+  int lg = 0;
+  int64_t ks = 0, max_items = 0;
+  __device__ __forceinline__ uint32_t slot0(uint32_t ent) const { return ent << lg; }  // first slot of the entry's block
+  __device__ __forceinline__ uint32_t fill(uint32_t ent) const { return (ent >> (32 - lg)) + 1; }
+};
+
+// Particles partitioned by tile (plan scratch; see sort_by_tile): a pool of
+// records of rw floats (x, y, z[, mass]), the tiles' block lists and work
+// items, and optionally the permutations input -> slot in the pool.
 struct TileOrder {
   const float *rec = nullptr;
   int rw = 0;
   bool has_mass = false, has_perm = false;
   const uint32_t *perm1 = nullptr, *perm2 = nullptr;
-  const uint32_t *tile_start = nullptr, *item_start = nullptr, *part_start = nullptr;
-  const uint32_t *item_tile = nullptr;  // tile of each work item (max_items entries)
+  TileList list;
+  const uint32_t *part_start = nullptr;  // first partial tile of each split tile
   const uint32_t *nheavy = nullptr, *heavy = nullptr;
   // with masses: [0] the bits of the largest |mass|, [1] those of the
   // smallest nonzero |mass| (0xffffffff when every mass is 0)
   const uint32_t *mrange = nullptr;
-  int64_t ks = 0, n = 0, max_items = 0;
-  uint32_t item_max = 0;  // records per work item at most (deposit_item_max)
+  int64_t n = 0, max_parts = 0;  // max_parts: bound of the partial tiles
 };
 
 // Tile order kept from the last deposit made with retain = true, for the
@@ -160,11 +173,12 @@ struct Plan {
   bool tiles_live = false;  // tiles hold deposits not yet folded
 
   // sort / deposit scratch
-  DevBuf recA, recB, table1, table2, seginfo, tile_start, item_start, part_start, heavy, partials, item_tile;
+  DevBuf recA, recB, table1, seginfo, item_start, heavy, partials, item_tile;
   DevBuf permA, permB;      // sort permutations kept for the adjoint gather
-  DevBuf dig2;              // low tile-key digit of each pass-1 output record (one byte)
-  DevBuf pages;             // paged first sort pass: block digits, fills and lists
-  DevBuf mrange;            // largest and smallest nonzero |mass| of the last sort (float bits)
+  DevBuf pages1, pages;     // block headers, counts and lists of a paged first and of the last sort pass
+  DevBuf sort_tot;          // bucket totals of the sort passes
+  int64_t sort_tot_zero = 0;  // bucket totals known to be zero (0: unknown)
+  DevBuf mrange;            // largest and smallest nonzero |mass| of the last sort (float bits), then per workgroup
   DevBuf nonfinite;         // flag of the last deposit: a particle position is not finite
   DevBuf scan_tmp;
   RetainedOrder order;

@@ -1,13 +1,16 @@
-// Partition of particles by deposit tile on gfx950: an MSD radix partition
-// of one or two passes over the tile key (upsweep histogram in LDS ->
-// offset scan -> downsweep that ranks records with LDS atomics, stages them
-// in LDS by digit and writes contiguous runs), then the work items of the
-// tile kernels.  Large two-pass sorts run their first pass paged: each
-// workgroup appends each digit's records to blocks of its own, so the
-// positions are read once (no histogram pass), and the second pass reads
-// every digit's blocks through a block list.  Global atomics are avoided:
-// on this chip they run at ~27 Gop/s.  The order of the records within one
-// tile is not specified (the tile kernels do not depend on it).
+// Partition of particles by deposit tile on gfx950: a radix partition of one
+// or two passes over the tile key.  The last pass is always paged: every
+// workgroup ranks the records of its chunk with LDS atomics, stages them in
+// LDS by digit and appends each digit's run to blocks of record slots that
+// it takes from a range of its own, so there is no histogram pass and no
+// shared cursor; a small directory (k_dir, k_list) then lists every tile's
+// blocks and its work items, and the tile kernels read the records through
+// that list.  A first pass is paged the same way where each workgroup holds
+// many records of each digit; elsewhere it counts first (k_upsweep, an
+// offset scan) and writes contiguous runs.  Global atomics are avoided but
+// for one per workgroup and digit: on this chip they run at ~27 Gop/s.  The
+// order of the records within one tile is not specified (the tile kernels
+// do not depend on it).
 #include "tilesort.h"
 
 #include <algorithm>
@@ -23,17 +26,10 @@ namespace {
 // ms for two 512-thread workgroups per CU staging 4096 records each).
 constexpr int SORT_THREADS = 1024;
 constexpr int SORT_WAVES = SORT_THREADS / 64;
-// Records per workgroup: from SORT_CHUNK_MIN (one sub-chunk of the
-// downsweep) up to SORT_CHUNK_MAX, the smallest that keeps at most four
-// chunks per CU (small sets then still spread over every CU).  32 Ki rather
-// than 64 Ki: the paged second pass's count kernel runs more, shorter
-// workgroups (2^27 particles at 512^3: 0.23 -> 0.17 ms) and the downsweeps
-// are unchanged or slightly faster; 16 Ki is no faster.
+// Records per workgroup of the counted first pass: from SORT_CHUNK_MIN (one
+// sub-chunk) up to SORT_CHUNK_MAX, the smallest that keeps at most four
+// chunks per CU (small sets then still spread over every CU).
 constexpr int64_t SORT_CHUNK_MIN = 8192, SORT_CHUNK_MAX = 32768;
-// The paged second pass's count kernel: four waves per workgroup, so that
-// eight workgroups (chunks) per CU overlap their memory round trips.
-constexpr int UP_THREADS = 256;
-constexpr int UP_WAVES = UP_THREADS / 64;
 
 // Source of records: either the caller's arrays (positions [n][3], optional
 // masses [n]) or a packed record buffer of RW floats per record.
@@ -62,80 +58,55 @@ struct Src {
   }
 };
 
-// Chunk range of workgroup g and the place of its digit counts in the
-// count table: counts of digit dg at tb + dg * ts.  Pass 1 chunks tile
-// [0, n) and its table is digit-major over all chunks (tb = g, ts = number
-// of chunks).  Pass 2 chunks tile each high-digit segment separately; its
-// table is segment-major, then digit, then chunk (tb = first chunk of the
-// segment * nlo + chunk within the segment, ts = chunks of the segment), so
-// one exclusive scan of the table gives every chunk's output offsets and
-// every tile's start.
-struct ChunkMap {
-  int64_t n;
-  int nseg;                    // 0: plain chunks of [0, n)
-  const uint32_t *seg_start;   // [nseg+1] record offsets of the segments
-  const uint32_t *chunk_start; // [nseg+1] first chunk of each segment
-  int64_t nchunks;             // pass 1: number of chunks
-  int nlo;                     // pass 2: digits
-  int64_t chunk;               // records per chunk (a multiple of the downsweep's sub-chunk)
-  __device__ __forceinline__ bool range(int64_t g, int64_t &b, int64_t &e, int64_t &tb, int64_t &ts) const {
-    if (nseg == 0) {
-      b = g * chunk;
-      e = min(n, b + chunk);
-      tb = g;
-      ts = nchunks;
-      return b < e;
-    }
-    if (g >= (int64_t)chunk_start[nseg]) return false;
-    int lo = 0, hi = nseg;  // find s with chunk_start[s] <= g < chunk_start[s+1]
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if ((int64_t)chunk_start[mid] <= g) lo = mid; else hi = mid;
-    }
-    const int s = lo;
-    const int64_t c0 = chunk_start[s];
-    b = (int64_t)seg_start[s] + (g - c0) * chunk;
-    e = min((int64_t)seg_start[s + 1], b + chunk);
-    tb = c0 * nlo + (g - c0);
-    ts = (int64_t)chunk_start[s + 1] - c0;
-    return b < e;
-  }
+// Input of a pass: workgroup g takes slots [g * chunk, (g + 1) * chunk).
+//   IN_RAW: slots are the caller's n records.
+//   IN_SEG / IN_LIST: slots are the records, or the record slots of the
+//   block-list entries (2^lg each), of a first pass's buckets, bucket s from
+//   record or entry start[s] on; first_seg[g] is the bucket of g's first slot.
+//   A workgroup handles the part of each bucket in its range as a piece of
+//   its own (a bucket's digits are not another's).
+enum { IN_RAW = 0, IN_SEG = 1, IN_LIST = 2 };
+struct InMap {
+  int64_t n = 0, chunk = 0;
+  int nseg = 0;
+  int lg = 0;
 };
 
-// Write target of the downsweep's staging positions past a sub-chunk's last
-// record (the write-out issues the same stores on every path): many
-// workgroups may write it at once, and nothing reads it.
-__device__ float sort_sink[SORT_THREADS * 8 * 4];
-__device__ uint8_t sort_sink_digits[SORT_THREADS * 8];
-
-// Paged pass 1 (MODE 1 and 2 of k_downsweep, two-pass sorts of many
-// records): the pass-1 output pool is cut into blocks of PG_BLOCK record
-// slots, Q per pass-1 workgroup.
-constexpr int PG_LOG = 10;
-constexpr uint32_t PG_BLOCK = 1u << PG_LOG;
-
-// A block-list entry: the block and its fill (1 to PG_BLOCK records) in one
-// word, so that one load gives both.
-__host__ __device__ constexpr uint32_t pg_entry(uint32_t blk, uint32_t fill) { return blk | (fill - 1) << 22; }
-__device__ __forceinline__ uint32_t pg_blk(uint32_t e) { return e & ((1u << 22) - 1); }
-__device__ __forceinline__ uint32_t pg_fill(uint32_t e) { return (e >> 22) + 1; }
-
-struct PgArgs {
-  uint32_t *hdr = nullptr;          // [G * Q] of each taken block: digit | (its number among the digit's blocks) << 8
-  uint32_t *fill = nullptr;         // [G * Q] records in each taken block
-  uint32_t *used = nullptr;         // [G] blocks taken by each pass-1 workgroup
-  int64_t Q = 0;                    // blocks per pass-1 workgroup
-  const uint32_t *blist = nullptr;  // pass 2: the taken blocks, segment (pass-1 digit) by segment (pg_entry)
+// Output of a paged pass: a pool of blocks of 2^lg record slots, in which
+// every piece (a workgroup's slots of one bucket) has a range large enough for
+// its full blocks and one partly filled block per digit.  Piece w + s is
+// workgroup w's of bucket s; its range starts at block (first slot >> lg) +
+// (w + s) (nb + 1).
+struct PgOut {
+  uint32_t *hdr = nullptr;    // of each taken block: digit | (its number among the piece's blocks of the digit) << 11
+  uint32_t *cnt = nullptr;    // [pieces * nb] records per digit of each piece (written where not 0)
+  uint32_t *base = nullptr;   // [pieces * nb] number of the piece's first block among its bucket's
+  uint4 *piece = nullptr;     // first block, blocks taken, bucket (blocks taken: 0 where there is no piece)
+  unsigned long long *tot = nullptr;  // per output bucket: blocks << 32 | records, summed over the pieces
+  int lg = 0;
 };
 
-// Tile key of a record with the cells along the axes not in `axes` (bit a:
-// axis a of x, y, z) taken as 0 and not computed.
+// A block-list entry: the block in the low 32 - lg bits, its fill (1 to 2^lg
+// records) less one above, so that one load gives both.
+__device__ __forceinline__ uint32_t pg_entry(uint32_t blk, uint32_t fill, int lg) { return blk | (fill - 1) << (32 - lg); }
+
+// Tile key of a position with the cells along the axes not in `axes` (bit a:
+// axis a of x, y, z) taken as 0 and not computed: cell_of's cells, with one
+// branch for the rare wrap of any of them into [0, d).
 __device__ __forceinline__ uint32_t key_on_axes(const float *r, const KeyGeom &g, int axes) {
-  double fr;
-  const int cx = (axes & 1) ? cell_of(r[0], g.units, g.d, fr) : 0;
-  const int cy = (axes & 2) ? cell_of(r[1], g.units, g.d, fr) : 0;
-  const int cz = (axes & 4) ? cell_of(r[2], g.units, g.d, fr) : 0;
-  return (uint32_t)((((cx >> g.sx) * g.nty + (cy >> g.sy)) * g.ntz) + (cz >> g.sz));
+  int c[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) c[a] = (axes >> a) & 1 ? (int)floor((double)r[a] * g.units) : 0;
+  const unsigned ud = (unsigned)g.d;
+  if (((unsigned)c[0] >= ud) | ((unsigned)c[1] >= ud) | ((unsigned)c[2] >= ud)) {
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+      if ((unsigned)c[a] >= ud) {
+        c[a] %= g.d;
+        if (c[a] < 0) c[a] += g.d;
+      }
+  }
+  return (uint32_t)((((c[0] >> g.sx) * g.nty + (c[1] >> g.sy)) * g.ntz) + (c[2] >> g.sz));
 }
 
 struct DigitSel {
@@ -174,14 +145,13 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// counts[tb + dg * ts] = number of records of chunk g with digit dg
+// counts[dg * G + g] = number of records of chunk g with digit dg
 template <int NM>
-__global__ void __launch_bounds__(SORT_THREADS) k_upsweep(Src<NM> src, ChunkMap cm, KeyGeom kg, DigitSel ds,
-                                                          int nb, uint32_t *__restrict__ counts) {
+__global__ void __launch_bounds__(SORT_THREADS) k_upsweep(Src<NM> src, InMap im, KeyGeom kg, DigitSel ds, int nb,
+                                                          uint32_t *__restrict__ counts) {
   constexpr int UNR = 8;
   extern __shared__ uint32_t hist[];
-  int64_t b, e, tb, ts;
-  if (!cm.range(blockIdx.x, b, e, tb, ts)) return;
+  const int64_t b = blockIdx.x * im.chunk, e = min(im.n, b + im.chunk);
   for (int i = threadIdx.x; i < nb; i += SORT_THREADS) hist[i] = 0;
   __syncthreads();
   for (int64_t base = b; base < e; base += SORT_THREADS * UNR) {
@@ -207,81 +177,29 @@ __global__ void __launch_bounds__(SORT_THREADS) k_upsweep(Src<NM> src, ChunkMap 
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < nb; i += SORT_THREADS)
-    counts[tb + (int64_t)i * ts] = hist[i];
-}
-
-// k_upsweep's counts for a digit of at most 8 bits from the digit bytes the
-// previous downsweep wrote beside its output records (digs[i]: digit of
-// record i), so the records themselves are not read.  Reads the 4-byte words
-// covering [b, e): digs holds at least 4 bytes past the last record.
-__global__ void __launch_bounds__(SORT_THREADS) k_upsweep_bytes(const uint8_t *__restrict__ digs, ChunkMap cm,
-                                                                int nb, uint32_t *__restrict__ counts) {
-  constexpr int UNR = 4;
-  extern __shared__ uint32_t hist[];
-  int64_t b, e, tb, ts;
-  if (!cm.range(blockIdx.x, b, e, tb, ts)) return;
-  for (int i = threadIdx.x; i < nb; i += SORT_THREADS) hist[i] = 0;
-  __syncthreads();
-  const uint32_t *words = reinterpret_cast<const uint32_t *>(digs);
-  const int64_t w0 = b >> 2, w1 = (e + 3) >> 2;
-  for (int64_t base = w0; base < w1; base += SORT_THREADS * UNR) {
-    uint32_t v[UNR];
-#pragma unroll
-    for (int u = 0; u < UNR; u++) {
-      const int64_t w = base + u * SORT_THREADS + threadIdx.x;
-      v[u] = w < w1 ? words[w] : 0u;
-    }
-#pragma unroll
-    for (int u = 0; u < UNR; u++) {
-      const int64_t w = base + u * SORT_THREADS + threadIdx.x;
-      // a word of four equal in-range digits adds them with one atomic, and
-      // a wavefront of such words of one digit with one atomic for all
-      const uint32_t d0 = v[u] & 0xffu;
-      const bool same4 = 4 * w >= b && 4 * w + 4 <= e && v[u] == d0 * 0x01010101u;
-      const uint32_t dw = __builtin_amdgcn_readfirstlane(d0);
-      if (__ballot(same4 && d0 == dw) == ~0ull) {
-        if ((threadIdx.x & 63) == 0) atomicAdd(&hist[dw], 256u);
-      } else if (same4) {
-        atomicAdd(&hist[d0], 4u);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int64_t i = 4 * w + j;
-          if (i >= b && i < e) atomicAdd(&hist[(v[u] >> (8 * j)) & 0xffu], 1u);
-        }
-      }
-    }
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < nb; i += SORT_THREADS)
-    counts[tb + (int64_t)i * ts] = hist[i];
+  for (int i = threadIdx.x; i < nb; i += SORT_THREADS) counts[(int64_t)i * gridDim.x + blockIdx.x] = hist[i];
 }
 
 // Rank of each of a lane's PL record slots among the wave's slots of its
 // digit in this sub-chunk, from LDS atomic adds that return the old count on
 // the wave's count row (a wave whose 64 slots share one digit adds them with
-// one atomic, from lane 0).  Slots it >= nv hold no record: they take the
+// one atomic, from lane 0).  Slots not in vm hold no record: they take the
 // digit `trash` (one past the last), so that they rank and stage like
 // records, after every real one.  Equal digits are ordered by the LDS unit's
 // processing order of one instruction's lanes and, where waves share a count
 // row, by the order in which they run: the order of the records within a
 // tile is not specified (the tile kernels do not depend on it).  pk
-// receives each slot's rank (bits 0-12, below the sub-chunk's 8192 slots),
-// its digit from bit 13 and, with `two` (digits of at most 8 bits, so the
-// digit takes bits 13-21), its digit of ds2 (from the same key) from bit 22:
-// one register per slot.  Called by whole waves.
+// receives each slot's rank (bits 0-12, below the sub-chunk's 8192 slots)
+// and its digit from bit 13: one register per slot.  Called by whole waves.
 template <int NM, int PL>
-__device__ __forceinline__ void rank_records(const float (&rec)[PL][Src<NM>::RW], uint32_t nv, const KeyGeom &kg,
-                                             const DigitSel &ds, const DigitSel &ds2, bool two, uint32_t trash,
-                                             uint32_t *wrow, uint32_t (&pk)[PL]) {
+__device__ __forceinline__ void rank_records(const float (&rec)[PL][Src<NM>::RW], uint32_t vm, const KeyGeom &kg,
+                                             const DigitSel &ds, uint32_t trash, uint32_t *wrow, uint32_t (&pk)[PL]) {
   const uint32_t lane = threadIdx.x & 63;
   uint32_t rnk[PL];
   uint32_t uni = 0;  // bit it: the wave's slots `it` share one digit
 #pragma unroll
   for (int it = 0; it < PL; it++) {
-    const uint32_t key = tile_key(rec[it], kg);
-    const uint32_t dg = (uint32_t)it < nv ? ds.of_key(key) : trash;
+    const uint32_t dg = (vm >> it) & 1u ? ds.of(rec[it], kg) : trash;
     const uint32_t d0 = __builtin_amdgcn_readfirstlane(dg);
     uint32_t r = 0;
     if (__ballot(dg == d0) == ~0ull) {
@@ -290,7 +208,7 @@ __device__ __forceinline__ void rank_records(const float (&rec)[PL][Src<NM>::RW]
     } else {
       r = atomicAdd(&wrow[dg], 1u);
     }
-    pk[it] = dg << 13 | (two ? ds2.of_key(key) << 22 : 0u);
+    pk[it] = dg << 13;
     rnk[it] = r;
   }
   // a one-digit wave's slots follow lane 0's old count
@@ -300,14 +218,24 @@ __device__ __forceinline__ void rank_records(const float (&rec)[PL][Src<NM>::RW]
 }
 
 // Per-row counts of digit dg -> per-row exclusive offsets in place; returns the total.
-__device__ __forceinline__ uint32_t wave_offsets(uint32_t *whist, int nb, int hw, int dg) {
+__device__ __forceinline__ uint32_t wave_offsets(uint32_t *whist, int nbt, int hw, int dg) {
   uint32_t tot = 0;
   for (int w = 0; w < hw; w++) {
-    const uint32_t t = whist[w * nb + dg];
-    whist[w * nb + dg] = tot;
+    const uint32_t t = whist[w * nbt + dg];
+    whist[w * nbt + dg] = tot;
     tot += t;
   }
   return tot;
+}
+
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t t = __shfl_up(v, off, 64);
+    if (lane >= off) v += t;
+  }
+  return v;
 }
 
 // One round of a block-wide exclusive scan (one value per thread), added to
@@ -316,12 +244,7 @@ __device__ __forceinline__ uint32_t wave_offsets(uint32_t *whist, int nb, int hw
 __device__ __forceinline__ uint32_t block_scan_round(uint32_t v, uint32_t (*wtot)[SORT_WAVES], int rd,
                                                      uint32_t &carry) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t incl = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t t = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += t;
-  }
+  const uint32_t incl = wave_incl_scan(v);
   if (lane == 63) wtot[rd & 1][wave] = incl;
   __syncthreads();
   uint32_t run = carry + incl - v, all = 0;
@@ -335,75 +258,71 @@ __device__ __forceinline__ uint32_t block_scan_round(uint32_t v, uint32_t (*wtot
   return run;
 }
 
-// Partition of each chunk by digit.  perm (optional): perm[i] = output
-// position of input record i.  Per sub-chunk of SORT_THREADS * PL record
-// slots (each wave owns 64 * PL consecutive ones): ranks (rank_records; the
-// slots past the chunk's end take the digit nb, one past the last), then one
-// thread per digit turns the per-wave counts into offsets and a block scan
-// gives the digit's start in a digit-sorted staging copy and dbase = (global
-// output offset - staging start) mod 2^32, records go to the staging copy,
-// and the staging copy's records (every slot before digit nb's start) are
-// written out as contiguous runs (record p goes to dbase[its digit] + p)
-// while the next sub-chunk's records load.  With DB the per-wave counts are
-// double-buffered: this sub-chunk's buffer is cleared during the write-out
-// and the next sub-chunk ranks into the other one, so no barrier separates
-// them.  hw count rows (a divisor of the wave count) serve the waves, wave w
-// on row w % hw.  A digit's staging start, global base, dbase and second
-// dbase sit together in one 16-byte LDS word (dinfo).
-//   MODE 0: the chunk's output offsets per digit are offsets[tb + dg * ts].
-//   MODE 1 (paged pass 1): workgroup g appends each digit's records to
-//     blocks of PG_BLOCK slots that it takes in order from its own range
-//     [g Q, g Q + Q) of the pool: the digit's current block until it is
-//     full, then new ones (a run then has two parts, the second from
-//     staging position dinfo[dg].y on, at dbase dinfo[dg].w).  Each block's
-//     digit and number among the digit's blocks go to pg.hdr, its fill to
-//     pg.fill, the number of blocks taken to pg.used[g].  No histogram pass
-//     and no global atomics.
-//   MODE 2 (paged pass 2): the chunk covers list slots of its segment's
-//     blocks (pg.blist); slot v is record (block of blist[v / PG_BLOCK], v %
-//     PG_BLOCK) when below that block's fill, and is skipped otherwise.
-//     perm is indexed by pool slot.
-template <int NM, int PL, bool DB, int MODE>
-__global__ void __launch_bounds__(SORT_THREADS, 4) k_downsweep(Src<NM> src, float *__restrict__ dst, ChunkMap cm,
-                                                               KeyGeom kg, DigitSel ds, int nb, int hw,
+// Partition of each piece by digit.  PERM: perm[i] = output
+// position of input record i (IN_LIST: of pool slot i).
+// Per sub-chunk of SORT_THREADS * PL record slots (each wave owns 64 * PL
+// consecutive ones): ranks (rank_records; the slots without a record take
+// the digit nb, one past the last), then one thread per digit turns the
+// per-wave counts into offsets and a block scan gives the digit's start in a
+// digit-sorted staging copy, records go to the staging copy, and the staging
+// copy's records (every slot before digit nb's start) are written out as
+// contiguous runs while the next sub-chunk's records load.  With DB the
+// per-wave counts are double-buffered: this sub-chunk's buffer is cleared
+// during the write-out and the next sub-chunk ranks into the other one, so
+// no barrier separates them.  hw count rows (a divisor of the wave count)
+// serve the waves, wave w on row w % hw.
+//   PAGED: each digit's records are appended to its current block of 2^lg
+//     slots until that is full, then to new blocks of the piece's own range of
+//     the pool: staging position p of digit dg goes to dinfo[dg].z + p below
+//     dinfo[dg].y, else to dinfo[dg].w + p (dinfo[dg].x is the digit's staging
+//     start).  At a piece's end its blocks and records of each digit are added
+//     to the bucket's totals with one atomic, whose old value numbers the
+//     piece's blocks among the bucket's.
+//   else: record p goes to dinfo[its digit].z + p, from the chunk's scanned
+//     offsets[dg * gridDim.x + g].
+// blist (IN_LIST): block and fill of each list entry (pg_entry).
+template <int NM, int PL, bool DB, int IN, bool PAGED, bool PERM>
+__global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__restrict__ pos,
+                                                               const float *__restrict__ masses,
+                                                               const uint32_t *__restrict__ blist,
+                                                               const uint32_t *__restrict__ start,
+                                                               const uint32_t *__restrict__ first_seg,
+                                                               float *__restrict__ dst, InMap im, KeyGeom kg,
+                                                               DigitSel ds, int nb, int hw,
                                                                const uint32_t *__restrict__ offsets,
                                                                uint32_t *__restrict__ perm,
-                                                               uint8_t *__restrict__ dig2, DigitSel ds2,
-                                                               uint32_t *__restrict__ mrange, PgArgs pg) {
+                                                               uint32_t *__restrict__ mrange_w, PgOut pg) {
   constexpr int RW = Src<NM>::RW;
+  const Src<NM> src{pos, masses, IN == IN_RAW};
   constexpr int SUBN = SORT_THREADS * PL;
   constexpr int NBUF = DB ? 2 : 1;
-  constexpr uint32_t NONE = 0xffffffffu;
-  static_assert(MODE != 2 || PL * 64 <= (int)PG_BLOCK, "a wave's records of a sub-chunk lie in one block");
   static_assert(SUBN <= 8192, "ranks take 13 bits (rank_records)");
   extern __shared__ uint4 sm4[];
   const int nbt = nb + 1;                                    // digits and the empty slots' digit nb
-  uint4 *dinfo = sm4;                                        // [nbt] staging start, gbase, dbase, dbase2
+  uint4 *dinfo = sm4;                                        // [nbt]
   uint32_t *whist_all = reinterpret_cast<uint32_t *>(dinfo + nbt);  // [NBUF][hw][nbt]
-  uint32_t *cur_blk = whist_all + NBUF * hw * nbt;           // MODE 1 [nb]: the digit's current block
-  uint32_t *cur_fill = cur_blk + (MODE == 1 ? nb : 0);       // MODE 1 [nb]: its fill (PG_BLOCK: none open)
-  uint32_t *dblocks = cur_fill + (MODE == 1 ? nb : 0);       // MODE 1 [nb]: blocks the digit took
-  uint16_t *sdig = reinterpret_cast<uint16_t *>(dblocks + (MODE == 1 ? nb : 0));  // [SUBN]
+  uint32_t *dcnt = whist_all + NBUF * hw * nbt;              // PAGED [nb]: records of the digit so far
+  uint32_t *dblk = dcnt + (PAGED ? nb : 0);                  // PAGED [nb]: the digit's last block
+  uint16_t *sdig = reinterpret_cast<uint16_t *>(dblk + (PAGED ? nb : 0));  // [SUBN]
   float *stage = reinterpret_cast<float *>(sdig + SUBN);      // [SUBN][RW]
   __shared__ uint32_t wtot[2][SORT_WAVES];
   __shared__ uint32_t smr[2];  // masses: largest, smallest nonzero |mass| bits of this chunk
 
-  int64_t cb, ce, tb, ts;
-  if (!cm.range(blockIdx.x, cb, ce, tb, ts)) return;
+  // this workgroup's slots, and the piece [., pe) of them in bucket seg
+  const int sh = IN == IN_LIST ? im.lg : 0;
+  const int64_t cb = blockIdx.x * im.chunk;
+  const int64_t ce = min(IN == IN_RAW ? im.n : (int64_t)start[im.nseg] << sh, cb + im.chunk);
+  if (cb >= ce) return;
+  uint32_t seg = IN == IN_RAW ? 0u : first_seg[blockIdx.x];
+  int64_t pe = IN == IN_RAW ? ce : min(ce, (int64_t)start[seg + 1] << sh);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // with dig2 (digits of at most 8 bits), sdig holds the digit and the ds2
-  // digit (paged pass 1 always writes dig2, paged pass 2 never)
-  const bool two = MODE == 1 ? true : MODE == 2 ? false : dig2 != nullptr;
-  if (MODE != 1)
-    for (int i = threadIdx.x; i < nb; i += SORT_THREADS) dinfo[i].y = offsets[tb + (int64_t)i * ts];
-  if (MODE == 1)
-    for (int i = threadIdx.x; i < nb; i += SORT_THREADS) {
-      cur_blk[i] = NONE;
-      cur_fill[i] = PG_BLOCK;
-      dblocks[i] = 0;
-    }
-  const uint32_t blk0 = MODE == 1 ? (uint32_t)(blockIdx.x * pg.Q) : 0u;  // this workgroup's block range
-  uint32_t taken = 0;                                                    // MODE 1: blocks taken so far
+  const uint32_t pb = 1u << pg.lg;
+  uint32_t blk0 = PAGED ? (uint32_t)(cb >> pg.lg) + (blockIdx.x + seg) * (uint32_t)(nb + 1) : 0u;  // the piece's blocks
+  uint32_t taken = 0;                                                                      // blocks taken so far
+  for (int i = threadIdx.x; i < nb; i += SORT_THREADS) {
+    if constexpr (PAGED) dcnt[i] = 0;
+    else dinfo[i].y = offsets[(int64_t)i * gridDim.x + blockIdx.x];
+  }
   for (int i = threadIdx.x; i < NBUF * hw * nbt; i += SORT_THREADS) whist_all[i] = 0;
   const int row = (wave % hw) * nbt;
   if (threadIdx.x == 0) {
@@ -413,102 +332,105 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_downsweep(Src<NM> src, floa
   uint32_t mx = 0u, mn = 0xffffffffu;
 
   float rec[PL][RW] = {};
-  uint32_t nv = 0;  // this lane's slots of the sub-chunk that hold records (a prefix: it < nv)
+  uint32_t vm = 0;  // bit it: this lane's slot `it` of the sub-chunk holds a record
   const int wbase = wave * (PL * 64) + lane;
-  // MODE 2: a wave's 64 * PL consecutive list slots (PL * 64 <= PG_BLOCK,
-  // sub-chunks start at multiples of PG_BLOCK) lie in one block: its pool
-  // offset and fill are looked up once per wave and sub-chunk
-  uint32_t wblk = 0, wfill = 0;
-  // records of the sub-chunk at s0 (MODE 2: through the block list)
-  auto load_sub = [&](int64_t s0) {
-    const int64_t i0 = s0 + wbase;
-    int64_t lim = ce - i0;  // slot i0 + 64 it holds a record iff 64 it < lim
-    if constexpr (MODE == 2) {
-      // the wave's first slot as a uniform value: the entry is a scalar load
+  // IN_LIST: blocks hold at least 64 slots and sub-chunks start at multiples
+  // of 64, so 64 consecutive slots lie in one block: the block is looked up
+  // once per wave and `it`, with scalar loads
+  uint32_t wslot[IN == IN_LIST ? PL : 1];  // pool slot of the wave's first slot `it`
+  // records of the sub-chunk at s0 of a piece that ends at `end`
+  auto load_sub = [&](int64_t s0, int64_t end) {
+    if constexpr (IN == IN_LIST) {
       const int64_t w0 = s0 + __builtin_amdgcn_readfirstlane(wave) * (PL * 64);
-      wfill = 0;
-      if (w0 < ce) {
-        const uint32_t ent = pg.blist[w0 >> PG_LOG];
-        wblk = pg_blk(ent);
-        wfill = pg_fill(ent);
-      }
-      lim = min(lim, (int64_t)wfill - (int64_t)((uint32_t)i0 & (PG_BLOCK - 1)));
-    }
-    nv = lim <= 0 ? 0u : (uint32_t)min((int64_t)PL, (lim + 63) >> 6);
+      const uint32_t ibm = (1u << im.lg) - 1;
+      uint32_t ent[PL];
 #pragma unroll
-    for (int it = 0; it < PL; it++) {
-      const int64_t i = i0 + it * 64;
-      if ((uint32_t)it < nv) {
-        if constexpr (MODE == 2) src.load(wblk * PG_BLOCK + ((uint32_t)i & (PG_BLOCK - 1)), rec[it]);
-        else src.load(i, rec[it]);
+      for (int it = 0; it < PL; it++) ent[it] = w0 + it * 64 < end ? blist[(w0 + it * 64) >> im.lg] : 0u;
+      vm = 0;
+#pragma unroll
+      for (int it = 0; it < PL; it++) {
+        const uint32_t in = (uint32_t)(w0 + it * 64) & ibm;  // slot within the block
+        const uint32_t fill = w0 + it * 64 < end ? (ent[it] >> (32 - im.lg)) + 1 : 0u;
+        wslot[it] = (ent[it] << im.lg) + in;
+        if (in + lane < fill) {
+          vm |= 1u << it;
+          src.load((int64_t)(wslot[it] + lane), rec[it]);
+        }
       }
+    } else {
+      const int64_t i0 = s0 + wbase;
+      const int64_t lim = end - i0;  // slot i0 + 64 it holds a record iff 64 it < lim
+      const uint32_t nv = lim <= 0 ? 0u : (uint32_t)min((int64_t)PL, (lim + 63) >> 6);
+      vm = (1u << nv) - 1;
+#pragma unroll
+      for (int it = 0; it < PL; it++)
+        if ((uint32_t)it < nv) src.load(i0 + it * 64, rec[it]);
     }
   };
-  load_sub(cb);
+  load_sub(cb, pe);
   // nothing in flight on entry to the loop, so that the wait for a
   // sub-chunk's records there is not a wait for the write-out's stores
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
 
   int sub = 0;
-  for (int64_t s0 = cb; s0 < ce; s0 += SUBN, sub++) {
+  for (int64_t s0 = cb; s0 < ce; sub++) {
+    // the next sub-chunk: of this piece, or the next piece's first
+    const bool last = s0 + SUBN >= pe;  // of the piece
+    const int64_t s1 = last ? pe : s0 + SUBN;
+    uint32_t nseg = seg;
+    int64_t npe = pe;
+    if (IN != IN_RAW && last && s1 < ce) {
+      do npe = (int64_t)start[++nseg + 1] << sh;
+      while (npe == s1);  // empty buckets
+      npe = min(npe, ce);
+    }
     uint32_t *whist = whist_all + (DB ? (sub & 1) * hw * nbt : 0);
     uint32_t pk[PL];
-    rank_records<NM, PL>(rec, nv, kg, ds, ds2, two, (uint32_t)nb, whist + row, pk);
+    rank_records<NM, PL>(rec, vm, kg, ds, (uint32_t)nb, whist + row, pk);
     __syncthreads();
-    {
-      uint32_t total = 0;  // slots of this sub-chunk (MODE 1: and blocks taken << 16)
-      for (int r0 = 0, rd = 0; r0 < nbt; r0 += SORT_THREADS, rd++) {
-        const int dg = r0 + threadIdx.x;
-        const uint32_t tot = dg < nbt ? wave_offsets(whist, nbt, hw, dg) : 0u;
-        if constexpr (MODE == 1) {
-          // the run fills the current block (a records), then `need` new
-          // blocks; counts and block numbers scan together (nb <= 256, one
-          // round: at most SUBN slots and SUBN / PG_BLOCK + nb blocks)
-          const bool real = dg < nb;
-          const uint32_t cf = real ? cur_fill[dg] : PG_BLOCK;
-          const uint32_t a = min(tot, PG_BLOCK - cf);
-          const uint32_t need = real ? (tot - a + PG_BLOCK - 1) >> PG_LOG : 0u;
-          const uint32_t run = block_scan_round(tot | need << 16, wtot, rd, total);
-          if (real) {
-            const uint32_t lr = run & 0xffffu, first = blk0 + taken + (run >> 16);
-            const uint32_t cbk = cur_blk[dg];
-            // dbase used only when a > 0, i.e. cbk is open
-            dinfo[dg] = make_uint4(lr, lr + a, cbk * PG_BLOCK + cf - lr, first * PG_BLOCK - (lr + a));
-            if (need) {
-              if (cbk != NONE) pg.fill[cbk] = PG_BLOCK;  // filled by this run
-              const uint32_t nd = dblocks[dg];
-              for (uint32_t k = 0; k < need; k++) {
-                pg.hdr[first + k] = (uint32_t)dg | (nd + k) << 8;
-                if (k + 1 < need) pg.fill[first + k] = PG_BLOCK;
-              }
-              dblocks[dg] = nd + need;
-              cur_blk[dg] = first + need - 1;
-              cur_fill[dg] = tot - a - (need - 1) * PG_BLOCK;
-            } else {
-              cur_fill[dg] = cf + tot;
-            }
-          } else if (dg == nb) {
-            dinfo[nb].x = run & 0xffffu;
+    uint32_t total = 0;  // records of this sub-chunk (PAGED: and blocks taken << 16)
+    if (threadIdx.x == SORT_THREADS - 1) wave_offsets(whist, nbt, hw, nb);
+    for (int r0 = 0, rd = 0; r0 < nb; r0 += SORT_THREADS, rd++) {
+      const int dg = r0 + threadIdx.x;
+      const uint32_t tot = dg < nb ? wave_offsets(whist, nbt, hw, dg) : 0u;
+      if constexpr (PAGED) {
+        // the run fills the open block (a records), then `need` new blocks;
+        // counts and block numbers scan together (at most SUBN slots and
+        // SUBN / 8 + nb blocks)
+        const uint32_t c0 = dg < nb ? dcnt[dg] : 0u;
+        const uint32_t f = c0 & (pb - 1);
+        const uint32_t a = f ? min(tot, pb - f) : 0u;
+        const uint32_t need = (tot - a + pb - 1) >> pg.lg;
+        const uint32_t run = block_scan_round(tot | need << 16, wtot, rd, total);
+        if (dg < nb) {
+          const uint32_t lr = run & 0xffffu, first = blk0 + taken + (run >> 16);
+          // the first part is used only when a > 0, i.e. the block is open
+          dinfo[dg] = make_uint4(lr, lr + a, ((f ? dblk[dg] : 0u) << pg.lg) + f - lr, (first << pg.lg) - (lr + a));
+          if (need) {
+            const uint32_t nd = (c0 + pb - 1) >> pg.lg;
+            for (uint32_t k = 0; k < need; k++) pg.hdr[first + k] = (uint32_t)dg | (nd + k) << 11;
+            dblk[dg] = first + need - 1;
           }
-        } else {
-          const uint32_t run = block_scan_round(tot, wtot, rd, total);
-          if (dg < nb) {
-            const uint32_t g = dinfo[dg].y;
-            dinfo[dg].x = run;
-            dinfo[dg].y = g + tot;
-            dinfo[dg].z = g - run;
-          } else if (dg == nb) {
-            dinfo[nb].x = run;
-          }
+          dcnt[dg] = c0 + tot;
+        }
+      } else {
+        const uint32_t run = block_scan_round(tot, wtot, rd, total);
+        if (dg < nb) {
+          const uint32_t g = dinfo[dg].y;
+          dinfo[dg].x = run;
+          dinfo[dg].y = g + tot;
+          dinfo[dg].z = g - run;
         }
       }
-      if constexpr (MODE == 1) taken += total >> 16;
     }
+    const uint32_t nrec = PAGED ? total & 0xffffu : total;  // staging positions [0, nrec) hold records
+    if constexpr (PAGED) taken += total >> 16;
+    if (threadIdx.x == SORT_THREADS - 1) dinfo[nb].x = nrec;
     __syncthreads();
     // output position of the record at staging position p of digit d
     auto dest_of = [&](uint32_t p, uint32_t d) -> uint32_t {
-      if constexpr (MODE == 1) {
+      if constexpr (PAGED) {
         const uint4 di = dinfo[d];
         return p < di.y ? di.z + p : di.w + p;
       } else {
@@ -518,12 +440,12 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_downsweep(Src<NM> src, floa
 #pragma unroll
     for (int it = 0; it < PL; it++) {
       const int loc = wbase + it * 64;
-      const uint32_t dg = two ? (pk[it] >> 13) & 0x1ffu : pk[it] >> 13;
+      const uint32_t dg = pk[it] >> 13;
       const uint32_t p = dinfo[dg].x + whist[row + dg] + (pk[it] & 0x1fffu);
 #pragma unroll
       for (int k = 0; k < RW; k++) stage[p * RW + k] = rec[it][k];
-      sdig[p] = (uint16_t)(two ? dg | (pk[it] >> 22) << 8 : dg);
-      if (dg < (uint32_t)nb) {
+      sdig[p] = (uint16_t)dg;
+      if ((vm >> it) & 1u) {
         if constexpr (NM == 1) {
           // |mass| as bits orders like the value (a NaN above every finite one)
           const uint32_t mb = __float_as_uint(rec[it][3]) & 0x7fffffffu;
@@ -531,579 +453,549 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_downsweep(Src<NM> src, floa
           if (mb) mn = min(mn, mb);
         }
         // where this record goes (coalesced writes, by input position or pool slot)
-        if (perm) perm[MODE == 2 ? (int64_t)(wblk * PG_BLOCK + ((uint32_t)(s0 + loc) & (PG_BLOCK - 1))) : s0 + loc] = dest_of(p, dg);
+        if constexpr (PERM) perm[IN == IN_LIST ? (int64_t)(wslot[IN == IN_LIST ? it : 0] + lane) : s0 + loc] = dest_of(p, dg);
       }
     }
     // the next sub-chunk loads during the barrier and the write-out
-    load_sub(s0 + SUBN);
+    load_sub(s1, npe);
     __syncthreads();
-    const uint32_t nrec = dinfo[nb].x;  // records of this sub-chunk: staging positions [0, nrec)
-    // record_p: staging position p holds a record (p < nrec); the others
-    // are written to the sink
-    auto put = [&](int p, bool record_p) {
-      const uint32_t sd = sdig[p];
-      const uint32_t dest = dest_of((uint32_t)p, record_p ? (two ? sd & 0xffu : sd) : 0u);
+    auto put = [&](int p) {
+      const uint32_t dest = dest_of((uint32_t)p, sdig[p]);
       float v[RW];
 #pragma unroll
       for (int k = 0; k < RW; k++) v[k] = stage[p * RW + k];
-      // the sink position from p computed in the loop (not hoisted out of it)
-      int ps = p;
-      asm volatile("" : "+v"(ps));
-      float *to = record_p ? dst + (int64_t)dest * RW : sort_sink + ps * RW;
 #pragma unroll
-      for (int k = 0; k < RW; k++) to[k] = v[k];
-      if (two) *(record_p ? dig2 + dest : sort_sink_digits + ps) = (uint8_t)(sd >> 8);
+      for (int k = 0; k < RW; k++) dst[(int64_t)dest * RW + k] = v[k];
     };
-    // With the sink (paged passes; pass 1 only with masses, where it measured
-    // faster), every lane stores for each of its staging positions, so that
-    // every path issues the same stores and the next sub-chunk's loads
-    // (issued before them) are waited for without waiting for these writes;
-    // elsewhere the extra registers cost more than that wait.  Pass 1's
-    // two-part runs write two positions at a time to keep the registers in
-    // bounds.
-    constexpr bool SINK = MODE == 2 || (MODE == 1 && NM == 1);
-    if constexpr (SINK && MODE == 1) {
-#pragma unroll 2
-      for (int it = 0; it < PL; it++) {
-        const int p = threadIdx.x + it * SORT_THREADS;
-        put(p, p < (int)nrec);
-      }
-    } else if constexpr (SINK) {
-#pragma unroll
-      for (int it = 0; it < PL; it++) {
-        const int p = threadIdx.x + it * SORT_THREADS;
-        put(p, p < (int)nrec);
-      }
-    } else if (nrec == SUBN) {
-      if constexpr (MODE == 1) {
-#pragma unroll 2
-        for (int it = 0; it < PL; it++) put(threadIdx.x + it * SORT_THREADS, true);
-      } else {
-#pragma unroll
-        for (int it = 0; it < PL; it++) put(threadIdx.x + it * SORT_THREADS, true);
-      }
+    // four stores in flight per lane (all eight cost pass 2 6.5 -> 7.0 ms at
+    // 2^30 records: registers); the last sub-chunk may be partial
+    if (nrec == SUBN) {
+#pragma unroll PAGED ? 4 : PL
+      for (int it = 0; it < PL; it++) put(threadIdx.x + it * SORT_THREADS);
     } else {
-      for (int p = threadIdx.x; p < (int)nrec; p += SORT_THREADS) put(p, true);
+      for (int p = threadIdx.x; p < (int)nrec; p += SORT_THREADS) put(p);
     }
     for (int i = threadIdx.x; i < hw * nbt; i += SORT_THREADS) whist[i] = 0;
+    if (PAGED && last) {
+      // the piece's totals (each digit's state is its own thread's)
+      const uint32_t p = blockIdx.x + seg;
+      for (int dg = threadIdx.x; dg < nb; dg += SORT_THREADS) {
+        const uint32_t c = dcnt[dg];
+        if (c == 0) continue;
+        dcnt[dg] = 0;
+        const unsigned long long add = (unsigned long long)((c + pb - 1) >> pg.lg) << 32 | c;
+        const int64_t at = (int64_t)p * nb + dg;
+        pg.cnt[at] = c;
+        pg.base[at] = (uint32_t)(atomicAdd(&pg.tot[(int64_t)seg * nb + dg], add) >> 32);
+      }
+      if (threadIdx.x == 0) pg.piece[p] = make_uint4(blk0, taken, seg, 0u);
+      blk0 = (uint32_t)(s1 >> pg.lg) + (blockIdx.x + nseg) * (uint32_t)(nb + 1);
+      taken = 0;
+    }
+    s0 = s1;
+    seg = nseg;
+    pe = npe;
     if (!DB) __syncthreads();
   }
-  if constexpr (MODE == 1) {
-    // the open blocks' fills (each digit's state is its own thread's)
-    for (int dg = threadIdx.x; dg < nb; dg += SORT_THREADS)
-      if (cur_blk[dg] != NONE) pg.fill[cur_blk[dg]] = cur_fill[dg];
-    if (threadIdx.x == 0) pg.used[blockIdx.x] = taken;
-  }
   if constexpr (NM == 1) {
-    if (mrange) {
+    if (mrange_w) {
       atomicMax(&smr[0], mx);
       atomicMin(&smr[1], mn);
       __syncthreads();
-      if (threadIdx.x == 0) {
-        atomicMax(&mrange[0], smr[0]);
-        atomicMin(&mrange[1], smr[1]);
-      }
+      if (threadIdx.x < 2) mrange_w[2 * (int64_t)blockIdx.x + threadIdx.x] = smr[threadIdx.x];
     }
   }
 }
 
-__global__ void k_mrange_init(uint32_t *mrange) {
-  mrange[0] = 0u;
-  mrange[1] = 0xffffffffu;
-}
-
-// Pass-2 segment bookkeeping from the scanned pass-1 table.
-__global__ void k_seginfo(const uint32_t *__restrict__ t1scan, int64_t g1, int nseg, int64_t n, int64_t chunk,
-                          uint32_t *__restrict__ seg_start, uint32_t *__restrict__ nchunks) {
+// Bucket totals of a counted first pass, from its scanned table: records in
+// both halves (one record per list entry).
+__global__ void k_seg_tot(const uint32_t *__restrict__ t1scan, int64_t g1, int nseg, int64_t n,
+                          unsigned long long *__restrict__ tot) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s > nseg) return;
-  if (s == nseg) {
-    seg_start[s] = (uint32_t)n;
-    nchunks[s] = 0;
-    return;
-  }
+  if (s >= nseg) return;
   const uint32_t st = t1scan[(int64_t)s * g1];
   const uint32_t en = (s + 1 < nseg) ? t1scan[(int64_t)(s + 1) * g1] : (uint32_t)n;
-  seg_start[s] = st;
-  nchunks[s] = (uint32_t)(((int64_t)en - st + chunk - 1) / chunk);
+  tot[s] = (unsigned long long)(en - st) << 32 | (en - st);
 }
 
-// Two-pass tile starts from the scanned pass-2 table: the offset of a tile's
-// first chunk, or the segment's first record (rec_start) when the segment is
-// empty; tile_start[ks] = n.
-__global__ void k_tile_start_2pass(const uint32_t *__restrict__ t2scan, const uint32_t *__restrict__ chunk_start,
-                                   const uint32_t *__restrict__ rec_start, int nhi, int nlo, int64_t n,
-                                   uint32_t *__restrict__ tile_start) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t ks = (int64_t)nhi * nlo;
-  if (t > ks) return;
-  if (t == ks) {
-    tile_start[t] = (uint32_t)n;
-    return;
+// Directory of the buckets of a pass, from their totals (list entries << 32
+// | records): every bucket's first list entry; of the segments of a second
+// pass, the bucket of each workgroup's first slot; of tiles, the work items
+// and the item -> tile table.  One workgroup: a bucket count of 65 536 is 16 rounds, and the
+// scans, tables and flags that it replaces were a dozen launches of 2 to 5
+// us each.  The totals are cleared for the next sort.
+struct DirArgs {
+  unsigned long long *tot;
+  int64_t nb, kreal;      // buckets; those below kreal are real tiles
+  uint32_t *start, *ustart, *utile;  // [nb + 1]; tiles: first item [nb + 1]; tile of each item or first_seg
+  uint32_t unit;          // segments: list entries per workgroup (0: tiles)
+  FastDiv funit;
+  uint4 *piece;           // segments: the second pass's pieces, cleared
+  int64_t npiece;
+  // tiles: items of at most 2^limax records and 2^17 record slots; store: every
+  // real tile gets at least one item (so untouched tiles are written as zeros)
+  int store, lg, limax;
+  uint32_t *pstart, *nheavy, *heavy;  // first partial tile of split tiles, and their list
+  uint32_t *nonfinite;
+  uint32_t *mrange;       // with masses: reduced from mrange_w[2 * nw]
+  const uint32_t *mrange_w;
+  int64_t nw;
+};
+constexpr int DIR_PER = 4;  // buckets per thread and round
+
+__global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
+  __shared__ uint32_t wt[2][3][SORT_WAVES];
+  __shared__ uint32_t hcount, smr[2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) {
+    hcount = 0;
+    smr[0] = 0u;
+    smr[1] = 0xffffffffu;
+    if (D.nonfinite) *D.nonfinite = 0u;
   }
-  const int hi = (int)(t / nlo), lo = (int)(t % nlo);
-  const int64_t c0 = chunk_start[hi], nc = (int64_t)chunk_start[hi + 1] - c0;
-  tile_start[t] = nc ? t2scan[c0 * nlo + lo * nc] : rec_start[hi];
-}
-
-// Paged pass 1's block directory.  Per pass-1 workgroup w (one workgroup
-// each): the blocks and records of each digit among the blocks it took, at
-// bcnt / rcnt[d * G + w]; entry nhi * G is zero, so that exclusive scans of
-// the nhi * G + 1 entries end in the totals.
-__global__ void __launch_bounds__(256) k_pg_count(PgArgs pg, int nhi, int64_t G, uint32_t *__restrict__ bcnt,
-                                                  uint32_t *__restrict__ rcnt) {
-  __shared__ uint32_t cb[256], cr[256];
-  const int64_t w = blockIdx.x;
-  for (int i = threadIdx.x; i < nhi; i += 256) cb[i] = cr[i] = 0;
-  __syncthreads();
-  const uint32_t used = (uint32_t)min((int64_t)pg.used[w], pg.Q);
-  const int64_t b0 = w * pg.Q;
-  for (uint32_t k = threadIdx.x; k < used; k += 256) {
-    const uint32_t d = pg.hdr[b0 + k] & 0xffu;
-    if (d < (uint32_t)nhi) {
-      atomicAdd(&cb[d], 1u);
-      atomicAdd(&cr[d], pg.fill[b0 + k]);
+  const uint32_t eslots = 1u << (LG_ITEM_MAX - D.lg);  // list entries of 2^17 record slots
+  uint32_t carry[3] = {0, 0, 0};
+  unsigned long long t[DIR_PER];
+  auto div_up = [&](uint32_t x) { return x == 0 ? 0u : D.funit.div(x - 1) + 1; };  // entries < 2^31
+  auto load = [&](int64_t r0) {
+#pragma unroll
+    for (int i = 0; i < DIR_PER; i++) {
+      const int64_t k = r0 + threadIdx.x * DIR_PER + i;
+      t[i] = k < D.nb ? D.tot[k] : 0ull;
     }
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < nhi; i += 256) {
-    bcnt[(int64_t)i * G + w] = cb[i];
-    rcnt[(int64_t)i * G + w] = cr[i];
-  }
-  if (w == 0 && threadIdx.x == 0) {
-    bcnt[(int64_t)nhi * G] = 0;
-    rcnt[(int64_t)nhi * G] = 0;
-  }
-}
-
-// The block list: digit d's blocks from pass-1 workgroup w at boff[d * G +
-// w] onwards, in the order the workgroup took them (each block's number
-// among its digit's blocks is in its header), so a segment lists its records
-// in input order, as the plain pass 1 writes them.
-__global__ void __launch_bounds__(256) k_pg_list(PgArgs pg, int nhi, int64_t G, const uint32_t *__restrict__ boff,
-                                                 uint32_t *__restrict__ blist) {
-  __shared__ uint32_t at[256], cnt[256];
-  const int64_t w = blockIdx.x;
-  for (int i = threadIdx.x; i < nhi; i += 256) {
-    at[i] = boff[(int64_t)i * G + w];
-    cnt[i] = boff[(int64_t)i * G + w + 1] - at[i];
-  }
-  __syncthreads();
-  const uint32_t used = (uint32_t)min((int64_t)pg.used[w], pg.Q);
-  const int64_t b0 = w * pg.Q;
-  for (uint32_t k = threadIdx.x; k < used; k += 256) {
-    const uint32_t h = pg.hdr[b0 + k], d = h & 0xffu;
-    if (d < (uint32_t)nhi && (h >> 8) < cnt[d]) blist[at[d] + (h >> 8)] = pg_entry((uint32_t)(b0 + k), pg.fill[b0 + k]);
-  }
-}
-
-// Pass-2 segments over the block list: segment s (pass-1 digit s) covers
-// list slots [seg_start[s], seg_start[s+1]) (PG_BLOCK per listed block), its
-// records start at rec_start[s] of the output, and it has nchunks[s] chunks
-// of `chunk` list slots.
-__global__ void k_pg_seginfo(const uint32_t *__restrict__ boff, const uint32_t *__restrict__ roff, int nhi,
-                             int64_t G, int64_t chunk, uint32_t *__restrict__ seg_start,
-                             uint32_t *__restrict__ rec_start, uint32_t *__restrict__ nchunks) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s > nhi) return;
-  const uint32_t b0 = boff[(int64_t)s * G];
-  seg_start[s] = b0 * PG_BLOCK;
-  rec_start[s] = roff[(int64_t)s * G];
-  nchunks[s] = s < nhi ? (uint32_t)(((int64_t)(boff[(int64_t)(s + 1) * G] - b0) * PG_BLOCK + chunk - 1) / chunk) : 0u;
-}
-
-// k_upsweep_bytes over the list slots of a paged pass 2: the digit bytes of
-// the listed blocks' filled slots.  Chunks start at multiples of PG_BLOCK
-// list slots; each wave takes whole blocks (one lookup of the block and its
-// fill), each lane 16 consecutive slots of it.
-__global__ void __launch_bounds__(UP_THREADS) k_upsweep_pages(const uint8_t *__restrict__ digs, ChunkMap cm,
-                                                                PgArgs pg, int nb, uint32_t *__restrict__ counts) {
-  static_assert(PG_BLOCK == 64 * 16, "one block per wave, 16 slots per lane");
-  extern __shared__ uint32_t hist[];
-  int64_t b, e, tb, ts;
-  if (!cm.range(blockIdx.x, b, e, tb, ts)) return;
-  for (int i = threadIdx.x; i < nb; i += UP_THREADS) hist[i] = 0;
-  __syncthreads();
-  // the wave as a uniform value: the block-list entries are scalar loads
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t k0 = b >> PG_LOG, k1 = (e + PG_BLOCK - 1) >> PG_LOG;  // list entries of the chunk
-  constexpr int UNR = 4;  // blocks per wave in flight
-  for (int64_t kb = k0 + wave; kb < k1; kb += UNR * UP_WAVES) {
-    uint32_t blk[UNR];
-    int nv[UNR];
-    uint4 v[UNR];
+  };
+  load(0);
+  int rd = 0;
+  for (int64_t r0 = 0; r0 < D.nb; r0 += SORT_THREADS * DIR_PER, rd ^= 1) {
+    const int64_t k0 = r0 + threadIdx.x * DIR_PER;
+    uint32_t v[3][DIR_PER], sum[3] = {0, 0, 0};
 #pragma unroll
-    for (int u = 0; u < UNR; u++) {
-      const int64_t k = kb + u * UP_WAVES;
-      const uint32_t ent = k < k1 ? pg.blist[k] : 0u;
-      blk[u] = pg_blk(ent);
-      // filled slots of this block inside the chunk, from this lane's 16
-      const int64_t lim = k < k1 ? min((int64_t)pg_fill(ent), e - (k << PG_LOG)) : 0;
-      nv[u] = (int)max((int64_t)0, min((int64_t)16, lim - 16 * lane));
+    for (int i = 0; i < DIR_PER; i++) {
+      const int64_t k = k0 + i;
+      const uint32_t ents = (uint32_t)(t[i] >> 32), recs = (uint32_t)t[i];
+      uint32_t m = 0;
+      if (D.unit == 0 && k < D.kreal) {
+        if (recs == 0) m = D.store ? 1u : 0u;
+        else m = max((recs + (1u << D.limax) - 1) >> D.limax, (ents + (eslots - 1)) >> (LG_ITEM_MAX - D.lg));
+      }
+      v[0][i] = ents;
+      v[1][i] = m;
+      v[2][i] = m > 1 ? m : 0u;
+      if (k < D.nb) D.tot[k] = 0ull;
+#pragma unroll
+      for (int j = 0; j < 3; j++) sum[j] += v[j][i];
     }
+    load(r0 + SORT_THREADS * DIR_PER);
+    uint32_t run[3];
 #pragma unroll
-    for (int u = 0; u < UNR; u++) {
-      v[u] = make_uint4(0u, 0u, 0u, 0u);
-      if (nv[u] > 0) v[u] = *reinterpret_cast<const uint4 *>(digs + (int64_t)blk[u] * PG_BLOCK + 16 * lane);
+    for (int j = 0; j < 3; j++) {
+      const uint32_t incl = wave_incl_scan(sum[j]);
+      run[j] = carry[j] + incl - sum[j];
+      if (lane == 63) wt[rd][j][wave] = incl;
     }
+    __syncthreads();
 #pragma unroll
-    for (int u = 0; u < UNR; u++) {
-      // 16 equal digits add with one atomic, and a wavefront of such lanes
-      // of one digit with one atomic for all
-      const uint32_t d0 = v[u].x & 0xffu;
-      const uint32_t rep = d0 * 0x01010101u;
-      const bool same16 = nv[u] == 16 && v[u].x == rep && v[u].y == rep && v[u].z == rep && v[u].w == rep;
-      const uint32_t dw = __builtin_amdgcn_readfirstlane(d0);
-      if (__ballot(same16 && d0 == dw) == ~0ull) {
-        if (lane == 0) atomicAdd(&hist[dw], 1024u);
-      } else if (same16) {
-        atomicAdd(&hist[d0], 16u);
-      } else {
+    for (int j = 0; j < 3; j++)
+      for (int w = 0; w < SORT_WAVES; w++) {
+        const uint32_t x = wt[rd][j][w];
+        if (w < wave) run[j] += x;
+        carry[j] += x;
+      }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const uint32_t wq = q == 0 ? v[u].x : q == 1 ? v[u].y : q == 2 ? v[u].z : v[u].w;
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            if (4 * q + j < nv[u]) atomicAdd(&hist[(wq >> (8 * j)) & 0xffu], 1u);
+    for (int i = 0; i < DIR_PER; i++) {
+      const int64_t k = k0 + i;
+      if (k < D.nb) {
+        D.start[k] = run[0];
+        if (D.unit) {
+          // the workgroups whose first entry lies in this bucket
+          const uint32_t w1 = div_up(run[0] + v[0][i]);
+          for (uint32_t w = div_up(run[0]); w < w1; w++) D.utile[w] = (uint32_t)k;
+        } else {
+          D.ustart[k] = run[1];
+          for (uint32_t u = 0; u < v[1][i]; u++) D.utile[run[1] + u] = (uint32_t)k;
+          D.pstart[k] = run[2];
+          if (v[1][i] > 1) D.heavy[atomicAdd(&hcount, 1u)] = (uint32_t)k;
         }
       }
+#pragma unroll
+      for (int j = 0; j < 3; j++) run[j] += v[j][i];
     }
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < nb; i += UP_THREADS)
-    counts[tb + (int64_t)i * ts] = hist[i];
-}
-
-// Single-pass tile starts: tile_start[k] = t1scan[k*g1] (chunk 0), tile_start[ks] = n
-__global__ void k_tile_start_1pass(const uint32_t *__restrict__ t1scan, int64_t g1, int ks, int64_t n,
-                                   uint32_t *__restrict__ tile_start) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > ks) return;
-  tile_start[k] = (k == ks) ? (uint32_t)n : t1scan[(int64_t)k * g1];
-}
-
-// Work items per tile, at most imax records each.  store mode: every real
-// tile gets at least one item (so untouched tiles are written as zeros); add
-// mode: empty tiles are skipped.
-__global__ void k_items(const uint32_t *__restrict__ tile_start, int64_t ks, int64_t kreal, int store, uint32_t imax,
-                        uint32_t *__restrict__ mcnt, uint32_t *__restrict__ pcnt, uint32_t *__restrict__ nheavy) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > ks) return;
-  if (k == ks) {
-    mcnt[k] = 0;
-    pcnt[k] = 0;
-    return;
+  if (threadIdx.x == 0) {
+    D.start[D.nb] = carry[0];
+    if (!D.unit) D.ustart[D.nb] = carry[1];
   }
-  const uint32_t c = tile_start[k + 1] - tile_start[k];
-  uint32_t m = 0;
-  if (k < kreal) m = c == 0 ? (store ? 1u : 0u) : (c + imax - 1) / imax;
-  mcnt[k] = m;
-  pcnt[k] = m > 1 ? m : 0;
-  if (k == 0) *nheavy = 0;
+  for (int64_t i = threadIdx.x; i < D.npiece; i += SORT_THREADS) D.piece[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (D.mrange) {
+    uint32_t mx = 0u, mn = 0xffffffffu;
+    for (int64_t i = threadIdx.x; i < D.nw; i += SORT_THREADS) {
+      mx = max(mx, D.mrange_w[2 * i]);
+      mn = min(mn, D.mrange_w[2 * i + 1]);
+    }
+    atomicMax(&smr[0], mx);
+    atomicMin(&smr[1], mn);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (D.nheavy) *D.nheavy = hcount;
+    if (D.mrange) {
+      D.mrange[0] = smr[0];
+      D.mrange[1] = smr[1];
+    }
+  }
 }
 
-// item_tile[i] = tile of work item i
-__global__ void k_item_tiles(const uint32_t *__restrict__ item_start, int64_t ks, uint32_t *__restrict__ item_tile) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ks) return;
-  for (uint32_t i = item_start[k]; i < item_start[k + 1]; i++) item_tile[i] = (uint32_t)k;
+// The block list: bucket k's blocks from list entry start[k] on, each piece's
+// of a digit in the order it took them.  One workgroup per piece.
+__global__ void __launch_bounds__(SORT_THREADS) k_list(PgOut pg, int nb, const uint32_t *__restrict__ start,
+                                                       uint32_t *__restrict__ blist) {
+  const int64_t p = blockIdx.x;
+  const uint4 pc = pg.piece[p];
+  const int64_t bucket0 = (int64_t)pc.z * nb;
+  for (uint32_t k = threadIdx.x; k < pc.y; k += SORT_THREADS) {
+    const uint32_t blk = pc.x + k;
+    const uint32_t h = pg.hdr[blk], d = h & 2047u, j = h >> 11;
+    const int64_t at = p * nb + d;
+    const uint32_t fill = min(1u << pg.lg, pg.cnt[at] - (j << pg.lg));
+    blist[start[bucket0 + d] + pg.base[at] + j] = pg_entry(blk, fill, pg.lg);
+  }
 }
 
-__global__ void k_heavy_list(const uint32_t *__restrict__ pcnt, int64_t ks, uint32_t *__restrict__ nheavy,
-                             uint32_t *__restrict__ heavy) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ks) return;
-  if (pcnt[k] > 1) heavy[atomicAdd(nheavy, 1u)] = (uint32_t)k;
-}
-
-struct DsShape {
+struct PtShape {
   int pl;
   bool db;
   int hw;
 };
 
-// LDS of a downsweep shape (nb digits and the empty slots' digit); MODE 1
-// keeps three more arrays per digit.
-size_t downsweep_lds(int nb, int rw, const DsShape &h, int mode = 0) {
+// LDS of a partition shape (nb digits and the empty slots' digit); a paged
+// pass keeps two more arrays per digit.
+size_t partition_lds(int nb, int rw, const PtShape &h, bool paged) {
   const size_t sub = (size_t)SORT_THREADS * h.pl, nbt = (size_t)nb + 1;
-  return ((4 + (h.db ? 2 : 1) * h.hw) * nbt + (mode == 1 ? 3 * (size_t)nb : 0)) * 4 + sub * 2 + sub * rw * 4;
+  return ((4 + (h.db ? 2 : 1) * h.hw) * nbt + (paged ? 2 * (size_t)nb : 0)) * 4 + sub * 2 + sub * rw * 4;
 }
 
 // The first shape whose LDS fits one workgroup per CU: four count rows (each
-// shared by four waves: 16 rows measured 0.1 ms slower per downsweep at 2^30
+// shared by four waves: 16 rows measured 0.1 ms slower per pass at 2^30
 // records, the per-digit offsets running over more rows), then the most
-// records per lane, then double-buffered counts.
-DsShape downsweep_shape(int nb, int rw, int mode = 0) {
-  const size_t cap = 160 * 1024 - 256;
+// records per lane (at most plmax), then double-buffered counts.
+PtShape partition_shape(int nb, int rw, bool paged, int plmax) {
+  const size_t cap = 160 * 1024 - 512;
   for (int hw : {SORT_WAVES / 4, 1})
     for (int pl : {8, 4, 2})
       for (bool db : {true, false}) {
-        const DsShape h{pl, db, hw};
-        if (downsweep_lds(nb, rw, h, mode) <= cap) return h;
+        const PtShape h{pl, db, hw};
+        if (pl <= plmax && !(pl == 2 && db) && partition_lds(nb, rw, h, paged) <= cap) return h;
       }
-  return DsShape{1, false, 1};
+  return PtShape{2, false, 1};
 }
 
-// MODE 1 and 2 run with 8 records per lane only (sub-chunks of 8192 records)
-template <int NM, int MODE = 0>
-void launch_downsweep(int64_t grid, hipStream_t s, Src<NM> src, float *dst, const ChunkMap &cm, const KeyGeom &kg,
-                      const DigitSel &ds, int nb, const uint32_t *offsets, uint32_t *perm,
-                      uint8_t *dig2 = nullptr, const DigitSel &ds2 = DigitSel{0, 0, 0},
-                      uint32_t *mrange = nullptr, const PgArgs &pg = PgArgs{}) {
-  GENPK_REQUIRE(nb <= 2 * SORT_THREADS, "sort digit too wide");
-  GENPK_REQUIRE(!dig2 || (nb <= 256 && ds2.mask <= 255u), "sort digit bytes need digits of at most 8 bits");
-  const DsShape h = downsweep_shape(nb, Src<NM>::RW, MODE);
-  const size_t lds = downsweep_lds(nb, Src<NM>::RW, h, MODE);
+// Records per lane and sub-chunk of a pass over n records: fewer for small
+// sets, so that they spread over the CUs.
+int partition_plmax(int64_t n) {
+  const int64_t per = n / (2 * (int64_t)num_cus());
+  return per <= 2 * SORT_THREADS ? 2 : per <= 4 * SORT_THREADS ? 4 : 8;
+}
+
+template <int NM, int IN, bool PAGED, bool PERM>
+void launch_partition_perm(int64_t grid, hipStream_t s, const float *pos, const float *masses, const uint32_t *blist,
+                           const uint32_t *start, const uint32_t *first_seg, float *dst, const InMap &im, const KeyGeom &kg, const DigitSel &ds, int nb,
+                           const PtShape &h, const uint32_t *offsets, uint32_t *perm, uint32_t *mrange_w,
+                           const PgOut &pg) {
+  GENPK_REQUIRE(nb <= 2048, "sort digit too wide");
+  const size_t lds = partition_lds(nb, Src<NM>::RW, h, PAGED);
+  GENPK_REQUIRE(lds <= 160 * 1024 - 512, "sort pass does not fit in LDS");
   const dim3 g((unsigned)grid), b(SORT_THREADS);
-  if constexpr (MODE != 0) {
-    GENPK_REQUIRE(h.pl == 8 && nb <= 256 && (MODE != 1 || dig2), "paged sort pass: unsupported shape");
-    if (h.db)
-      hipLaunchKernelGGL((k_downsweep<NM, 8, true, MODE>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets,
-                         perm, dig2, ds2, mrange, pg);
-    else
-      hipLaunchKernelGGL((k_downsweep<NM, 8, false, MODE>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets,
-                         perm, dig2, ds2, mrange, pg);
-  } else if (h.pl == 8 && h.db) {
-    hipLaunchKernelGGL((k_downsweep<NM, 8, true, 0>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets, perm,
-                       dig2, ds2, mrange, pg);
-  } else if (h.pl == 8) {
-    hipLaunchKernelGGL((k_downsweep<NM, 8, false, 0>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets, perm,
-                       dig2, ds2, mrange, pg);
-  } else if (h.pl == 4 && h.db) {
-    hipLaunchKernelGGL((k_downsweep<NM, 4, true, 0>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets, perm,
-                       dig2, ds2, mrange, pg);
-  } else if (h.pl == 4) {
-    hipLaunchKernelGGL((k_downsweep<NM, 4, false, 0>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets, perm,
-                       dig2, ds2, mrange, pg);
-  } else if (h.pl == 2) {
-    hipLaunchKernelGGL((k_downsweep<NM, 2, false, 0>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets, perm,
-                       dig2, ds2, mrange, pg);
-  } else {
-    hipLaunchKernelGGL((k_downsweep<NM, 1, false, 0>), g, b, lds, s, src, dst, cm, kg, ds, nb, h.hw, offsets, perm,
-                       dig2, ds2, mrange, pg);
-  }
+#define GENPK_PART(PL, DB)                                                                                       \
+  hipLaunchKernelGGL((k_partition<NM, PL, DB, IN, PAGED, PERM>), g, b, lds, s, pos, masses, blist, start, first_seg, \
+                     dst, im, kg, ds, nb, h.hw, offsets, perm, mrange_w, pg)
+  if (h.pl == 8 && h.db) GENPK_PART(8, true);
+  else if (h.pl == 8) GENPK_PART(8, false);
+  else if (h.pl == 4 && h.db) GENPK_PART(4, true);
+  else if (h.pl == 4) GENPK_PART(4, false);
+  else GENPK_PART(2, false);
+#undef GENPK_PART
   GENPK_LAUNCH_CHECK();
 }
 
-// Whether and how a sort runs its first pass paged: two passes with digits
-// of at most 8 bits, and so many records that the partly filled blocks (at
-// most one per pass-1 workgroup and digit) leave fewer empty slots than 1/4
-// of the records (half that on average).  G = twice the CU count workgroups
-// (two rounds of one per CU even out their finishing times: 7.8 -> 7.5 ms
-// at 2^30 records) take `chunk` records each (whole sub-chunks) and Q =
-// chunk / PG_BLOCK + nhi blocks: every digit's blocks but its last are
-// full.  With masses (16-byte records) the paged downsweeps keep a few
-// registers in scratch and are still faster than the histogram pass they
-// replace (37.5 -> 36.3 ms per retaining forward at 2^30).
+template <int NM, int IN, bool PAGED>
+void launch_partition(int64_t grid, hipStream_t s, const float *pos, const float *masses, const uint32_t *blist,
+                      const uint32_t *start, const uint32_t *first_seg, float *dst, const InMap &im, const KeyGeom &kg, const DigitSel &ds, int nb, const PtShape &h,
+                      const uint32_t *offsets, uint32_t *perm, uint32_t *mrange_w, const PgOut &pg) {
+  if (perm)
+    launch_partition_perm<NM, IN, PAGED, true>(grid, s, pos, masses, blist, start, first_seg, dst, im, kg, ds, nb, h,
+                                               offsets, perm,
+                                               mrange_w, pg);
+  else
+    launch_partition_perm<NM, IN, PAGED, false>(grid, s, pos, masses, blist, start, first_seg, dst, im, kg, ds, nb, h,
+                                               offsets, perm,
+                                                mrange_w, pg);
+}
+
+// log2 of a paged pass's block: a quarter to a half of the records that a
+// piece holds of a digit on average.  Longer blocks write faster (2^30
+// records: pass 2 7.1, 6.8, 6.5 ms with an eighth to a sixteenth, a quarter
+// to an eighth, and this), shorter ones leave fewer slots empty.
+int pick_lg(int64_t recs, int64_t nb, int lo, int hi) {
+  int lg = 0;
+  while (((int64_t)2 << (lg + 1)) * nb <= recs) lg++;
+  return std::min(std::max(lg, lo), hi);
+}
+
+// Shape of a paged pass: G workgroups of `chunk` input slots each, and the
+// pool of its pieces' blocks of 2^lg record slots.
 struct PgLayout {
-  bool on = false;
-  int64_t G = 0, chunk = 0, Q = 0;
-  int64_t slots = 0;  // G * Q * PG_BLOCK record slots of the pass-1 output
+  PtShape h;
+  int64_t G = 0, chunk = 0, pieces = 0, blocks = 0;
+  int lg = 0;
+  int64_t slots() const { return blocks << lg; }
 };
 
-PgLayout pg_layout(const Plan &p, int64_t n, int rw) {
+// A paged pass over at most `slots` input slots in nseg buckets.  Every
+// workgroup takes the same number of slots: one round of one workgroup per
+// CU, or more rounds as long as each workgroup keeps minsub sub-chunks and
+// the partly filled blocks (one per piece and digit at most) stay below a
+// sixth of the slots (or 2^26: about 1 GB).  Shorter ranges run beside each other in time on
+// neighbouring parts of the pools, and finish evenly: with two rounds instead
+// of eight the first pass takes 0.80 instead of 0.74 ms (2^27 records, 64
+// digits), with two instead of 16 the second 7.2 instead of 6.5 ms (2^30
+// records).
+PgLayout paged_layout(int64_t slots, int64_t nseg, int nb, int rw, int lo, int hi, int minsub) {
   PgLayout L;
-  const TileGeom &tg = p.tg;
-  if (tg.passes != 2 || tg.hi_bits > 8 || tg.lo_bits > 8) return L;
-  const int64_t nhi = (int64_t)1 << tg.hi_bits, cus = num_cus();
-  if (2 * cus * nhi * (int64_t)PG_BLOCK > n / 4) return L;
-  for (int mode : {1, 2})
-    if (downsweep_shape((int)nhi, rw, mode).pl != 8) return L;
-  constexpr int64_t SUBN = (int64_t)SORT_THREADS * 8;
-  L.chunk = ceil_div(ceil_div(n, 2 * cus), SUBN) * SUBN;
-  L.G = ceil_div(n, L.chunk);
-  L.Q = L.chunk / PG_BLOCK + nhi;
-  L.slots = L.G * L.Q * PG_BLOCK;
-  L.on = L.slots <= ((int64_t)1 << 32);  // block numbers below 2^22 (pg_entry)
+  L.h = partition_shape(nb, rw, true, partition_plmax(slots));
+  const int64_t subn = (int64_t)SORT_THREADS * L.h.pl, cus = num_cus();
+  for (int64_t rounds = 1; rounds <= 16; rounds *= 2) {
+    PgLayout M = L;
+    M.chunk = std::max(subn, ceil_div(ceil_div(slots, rounds * cus), subn) * subn);
+    M.G = ceil_div(slots, M.chunk);
+    M.pieces = nseg > 1 ? M.G + nseg : M.G;
+    M.lg = pick_lg(slots / M.pieces, nb, lo, hi);
+    const int64_t partial = M.pieces * (nb + 1);
+    M.blocks = (slots >> M.lg) + partial + 1;
+    if (rounds > 1 && (M.chunk < minsub * subn || (partial << M.lg) > std::max(slots / 6, (int64_t)1 << 26))) break;
+    L = M;
+  }
   return L;
+}
+
+// Whether the first of two passes is paged (of 2^hi_bits digits): each
+// workgroup has to hold many records of a digit.  With 256 digits the counted
+// pass keeps sorts below 2^29 records, which the tests compare with paged
+// ones.
+bool first_paged(const Plan &p, int64_t n) {
+  const int64_t nhi = (int64_t)1 << p.tg.hi_bits, cus = num_cus();
+  if (nhi > 256) return false;
+  if (nhi == 256) return 2 * cus * nhi * 1024 <= n / 4;
+  return n >= cus * nhi * 128;
+}
+
+// Workspace of a paged pass in one buffer: pieces, headers, per-piece counts
+// and bases, and the block list.
+uint32_t *pg_buffers(DevBuf &buf, const PgLayout &L, int nb, PgOut &pg, unsigned long long *tot) {
+  const size_t blocks = (size_t)L.blocks, wd = (size_t)L.pieces * nb;
+  GENPK_REQUIRE((uint64_t)L.slots() <= ((uint64_t)1 << 32), "sort pool too large");
+  uint32_t *b = static_cast<uint32_t *>(buf.ensure((4 * (size_t)L.pieces + 2 * blocks + 2 * wd) * 4));
+  pg.piece = reinterpret_cast<uint4 *>(b);
+  pg.hdr = b + 4 * L.pieces;
+  pg.cnt = pg.hdr + blocks;
+  pg.base = pg.cnt + wd;
+  pg.tot = tot;
+  pg.lg = L.lg;
+  return pg.base + wd;  // the block list
+}
+
+void launch_dir(const DirArgs &D, hipStream_t s) {
+  hipLaunchKernelGGL(k_dir, dim3(1), dim3(SORT_THREADS), 0, s, D);
+  GENPK_LAUNCH_CHECK();
+}
+
+// Counted first pass: chunk size and count.
+int64_t counted_chunk(int64_t n) {
+  int64_t chunk = SORT_CHUNK_MIN;
+  while (chunk < SORT_CHUNK_MAX && chunk * 4 * num_cus() < n) chunk *= 2;
+  return chunk;
+}
+
+struct SortLayout {
+  bool two = false, paged1 = false;
+  PgLayout L1, L2;  // paged first pass (of two), last pass
+  int64_t slots1 = 0;  // slots that a first pass of two writes
+};
+
+SortLayout sort_layout(const Plan &p, int64_t n, int rw) {
+  SortLayout S;
+  const TileGeom &tg = p.tg;
+  const int nhi = 1 << tg.hi_bits, nlo = 1 << tg.lo_bits;
+  S.two = tg.passes == 2;
+  if (!S.two) {
+    S.L2 = paged_layout(n, 1, nhi, rw, 3, 8, 8);
+    return S;
+  }
+  S.paged1 = first_paged(p, n);
+  if (S.paged1) {
+    S.L1 = paged_layout(n, 1, nhi, rw, 6, 8, 8);
+    S.slots1 = S.L1.slots();
+    S.paged1 = S.slots1 <= ((int64_t)1 << 32);
+  }
+  if (!S.paged1) S.slots1 = n;
+  S.L2 = paged_layout(S.slots1, nhi, nlo, rw, 3, 8, 2);
+  return S;
 }
 
 template <int NM>
 TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, const float *masses, bool with_perm,
-                    bool every_tile, const PgLayout &L) {
+                    bool every_tile, const SortLayout &S) {
+  constexpr int RW = Src<NM>::RW;
   hipStream_t s = p.stream;
   const TileGeom &tg = p.tg;
-
+  const int nhi = 1 << tg.hi_bits, nlo = 1 << tg.lo_bits;
+  const int64_t ks = (int64_t)nhi * nlo;
   float *A = p.recA.as<float>();
   float *B = p.recB.as<float>();
-  int64_t chunk = SORT_CHUNK_MIN;
-  while (chunk < SORT_CHUNK_MAX && chunk * 4 * num_cus() < n) chunk *= 2;
-  const int64_t g1 = ceil_div(n, chunk);
   Src<NM> raw{pos, masses, true};
   uint32_t *perm1 = with_perm ? p.permA.as<uint32_t>() : nullptr;
-  uint32_t *perm2 = (with_perm && tg.passes == 2) ? p.permB.as<uint32_t>() : nullptr;
-  const float *sorted = nullptr;
-  uint32_t *tile_start = nullptr;
-  int64_t ks = 0;
+  uint32_t *perm2 = (with_perm && S.two) ? p.permB.as<uint32_t>() : nullptr;
+
+  // bucket totals, of the tiles and of a first pass's segments: zero between
+  // sorts (k_dir clears what it read)
+  const int64_t ntot = ks + (S.two ? nhi : 0);
+  unsigned long long *tot = static_cast<unsigned long long *>(p.sort_tot.ensure((size_t)ntot * 8));
+  if (p.sort_tot_zero != ntot) fill_zero(tot, (size_t)ntot * 8, s);
+  p.sort_tot_zero = 0;
+
   // with masses, pass 1 (which reads every mass) records their range for the deposit
-  uint32_t *mrange = nullptr;
+  const int64_t chunk1 = S.two && !S.paged1 ? counted_chunk(n) : 0;
+  const int64_t g1 = !S.two ? S.L2.G : S.paged1 ? S.L1.G : ceil_div(n, chunk1);
+  uint32_t *mrange = nullptr, *mrange_w = nullptr;
   if (NM == 1) {
-    mrange = static_cast<uint32_t *>(p.mrange.ensure(64));
-    hipLaunchKernelGGL(k_mrange_init, dim3(1), dim3(1), 0, s, mrange);
-    GENPK_LAUNCH_CHECK();
+    mrange = static_cast<uint32_t *>(p.mrange.ensure((size_t)(2 + 2 * g1) * 4));
+    mrange_w = mrange + 2;
   }
 
-  if (tg.passes == 1) {
-    const int nb = 1 << tg.hi_bits;
-    ks = nb;
-    uint32_t *t1 = static_cast<uint32_t *>(p.table1.ensure((size_t)nb * g1 * 4));
-    const DigitSel dsel = digit_sel(kg, 0, tg.hi_bits);
-    ChunkMap cm{n, 0, nullptr, nullptr, g1, 0, chunk};
-    {
-      Stage st(p, "sort_upsweep1");
-      hipLaunchKernelGGL((k_upsweep<NM>), dim3((unsigned)g1), dim3(SORT_THREADS), nb * 4, s, raw, cm, kg, dsel, nb, t1);
-      GENPK_LAUNCH_CHECK();
-    }
-    exclusive_scan_u32(t1, t1, (int64_t)nb * g1, p.scan_tmp, s);
-    {
-      Stage st(p, "sort_downsweep1");
-      launch_downsweep<NM>(g1, s, raw, A, cm, kg, dsel, nb, t1, perm1, nullptr, DigitSel{0, 0, 0}, mrange);
-    }
-    tile_start = static_cast<uint32_t *>(p.tile_start.ensure((size_t)(ks + 1) * 4));
-    hipLaunchKernelGGL(k_tile_start_1pass, dim3((unsigned)ceil_div(ks + 1, 256)), dim3(256), 0, s, t1, g1, (int)ks,
-                       n, tile_start);
-    GENPK_LAUNCH_CHECK();
-    sorted = A;
+  PgOut pg2;
+  uint32_t *blist = pg_buffers(p.pages, S.L2, S.two ? nlo : nhi, pg2, tot);
+  const DigitSel dlo = digit_sel(kg, 0, S.two ? tg.lo_bits : tg.hi_bits);
+  float *out;
+  if (!S.two) {
+    out = A;
+    Stage st(p, "sort_downsweep1");
+    InMap im;
+    im.n = n;
+    im.chunk = S.L2.chunk;
+    launch_partition<NM, IN_RAW, true>(S.L2.G, s, pos, masses, nullptr, nullptr, nullptr, out, im, kg, dlo, nhi, S.L2.h, nullptr, perm1, mrange_w, pg2);
   } else {
-    const int nhi = 1 << tg.hi_bits, nlo = 1 << tg.lo_bits;
-    ks = (int64_t)nhi * nlo;
-    const DigitSel d1 = digit_sel(kg, tg.lo_bits, tg.hi_bits);
-    const DigitSel d2 = digit_sel(kg, 0, tg.lo_bits);
-    // with digits of at most 8 bits, pass 1 writes each record's low digit as
-    // a byte beside it (in its output slot), and pass 2 counts those bytes
-    // instead of reading the records
-    const int64_t slots = L.on ? L.slots : n;  // pass-1 output slots
-    uint8_t *dig2 = tg.lo_bits <= 8 && tg.hi_bits <= 8
-                        ? static_cast<uint8_t *>(p.dig2.ensure((size_t)slots + 64))
-                        : nullptr;
-    // segments of pass 2 (one per pass-1 digit): start (records, or list
-    // slots when paged), chunk count and first chunk, first record
-    uint32_t *seg = static_cast<uint32_t *>(p.seginfo.ensure((size_t)(nhi + 1) * 4 * 4));
-    uint32_t *seg_start = seg, *nchunks = seg + (nhi + 1), *chunk_start = seg + 2 * (nhi + 1);
-    uint32_t *rec_start = seg_start;
-    int64_t g2 = 0;  // upper bound of pass-2 chunks
-    PgArgs pg;
-    if (L.on) {
+    out = B;
+    const DigitSel dhi = digit_sel(kg, tg.lo_bits, tg.hi_bits);
+    // segments of pass 2: first list entry (or record), and the segment of
+    // each workgroup's first
+    const int64_t ss = nhi + 4;
+    uint32_t *sb = static_cast<uint32_t *>(p.seginfo.ensure((size_t)(ss + S.L2.G) * 4));
+    InMap im1, im2;
+    const uint32_t *list1 = nullptr;
+    im1.n = n;
+    im1.chunk = S.paged1 ? S.L1.chunk : chunk1;
+    im2.nseg = nhi;
+    im2.chunk = S.L2.chunk;
+    DirArgs D{};
+    D.tot = tot + ks;
+    D.nb = D.kreal = nhi;
+    D.start = sb;
+    D.utile = sb + ss;
+    D.piece = pg2.piece;
+    D.npiece = S.L2.pieces;
+    if (S.paged1) {
       // pass 1, paged: the positions are read once
-      GENPK_REQUIRE(chunk % PG_BLOCK == 0, "paged sort: pass-2 chunks must be whole blocks");
-      const int64_t nbk = L.G * L.Q, nt = (int64_t)nhi * L.G + 1;
-      uint32_t *pb = static_cast<uint32_t *>(p.pages.ensure((size_t)(4 * nbk + L.G + 4 * nt) * 4));
-      pg.hdr = pb;
-      pg.fill = pb + nbk;
-      pg.used = pb + 2 * nbk;
-      pg.Q = L.Q;
-      uint32_t *blist = pg.used + L.G;
-      uint32_t *bcnt = blist + nbk, *rcnt = bcnt + nt, *boff = rcnt + nt, *roff = boff + nt;
-      rec_start = seg + 3 * (nhi + 1);
-      ChunkMap cm1{n, 0, nullptr, nullptr, L.G, 0, L.chunk};
+      PgOut pg1;
+      uint32_t *blist1 = pg_buffers(p.pages1, S.L1, nhi, pg1, tot + ks);
       {
         Stage st(p, "sort_downsweep1");
-        launch_downsweep<NM, 1>(L.G, s, raw, A, cm1, kg, d1, nhi, nullptr, perm1, dig2, d2, mrange, pg);
+        launch_partition<NM, IN_RAW, true>(S.L1.G, s, pos, masses, nullptr, nullptr, nullptr, A, im1, kg, dhi, nhi, S.L1.h, nullptr, perm1, mrange_w,
+                                           pg1);
       }
-      {
-        Stage st(p, "sort_pages");
-        hipLaunchKernelGGL(k_pg_count, dim3((unsigned)L.G), dim3(256), 0, s, pg, nhi, L.G, bcnt, rcnt);
-        GENPK_LAUNCH_CHECK();
-        exclusive_scan_u32(bcnt, boff, nt, p.scan_tmp, s);
-        exclusive_scan_u32(rcnt, roff, nt, p.scan_tmp, s);
-        hipLaunchKernelGGL(k_pg_list, dim3((unsigned)L.G), dim3(256), 0, s, pg, nhi, L.G, boff, blist);
-        GENPK_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_pg_seginfo, dim3((unsigned)ceil_div(nhi + 1, 256)), dim3(256), 0, s, boff, roff, nhi,
-                           L.G, chunk, seg_start, rec_start, nchunks);
-        GENPK_LAUNCH_CHECK();
-      }
-      pg.blist = blist;
-      g2 = ceil_div(nbk * PG_BLOCK, chunk) + nhi;
+      Stage st(p, "sort_pages");
+      D.unit = (uint32_t)(S.L2.chunk >> S.L1.lg);
+      D.funit = FastDiv(D.unit);
+      launch_dir(D, s);
+      hipLaunchKernelGGL(k_list, dim3((unsigned)S.L1.pieces), dim3(SORT_THREADS), 0, s, pg1, nhi, D.start, blist1);
+      GENPK_LAUNCH_CHECK();
+      list1 = blist1;
+      im2.lg = S.L1.lg;
     } else {
-      // pass 1: high digit over [0, n)
+      // pass 1, counted
       uint32_t *t1 = static_cast<uint32_t *>(p.table1.ensure((size_t)nhi * g1 * 4));
-      ChunkMap cm1{n, 0, nullptr, nullptr, g1, 0, chunk};
       {
         Stage st(p, "sort_upsweep1");
-        hipLaunchKernelGGL((k_upsweep<NM>), dim3((unsigned)g1), dim3(SORT_THREADS), nhi * 4, s, raw, cm1, kg, d1,
+        hipLaunchKernelGGL((k_upsweep<NM>), dim3((unsigned)g1), dim3(SORT_THREADS), nhi * 4, s, raw, im1, kg, dhi,
                            nhi, t1);
         GENPK_LAUNCH_CHECK();
       }
       exclusive_scan_u32(t1, t1, (int64_t)nhi * g1, p.scan_tmp, s);
       {
         Stage st(p, "sort_downsweep1");
-        launch_downsweep<NM>(g1, s, raw, A, cm1, kg, d1, nhi, t1, perm1, dig2, d2, mrange);
+        launch_partition<NM, IN_RAW, false>(g1, s, pos, masses, nullptr, nullptr, nullptr, A, im1, kg, dhi, nhi, partition_shape(nhi, RW, false, 8), t1,
+                                            perm1, mrange_w, PgOut{});
       }
-      hipLaunchKernelGGL(k_seginfo, dim3((unsigned)ceil_div(nhi + 1, 256)), dim3(256), 0, s, t1, g1, nhi, n, chunk,
-                         seg_start, nchunks);
+      hipLaunchKernelGGL(k_seg_tot, dim3((unsigned)ceil_div(nhi, 256)), dim3(256), 0, s, t1, g1, nhi, n, tot + ks);
       GENPK_LAUNCH_CHECK();
-      g2 = g1 + nhi;
+      D.unit = (uint32_t)S.L2.chunk;
+      D.funit = FastDiv(D.unit);
+      launch_dir(D, s);
     }
-    exclusive_scan_u32(nchunks, chunk_start, nhi + 1, p.scan_tmp, s);
-    uint32_t *t2 = static_cast<uint32_t *>(p.table2.ensure((size_t)g2 * nlo * 4));
-    ChunkMap cm2{n, nhi, seg_start, chunk_start, 0, nlo, chunk};
-    Src<NM> pa{A, nullptr, false};
-    {
-      Stage st(p, "sort_upsweep2");
-      if (L.on)
-        hipLaunchKernelGGL(k_upsweep_pages, dim3((unsigned)g2), dim3(UP_THREADS), nlo * 4, s, dig2, cm2, pg, nlo,
-                           t2);
-      else if (dig2)
-        hipLaunchKernelGGL(k_upsweep_bytes, dim3((unsigned)g2), dim3(SORT_THREADS), nlo * 4, s, dig2, cm2, nlo, t2);
-      else
-        hipLaunchKernelGGL((k_upsweep<NM>), dim3((unsigned)g2), dim3(SORT_THREADS), nlo * 4, s, pa, cm2, kg, d2, nlo,
-                           t2);
-      GENPK_LAUNCH_CHECK();
-    }
-    // the written part of the table is its first (pass-2 chunks) * nlo entries;
-    // the rest, scanned along, is never read
-    exclusive_scan_u32(t2, t2, g2 * nlo, p.scan_tmp, s);
-    tile_start = static_cast<uint32_t *>(p.tile_start.ensure((size_t)(ks + 1) * 4));
-    hipLaunchKernelGGL(k_tile_start_2pass, dim3((unsigned)ceil_div(ks + 1, 256)), dim3(256), 0, s, t2, chunk_start,
-                       rec_start, nhi, nlo, n, tile_start);
-    GENPK_LAUNCH_CHECK();
-    {
-      Stage st(p, "sort_downsweep2");
-      if (L.on)
-        launch_downsweep<NM, 2>(g2, s, pa, B, cm2, kg, d2, nlo, t2, perm2, nullptr, DigitSel{0, 0, 0}, nullptr, pg);
-      else
-        launch_downsweep<NM>(g2, s, pa, B, cm2, kg, d2, nlo, t2, perm2);
-    }
-    sorted = B;
+    Stage st(p, "sort_downsweep2");
+    if (S.paged1)
+      launch_partition<NM, IN_LIST, true>(S.L2.G, s, A, nullptr, list1, sb, sb + ss, out, im2, kg, dlo, nlo, S.L2.h, nullptr, perm2, nullptr, pg2);
+    else
+      launch_partition<NM, IN_SEG, true>(S.L2.G, s, A, nullptr, list1, sb, sb + ss, out, im2, kg, dlo, nlo, S.L2.h, nullptr, perm2, nullptr, pg2);
   }
 
-  // work items
-  const int store = every_tile ? 1 : 0;
-  uint32_t *ib = static_cast<uint32_t *>(p.item_start.ensure((size_t)(ks + 1) * 4 * 4 + 64));
-  uint32_t *mcnt = ib, *item_start = ib + (ks + 1), *pcnt = ib + 2 * (ks + 1), *part_start = ib + 3 * (ks + 1);
-  uint32_t *hv = static_cast<uint32_t *>(p.heavy.ensure((size_t)(ks + 2) * 4));
-  uint32_t *nheavy = hv, *heavy = hv + 1;
-  const uint32_t imax = deposit_item_max(n, tg.K);
-  hipLaunchKernelGGL(k_items, dim3((unsigned)ceil_div(ks + 1, 256)), dim3(256), 0, s, tile_start, ks, tg.K, store,
-                     imax, mcnt, pcnt, nheavy);
-  GENPK_LAUNCH_CHECK();
-  exclusive_scan_u32(mcnt, item_start, ks + 1, p.scan_tmp, s);
-  exclusive_scan_u32(pcnt, part_start, ks + 1, p.scan_tmp, s);
-  hipLaunchKernelGGL(k_heavy_list, dim3((unsigned)ceil_div(ks, 256)), dim3(256), 0, s, pcnt, ks, nheavy, heavy);
-  GENPK_LAUNCH_CHECK();
-  const int64_t max_items = tg.K + ceil_div(n, (int64_t)imax);
-  uint32_t *item_tile = static_cast<uint32_t *>(p.item_tile.ensure((size_t)max_items * 4));
-  hipLaunchKernelGGL(k_item_tiles, dim3((unsigned)ceil_div(ks, 256)), dim3(256), 0, s, item_start, ks, item_tile);
-  GENPK_LAUNCH_CHECK();
-
+  // the tiles' block lists and work items
   TileOrder o;
-  o.rec = sorted;
-  o.rw = Src<NM>::RW;
+  const uint32_t imax = deposit_item_max(n, tg.K);
+  const int64_t slots = S.L2.slots();
+  // split tiles have m > 1 items, at most twice the item sizes that fill them
+  o.max_parts = 2 * ((imax < (uint32_t)DEPOSIT_ITEM_MAX ? ceil_div(n, (int64_t)imax) : 0) +
+                     ceil_div(slots, (int64_t)DEPOSIT_ITEM_MAX));
+  const int64_t max_items = tg.K + o.max_parts;
+  const int64_t ts = (ks + 4) / 4 * 4;
+  uint32_t *ib = static_cast<uint32_t *>(p.item_start.ensure((size_t)ts * 4 * 4 + 64));
+  uint32_t *item_tile = static_cast<uint32_t *>(p.item_tile.ensure((size_t)max_items * 4));
+  DirArgs D{};
+  D.tot = tot;
+  D.nb = ks;
+  D.kreal = tg.K;
+  D.start = ib;
+  D.ustart = ib + ts;
+  D.utile = item_tile;
+  D.store = every_tile ? 1 : 0;
+  D.lg = S.L2.lg;
+  D.limax = ilog2(imax);
+  D.pstart = ib + 2 * ts;
+  D.heavy = ib + 3 * ts;
+  D.nheavy = static_cast<uint32_t *>(p.heavy.ensure(64));
+  D.nonfinite = static_cast<uint32_t *>(p.nonfinite.ensure(64));
+  D.mrange = mrange;
+  D.mrange_w = mrange_w;
+  D.nw = g1;
+  {
+    Stage st(p, "sort_tiles");
+    launch_dir(D, s);
+    hipLaunchKernelGGL(k_list, dim3((unsigned)S.L2.pieces), dim3(SORT_THREADS), 0, s, pg2, S.two ? nlo : nhi,
+                       D.start, blist);
+    GENPK_LAUNCH_CHECK();
+  }
+  p.sort_tot_zero = ntot;
+
+  o.rec = out;
+  o.rw = RW;
   o.has_mass = NM != 0;
   o.has_perm = with_perm;
   o.perm1 = perm1;
   o.perm2 = perm2;
-  o.tile_start = tile_start;
-  o.item_start = item_start;
-  o.item_tile = item_tile;
-  o.part_start = part_start;
-  o.nheavy = nheavy;
-  o.heavy = heavy;
+  o.list = {D.start, D.ustart, item_tile, blist, S.L2.lg, ks, max_items};
+  o.part_start = D.pstart;
+  o.nheavy = D.nheavy;
+  o.heavy = D.heavy;
   o.mrange = mrange;
-  o.ks = ks;
   o.n = n;
-  o.max_items = max_items;
-  o.item_max = imax;
   return o;
 }
 }  // namespace
@@ -1129,19 +1021,25 @@ TileOrder sort_by_tile(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, 
                        bool every_tile) {
   GENPK_REQUIRE(n > 0 && n <= ((int64_t)1 << 31), "sort_by_tile: particle count out of range");
   const int rw = 3 + (masses ? 1 : 0);
-  const PgLayout L = pg_layout(p, n, rw);
-  // with the permutations, both record buffers can also take the adjoint
-  // gather's output records (up to 4 floats); recA holds the pass-1 output
-  // (paged: L.slots record slots), perm2 is indexed by its slots
-  const size_t rec_bytes = (size_t)n * (with_perm ? 4 : rw) * 4;
-  p.recA.ensure(L.on ? std::max(rec_bytes, (size_t)L.slots * rw * 4) : rec_bytes);
-  if (p.tg.passes == 2 || with_perm) p.recB.ensure(rec_bytes);
+  const SortLayout S = sort_layout(p, n, rw);
+  // the first pass of two writes recA and the last pass recB (a single pass:
+  // recA); with the permutations the other one also takes the adjoint
+  // gather's output records (up to 4 floats per slot of the sorted pool).
+  // perm2 is indexed by pass-1 slots.
+  const size_t last = (size_t)S.L2.slots(), gather = with_perm ? last * 16 : 0;
+  if (S.two) {
+    p.recA.ensure(std::max((size_t)S.slots1 * rw * 4, gather));
+    p.recB.ensure(last * rw * 4);
+  } else {
+    p.recA.ensure(last * rw * 4);
+    if (with_perm) p.recB.ensure(gather);
+  }
   if (with_perm) {
     p.permA.ensure((size_t)n * 4);
-    if (p.tg.passes == 2) p.permB.ensure((size_t)(L.on ? L.slots : n) * 4);
+    if (S.two) p.permB.ensure((size_t)S.slots1 * 4);
   }
-  if (masses) return sort_impl<1>(p, kg, n, pos, masses, with_perm, every_tile, L);
-  return sort_impl<0>(p, kg, n, pos, nullptr, with_perm, every_tile, L);
+  if (masses) return sort_impl<1>(p, kg, n, pos, masses, with_perm, every_tile, S);
+  return sort_impl<0>(p, kg, n, pos, nullptr, with_perm, every_tile, S);
 }
 
 }  // namespace genpk

@@ -1,0 +1,90 @@
+"""The tile partition at the edges of its shapes: particle counts around one
+sub-chunk (1024 threads x 2, 4 or 8 records), around the counts where
+the records per lane and the first pass's form change, tile counts around
+the one-pass limit (1024 tiles), all particles in one cell (split tiles),
+with and without masses.
+
+Deposits of the same particles under two tile shapes go through different
+partitions (digits, passes, blocks); with one mass the per-cell sums are
+exact integers (2^-36 per weight, below 2^53), so the FP64 densities are
+equal bit for bit.  With masses in [0.5, 1) every term is a multiple of
+2^-45, so that cells below 2^7 (2^52 such units) are equal too; fuller cells
+round as they convert and as tiles' halos are added, which differs between
+the tilings, and are checked against the oracle only.  The adjoint gather's gradients of one dL/drho depend on no order.  One
+density per case is compared with the FP64 CPU oracle: each of a cell's c
+terms is rounded by at most 2^-37, so the difference is below c 2^-37 (and
+FP64 rounding), with c at most the particles of the fullest cell's
+neighbourhood."""
+import numpy as np
+import pytest
+
+import genpk_amd
+import oracle
+
+BOX = 100.0
+# n around sub-chunks of 2048 and 8192 records, 512 workgroups of them
+# (2^20, 2^21), and the paged first pass's bound for 32 digits (2^20)
+CASES = [(1, 64), (63, 33), (2048, 64), (2049, 200), (8193, 256), (65537, 256), (300001, 257), (1048575, 264),
+         (1048577, 264), (2097153, 200), (1300000, 320)]
+
+
+def _positions(torch, n, kind):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    if kind == "cell":
+        return (torch.rand((n, 3), device="cuda", generator=g) * 0.2 + 31.1).contiguous()
+    pos = torch.rand((n, 3), device="cuda", generator=g) * BOX
+    if n > 100:
+        # a tenth outside the box (wrapped), a tenth in one clump
+        pos[: n // 10] += BOX * torch.randint(-2, 3, (n // 10, 3), device="cuda", generator=g)
+        pos[n // 10: n // 5] = torch.randn((n // 5 - n // 10, 3), device="cuda", generator=g) * 0.3 + 50.0
+    return pos.contiguous()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,d", CASES)
+@pytest.mark.parametrize("kind", ["spread", "cell"])
+@pytest.mark.parametrize("masses", [False, True])
+def test_partition_edges(gpu, n, d, kind, masses):
+    import torch
+    if kind == "cell" and n > 300001:
+        pytest.skip("one cell: covered by the smaller counts")
+    print("CASE", n, d, kind, masses, flush=True)
+    pos = _positions(torch, n, kind)
+    m = None
+    if masses:
+        m = torch.rand(n, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)) * 0.5 + 0.5
+    a, b = genpk_amd.Plan(d, "f64"), genpk_amd.Plan(d, "f64").set_options((8, 16, 32))
+    got = []
+    for p in (a, b):
+        p.clear()
+        p.deposit(pos, BOX, m, retain=True)
+        got.append(p.export_density().clone())
+    if masses:
+        few = got[0] < 2.0 ** 7
+        assert torch.equal(got[0][few], got[1][few])
+    else:
+        assert torch.equal(got[0], got[1])
+    # the kept order deposits again
+    a.clear()
+    a.redeposit()
+    assert torch.equal(a.export_density(), got[0])
+    # gradients of one dL/drho through the kept order and a fresh partition
+    G = torch.randn(got[0].shape, dtype=torch.float64, device="cuda",
+                    generator=torch.Generator(device="cuda").manual_seed(5))
+    a.clear()
+    a.deposit(pos, BOX, m, retain=True)
+    grads = []
+    for p in (a, b):
+        p.import_density(G)
+        grads.append(p.adjoint_gather(pos, BOX, m))
+    assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
+    if n > 300001:
+        return
+    ref = oracle.new_field(d)
+    oracle.fieldize(BOX, d, ref, pos.cpu().numpy(), None if m is None else m.cpu().numpy(), 1.0, 1)
+    ref = np.asarray(ref).reshape(d, d, -1)[:, :, :d]
+    dens = got[0].cpu().numpy().reshape(d, d, -1)[:, :, :d]
+    cells = (np.floor(pos.cpu().numpy().astype(np.float64) * (d / BOX)).astype(np.int64)) % d
+    _, c = np.unique((cells[:, 0] * d + cells[:, 1]) * d + cells[:, 2], return_counts=True)
+    terms = 8 * c.max()
+    assert np.abs(dens - ref).max() <= terms * 2.0 ** -37 + 2.0 ** -45 * ref.max()
