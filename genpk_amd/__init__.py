@@ -201,10 +201,11 @@ class Plan:
 
     def _outputs(self, nrbins, cross):
         t = self.torch
+        # every value is written by the binning
         f64 = dict(dtype=t.float64, device=self.device)
-        pw = [t.zeros(nrbins, **f64) for _ in range(3 if cross else 1)]
-        count = t.zeros(nrbins, dtype=t.int32, device=self.device)
-        keffs = t.zeros(nrbins, **f64)
+        pw = [t.empty(nrbins, **f64) for _ in range(3 if cross else 1)]
+        count = t.empty(nrbins, dtype=t.int32, device=self.device)
+        keffs = t.empty(nrbins, **f64)
         return pw, count, keffs
 
     def bin(self, nrbins=None, other=None, mass=1.0, other_mass=None):

@@ -383,45 +383,55 @@ __global__ void __launch_bounds__(BIN_THREADS) k_bin_stored(const typename Cx<T>
 }
 
 // Sum per-workgroup partials (fixed order) and normalise (powerspectrum.c:102-108).
-__global__ void k_bin_finish(int nrbins, int ns, int G, const double *__restrict__ part,
+// One workgroup per FIN_BINS bins and spectrum: FIN_SLICES threads per bin sum
+// a contiguous range of the partials each, eight loads in flight, and the
+// slices add in order.  (One thread per bin summing all G partials was a
+// chain of G / 8 memory round trips in one to four workgroups: 14 us for 256
+// partials, 26 for 512; this 4.)
+constexpr int FIN_BINS = 16, FIN_SLICES = 16;
+__global__ void __launch_bounds__(FIN_BINS * FIN_SLICES) k_bin_finish(int nrbins, int ns, int G, const double *__restrict__ part,
                              const int *__restrict__ count, const double *__restrict__ keffsum, double m_aa,
                              double m_bb, double m_ab, double *__restrict__ p_aa, double *__restrict__ p_bb,
                              double *__restrict__ p_ab, int *__restrict__ count_out, double *__restrict__ keffs_out) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nrbins) return;
-  // eight partials in flight per thread; each sum adds in the order gi = 0, 1, ...
-  double s[3] = {0, 0, 0};
+  __shared__ double sums[FIN_SLICES][FIN_BINS];
+  const int lb = threadIdx.x % FIN_BINS, sl = threadIdx.x / FIN_BINS;
+  const int b = blockIdx.x * FIN_BINS + lb, k = blockIdx.y;
   const int64_t gs = (int64_t)ns * nrbins;
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    if (k >= ns) break;
+  double acc = 0;
+  if (b < nrbins) {
     const double *pk = part + (int64_t)k * nrbins + b;
-    double acc = 0;
-    int gi = 0;
-    for (; gi + 8 <= G; gi += 8) {
+    const int per = (G + FIN_SLICES - 1) / FIN_SLICES;
+    const int g1 = min(G, (sl + 1) * per);
+    int gi = sl * per;
+    for (; gi + 8 <= g1; gi += 8) {
       double t[8];
 #pragma unroll
       for (int q = 0; q < 8; q++) t[q] = pk[(int64_t)(gi + q) * gs];
 #pragma unroll
       for (int q = 0; q < 8; q++) acc += t[q];
     }
-    for (; gi < G; gi++) acc += pk[(int64_t)gi * gs];
-    s[k] = acc;
+    for (; gi < g1; gi++) acc += pk[(int64_t)gi * gs];
   }
+  sums[sl][lb] = acc;
+  __syncthreads();
+  if (sl != 0 || b >= nrbins) return;
+  double s = 0;
+  for (int i = 0; i < FIN_SLICES; i++) s += sums[i][lb];
   const int c = count[b];
-  double *outs[3] = {p_aa, p_bb, p_ab};
-  const double ms[3] = {m_aa, m_bb, m_ab};
-  for (int k = 0; k < ns; k++) {
-    if (!outs[k]) continue;
+  double *out = k == 0 ? p_aa : k == 1 ? p_bb : p_ab;
+  const double m = k == 0 ? m_aa : k == 1 ? m_bb : m_ab;
+  if (out) {
     double v = 0;
     if (c) {
-      v = s[k] / ms[k];
+      v = s / m;
       v /= c;
     }
-    outs[k][b] = v;
+    out[b] = v;
   }
-  if (count_out) count_out[b] = c;
-  if (keffs_out) keffs_out[b] = c ? keffsum[b] / c : 0.0;
+  if (k == 0) {
+    if (count_out) count_out[b] = c;
+    if (keffs_out) keffs_out[b] = c ? keffsum[b] / c : 0.0;
+  }
 }
 
 }  // namespace
@@ -717,7 +727,7 @@ void bin_spectra(Plan &a, Plan *b, int nrbins, bool fused_xpass, double *pow_aa,
       if (b) launch_stored<double, 2>(a, b, bt, part, G); else launch_stored<double, 1>(a, b, bt, part, G);
     }
   }
-  hipLaunchKernelGGL(k_bin_finish, dim3((unsigned)ceil_div(nrbins, 256)), dim3(256), 0, a.stream, nrbins, ns, G, part,
+  hipLaunchKernelGGL(k_bin_finish, dim3((unsigned)ceil_div(nrbins, FIN_BINS), (unsigned)ns), dim3(FIN_BINS * FIN_SLICES), 0, a.stream, nrbins, ns, G, part,
                      bt.count.as<int>(), bt.keffsum.as<double>(), b ? ma * ma : ma * mb, mb * mb, ma * mb, pow_aa,
                      b ? pow_bb : (double *)nullptr, b ? pow_ab : (double *)nullptr, count, keffs);
   GENPK_LAUNCH_CHECK();
