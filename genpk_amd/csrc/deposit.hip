@@ -10,9 +10,8 @@
 //    split; their items write their raw accumulators as partial tiles, which a
 //    reduction sums exactly (fixed point) whatever records formed each item.
 // 3. Fold.  Grid cell values are assembled from the tile store by adding the
-//    halo cells of the previous tiles onto each tile's low faces: y and x
-//    halos in place after the deposit (k_fold_axis), z halos by the readers
-//    (the transform's z pass while loading, export with fold_value).
+//    halo cells of the previous tiles onto each tile's low faces, by the
+//    readers while they load (the transform's z pass, the export; tiles.h).
 //
 // Per-particle index and weight arithmetic follows fieldize.cpp:63-92:
 // u = (double)pos * (d/box); i0 = floor(u) wrapped into [0,d), i1 = i0+1
@@ -426,59 +425,63 @@ __global__ void __launch_bounds__(256) k_poison(const float *__restrict__ rec, i
   }
 }
 
-// In-place halo folds along y, then x.  fold_y: one workgroup per tile t adds
-// the y-halo rows (local y = width of the previous tile along y) of that
-// tile into t's rows at local y = 0, for every local x including t's x-halo
-// row, and for the z-halo plane entries of those rows, zeroing the sources.
-// fold_x then adds the previous tile along x's x-halo rows (every local y)
-// into t's rows at local x = 0.  Corner contributions travel through both
-// steps; z halos stay in place for the readers.  Each source row has one
-// destination and sources and destinations never coincide (a width is >= 1),
-// so workgroups do not race; zeroed sources let later deposits accumulate.
-template <typename Real, int AXIS>
-__global__ void __launch_bounds__(256) k_fold_axis(Real *__restrict__ tiles, FoldGeom P) {
-  const int64_t t = blockIdx.x;
-  const int tz = (int)(t % P.ntz);
-  const int ty = (int)((t / P.ntz) % P.nty);
-  const int tx = (int)(t / ((int64_t)P.ntz * P.nty));
-  const int HX = P.TX + 1;
-  int64_t src;
-  int h;
-  if (AXIS == 1) {
-    const int typ = ty == 0 ? P.nty - 1 : ty - 1;
-    h = min(P.TY, P.d - typ * P.TY);
-    src = ((int64_t)tx * P.nty + typ) * P.ntz + tz;
-  } else {
-    const int txp = tx == 0 ? P.ntx - 1 : tx - 1;
-    h = min(P.TX, P.d - txp * P.TX);
-    src = ((int64_t)txp * P.nty + ty) * P.ntz + tz;
+// Fold the halo'd tiles into a padded real grid [d][d][out_rowlen].  Each
+// thread takes pairs of cells along z (one tile row holds both: tile edges
+// are even), FOLD_UNR of them in flight; VEC: pairs are stored as one 8- or
+// 16-byte word (even row length, aligned out).  (One cell per thread with
+// two workgroups per line and 64-bit index divisions ran at 1.4 TB/s: 0.32 ->
+// 0.10 ms at 384^3 FP32.)
+constexpr int FOLD_UNR = 4;
+template <typename Real, bool VEC>
+__global__ void __launch_bounds__(FOLD_THREADS) k_fold(const Real *__restrict__ tiles, FoldGeom P, FastDiv fnp,
+                                                       int64_t out_rowlen, int accumulate, Real *__restrict__ out) {
+  using C = typename Cx<Real>::C;
+  const int x = blockIdx.y;
+  const int np = (P.d + 1) / 2;  // pairs per line
+  const uint32_t total = (uint32_t)P.d * (uint32_t)np;
+  const uint32_t i0 = blockIdx.x * (FOLD_THREADS * FOLD_UNR) + threadIdx.x;
+  C v[FOLD_UNR];
+  Real zh[FOLD_UNR];
+#pragma unroll
+  for (int u = 0; u < FOLD_UNR; u++) {
+    const uint32_t i = i0 + u * FOLD_THREADS;
+    v[u] = C{0, 0};
+    zh[u] = 0;
+    if (i < total) {
+      const int y = (int)fnp.div(i), z = 2 * (int)(i - (uint32_t)y * (uint32_t)np);
+      const RowFold rf = row_fold(P, x, y);
+      const ZPlace zp = z_place(P, z);
+      const int64_t at = row_at(P, rf.t, rf.r, zp);
+      v[u] = C{tiles[at], tiles[at + 1]};
+      if (zp.halo) zh[u] = tiles[row_halo_at(P, rf.t, rf.r, zp)];
+    }
   }
-  // rows: AXIS 1 -> (lx, h) onto (lx, 0), lx < HX; AXIS 0 -> (h, ly) onto (0, ly), ly < HY
-  const int nrows = AXIS == 1 ? HX : P.HY;
-  const int per_row = P.TZ + 1;  // TZ row values, then the z-halo plane entry
-  for (int i = threadIdx.x; i < nrows * per_row; i += 256) {
-    const int r = i / per_row, z = i - r * per_row;
-    const int sl = AXIS == 1 ? r * P.HY + h : h * P.HY + r;   // source row (lx*HY + ly)
-    const int dl = AXIS == 1 ? r * P.HY : r;                    // destination row
-    const int64_t sa = z < P.TZ ? src * P.cm + (int64_t)sl * P.TZ + z : P.zoff + src * P.cz + sl;
-    const int64_t da = z < P.TZ ? t * P.cm + (int64_t)dl * P.TZ + z : P.zoff + t * P.cz + dl;
-    const Real v = tiles[sa];
-    tiles[sa] = (Real)0;
-    tiles[da] = (Real)((double)tiles[da] + (double)v);
+#pragma unroll
+  for (int u = 0; u < FOLD_UNR; u++) {
+    const uint32_t i = i0 + u * FOLD_THREADS;
+    if (i >= total) continue;
+    const int y = (int)fnp.div(i), z = 2 * (int)(i - (uint32_t)y * (uint32_t)np);
+    const RowFold rf = row_fold(P, x, y);
+    if (rf.fx || rf.fy) {
+      C w[1] = {v[u]};
+      Real wh[1] = {zh[u]};
+      add_halo_rows<Real, 1, 1>(tiles, P, rf, [&](int) { return z; }, w, wh);
+      v[u] = w[0];
+      zh[u] = wh[0];
+    }
+    Real *o = out + ((int64_t)x * P.d + y) * out_rowlen + z;
+    const bool two = z + 1 < P.d;
+    C prev = C{0, 0};
+    if (accumulate) prev = VEC && two ? *reinterpret_cast<const C *>(o) : C{o[0], two ? o[1] : (Real)0};
+    // one rounding of own cell + z halo (+ previous value)
+    const C s = C{(Real)((double)prev.x + ((double)v[u].x + (double)zh[u])), (Real)((double)prev.y + (double)v[u].y)};
+    if (VEC && two) {
+      *reinterpret_cast<C *>(o) = s;
+    } else {
+      o[0] = s.x;
+      if (two) o[1] = s.y;
+    }
   }
-}
-
-// Fold the halo'd tiles into a padded real grid [d][d][out_rowlen].
-template <typename Real, typename Out>
-__global__ void __launch_bounds__(FOLD_THREADS) k_fold(const Real *__restrict__ tiles, FoldGeom P, int64_t out_rowlen,
-                                                       int accumulate, Out *__restrict__ out) {
-  const int64_t line = blockIdx.y + (int64_t)blockIdx.z * gridDim.y;  // x*d + y
-  const int z = blockIdx.x * FOLD_THREADS + threadIdx.x;
-  if (z >= P.d || line >= (int64_t)P.d * P.d) return;
-  const int x = (int)(line / P.d), y = (int)(line % P.d);
-  const double v = fold_value(tiles, P, x, y, z);
-  Out *o = out + line * out_rowlen + z;
-  *o = accumulate ? (Out)((double)*o + v) : (Out)v;
 }
 
 // Persistent grid of the deposit: the workgroups that stay resident (one
@@ -565,24 +568,6 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
     else
       hipLaunchKernelGGL(k_poison<double>, dim3(grid), dim3(256), 0, s, sorted, o.rw, o.list, kg, fg, P.nonfinite,
                          p.tiles.as<double>());
-    GENPK_LAUNCH_CHECK();
-  }
-  {
-    Stage st(p, "fold_y");
-    const FoldGeom fg = fold_geom(p);
-    if (p.prec == 4)
-      hipLaunchKernelGGL((k_fold_axis<float, 1>), dim3((unsigned)tg.K), dim3(256), 0, s, p.tiles.as<float>(), fg);
-    else
-      hipLaunchKernelGGL((k_fold_axis<double, 1>), dim3((unsigned)tg.K), dim3(256), 0, s, p.tiles.as<double>(), fg);
-    GENPK_LAUNCH_CHECK();
-  }
-  {
-    Stage st(p, "fold_x");
-    const FoldGeom fg = fold_geom(p);
-    if (p.prec == 4)
-      hipLaunchKernelGGL((k_fold_axis<float, 0>), dim3((unsigned)tg.K), dim3(256), 0, s, p.tiles.as<float>(), fg);
-    else
-      hipLaunchKernelGGL((k_fold_axis<double, 0>), dim3((unsigned)tg.K), dim3(256), 0, s, p.tiles.as<double>(), fg);
     GENPK_LAUNCH_CHECK();
   }
 }
@@ -681,17 +666,24 @@ void fold_tiles(Plan &p, void *out, int64_t out_rowlen, bool accumulate) {
     return;
   }
   const FoldGeom F = fold_geom(p);
-  const int64_t lines = p.d * p.d;
-  const unsigned gy = (unsigned)std::min<int64_t>(lines, 65535);
-  const unsigned gz = (unsigned)ceil_div(lines, gy);
-  dim3 grid((unsigned)ceil_div(p.d, FOLD_THREADS), gy, gz);
+  const int64_t np = (p.d + 1) / 2;
+  const dim3 grid((unsigned)ceil_div(p.d * np, FOLD_THREADS * FOLD_UNR), (unsigned)p.d);
+  const bool vec = out_rowlen % 2 == 0 && reinterpret_cast<uintptr_t>(out) % (2 * (size_t)p.prec) == 0;
+  const FastDiv fnp((uint32_t)np);
+  const int acc = accumulate ? 1 : 0;
   Stage st(p, "fold");
-  if (p.prec == 4)
-    hipLaunchKernelGGL((k_fold<float, float>), grid, dim3(FOLD_THREADS), 0, p.stream, p.tiles.as<float>(), F,
-                       out_rowlen, accumulate ? 1 : 0, static_cast<float *>(out));
+  if (p.prec == 4 && vec)
+    hipLaunchKernelGGL((k_fold<float, true>), grid, dim3(FOLD_THREADS), 0, p.stream, p.tiles.as<float>(), F, fnp,
+                       out_rowlen, acc, static_cast<float *>(out));
+  else if (p.prec == 4)
+    hipLaunchKernelGGL((k_fold<float, false>), grid, dim3(FOLD_THREADS), 0, p.stream, p.tiles.as<float>(), F, fnp,
+                       out_rowlen, acc, static_cast<float *>(out));
+  else if (vec)
+    hipLaunchKernelGGL((k_fold<double, true>), grid, dim3(FOLD_THREADS), 0, p.stream, p.tiles.as<double>(), F, fnp,
+                       out_rowlen, acc, static_cast<double *>(out));
   else
-    hipLaunchKernelGGL((k_fold<double, double>), grid, dim3(FOLD_THREADS), 0, p.stream, p.tiles.as<double>(), F,
-                       out_rowlen, accumulate ? 1 : 0, static_cast<double *>(out));
+    hipLaunchKernelGGL((k_fold<double, false>), grid, dim3(FOLD_THREADS), 0, p.stream, p.tiles.as<double>(), F, fnp,
+                       out_rowlen, acc, static_cast<double *>(out));
   GENPK_LAUNCH_CHECK();
 }
 
