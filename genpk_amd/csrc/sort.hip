@@ -78,8 +78,9 @@ struct InMap {
 // workgroup w's of bucket s; its range starts at block (first slot >> lg) +
 // (w + s) (nb + 1).
 struct PgOut {
-  uint32_t *hdr = nullptr;    // of each taken block: digit | (its number among the piece's blocks of the digit) << 11
+  uint16_t *hdr = nullptr;    // digit of each taken block, written with the block's first record
   uint32_t *cnt = nullptr;    // [pieces * nb] records per digit of each piece (written where not 0)
+  uint32_t *last = nullptr;   // [pieces * nb] the digit's last block (the one that may be partly filled)
   uint32_t *base = nullptr;   // [pieces * nb] number of the piece's first block among its bucket's
   uint4 *piece = nullptr;     // first block, blocks taken, bucket (blocks taken: 0 where there is no piece)
   unsigned long long *tot = nullptr;  // per output bucket: blocks << 32 | records, summed over the pieces
@@ -407,11 +408,7 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__re
           const uint32_t lr = run & 0xffffu, first = blk0 + taken + (run >> 16);
           // the first part is used only when a > 0, i.e. the block is open
           dinfo[dg] = make_uint4(lr, lr + a, ((f ? dblk[dg] : 0u) << pg.lg) + f - lr, (first << pg.lg) - (lr + a));
-          if (need) {
-            const uint32_t nd = (c0 + pb - 1) >> pg.lg;
-            for (uint32_t k = 0; k < need; k++) pg.hdr[first + k] = (uint32_t)dg | (nd + k) << 11;
-            dblk[dg] = first + need - 1;
-          }
+          if (need) dblk[dg] = first + need - 1;
           dcnt[dg] = c0 + tot;
         }
       } else {
@@ -460,7 +457,12 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__re
     load_sub(s1, npe);
     __syncthreads();
     auto put = [&](int p) {
-      const uint32_t dest = dest_of((uint32_t)p, sdig[p]);
+      const uint32_t sd = sdig[p], dest = dest_of((uint32_t)p, sd);
+      // a block's first record names its digit (one thread per digit naming
+      // all its new blocks was a serial loop of up to 512 stores where a
+      // sub-chunk's records share few digits: 57 -> 32 us for 1.2e6 clumped
+      // records in 637 tiles)
+      if (PAGED && (dest & (pb - 1)) == 0) pg.hdr[dest >> pg.lg] = (uint16_t)sd;
       float v[RW];
 #pragma unroll
       for (int k = 0; k < RW; k++) v[k] = stage[p * RW + k];
@@ -486,6 +488,7 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__re
         const unsigned long long add = (unsigned long long)((c + pb - 1) >> pg.lg) << 32 | c;
         const int64_t at = (int64_t)p * nb + dg;
         pg.cnt[at] = c;
+        pg.last[at] = dblk[dg];
         pg.base[at] = (uint32_t)(atomicAdd(&pg.tot[(int64_t)seg * nb + dg], add) >> 32);
       }
       if (threadIdx.x == 0) pg.piece[p] = make_uint4(blk0, taken, seg, 0u);
@@ -646,18 +649,22 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
 }
 
 // The block list: bucket k's blocks from list entry start[k] on, each piece's
-// of a digit in the order it took them.  One workgroup per piece.
+// of a digit side by side in any order.  One workgroup per piece.
 __global__ void __launch_bounds__(SORT_THREADS) k_list(PgOut pg, int nb, const uint32_t *__restrict__ start,
                                                        uint32_t *__restrict__ blist) {
+  extern __shared__ uint32_t lcnt[];  // [nb]
   const int64_t p = blockIdx.x;
   const uint4 pc = pg.piece[p];
+  if (pc.y == 0) return;
+  for (int i = threadIdx.x; i < nb; i += SORT_THREADS) lcnt[i] = 0;
+  __syncthreads();
   const int64_t bucket0 = (int64_t)pc.z * nb;
   for (uint32_t k = threadIdx.x; k < pc.y; k += SORT_THREADS) {
-    const uint32_t blk = pc.x + k;
-    const uint32_t h = pg.hdr[blk], d = h & 2047u, j = h >> 11;
+    const uint32_t blk = pc.x + k, d = pg.hdr[blk];
     const int64_t at = p * nb + d;
-    const uint32_t fill = min(1u << pg.lg, pg.cnt[at] - (j << pg.lg));
-    blist[start[bucket0 + d] + pg.base[at] + j] = pg_entry(blk, fill, pg.lg);
+    const uint32_t part = pg.cnt[at] & ((1u << pg.lg) - 1);
+    const uint32_t fill = part && blk == pg.last[at] ? part : 1u << pg.lg;
+    blist[start[bucket0 + d] + pg.base[at] + atomicAdd(&lcnt[d], 1u)] = pg_entry(blk, fill, pg.lg);
   }
 }
 
@@ -788,19 +795,21 @@ bool first_paged(const Plan &p, int64_t n) {
   return n >= cus * nhi * 128;
 }
 
-// Workspace of a paged pass in one buffer: pieces, headers, per-piece counts
-// and bases, and the block list.
+// Workspace of a paged pass in one buffer: pieces, per-piece counts, last
+// blocks and bases, the block list and the blocks' digits.
 uint32_t *pg_buffers(DevBuf &buf, const PgLayout &L, int nb, PgOut &pg, unsigned long long *tot) {
   const size_t blocks = (size_t)L.blocks, wd = (size_t)L.pieces * nb;
   GENPK_REQUIRE((uint64_t)L.slots() <= ((uint64_t)1 << 32), "sort pool too large");
-  uint32_t *b = static_cast<uint32_t *>(buf.ensure((4 * (size_t)L.pieces + 2 * blocks + 2 * wd) * 4));
+  uint32_t *b = static_cast<uint32_t *>(buf.ensure((4 * (size_t)L.pieces + 3 * wd + blocks + (blocks + 1) / 2) * 4));
   pg.piece = reinterpret_cast<uint4 *>(b);
-  pg.hdr = b + 4 * L.pieces;
-  pg.cnt = pg.hdr + blocks;
-  pg.base = pg.cnt + wd;
+  pg.cnt = b + 4 * L.pieces;
+  pg.last = pg.cnt + wd;
+  pg.base = pg.last + wd;
+  uint32_t *blist = pg.base + wd;
+  pg.hdr = reinterpret_cast<uint16_t *>(blist + blocks);
   pg.tot = tot;
   pg.lg = L.lg;
-  return pg.base + wd;  // the block list
+  return blist;
 }
 
 void launch_dir(const DirArgs &D, hipStream_t s) {
@@ -915,7 +924,7 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
       D.unit = (uint32_t)(S.L2.chunk >> S.L1.lg);
       D.funit = FastDiv(D.unit);
       launch_dir(D, s);
-      hipLaunchKernelGGL(k_list, dim3((unsigned)S.L1.pieces), dim3(SORT_THREADS), 0, s, pg1, nhi, D.start, blist1);
+      hipLaunchKernelGGL(k_list, dim3((unsigned)S.L1.pieces), dim3(SORT_THREADS), nhi * 4, s, pg1, nhi, D.start, blist1);
       GENPK_LAUNCH_CHECK();
       list1 = blist1;
       im2.lg = S.L1.lg;
@@ -978,7 +987,7 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   {
     Stage st(p, "sort_tiles");
     launch_dir(D, s);
-    hipLaunchKernelGGL(k_list, dim3((unsigned)S.L2.pieces), dim3(SORT_THREADS), 0, s, pg2, S.two ? nlo : nhi,
+    hipLaunchKernelGGL(k_list, dim3((unsigned)S.L2.pieces), dim3(SORT_THREADS), (S.two ? nlo : nhi) * 4, s, pg2, S.two ? nlo : nhi,
                        D.start, blist);
     GENPK_LAUNCH_CHECK();
   }
