@@ -64,6 +64,43 @@ struct AdjWeight {
   }
 };
 
+// The adjoint weight from LDS: the per-bin factors 2 lambda_b / (M^2 C_b), the
+// window factors and the bin thresholds, so that a mode's weight costs no
+// global read and no division.
+struct LdsWeight {
+  double *sfb;  // [nrbins]
+  float *swt;   // [d]
+  int *sthr;    // [nrbins + 1]
+  int nrbins;
+  float lq;
+  static size_t bytes(int64_t d, int nrbins) { return (size_t)nrbins * 8 + (size_t)d * 4 + (size_t)(nrbins + 1) * 4; }
+  // fill the tables (16-byte aligned at) with the whole workgroup; no barrier
+  __device__ __forceinline__ void init(void *at, const AdjWeight &w, int64_t d) {
+    sfb = static_cast<double *>(at);
+    swt = reinterpret_cast<float *>(sfb + w.nrbins);
+    sthr = reinterpret_cast<int *>(swt + d);
+    nrbins = w.nrbins;
+    lq = w.lq;
+    for (int i = threadIdx.x; i < w.nrbins; i += blockDim.x) {
+      const int c = w.count[i];
+      sfb[i] = c ? 2.0 * w.lambda[i] * w.inv_m2 / (double)c : 0.0;
+    }
+    for (int i = threadIdx.x; i < d; i += blockDim.x) swt[i] = w.wtab[i];
+    for (int i = threadIdx.x; i <= w.nrbins; i += blockDim.x) sthr[i] = (int)w.thr[i];
+  }
+  // weight of array index xi along x of a column with a = ky^2 + kz^2 and
+  // window factors wy, wz; bt tracks the bin along the column
+  __device__ __forceinline__ double at(int xi, int n, int a, float wy, float wz, BinTrackLds &bt) const {
+    const int kx = xi <= n / 2 ? xi : xi - n;
+    const int qk = a + kx * kx;
+    if (qk == 0) return 0.0;
+    const float gw = (swt[xi] * wy) * wz;  // the forward's ((wx*wy)*wz) in float
+    double g = (double)gw * (double)gw;
+    g *= g;
+    return g * sfb[bt.of(qk, sthr, nrbins, lq)];
+  }
+};
+
 template <typename T>
 __global__ void k_weight(typename Cx<T>::C *__restrict__ f, int64_t d, int64_t hz, AdjWeight w) {
   using C = typename Cx<T>::C;
@@ -81,10 +118,12 @@ __global__ void k_weight(typename Cx<T>::C *__restrict__ f, int64_t d, int64_t h
 // per column block (fixed y, B consecutive kz), forward length-d FFT along
 // x, multiply by the adjoint weight, inverse FFT, store back.  One block
 // per workgroup, the stages in place in one LDS buffer (k_adjoint_x_pp
-// covers the usual shapes).
-template <typename T>
+// covers the usual shapes).  LW: the weight from LDS tables (where they fit
+// beside the columns; with six global reads and a division per mode the pass
+// took 0.27 ms at 360^3 FP32, with the tables 0.24).
+template <typename T, bool LW>
 __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__restrict__ f, int64_t d, int64_t hz,
-                                                          int lgb, int nkb, RadixPlan rp,
+                                                          int lgb, int nkb, FastDiv fnkb, RadixPlan rp,
                                                           const typename Cx<T>::C *__restrict__ tw, AdjWeight w) {
   using C = typename Cx<T>::C;
   constexpr int MAXE = AdjCfg<T>::MAXE;
@@ -93,30 +132,43 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
   const int n = rp.n;
   const int B = 1 << lgb;
   const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-  const int64_t y = blk / nkb;
-  const int kb = (int)(blk - y * nkb);
-  const int64_t kz0 = (int64_t)kb * B;
+  const uint32_t yb = fnkb.div(blk);
+  const int64_t y = yb;
+  const int64_t kz0 = (int64_t)(blk - yb * (uint32_t)nkb) * B;
   const int nb = (int)min((int64_t)B, hz - kz0);
   const int64_t estride = d * hz;
   C *base = f + y * hz + kz0;
   const int tot = n * B;
+  C v[MAXE];
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
     const int i = threadIdx.x + q * ADJ_THREADS;
     const int e = i >> lgb, b = i & (B - 1);
-    if (i < tot) buf[i] = b < nb ? base[e * estride + b] : C{0, 0};
+    v[q] = i < tot && b < nb ? base[e * estride + b] : C{0, 0};
+  }
+#pragma unroll
+  for (int q = 0; q < MAXE; q++) {
+    const int i = threadIdx.x + q * ADJ_THREADS;
+    if (i < tot) buf[i] = v[q];
   }
   C *stw = buf + tot;
   for (int i = threadIdx.x; i < n; i += ADJ_THREADS) stw[i] = tw[i];
+  LdsWeight lw;
+  if constexpr (LW) lw.init(stw + n, w, d);
   __syncthreads();
   lds_fft<-1, true, MAXE>(buf, rp, B, lgb, B, 1, stw);
   __syncthreads();
-  for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
-    const int e = i >> lgb, b = i & (B - 1);
-    if (b < nb) {
-      const double s = w.at(e, y, kz0 + b, d);
-      const C a = buf[i];
-      buf[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
+  {
+    // ADJ_THREADS is a multiple of B: a thread's elements lie in one column
+    const int b = threadIdx.x & (B - 1), kz = (int)kz0 + b, ky = (int)kv(y, d);
+    BinTrackLds bt;
+    for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
+      const int e = i >> lgb;
+      if (b < nb) {
+        const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[y], lw.swt[kz], bt) : w.at(e, y, kz, d);
+        const C a = buf[i];
+        buf[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
+      }
     }
   }
   __syncthreads();
@@ -134,13 +186,11 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
 // stage runs from the loaded registers, the stages alternate between two
 // LDS buffers (one barrier each), and the next block's loads are in flight
 // during this block's inverse transform and stores.
-// LT (a last radix 2): the last forward stage runs in registers with the
-// weight; the per-bin factors 2 lambda_b / (M^2 C_b), the window factors
-// and the bin thresholds are staged in LDS, and each thread's modes find
-// their bin by tracking the thresholds along kx, so a mode's weight costs
-// no global read and no division.  (Compile-time stages for n = 1024 spill
+// LW: the weight from LDS tables.  LT (with LW, a last radix 2): the last forward stage runs in registers with the
+// weight (LdsWeight), and each thread's modes find their bin by tracking the
+// thresholds along kx.  (Compile-time stages for n = 1024 spill
 // registers here: 5.2 -> 7.3 ms at 1024^3, against 4.3 ms without.)
-template <typename T, bool LT>
+template <typename T, bool LT, bool LW>
 __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C *__restrict__ f, int64_t d,
                                                              int64_t hz, int lgb, int nkb, FastDiv fnkb, RadixPlan rp,
                                                              const typename Cx<T>::C *__restrict__ tw, AdjWeight w) {
@@ -154,17 +204,8 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
   C *buf2 = buf + tot;
   C *stw = buf2 + tot;
   for (int i = threadIdx.x; i < n; i += ADJ_THREADS) stw[i] = tw[i];
-  double *sfb = reinterpret_cast<double *>(stw + n);  // [nrbins]
-  float *swt = reinterpret_cast<float *>(sfb + w.nrbins);  // [d]
-  int *sthr = reinterpret_cast<int *>(swt + d);  // [nrbins + 1]
-  if constexpr (LT) {
-    for (int i = threadIdx.x; i < w.nrbins; i += ADJ_THREADS) {
-      const int c = w.count[i];
-      sfb[i] = c ? 2.0 * w.lambda[i] * w.inv_m2 / (double)c : 0.0;
-    }
-    for (int i = threadIdx.x; i < d; i += ADJ_THREADS) swt[i] = w.wtab[i];
-    for (int i = threadIdx.x; i <= w.nrbins; i += ADJ_THREADS) sthr[i] = (int)w.thr[i];
-  }
+  LdsWeight lw;
+  if constexpr (LW) lw.init(stw + n, w, d);
   const int64_t estride = d * hz;
   const int64_t nblk = d * nkb;
   const int b = threadIdx.x & (B - 1);
@@ -210,17 +251,8 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
       // each keep a bin tracker along their run
       const int kz = (int)kz0 + b, ky = (int)kv(y, d);
       const int a = ky * ky + kz * kz;
-      const float wy = swt[y], wz = swt[min(kz, (int)d - 1)];
+      const float wy = lw.swt[y], wz = lw.swt[min(kz, (int)d - 1)];
       BinTrackLds t0, t1;
-      auto lds_weight = [&](int xi, BinTrackLds &bt) -> double {
-        const int kx = xi <= half ? xi : xi - n;
-        const int qk = a + kx * kx;
-        if (qk == 0) return 0.0;
-        const float gw = (swt[xi] * wy) * wz;  // the forward's ((wx*wy)*wz) in float
-        double g = (double)gw * (double)gw;
-        g *= g;
-        return g * sfb[bt.of(qk, sthr, w.nrbins, w.lq)];
-      };
 #pragma unroll
       for (int q = 0; q < HB; q++) {
         const int jj = jb + q;
@@ -228,8 +260,8 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
         const C v1 = cmul(x[(jj + half) * B + b], stw[jj]);
         C o0 = cadd(a0, v1), o1 = csub(a0, v1);
         if (b < nb) {
-          const double s0 = lds_weight(jj, t0);
-          const double s1 = lds_weight(jj + half, t1);
+          const double s0 = lw.at(jj, n, a, wy, wz, t0);
+          const double s1 = lw.at(jj + half, n, a, wy, wz, t1);
           o0 = C{(T)((double)o0.x * s0), (T)((double)o0.y * s0)};
           o1 = C{(T)((double)o1.x * s1), (T)((double)o1.y * s1)};
         }
@@ -238,10 +270,12 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
       }
     } else {
       res = lds_fft_pp<-1, true, MAXE>(buf2, buf, rp, B, lgb, B, 1, stw, 1);
+      const int kz = (int)kz0 + b, ky = (int)kv(y, d);
+      BinTrackLds bt;
       for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
         const int e = i >> lgb;
         if (b < nb) {
-          const double s = w.at(e, y, kz0 + b, d);
+          const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[y], lw.swt[kz], bt) : w.at(e, y, kz, d);
           const C a = res[i];
           res[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
         }
@@ -459,36 +493,50 @@ void adjoint_x_impl(Plan &p, const AdjWeight &w) {
   using C = typename Cx<T>::C;
   const int B = col_block(p.prec, p.d, p.hz);
   const int nkb = (int)ceil_div(p.hz, B);
-  const RadixPlan &rp = p.rp_d;
   const C *tw = (p.prec == 4) ? (const C *)p.fft.tw_d_f32.ptr : (const C *)p.fft.tw_d_f64.ptr;
-  GENPK_REQUIRE((int64_t)p.d * B <= (int64_t)AdjCfg<T>::MAXE * ADJ_THREADS, "adjoint x pass: column block too large");
-  Stage st(p, "adjoint_x");
   const int64_t tot = p.d * B;
-  const bool pp = rp.st[0].R == AdjCfg<T>::MAXE && tot == (int64_t)ADJ_THREADS * AdjCfg<T>::MAXE &&
-                  (size_t)(2 * tot + p.d) * sizeof(C) <= 160 * 1024;
-  const dim3 grid((unsigned)(p.d * nkb));
-  // the LDS tables of the fused weight: per-bin factors, window factors, thresholds
-  const size_t lds_lt = (size_t)(2 * tot + p.d) * sizeof(C) + (size_t)w.nrbins * 8 + (size_t)p.d * 4 +
-                        (size_t)(w.nrbins + 1) * 4;
-  const bool lt = pp && rp.st[rp.nst - 1].R == 2 && w.nrbins >= 1 && lds_lt <= 160 * 1024;
+  GENPK_REQUIRE(tot <= (int64_t)AdjCfg<T>::MAXE * ADJ_THREADS, "adjoint x pass: column block too large");
+  Stage st(p, "adjoint_x");
+  const size_t lds_w = LdsWeight::bytes(p.d, w.nrbins), lds_pp = (size_t)(2 * tot + p.d) * sizeof(C), cap = 160 * 1024;
+  // the register first stage takes a plan of its length with a first radix of
+  // MAXE; FP32: one that also ends in a radix 2, where the plan's own (the
+  // column passes') does not (512 = 8 8 8 -> 8 8 4 2: 0.56 -> 0.48 ms at 512^3)
+  RadixPlan rp = p.rp_d;
+  auto last2 = [](const RadixPlan &r) { return r.st[r.nst - 1].R == 2; };
+  if (sizeof(T) == 4 && !(rp.st[0].R == 8 && last2(rp))) {
+    const RadixPlan xp = radix_plan_8_to_2((int)p.d);
+    if (xp.nst > 0) rp = xp;
+  }
+  const bool pp = rp.st[0].R == AdjCfg<T>::MAXE && tot == (int64_t)ADJ_THREADS * AdjCfg<T>::MAXE && lds_pp <= cap;
+  const bool lw = lds_pp + lds_w <= cap, lt = lw && last2(rp);
   if (pp) {
     // persistent: as many workgroups as stay resident, at most one per column block
     // (4.3 ms at 1024^3 against 5.2 ms for one workgroup per block)
-    const void *fn = lt ? reinterpret_cast<const void *>(&k_adjoint_x_pp<T, true>)
-                        : reinterpret_cast<const void *>(&k_adjoint_x_pp<T, false>);
-    const size_t lds = lt ? lds_lt : (size_t)(2 * tot + p.d) * sizeof(C);
+    const void *fn = lt   ? reinterpret_cast<const void *>(&k_adjoint_x_pp<T, true, true>)
+                     : lw ? reinterpret_cast<const void *>(&k_adjoint_x_pp<T, false, true>)
+                          : reinterpret_cast<const void *>(&k_adjoint_x_pp<T, false, false>);
+    const size_t lds = lw ? lds_pp + lds_w : lds_pp;
     int per_cu = 0;
     GENPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, ADJ_THREADS, lds));
     const dim3 g((unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), p.d * nkb)));
     if (lt)
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d, p.hz,
+      hipLaunchKernelGGL((k_adjoint_x_pp<T, true, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d, p.hz,
                          ilog2(B), nkb, FastDiv((uint32_t)nkb), rp, tw, w);
+    else if (lw)
+      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d,
+                         p.hz, ilog2(B), nkb, FastDiv((uint32_t)nkb), rp, tw, w);
     else
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, false>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d, p.hz,
-                         ilog2(B), nkb, FastDiv((uint32_t)nkb), rp, tw, w);
+      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, false>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d,
+                         p.hz, ilog2(B), nkb, FastDiv((uint32_t)nkb), rp, tw, w);
   } else {
-    hipLaunchKernelGGL((k_adjoint_x<T>), grid, dim3(ADJ_THREADS), (size_t)(tot + p.d) * sizeof(C), p.stream,
-                       p.field.as<C>(), p.d, p.hz, ilog2(B), nkb, rp, tw, w);
+    const dim3 grid((unsigned)(p.d * nkb));
+    const size_t lds = (size_t)(tot + p.d) * sizeof(C);
+    if (lds + lds_w <= cap)
+      hipLaunchKernelGGL((k_adjoint_x<T, true>), grid, dim3(ADJ_THREADS), lds + lds_w, p.stream, p.field.as<C>(), p.d,
+                         p.hz, ilog2(B), nkb, FastDiv((uint32_t)nkb), p.rp_d, tw, w);
+    else
+      hipLaunchKernelGGL((k_adjoint_x<T, false>), grid, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d, p.hz,
+                         ilog2(B), nkb, FastDiv((uint32_t)nkb), p.rp_d, tw, w);
   }
   GENPK_LAUNCH_CHECK();
 }
