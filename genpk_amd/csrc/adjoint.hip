@@ -120,31 +120,29 @@ __global__ void k_weight(typename Cx<T>::C *__restrict__ f, int64_t d, int64_t h
 // per workgroup, the stages in place in one LDS buffer (k_adjoint_x_pp
 // covers the usual shapes).  LW: the weight from LDS tables (where they fit
 // beside the columns; with six global reads and a division per mode the pass
-// took 0.27 ms at 360^3 FP32, with the tables 0.24).
+// took 0.27 ms at 360^3 FP32, with the tables 0.24, and
+// 0.15 with all loads in flight together and no 64-bit division).
 template <typename T, bool LW>
-__global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__restrict__ f, int64_t d, int64_t hz,
-                                                          int lgb, int nkb, FastDiv fnkb, RadixPlan rp,
+__global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__restrict__ f, ColMap cm, RadixPlan rp,
                                                           const typename Cx<T>::C *__restrict__ tw, AdjWeight w) {
   using C = typename Cx<T>::C;
   constexpr int MAXE = AdjCfg<T>::MAXE;
   extern __shared__ unsigned char lds_raw[];
   C *buf = reinterpret_cast<C *>(lds_raw);  // [n][B]
   const int n = rp.n;
-  const int B = 1 << lgb;
-  const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-  const uint32_t yb = fnkb.div(blk);
-  const int64_t y = yb;
-  const int64_t kz0 = (int64_t)(blk - yb * (uint32_t)nkb) * B;
-  const int nb = (int)min((int64_t)B, hz - kz0);
+  const int lgb = cm.lgb, B = 1 << lgb;
+  const int64_t d = cm.d, hz = cm.hz;
+  const ColMap::Block c = cm.at(xcd_block(blockIdx.x, gridDim.x));
   const int64_t estride = d * hz;
-  C *base = f + y * hz + kz0;
+  C *base = f + (int64_t)c.outer * hz + c.kz0;
+  // ADJ_THREADS is a multiple of B: a thread's elements lie in one column
+  const int b = threadIdx.x & (B - 1);
   const int tot = n * B;
   C v[MAXE];
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
     const int i = threadIdx.x + q * ADJ_THREADS;
-    const int e = i >> lgb, b = i & (B - 1);
-    v[q] = i < tot && b < nb ? base[e * estride + b] : C{0, 0};
+    v[q] = i < tot && b < c.nb ? base[(i >> lgb) * estride + b] : C{0, 0};
   }
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
@@ -158,17 +156,14 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
   __syncthreads();
   lds_fft<-1, true, MAXE>(buf, rp, B, lgb, B, 1, stw);
   __syncthreads();
-  {
-    // ADJ_THREADS is a multiple of B: a thread's elements lie in one column
-    const int b = threadIdx.x & (B - 1), kz = (int)kz0 + b, ky = (int)kv(y, d);
+  if (b < c.nb) {
+    const int ky = (int)kv(c.outer, d), kz = (int)c.kz0 + b;
     BinTrackLds bt;
     for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
       const int e = i >> lgb;
-      if (b < nb) {
-        const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[y], lw.swt[kz], bt) : w.at(e, y, kz, d);
-        const C a = buf[i];
-        buf[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
-      }
+      const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[c.outer], lw.swt[kz], bt) : w.at(e, c.outer, kz, d);
+      const C a = buf[i];
+      buf[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
     }
   }
   __syncthreads();
@@ -176,8 +171,7 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
     const int i = threadIdx.x + q * ADJ_THREADS;
-    const int e = i >> lgb, b = i & (B - 1);
-    if (i < tot && b < nb) base[e * estride + b] = buf[i];
+    if (i < tot && b < c.nb) base[(i >> lgb) * estride + b] = buf[i];
   }
 }
 
@@ -191,14 +185,14 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
 // thresholds along kx.  (Compile-time stages for n = 1024 spill
 // registers here: 5.2 -> 7.3 ms at 1024^3, against 4.3 ms without.)
 template <typename T, bool LT, bool LW>
-__global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C *__restrict__ f, int64_t d,
-                                                             int64_t hz, int lgb, int nkb, FastDiv fnkb, RadixPlan rp,
-                                                             const typename Cx<T>::C *__restrict__ tw, AdjWeight w) {
+__global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C *__restrict__ f, ColMap cm,
+                                                             RadixPlan rp, const typename Cx<T>::C *__restrict__ tw, AdjWeight w) {
   using C = typename Cx<T>::C;
   constexpr int MAXE = AdjCfg<T>::MAXE;
   extern __shared__ unsigned char lds_raw[];
   const int n = rp.n;
-  const int B = 1 << lgb;
+  const int lgb = cm.lgb, B = 1 << lgb;
+  const int64_t d = cm.d, hz = cm.hz;
   const int tot = n * B;
   C *buf = reinterpret_cast<C *>(lds_raw);  // [n][B]
   C *buf2 = buf + tot;
@@ -207,33 +201,25 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
   LdsWeight lw;
   if constexpr (LW) lw.init(stw + n, w, d);
   const int64_t estride = d * hz;
-  const int64_t nblk = d * nkb;
+  const int64_t nblk = cm.nblk;
   const int b = threadIdx.x & (B - 1);
   C v[MAXE];
   // column block vb's loads: the inputs of this thread's first-stage butterfly
   // (a grid that is a multiple of the XCD count keeps vb on this workgroup's XCD)
   auto load = [&](int64_t vb) {
-    const uint32_t blk = xcd_block((uint32_t)vb, (uint32_t)nblk);
-    const uint32_t yb = fnkb.div(blk);  // a multiply-high, not a division loop
-    const int64_t y = yb;
-    const int64_t kz0 = (int64_t)(blk - yb * (uint32_t)nkb) * B;
-    const int nb = (int)min((int64_t)B, hz - kz0);
-    const C *src = f + y * hz + kz0;
+    const ColMap::Block c = cm.at(xcd_block((uint32_t)vb, (uint32_t)nblk));
+    const C *src = f + (int64_t)c.outer * hz + c.kz0;
 #pragma unroll
     for (int q = 0; q < MAXE; q++) {
       const int i = threadIdx.x + q * ADJ_THREADS;
-      const int e = i >> lgb;
-      v[q] = b < nb ? src[e * estride + b] : C{0, 0};
+      v[q] = b < c.nb ? src[(i >> lgb) * estride + b] : C{0, 0};
     }
   };
   if ((int64_t)blockIdx.x < nblk) load(blockIdx.x);
   for (int64_t vb = blockIdx.x; vb < nblk; vb += gridDim.x) {
-    const uint32_t blk = xcd_block((uint32_t)vb, (uint32_t)nblk);
-    const uint32_t yb = fnkb.div(blk);
-    const int64_t y = yb;
-    const int64_t kz0 = (int64_t)(blk - yb * (uint32_t)nkb) * B;
-    const int nb = (int)min((int64_t)B, hz - kz0);
-    C *base = f + y * hz + kz0;
+    const ColMap::Block c = cm.at(xcd_block((uint32_t)vb, (uint32_t)nblk));
+    const int64_t y = c.outer;
+    C *base = f + y * hz + c.kz0;
     // the previous block's stores have read their buffer before this barrier
     fft_first_regs<MAXE, -1>(v, buf2, B, lgb, B, 1);
     __syncthreads();
@@ -249,7 +235,7 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
       const int jb = (threadIdx.x >> lgb) * HB;
       // modes jj (kx = jj) and jj + n/2 (kx = jj - n/2, kx = n/2 at jj = 0)
       // each keep a bin tracker along their run
-      const int kz = (int)kz0 + b, ky = (int)kv(y, d);
+      const int kz = (int)c.kz0 + b, ky = (int)kv(y, d);
       const int a = ky * ky + kz * kz;
       const float wy = lw.swt[y], wz = lw.swt[min(kz, (int)d - 1)];
       BinTrackLds t0, t1;
@@ -259,7 +245,7 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
         const C a0 = x[jj * B + b];
         const C v1 = cmul(x[(jj + half) * B + b], stw[jj]);
         C o0 = cadd(a0, v1), o1 = csub(a0, v1);
-        if (b < nb) {
+        if (b < c.nb) {
           const double s0 = lw.at(jj, n, a, wy, wz, t0);
           const double s1 = lw.at(jj + half, n, a, wy, wz, t1);
           o0 = C{(T)((double)o0.x * s0), (T)((double)o0.y * s0)};
@@ -270,11 +256,11 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
       }
     } else {
       res = lds_fft_pp<-1, true, MAXE>(buf2, buf, rp, B, lgb, B, 1, stw, 1);
-      const int kz = (int)kz0 + b, ky = (int)kv(y, d);
+      const int kz = (int)c.kz0 + b, ky = (int)kv(y, d);
       BinTrackLds bt;
       for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
         const int e = i >> lgb;
-        if (b < nb) {
+        if (b < c.nb) {
           const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[y], lw.swt[kz], bt) : w.at(e, y, kz, d);
           const C a = res[i];
           res[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
@@ -289,7 +275,7 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
     for (int q = 0; q < MAXE; q++) {
       const int i = threadIdx.x + q * ADJ_THREADS;
       const int e = i >> lgb;
-      if (b < nb) base[e * estride + b] = res[i];
+      if (b < c.nb) base[e * estride + b] = res[i];
     }
   }
 }
@@ -492,7 +478,7 @@ template <typename T>
 void adjoint_x_impl(Plan &p, const AdjWeight &w) {
   using C = typename Cx<T>::C;
   const int B = col_block(p.prec, p.d, p.hz);
-  const int nkb = (int)ceil_div(p.hz, B);
+  const ColMap cm = col_map(p.d, p.hz, B);
   const C *tw = (p.prec == 4) ? (const C *)p.fft.tw_d_f32.ptr : (const C *)p.fft.tw_d_f64.ptr;
   const int64_t tot = p.d * B;
   GENPK_REQUIRE(tot <= (int64_t)AdjCfg<T>::MAXE * ADJ_THREADS, "adjoint x pass: column block too large");
@@ -518,25 +504,20 @@ void adjoint_x_impl(Plan &p, const AdjWeight &w) {
     const size_t lds = lw ? lds_pp + lds_w : lds_pp;
     int per_cu = 0;
     GENPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, ADJ_THREADS, lds));
-    const dim3 g((unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), p.d * nkb)));
+    const dim3 g((unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), (int64_t)cm.nblk)));
     if (lt)
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, true, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d, p.hz,
-                         ilog2(B), nkb, FastDiv((uint32_t)nkb), rp, tw, w);
+      hipLaunchKernelGGL((k_adjoint_x_pp<T, true, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, rp, tw, w);
     else if (lw)
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d,
-                         p.hz, ilog2(B), nkb, FastDiv((uint32_t)nkb), rp, tw, w);
+      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, rp, tw, w);
     else
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, false>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d,
-                         p.hz, ilog2(B), nkb, FastDiv((uint32_t)nkb), rp, tw, w);
+      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, false>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, rp, tw, w);
   } else {
-    const dim3 grid((unsigned)(p.d * nkb));
+    const dim3 grid(cm.nblk);
     const size_t lds = (size_t)(tot + p.d) * sizeof(C);
     if (lds + lds_w <= cap)
-      hipLaunchKernelGGL((k_adjoint_x<T, true>), grid, dim3(ADJ_THREADS), lds + lds_w, p.stream, p.field.as<C>(), p.d,
-                         p.hz, ilog2(B), nkb, FastDiv((uint32_t)nkb), p.rp_d, tw, w);
+      hipLaunchKernelGGL((k_adjoint_x<T, true>), grid, dim3(ADJ_THREADS), lds + lds_w, p.stream, p.field.as<C>(), cm, p.rp_d, tw, w);
     else
-      hipLaunchKernelGGL((k_adjoint_x<T, false>), grid, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), p.d, p.hz,
-                         ilog2(B), nkb, FastDiv((uint32_t)nkb), p.rp_d, tw, w);
+      hipLaunchKernelGGL((k_adjoint_x<T, false>), grid, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, p.rp_d, tw, w);
   }
   GENPK_LAUNCH_CHECK();
 }

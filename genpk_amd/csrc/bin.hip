@@ -147,8 +147,8 @@ struct BinTrack {
 // that the next first stage never writes the buffer being binned.
 template <typename T, int NF, bool REG1, bool R2L = false, int CT = 0>
 __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__restrict__ fa,
-                                                            typename Cx<T>::C *__restrict__ fb, BinGeom g, int B,
-                                                            int nkb, FastDiv fnkb, RadixPlan rp,
+                                                            typename Cx<T>::C *__restrict__ fb, BinGeom g, ColMap cm,
+                                                            RadixPlan rp,
                                                             const typename Cx<T>::C *__restrict__ tw, int keep,
                                                             int pp, double *__restrict__ part) {
   using C = typename Cx<T>::C;
@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
   double *bins = reinterpret_cast<double *>(lds_raw);
   C *buf = reinterpret_cast<C *>(bins + ((NS * g.nrbins + 1) & ~1));  // [NF][n][B], 16-byte aligned
   const int n = CT ? CT : rp.n;
-  const int lgb = ilog2(B);
+  const int lgb = cm.lgb, B = 1 << lgb;
   // pp (one field): a second buffer lets the FFT stages alternate (one barrier each)
   C *buf2 = buf + (size_t)NF * n * B;
   C *stw = buf2 + (pp ? (size_t)n * B : 0);  // twiddles staged in LDS
@@ -170,7 +170,7 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
   for (int i = threadIdx.x; i < g.nrbins; i += BIN_THREADS) thr32[i] = (int)g.thr[i];
   const int64_t d = g.d, hz = g.hz;
   const int64_t estride = d * hz;
-  const int64_t nblk = d * nkb;
+  const int64_t nblk = cm.nblk;
   // bin-phase mapping: thread -> column b, contiguous run of e
   const int tpc = BIN_THREADS / B;               // threads per column (B divides BIN_THREADS)
   const int my_b = threadIdx.x % B;
@@ -185,32 +185,24 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
   C va[MAXE], vb[NF == 2 ? MAXE : 1];
   auto load = [&](int64_t v) {
     // a grid that is a multiple of the XCD count keeps v on this workgroup's XCD
-    const uint32_t blk = xcd_block((uint32_t)v, (uint32_t)nblk);
-    const uint32_t yb = fnkb.div(blk);  // 32-bit: a 64-bit division costs ~130 scalar instructions
-    const int64_t y = yb;
-    const int64_t kz0 = (int64_t)(blk - yb * (uint32_t)nkb) * B;
-    const int nb = (int)min((int64_t)B, hz - kz0);
-    const int64_t off = y * hz + kz0;
+    const ColMap::Block c = cm.at(xcd_block((uint32_t)v, (uint32_t)nblk));
+    const int64_t off = (int64_t)c.outer * hz + c.kz0;
 #pragma unroll
     for (int q = 0; q < MAXE; q++) {
       const int i = threadIdx.x + q * lst;
-      const int e = i >> lgb, b = i & (B - 1);
-      const bool ok = loader && i < tot && b < nb;
-      va[q] = ok ? fa[off + e * estride + b] : C{0, 0};
-      if (NF == 2) vb[NF == 2 ? q : 0] = ok ? fb[off + e * estride + b] : C{0, 0};
+      const int e = i >> lgb;  // of column my_b
+      const bool ok = loader && i < tot && my_b < c.nb;
+      va[q] = ok ? fa[off + e * estride + my_b] : C{0, 0};
+      if (NF == 2) vb[NF == 2 ? q : 0] = ok ? fb[off + e * estride + my_b] : C{0, 0};
     }
   };
   // block v + gridDim.x loads into the registers while block v is binned
   // (their live range misses the FFT stages, where the registers peak)
   if ((int64_t)blockIdx.x < nblk) load(blockIdx.x);
   for (int64_t v = blockIdx.x; v < nblk; v += gridDim.x) {
-    const uint32_t blk = xcd_block((uint32_t)v, (uint32_t)nblk);
-    const uint32_t yb = fnkb.div(blk);
-    const int64_t y = yb;
-    const int kb = (int)(blk - yb * (uint32_t)nkb);
-    const int64_t kz0 = (int64_t)kb * B;
-    const int nb = (int)min((int64_t)B, hz - kz0);
-    const int64_t off = y * hz + kz0;
+    const ColMap::Block c = cm.at(xcd_block((uint32_t)v, (uint32_t)nblk));
+    const int64_t y = c.outer;
+    const int64_t off = y * hz + c.kz0;
     C *res = buf;
     if constexpr (REG1) {
       if (loader) fft_first_regs<MAXE, -1>(va, buf2, B, lgb, B, 1);
@@ -239,16 +231,16 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
     }
     if (keep) {
       for (int i = threadIdx.x; i < n * B; i += BIN_THREADS) {
-        const int e = i >> lgb, b = i & (B - 1);
-        if (b < nb) {
-          fa[off + e * estride + b] = res[i];
-          if (NF == 2) fb[off + e * estride + b] = res[n * B + i];
+        const int e = i >> lgb;  // of column my_b
+        if (my_b < c.nb) {
+          fa[off + e * estride + my_b] = res[i];
+          if (NF == 2) fb[off + e * estride + my_b] = res[n * B + i];
         }
       }
     }
     if (v + gridDim.x < nblk) load(v + gridDim.x);
-    if (my_b < nb) {
-      const int kz = (int)(kz0 + my_b);
+    if (my_b < c.nb) {
+      const int kz = (int)c.kz0 + my_b;
       const int ky = (int)kval(y, d);
       const double h = (kz == 0 || kz == d / 2) ? 1.0 : 2.0;
       const int a = ky * ky + kz * kz;
@@ -284,9 +276,9 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
             const float gw = (wt[e] * wy) * wz;  // the reference's ((wx*wy)*wz) in float
             double dc = (double)gw * (double)gw;
             dc *= dc;
-            double c[3];
-            mode_terms<C, NF>(mo[q], mo[q], h, dc, c);
-            run_add<NS>(r, bn, c, bins, g.nrbins);
+            double t[3];
+            mode_terms<C, NF>(mo[q], mo[q], h, dc, t);
+            run_add<NS>(r, bn, t, bins, g.nrbins);
           }
         }
         }
@@ -318,9 +310,9 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
             dc *= dc;
             const C fa_m = BATCH ? ma[BATCH ? j : 0] : res[e * B + my_b];
             const C fb_m = NF == 2 ? res[n * B + e * B + my_b] : fa_m;
-            double c[3];
-            mode_terms<C, NF>(fa_m, fb_m, h, dc, c);
-            run_add<NS>(r, b, c, bins, g.nrbins);
+            double t[3];
+            mode_terms<C, NF>(fa_m, fb_m, h, dc, t);
+            run_add<NS>(r, b, t, bins, g.nrbins);
           }
         }
       }
@@ -588,7 +580,7 @@ static int fused_grid(const Plan &a, int B, int nrbins, bool pp) {
   GENPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu,
                                                           reinterpret_cast<const void *>(&k_xpass_bin<T, NF, REG1, R2L, CT>),
                                                           BIN_THREADS, fused_lds<T, NF>(a, B, nrbins, pp)));
-  const int64_t nblk = a.d * ceil_div(a.hz, B);
+  const int64_t nblk = col_map(a.d, a.hz, B).nblk;
   return (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), nblk));
 }
 
@@ -599,13 +591,12 @@ static void launch_fused(Plan &a, Plan *b, const BinTables &bt, const RadixPlan 
   constexpr int NS = NF == 1 ? 1 : 3;
   // the R2L instance finishes the transform only in registers for the binning
   GENPK_REQUIRE(!(R2L && keep), "the fused pass cannot keep the spectrum with the last stage in the binning");
-  const int nkb = (int)ceil_div(a.hz, B);
   const C *tw = (a.prec == 4) ? (const C *)a.fft.tw_d_f32.ptr : (const C *)a.fft.tw_d_f64.ptr;
   BinGeom g{a.d, a.hz, bt.nrbins, bt.q2bin.as<int>(), bt.thr.as<int64_t>(), a.wtab.as<float>(), bt.lq};
   const size_t lds = fused_lds<T, NF>(a, B, bt.nrbins, pp);
   Stage st(a, "xpass_bin");
   hipLaunchKernelGGL((k_xpass_bin<T, NF, REG1, R2L, CT>), dim3(G), dim3(BIN_THREADS), lds, a.stream, a.field.as<C>(),
-                     b ? b->field.as<C>() : (C *)nullptr, g, B, nkb, FastDiv((uint32_t)nkb), rp, tw, keep ? 1 : 0, pp ? 1 : 0, part);
+                     b ? b->field.as<C>() : (C *)nullptr, g, col_map(a.d, a.hz, B), rp, tw, keep ? 1 : 0, pp ? 1 : 0, part);
   GENPK_LAUNCH_CHECK();
 }
 

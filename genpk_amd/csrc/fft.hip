@@ -298,140 +298,90 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
   }
 }
 
-// Elements of the inverse z pass's row buffer: L rows of M + 1 while the
-// half spectrum is unfolded, then L padded rows of M for the transform.
-__host__ __device__ inline int64_t c2r_span(int64_t L, int64_t M) {
-  return L * (M + 1) > lds_len<true>(L * M) ? L * (M + 1) : lds_len<true>(L * M);
-}
-
 // z pass, inverse: d/2+1 complex -> d reals (unnormalised c2r); the
 // imaginary parts of kz = 0 and kz = d/2 do not contribute.
+//   Z_k = (X_k + conj X_{M-k}) + i w^-k (X_k - conj X_{M-k}),  w = exp(-2 pi i / d)
+// Each thread reads the pairs X_k, X_{M-k} (k <= M/2) of a row and forms Z_k and
+// Z_{M-k} from them in registers, so that the half spectrum takes no round
+// trip through LDS of its own (0.49 ms at 512^3 FP32 with it and with
+// element-wise 4-byte accesses, 0.28 now).
 template <typename T>
 __global__ void __launch_bounds__(FFT_THREADS) k_c2r_z(T *__restrict__ field, int64_t rowlen, int64_t nrows, int L,
-                                                      FastDiv fdM, FastDiv fdM1, RadixPlan rp,
+                                                      FastDiv fdM, FastDiv fdP, RadixPlan rp,
                                                       const typename Cx<T>::C *__restrict__ twM,
                                                       const typename Cx<T>::C *__restrict__ twd) {
   using C = typename Cx<T>::C;
-  constexpr int MAXE = FftCfg<T>::MAXE;
+  constexpr int U = FftCfg<T>::MAXE / 2;  // pairs in flight per thread
   extern __shared__ unsigned char lds_raw[];
-  C *buf = reinterpret_cast<C *>(lds_raw);  // [L][M+1]
-  const int M = rp.n;
-  const int W = M + 1;
+  C *buf = reinterpret_cast<C *>(lds_raw);  // L padded rows of M (lds_ix)
+  const int M = rp.n, NP = M / 2 + 1;       // pairs per row (k = 0 with M, M/2 with itself)
+  C *stw = buf + lds_len<true>((int64_t)L * M);
   const int64_t row0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * L;
-  const int nl = (int)min((int64_t)L, nrows - row0);
-  // one row element is one thread's column (M == FFT_THREADS, L <= MAXE
-  // rows): element k = threadIdx.x of every row as one 8- or 16-byte load,
-  // k = M by thread 0; no index division
-  const bool colwise = M == FFT_THREADS && L <= MAXE;
-  if (colwise) {
-    const int k = threadIdx.x;
-    C v[MAXE];
-#pragma unroll
-    for (int l = 0; l < MAXE; l++) {
-      v[l] = C{0, 0};
-      if (l < nl) v[l] = reinterpret_cast<const C *>(field + (row0 + l) * rowlen)[k];
-    }
-#pragma unroll
-    for (int l = 0; l < MAXE; l++) {
-      if (l < L) {
-        if (k == 0) v[l].y = (T)0;
-        buf[l * W + k] = v[l];
-      }
-    }
-    if (k == 0)
-      for (int l = 0; l < L; l++)
-        buf[l * W + M] = l < nl ? C{field[(row0 + l) * rowlen + 2 * M], (T)0} : C{0, 0};
-  } else {
-    for (int i = threadIdx.x; i < L * W; i += FFT_THREADS) {
-      const int l = (int)fdM1.div((uint32_t)i), k = i - l * W;
-      C v = C{0, 0};
-      if (l < nl) {
-        const T *row = field + (row0 + l) * rowlen;
-        v = C{row[2 * k], (k == 0 || k == M) ? (T)0 : row[2 * k + 1]};
-      }
-      buf[i] = v;
-    }
-  }
-  __syncthreads();
-  // Z_k = (X_k + conj X_{M-k}) + i w^-k (X_k - conj X_{M-k}), k < M; staged in registers
-  C z[MAXE];
-#pragma unroll
-  for (int q = 0; q < MAXE; q++) {
-    const int i = threadIdx.x + q * FFT_THREADS;
-    if (i < L * M) {
-      const int l = colwise ? q : (int)fdM.div((uint32_t)i), k = colwise ? (int)threadIdx.x : i - l * M;
-      const C xk = buf[l * W + k];
-      const C xc = cconj(buf[l * W + (M - k)]);
-      const C s = cadd(xk, xc);
-      C dd = csub(xk, xc);
-      const C t = twd[k];
-      dd = cmul(dd, C{t.x, -t.y});                 // times exp(+2 pi i k / d)
-      z[q] = C{s.x - dd.y, s.y + dd.x};            // s + i*dd
-    }
-  }
-  __syncthreads();
-  // the transform runs on padded rows (lds_ix), as the forward z pass
-#pragma unroll
-  for (int q = 0; q < MAXE; q++) {
-    const int i = threadIdx.x + q * FFT_THREADS;
-    if (i < L * M) buf[lds_ix<true>(i)] = z[q];
-  }
-  C *stw = buf + c2r_span(L, M);
+  const int nl = (int)min((int64_t)L, nrows - row0), np = nl * NP;
   for (int i = threadIdx.x; i < M; i += FFT_THREADS) stw[i] = twM[i];
-  __syncthreads();
-  lds_fft<+1, false, MAXE, C, true>(buf, rp, L, 0, 1, M, stw);
-  if (colwise) {
-    const int m = threadIdx.x;
+  for (int i0 = threadIdx.x; i0 < np; i0 += FFT_THREADS * U) {
+    C xa[U], xb[U];
 #pragma unroll
-    for (int l = 0; l < MAXE; l++) {
-      if (l < nl) {
-        C *row = reinterpret_cast<C *>(field + (row0 + l) * rowlen);
-        row[m] = buf[lds_ix<true>(l * M + m)];
-        if (m == 0) row[M] = C{0, 0};
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * FFT_THREADS;
+      xa[u] = xb[u] = C{0, 0};
+      if (i < np) {
+        const int l = (int)fdP.div((uint32_t)i), k = i - l * NP;
+        const C *row = reinterpret_cast<const C *>(field + (row0 + l) * rowlen);
+        xa[u] = row[k];
+        xb[u] = row[M - k];
       }
     }
-    return;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * FFT_THREADS;
+      if (i >= np) continue;
+      const int l = (int)fdP.div((uint32_t)i), k = i - l * NP;
+      if (k == 0) xa[u].y = xb[u].y = (T)0;
+      const C t = twd[k];
+      auto zof = [&](C x, C y, C w) {  // x = X_k, y = X_{M-k}, w = w^-k
+        const C yc = cconj(y);
+        const C s = cadd(x, yc), dd = cmul(csub(x, yc), w);
+        return C{s.x - dd.y, s.y + dd.x};
+      };
+      buf[lds_ix<true>(l * M + k)] = zof(xa[u], xb[u], C{t.x, -t.y});
+      // w^-(M-k) = -conj(w^-k)
+      if (k != 0 && 2 * k != M) buf[lds_ix<true>(l * M + M - k)] = zof(xb[u], xa[u], C{-t.x, -t.y});
+    }
   }
+  __syncthreads();
+  lds_fft<+1, false, FftCfg<T>::MAXE, C, true>(buf, rp, nl, 0, 1, M, stw);
   for (int i = threadIdx.x; i < nl * M; i += FFT_THREADS) {
     const int l = (int)fdM.div((uint32_t)i), m = i - l * M;
-    const C v = buf[lds_ix<true>(i)];
-    T *row = field + (row0 + l) * rowlen;
-    row[2 * m] = v.x;
-    row[2 * m + 1] = v.y;
-    if (m == 0) {
-      row[2 * M] = 0;
-      row[2 * M + 1] = 0;
-    }
+    C *row = reinterpret_cast<C *>(field + (row0 + l) * rowlen);
+    row[m] = buf[lds_ix<true>(i)];
+    if (m == 0) row[M] = C{0, 0};
   }
 }
 
-// c2c along y (axis = 1) or x (axis = 0) over column blocks of B = 1 << lgb
-// consecutive kz values.  CT = 1024: the plan is n = 1024 = 8 * 8 * 8 * 2,
-// run with compile-time stages; 0: any plan.
+// c2c along y (axis = 1) or x (axis = 0) over column blocks (ColMap).  CT =
+// 1024: the plan is n = 1024 = 8 * 8 * 8 * 2, run with compile-time stages; 0:
+// any plan.
 template <typename T, int SIGN, int CT = 0>
-__global__ void __launch_bounds__(COL_THREADS) k_cols(typename Cx<T>::C *__restrict__ f, int64_t d, int64_t hz,
-                                                     int lgb, int nkb, int axis, RadixPlan rp,
-                                                     const typename Cx<T>::C *__restrict__ tw) {
+__global__ void __launch_bounds__(COL_THREADS) k_cols(typename Cx<T>::C *__restrict__ f, ColMap cm, int axis,
+                                                     RadixPlan rp, const typename Cx<T>::C *__restrict__ tw) {
   using C = typename Cx<T>::C;
   constexpr int MAXE = FftCfg<T>::COLE;
   extern __shared__ unsigned char lds_raw[];
   C *buf = reinterpret_cast<C *>(lds_raw);  // [n][B]
   const int n = CT ? CT : rp.n;
-  const int B = 1 << lgb;
-  const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-  const int64_t outer = blk / nkb;
-  const int kb = (int)(blk - outer * nkb);
-  const int64_t kz0 = (int64_t)kb * B;
-  const int nb = (int)min((int64_t)B, hz - kz0);
+  const int lgb = cm.lgb, B = 1 << lgb;
+  const int64_t d = cm.d, hz = cm.hz;
+  const ColMap::Block c = cm.at(xcd_block(blockIdx.x, gridDim.x));
   const int64_t estride = axis == 1 ? hz : d * hz;
-  C *base = f + (axis == 1 ? outer * d * hz : outer * hz) + kz0;
+  C *base = f + (int64_t)c.outer * (axis == 1 ? d * hz : hz) + c.kz0;
+  const int b = threadIdx.x & (B - 1);  // a thread's elements lie in one column
   const int tot = n * B;
   C v[MAXE];
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
     const int i = threadIdx.x + q * COL_THREADS;
-    const int e = i >> lgb, b = i & (B - 1);
-    v[q] = (i < tot && b < nb) ? base[e * estride + b] : C{0, 0};
+    v[q] = (i < tot && b < c.nb) ? base[(i >> lgb) * estride + b] : C{0, 0};
   }
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
@@ -448,43 +398,40 @@ __global__ void __launch_bounds__(COL_THREADS) k_cols(typename Cx<T>::C *__restr
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
     const int i = threadIdx.x + q * COL_THREADS;
-    const int e = i >> lgb, b = i & (B - 1);
-    if (i < tot && b < nb) base[e * estride + b] = buf[i];
+    if (i < tot && b < c.nb) base[(i >> lgb) * estride + b] = buf[i];
   }
 }
 
-// k_cols for n * B = COL_THREADS * COLE and a first radix of COLE: every
-// thread loads exactly the inputs of one first-stage butterfly (elements
-// j + q * n/R of column b, j = tid >> lgb, b = tid & (B-1): the same
-// addresses as k_cols' element-wise load), so the first stage runs from
+// k_cols for a first radix of COLE: every thread (below n * B / COLE) loads
+// exactly the inputs of one first-stage butterfly (elements j + q * n/R of
+// column b, j = tid >> lgb, b = tid & (B-1)), so the first stage runs from
 // registers and the load's LDS round trip and two barriers are saved.
 // L2 (last radix 2): the last stage's butterflies (rows k and k + n/2 of a
 // column, twiddle w^k) write their outputs straight to global memory.
-// CT = 1024: compile-time stages for n = 1024 as 8, 8, 8, 2 (FP32, with L2)
-// or 4, 8, 8, 4 (FP64 without L2).
-template <typename T, int SIGN, bool L2, int CT = 0>
-__global__ void __launch_bounds__(COL_THREADS) k_cols_r1(typename Cx<T>::C *__restrict__ f, int64_t d, int64_t hz,
-                                                        int lgb, int nkb, int axis, RadixPlan rp,
-                                                        const typename Cx<T>::C *__restrict__ tw) {
+// FULL: n * B / COLE is the thread count (else smaller, and guarded).  CT =
+// 1024 (with FULL): compile-time stages for n = 1024 as 8, 8, 8, 2 (FP32, with
+// L2) or 4, 8, 8, 4 (FP64 without L2).
+template <typename T, int SIGN, bool L2, bool FULL, int CT = 0>
+__global__ void __launch_bounds__(COL_THREADS) k_cols_r1(typename Cx<T>::C *__restrict__ f, ColMap cm, int axis,
+                                                        RadixPlan rp, const typename Cx<T>::C *__restrict__ tw) {
   using C = typename Cx<T>::C;
   constexpr int R = FftCfg<T>::COLE;
   extern __shared__ unsigned char lds_raw[];
   C *buf = reinterpret_cast<C *>(lds_raw);  // [n][B]
   const int n = CT ? CT : rp.n;
-  const int B = 1 << lgb;
-  const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
-  const int64_t outer = blk / nkb;
-  const int64_t kz0 = (int64_t)(blk - outer * nkb) * B;
-  const int nb = (int)min((int64_t)B, hz - kz0);
-  const int64_t estride = axis == 1 ? hz : d * hz;
-  C *base = f + (axis == 1 ? outer * d * hz : outer * hz) + kz0;
+  const int lgb = cm.lgb, B = 1 << lgb;
+  const int64_t d = cm.d, hz = cm.hz;
   const int b = threadIdx.x & (B - 1), j = threadIdx.x >> lgb, nq = n / R;
+  const ColMap::Block c = cm.at(xcd_block(blockIdx.x, gridDim.x));
+  const int64_t estride = axis == 1 ? hz : d * hz;
+  C *base = f + (int64_t)c.outer * (axis == 1 ? d * hz : hz) + c.kz0;
+  const bool mine = FULL || j < nq;
   C v[R];
 #pragma unroll
-  for (int q = 0; q < R; q++) v[q] = b < nb ? base[(int64_t)(j + q * nq) * estride + b] : C{0, 0};
+  for (int q = 0; q < R; q++) v[q] = mine && b < c.nb ? base[(int64_t)(j + q * nq) * estride + b] : C{0, 0};
   C *stw = buf + (int64_t)n * B;  // twiddles staged in LDS
   for (int i = threadIdx.x; i < n; i += COL_THREADS) stw[i] = tw[i];
-  fft_first_regs<R, SIGN>(v, buf, B, lgb, B, 1);
+  if (mine) fft_first_regs<R, SIGN>(v, buf, B, lgb, B, 1);
   __syncthreads();
   if constexpr (CT == 1024 && L2 && R == 8)
     lds_fft_ct<1024, 8, SIGN, true, R, false, C, false, 8, 8>(buf, buf, B, lgb, stw);
@@ -498,11 +445,12 @@ __global__ void __launch_bounds__(COL_THREADS) k_cols_r1(typename Cx<T>::C *__re
 #pragma unroll
     for (int i = 0; i < R / 2; i++) {
       const int k = j + i * (COL_THREADS >> lgb);  // butterfly b + k * B of B * n/2
+      if (!FULL && k >= h) continue;
       C t = stw[k];
       if (SIGN > 0) t.y = -t.y;
       C w[2] = {buf[k * B + b], cmul(buf[(k + h) * B + b], t)};
       Dft<2, SIGN, C>::run(w);
-      if (b < nb) {
+      if (b < c.nb) {
         base[(int64_t)k * estride + b] = w[0];
         base[(int64_t)(k + h) * estride + b] = w[1];
       }
@@ -510,27 +458,38 @@ __global__ void __launch_bounds__(COL_THREADS) k_cols_r1(typename Cx<T>::C *__re
   } else {
 #pragma unroll
     for (int q = 0; q < R; q++) {
-      const int e = (threadIdx.x + q * COL_THREADS) >> lgb;
-      if (b < nb) base[(int64_t)e * estride + b] = buf[threadIdx.x + q * COL_THREADS];
+      const int i = threadIdx.x + q * COL_THREADS, e = i >> lgb;
+      if ((FULL || e < n) && b < c.nb) base[(int64_t)e * estride + b] = buf[i];
     }
   }
 }
 
+// Rows per workgroup of the z passes: as many as the registers take (ELEMS
+// complex values, in LDS that lets two workgroups share a CU; one less of the
+// longest rows: 2.28 -> 2.05 ms at 1024^3 FP32 with 15 rows), no more than
+// spread the rows over every CU.  At 256^3 FP32 64 rows make two whole rounds
+// of workgroups (63 left a third round of 17: 61 -> 50 us).
 template <typename T>
-int rows_per_block(int64_t M) {
-  return (int)std::max<int64_t>(1, FftCfg<T>::ELEMS / std::max<int64_t>(M + 1, 1));
+int rows_per_block(int64_t M, int64_t nrows) {
+  const int64_t m = std::max<int64_t>(M, 1);
+  int64_t L = std::max<int64_t>(1, FftCfg<T>::ELEMS / (m + (m >= 512 ? 1 : 0)));
+  while (L > 1 && (lds_len<true>(L * m) + 2 * m + 1) * 2 * (int64_t)sizeof(T) > 80 * 1024) L--;
+  return (int)std::min(L, std::max<int64_t>(1, ceil_div(nrows, num_cus())));
 }
 
 }  // namespace
 
+// Columns per block of the y and x passes: as many as the registers take,
+// fewer where the blocks would not cover the CUs, down to one 64- or 128-byte
+// piece of a row.  (Sharing blocks between the outer indices for the last kz,
+// alone in its block where B divides d/2, measured slower: 33 -> 46 us at
+// 256^3 FP32, its single-element reads in a few late blocks.)
 int col_block(int prec, int64_t d, int64_t hz) {
   const int elems = prec == 4 ? FftCfg<float>::ELEMS : FftCfg<double>::ELEMS;
+  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(64, hz - 1));  // most blocks are full
   int B = 1;
-  while (B * 2 * d <= elems && B * 2 <= 64) B *= 2;
-  if (B > hz) {
-    B = 1;
-    while (B < hz) B *= 2;
-  }
+  while (B * 2 * d <= elems && B * 2 <= most) B *= 2;
+  while (B > 8 && d * ceil_div(hz - 1, B) < num_cus()) B /= 2;
   return B;
 }
 
@@ -567,8 +526,8 @@ template <typename T>
 static void r2c_z_impl(Plan &p, bool from_tiles) {
   using C = typename Cx<T>::C;
   const int64_t M = p.d / 2;
-  const int L = rows_per_block<T>(M);
   const int64_t nrows = p.d * p.d;
+  const int L = rows_per_block<T>(M, nrows);
   const RadixPlan &rp = p.rp_h;
   const C *twM = (p.prec == 4) ? (const C *)p.fft.tw_h_f32.ptr : (const C *)p.fft.tw_h_f64.ptr;
   const C *twd = (p.prec == 4) ? (const C *)p.fft.tw_d_f32.ptr : (const C *)p.fft.tw_d_f64.ptr;
@@ -625,15 +584,15 @@ template <typename T>
 static void c2r_z_impl(Plan &p) {
   using C = typename Cx<T>::C;
   const int64_t M = p.d / 2;
-  const int L = rows_per_block<T>(M);
   const int64_t nrows = p.d * p.d;
+  const int L = rows_per_block<T>(M, nrows);
   const RadixPlan &rp = p.rp_h;
   const C *twM = (p.prec == 4) ? (const C *)p.fft.tw_h_f32.ptr : (const C *)p.fft.tw_h_f64.ptr;
   const C *twd = (p.prec == 4) ? (const C *)p.fft.tw_d_f32.ptr : (const C *)p.fft.tw_d_f64.ptr;
   Stage st(p, "ifft_z");
   hipLaunchKernelGGL(k_c2r_z<T>, dim3((unsigned)ceil_div(nrows, L)), dim3(FFT_THREADS),
-                     ((size_t)c2r_span(L, M) + M) * sizeof(C), p.stream, p.field.as<T>(), p.rowlen, nrows, L,
-                     FastDiv((uint32_t)M), FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                     ((size_t)lds_len<true>((int64_t)L * M) + M) * sizeof(C), p.stream, p.field.as<T>(), p.rowlen,
+                     nrows, L, FastDiv((uint32_t)M), FastDiv((uint32_t)(M / 2 + 1)), rp, twM, twd);
   GENPK_LAUNCH_CHECK();
 }
 
@@ -641,32 +600,31 @@ template <typename T, int SIGN>
 static void cols_impl(Plan &p, int axis) {
   using C = typename Cx<T>::C;
   const int B = col_block(p.prec, p.d, p.hz);
-  const int nkb = (int)ceil_div(p.hz, B);
+  const ColMap cm = col_map(p.d, p.hz, B);
   const RadixPlan &rp = p.rp_d;
   const C *tw = (p.prec == 4) ? (const C *)p.fft.tw_d_f32.ptr : (const C *)p.fft.tw_d_f64.ptr;
   const size_t lds = (size_t)p.d * (B + 1) * sizeof(C);
-  const int64_t nblk = p.d * nkb;
+  const dim3 grid(cm.nblk), block(COL_THREADS);
   Stage st(p, axis == 1 ? (SIGN < 0 ? "fft_y" : "ifft_y") : (SIGN < 0 ? "fft_x" : "ifft_x"));
-  const bool ct1024 = is_plan_8882(rp);
-  if (rp.st[0].R == FftCfg<T>::COLE && p.d * B == (int64_t)COL_THREADS * FftCfg<T>::COLE) {
-    if (rp.st[rp.nst - 1].R == 2 && ct1024)
-      hipLaunchKernelGGL((k_cols_r1<T, SIGN, true, 1024>), dim3((unsigned)nblk), dim3(COL_THREADS), lds, p.stream,
-                         p.field.as<C>(), p.d, p.hz, ilog2(B), nkb, axis, rp, tw);
-    else if (rp.st[rp.nst - 1].R == 2)
-      hipLaunchKernelGGL((k_cols_r1<T, SIGN, true>), dim3((unsigned)nblk), dim3(COL_THREADS), lds, p.stream,
-                         p.field.as<C>(), p.d, p.hz, ilog2(B), nkb, axis, rp, tw);
-    else if (FftCfg<T>::COLE == 4 && is_plan_4884(rp))
-      hipLaunchKernelGGL((k_cols_r1<T, SIGN, false, FftCfg<T>::COLE == 4 ? 1024 : 0>), dim3((unsigned)nblk),
-                         dim3(COL_THREADS), lds, p.stream, p.field.as<C>(), p.d, p.hz, ilog2(B), nkb, axis, rp, tw);
-    else
-      hipLaunchKernelGGL((k_cols_r1<T, SIGN, false>), dim3((unsigned)nblk), dim3(COL_THREADS), lds, p.stream,
-                         p.field.as<C>(), p.d, p.hz, ilog2(B), nkb, axis, rp, tw);
+  // the compile-time instances fill every thread (n * B = COL_THREADS * COLE)
+  const bool full = p.d * B == (int64_t)COL_THREADS * FftCfg<T>::COLE;
+  const bool ct1024 = is_plan_8882(rp) && full;
+  if (rp.st[0].R == FftCfg<T>::COLE && p.d * B <= (int64_t)COL_THREADS * FftCfg<T>::COLE) {
+    const bool l2 = rp.nst > 1 && rp.st[rp.nst - 1].R == 2;
+    constexpr int CT4 = FftCfg<T>::COLE == 4 ? 1024 : 0;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, lds, p.stream, p.field.as<C>(), cm, axis, rp, tw);
+    };
+    if (l2 && ct1024) go(k_cols_r1<T, SIGN, true, true, 1024>);
+    else if (l2 && full) go(k_cols_r1<T, SIGN, true, true>);
+    else if (l2) go(k_cols_r1<T, SIGN, true, false>);
+    else if (CT4 && full && is_plan_4884(rp)) go(k_cols_r1<T, SIGN, false, true, CT4>);
+    else if (full) go(k_cols_r1<T, SIGN, false, true>);
+    else go(k_cols_r1<T, SIGN, false, false>);
   } else if (ct1024) {
-    hipLaunchKernelGGL((k_cols<T, SIGN, 1024>), dim3((unsigned)nblk), dim3(COL_THREADS), lds, p.stream,
-                       p.field.as<C>(), p.d, p.hz, ilog2(B), nkb, axis, rp, tw);
+    hipLaunchKernelGGL((k_cols<T, SIGN, 1024>), grid, block, lds, p.stream, p.field.as<C>(), cm, axis, rp, tw);
   } else {
-    hipLaunchKernelGGL((k_cols<T, SIGN>), dim3((unsigned)nblk), dim3(COL_THREADS), lds, p.stream, p.field.as<C>(), p.d,
-                       p.hz, ilog2(B), nkb, axis, rp, tw);
+    hipLaunchKernelGGL((k_cols<T, SIGN>), grid, block, lds, p.stream, p.field.as<C>(), cm, axis, rp, tw);
   }
   GENPK_LAUNCH_CHECK();
 }
