@@ -89,15 +89,15 @@ struct LdsWeight {
     for (int i = threadIdx.x; i <= w.nrbins; i += blockDim.x) sthr[i] = (int)w.thr[i];
   }
   // weight of array index xi along x of a column with a = ky^2 + kz^2 and
-  // window factors wy, wz; bt tracks the bin along the column
-  __device__ __forceinline__ double at(int xi, int n, int a, float wy, float wz, BinTrackLds &bt) const {
+  // window factors wy, wz
+  __device__ __forceinline__ double at(int xi, int n, int a, float wy, float wz) const {
     const int kx = xi <= n / 2 ? xi : xi - n;
     const int qk = a + kx * kx;
-    if (qk == 0) return 0.0;
     const float gw = (swt[xi] * wy) * wz;  // the forward's ((wx*wy)*wz) in float
     double g = (double)gw * (double)gw;
     g *= g;
-    return g * sfb[bt.of(qk, sthr, nrbins, lq)];
+    const double s = g * sfb[bin_lds(max(qk, 1), sthr, nrbins, lq)];
+    return qk ? s : 0.0;
   }
 };
 
@@ -158,10 +158,9 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
   __syncthreads();
   if (b < c.nb) {
     const int ky = (int)kv(c.outer, d), kz = (int)c.kz0 + b;
-    BinTrackLds bt;
     for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
       const int e = i >> lgb;
-      const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[c.outer], lw.swt[kz], bt) : w.at(e, c.outer, kz, d);
+      const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[c.outer], lw.swt[kz]) : w.at(e, c.outer, kz, d);
       const C a = buf[i];
       buf[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
     }
@@ -238,7 +237,6 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
       const int kz = (int)c.kz0 + b, ky = (int)kv(y, d);
       const int a = ky * ky + kz * kz;
       const float wy = lw.swt[y], wz = lw.swt[min(kz, (int)d - 1)];
-      BinTrackLds t0, t1;
 #pragma unroll
       for (int q = 0; q < HB; q++) {
         const int jj = jb + q;
@@ -246,8 +244,8 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
         const C v1 = cmul(x[(jj + half) * B + b], stw[jj]);
         C o0 = cadd(a0, v1), o1 = csub(a0, v1);
         if (b < c.nb) {
-          const double s0 = lw.at(jj, n, a, wy, wz, t0);
-          const double s1 = lw.at(jj + half, n, a, wy, wz, t1);
+          const double s0 = lw.at(jj, n, a, wy, wz);
+          const double s1 = lw.at(jj + half, n, a, wy, wz);
           o0 = C{(T)((double)o0.x * s0), (T)((double)o0.y * s0)};
           o1 = C{(T)((double)o1.x * s1), (T)((double)o1.y * s1)};
         }
@@ -257,11 +255,10 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
     } else {
       res = lds_fft_pp<-1, true, MAXE>(buf2, buf, rp, B, lgb, B, 1, stw, 1);
       const int kz = (int)c.kz0 + b, ky = (int)kv(y, d);
-      BinTrackLds bt;
-      for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
+        for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
         const int e = i >> lgb;
         if (b < c.nb) {
-          const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[y], lw.swt[kz], bt) : w.at(e, y, kz, d);
+          const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[y], lw.swt[kz]) : w.at(e, y, kz, d);
           const C a = res[i];
           res[i] = C{(T)((double)a.x * s), (T)((double)a.y * s)};
         }

@@ -36,6 +36,7 @@ namespace {
 // x 32 values (x pass + bin 4.0 -> 3.4 ms at 1024^3).
 constexpr int BIN_THREADS = 1024;
 constexpr int LDS_LIMIT = 160 * 1024;
+constexpr int LGC_MAX = 3;
 template <typename T> struct BinCfg;
 template <> struct BinCfg<float> { static constexpr int ELEMS = 8192; static constexpr int MAXE = 8; };
 template <> struct BinCfg<double> { static constexpr int ELEMS = 4096; static constexpr int MAXE = 4; };
@@ -73,18 +74,23 @@ struct RunAcc {
   double v[3] = {0, 0, 0};
 };
 
+// bins: this lane's copy of the LDS bins, 1 << lgc copies side by side.  Lanes
+// beside each other mostly end runs of one bin together, and their adds to
+// one address are taken one after another: with up to eight copies, as the
+// LDS has room, the x pass + bin takes 2.41 -> 2.23 ms at 1024^3 FP32, 0.74 ->
+// 0.68 with two fields at 512^3, and leaving the adds out saves no more.
 template <int NS>
-__device__ __forceinline__ void run_flush(RunAcc &r, double *bins, int nrbins) {
+__device__ __forceinline__ void run_flush(RunAcc &r, double *bins, int nrbins, int lgc) {
   if (r.cur >= 0) {
 #pragma unroll
-    for (int s = 0; s < NS; s++) atomicAdd(&bins[s * nrbins + r.cur], r.v[s]);
+    for (int s = 0; s < NS; s++) atomicAdd(&bins[(s * nrbins + r.cur) << lgc], r.v[s]);
   }
 }
 
 template <int NS>
-__device__ __forceinline__ void run_add(RunAcc &r, int b, const double *c, double *bins, int nrbins) {
+__device__ __forceinline__ void run_add(RunAcc &r, int b, const double *c, double *bins, int nrbins, int lgc) {
   if (b != r.cur) {
-    run_flush<NS>(r, bins, nrbins);
+    run_flush<NS>(r, bins, nrbins, lgc);
     r.cur = b;
 #pragma unroll
     for (int s = 0; s < NS; s++) r.v[s] = 0;
@@ -133,49 +139,56 @@ struct BinTrack {
 // Fused final FFT pass along x + deconvolved binning.  NF fields (1: auto,
 // 2: auto a, auto b and cross a.b*).  Persistent over column blocks.
 //
-// REG1 (one field, ping-pong buffers, n * B <= BIN_THREADS * MAXE, a first
-// stage of radix MAXE and an even number of stages): the MAXE loaded
-// elements of each thread below n * B / MAXE are the inputs of its butterfly
+// REG1 (a first stage of radix MAXE; one field: ping-pong buffers): the MAXE
+// loaded elements of each thread below n * B / MAXE are the inputs of its butterfly
 // in the first stage, which then runs from registers into buf2 (the threads
-// above it load nothing and bin nothing).  The previous block no longer reads
-// buf2 (an even number of stages leaves its result in buf), so no barrier
-// comes before that stage.
+// above it load nothing).  Where the binning reads buf2 (an odd number of
+// stages, or the last one left to the binning) the buffers swap roles
+// between blocks, so no barrier comes before that stage.  FP32 360^3: 0.15 ->
+// 0.11 ms; FP64 200^3 0.044 -> 0.036, 64^3 (three stages) 0.012 -> 0.010.  With
+// two fields the first stage runs from registers in place: 0.58 -> 0.53 ms
+// at 512^3 FP32.
 //
 // R2L (with REG1, a last stage of radix 2): the last stage runs in the
 // binning, each thread pairing stage inputs j and j + n/2 into modes j and
-// j + n/2 in registers; the two buffers then swap roles between blocks so
-// that the next first stage never writes the buffer being binned.
+// j + n/2 in registers.
+//
+// The registers hold the next block's loads while a block is binned: a
+// spilled value read back there waits for all of them (one spilled register
+// made the binning of a block 4.9 us instead of 2.7 at 1024^3 FP32), so each
+// element's address is one column address plus a scalar multiple.
 template <typename T, int NF, bool REG1, bool R2L = false, int CT = 0>
 __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__restrict__ fa,
                                                             typename Cx<T>::C *__restrict__ fb, BinGeom g, ColMap cm,
                                                             RadixPlan rp,
                                                             const typename Cx<T>::C *__restrict__ tw, int keep,
-                                                            int pp, double *__restrict__ part) {
+                                                            int pp, int lgc, double *__restrict__ part) {
   using C = typename Cx<T>::C;
   constexpr int NS = NF == 1 ? 1 : 3;
   static_assert(!R2L || REG1, "the radix-2 last stage in the binning needs the register first stage");
   extern __shared__ unsigned char lds_raw[];
   double *bins = reinterpret_cast<double *>(lds_raw);
-  C *buf = reinterpret_cast<C *>(bins + ((NS * g.nrbins + 1) & ~1));  // [NF][n][B], 16-byte aligned
+  C *buf = reinterpret_cast<C *>(bins + (((NS * g.nrbins << lgc) + 1) & ~1));  // [NF][n][B], 16-byte aligned
   const int n = CT ? CT : rp.n;
   const int lgb = cm.lgb, B = 1 << lgb;
   // pp (one field): a second buffer lets the FFT stages alternate (one barrier each)
   C *buf2 = buf + (size_t)NF * n * B;
   C *stw = buf2 + (pp ? (size_t)n * B : 0);  // twiddles staged in LDS
   float *wt = reinterpret_cast<float *>(stw + n);  // deconvolution weights [d]
-  int *thr32 = reinterpret_cast<int *>(wt + g.d);  // bin thresholds [nrbins]
+  int *thr32 = reinterpret_cast<int *>(wt + g.d);  // bin thresholds
   for (int i = threadIdx.x; i < n; i += BIN_THREADS) stw[i] = tw[i];
-  for (int i = threadIdx.x; i < NS * g.nrbins; i += BIN_THREADS) bins[i] = 0;
+  for (int i = threadIdx.x; i < NS * g.nrbins << lgc; i += BIN_THREADS) bins[i] = 0;
+  double *my_bins = bins + (threadIdx.x & ((1 << lgc) - 1));
   for (int i = threadIdx.x; i < g.d; i += BIN_THREADS) wt[i] = g.wtab[i];
-  for (int i = threadIdx.x; i < g.nrbins; i += BIN_THREADS) thr32[i] = (int)g.thr[i];
+  for (int i = threadIdx.x; i < bin_lds_slots(g.nrbins); i += BIN_THREADS) thr32[i] = (int)g.thr[i];
   const int64_t d = g.d, hz = g.hz;
   const int64_t estride = d * hz;
   const int64_t nblk = cm.nblk;
   // bin-phase mapping: thread -> column b, contiguous run of e
-  const int tpc = BIN_THREADS / B;               // threads per column (B divides BIN_THREADS)
-  const int my_b = threadIdx.x % B;
+  const int tpc = BIN_THREADS >> lgb;            // threads per column (B divides BIN_THREADS)
+  const int my_b = threadIdx.x & (B - 1);
   const int per = (n + tpc - 1) / tpc;
-  const int e0 = (threadIdx.x / B) * per;
+  const int e0 = (int)(threadIdx.x >> lgb) * per;
   // register-staged loads of column block v: all its global reads in flight
   // together; with REG1 at a stride of the first stage's butterfly count
   constexpr int MAXE = BinCfg<T>::MAXE;
@@ -183,17 +196,18 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
   const int lst = REG1 ? tot / MAXE : BIN_THREADS;
   const bool loader = !REG1 || (int)threadIdx.x < lst;
   C va[MAXE], vb[NF == 2 ? MAXE : 1];
+  const int64_t my_off = (threadIdx.x >> lgb) * estride + my_b, qstep = (int64_t)(lst >> lgb) * estride;
   auto load = [&](int64_t v) {
     // a grid that is a multiple of the XCD count keeps v on this workgroup's XCD
     const ColMap::Block c = cm.at(xcd_block((uint32_t)v, (uint32_t)nblk));
     const int64_t off = (int64_t)c.outer * hz + c.kz0;
+    const C *pa = fa + off + my_off, *pb = fb + off + my_off;
+    const bool ok = loader && my_b < c.nb;
 #pragma unroll
     for (int q = 0; q < MAXE; q++) {
-      const int i = threadIdx.x + q * lst;
-      const int e = i >> lgb;  // of column my_b
-      const bool ok = loader && i < tot && my_b < c.nb;
-      va[q] = ok ? fa[off + e * estride + my_b] : C{0, 0};
-      if (NF == 2) vb[NF == 2 ? q : 0] = ok ? fb[off + e * estride + my_b] : C{0, 0};
+      const bool okq = ok && (REG1 || (int)threadIdx.x + q * lst < tot);
+      va[q] = okq ? pa[q * qstep] : C{0, 0};
+      if (NF == 2) vb[NF == 2 ? q : 0] = okq ? pb[q * qstep] : C{0, 0};
     }
   };
   // block v + gridDim.x loads into the registers while block v is binned
@@ -204,7 +218,17 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
     const int64_t y = c.outer;
     const int64_t off = y * hz + c.kz0;
     C *res = buf;
-    if constexpr (REG1) {
+    if constexpr (REG1 && NF == 2) {
+      __syncthreads();  // the previous block's binning is done with buf
+      if (loader) {
+        fft_first_regs<MAXE, -1>(va, buf, B, lgb, B, 1);
+        fft_first_regs<MAXE, -1>(vb, buf + tot, B, lgb, B, 1);
+      }
+      __syncthreads();
+      for (int s = 1; s < rp.nst; s++)
+        for (int f = 0; f < 2; f++)
+          fft_stage_r<-1, true, MAXE, false, C>(rp.st[s].R, buf + f * tot, buf + f * tot, B, lgb, B, 1, rp.st[s], stw);
+    } else if constexpr (REG1) {
       if (loader) fft_first_regs<MAXE, -1>(va, buf2, B, lgb, B, 1);
       __syncthreads();
       if constexpr (CT == 1024 && R2L && MAXE == 8)
@@ -246,7 +270,6 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
       const int a = ky * ky + kz * kz;
       const float wy = wt[y], wz = wt[kz];
       RunAcc r;
-      BinTrackLds bt;
       // this thread's run of at most MAXE modes along x (per <= MAXE as
       // n * B <= BIN_THREADS * MAXE); with one field all its LDS reads are
       // issued first (two fields would not fit the registers)
@@ -255,34 +278,39 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
         // (the latter times w^jj) into modes jj and jj + n/2
         constexpr int HB = MAXE / 2;
         const int half = n / 2;
-        const int jb = (threadIdx.x / B) * HB;  // below half exactly for the loaders
+        const int jb = (int)(threadIdx.x >> lgb) * HB;  // below half exactly for the loaders
         C mo[MAXE];
         if (loader) {
 #pragma unroll
         for (int q = 0; q < HB; q++) {
           const int jj = jb + q;
-          const C a0 = res[jj * B + my_b];
-          const C v1 = cmul(res[(jj + half) * B + my_b], stw[jj]);
+          const C a0 = res[(jj << lgb) + my_b];
+          const C v1 = cmul(res[((jj + half) << lgb) + my_b], stw[jj]);
           mo[q] = cadd(a0, v1);
           mo[q + HB] = csub(a0, v1);
         }
+        // half the modes at a time: their bins, then their terms (all eight
+        // bins at once spill registers with the compile-time stages)
 #pragma unroll
-        for (int q = 0; q < MAXE; q++) {
-          const int e = q < HB ? jb + q : jb + (q - HB) + half;
-          const int kx = e <= d / 2 ? e : e - (int)d;
-          const int qk = a + kx * kx;
-          if (qk != 0) {
-            const int bn = bt.of(qk, thr32, g.nrbins, g.lq);
-            const float gw = (wt[e] * wy) * wz;  // the reference's ((wx*wy)*wz) in float
-            double dc = (double)gw * (double)gw;
-            dc *= dc;
-            double t[3];
-            mode_terms<C, NF>(mo[q], mo[q], h, dc, t);
-            run_add<NS>(r, bn, t, bins, g.nrbins);
+        for (int m = 0; m < MAXE; m += HB) {
+          const int eb = m ? jb + half : jb, kb = m ? jb - half : jb;  // d / 2 counts as -d / 2
+          int bq[HB];
+#pragma unroll
+          for (int q = 0; q < HB; q++) bq[q] = bin_lds(max(a + (kb + q) * (kb + q), 1), thr32, g.nrbins, g.lq);
+#pragma unroll
+          for (int q = 0; q < HB; q++) {
+            if (a != 0 || eb + q != 0) {
+              const float gw = (wt[eb + q] * wy) * wz;  // the reference's ((wx*wy)*wz) in float
+              double dc = (double)gw * (double)gw;
+              dc *= dc;
+              double t[3];
+              mode_terms<C, NF>(mo[m + q], mo[m + q], h, dc, t);
+              run_add<NS>(r, bq[q], t, my_bins, g.nrbins, lgc);
+            }
           }
         }
         }
-        run_flush<NS>(r, bins, g.nrbins);
+        run_flush<NS>(r, my_bins, g.nrbins, lgc);
       } else {
       constexpr bool BATCH = NF == 1;
       C ma[BATCH ? MAXE : 1];
@@ -292,7 +320,7 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
         for (int j = 0; j < MAXE; j++) {
           const int e = e0 + j;
           if (j < per && e < n) {
-            ma[BATCH ? j : 0] = res[e * B + my_b];
+            ma[BATCH ? j : 0] = res[(e << lgb) + my_b];
             if (!REG1) wx[BATCH ? j : 0] = wt[e];
           }
         }
@@ -304,22 +332,22 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
           const int kx = e <= d / 2 ? e : e - (int)d;
           const int q = a + kx * kx;
           if (q != 0) {
-            const int b = bt.of(q, thr32, g.nrbins, g.lq);
+            const int b = bin_lds(q, thr32, g.nrbins, g.lq);
             const float gw = ((BATCH && !REG1 ? wx[BATCH ? j : 0] : wt[e]) * wy) * wz;  // the reference's ((wx*wy)*wz) in float
             double dc = (double)gw * (double)gw;
             dc *= dc;
-            const C fa_m = BATCH ? ma[BATCH ? j : 0] : res[e * B + my_b];
-            const C fb_m = NF == 2 ? res[n * B + e * B + my_b] : fa_m;
+            const C fa_m = BATCH ? ma[BATCH ? j : 0] : res[(e << lgb) + my_b];
+            const C fb_m = NF == 2 ? res[tot + (e << lgb) + my_b] : fa_m;
             double t[3];
             mode_terms<C, NF>(fa_m, fb_m, h, dc, t);
-            run_add<NS>(r, b, t, bins, g.nrbins);
+            run_add<NS>(r, b, t, my_bins, g.nrbins, lgc);
           }
         }
       }
-      run_flush<NS>(r, bins, g.nrbins);
+      run_flush<NS>(r, my_bins, g.nrbins, lgc);
       }
     }
-    if constexpr (R2L) {
+    if constexpr (REG1 && NF == 1) {
       // the next first stage writes the buffer the binning did not read
       if (res == buf2) {
         C *t = buf;
@@ -329,7 +357,11 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < NS * g.nrbins; i += BIN_THREADS) part[(int64_t)blockIdx.x * NS * g.nrbins + i] = bins[i];
+  for (int i = threadIdx.x; i < NS * g.nrbins; i += BIN_THREADS) {
+    double t = 0;
+    for (int k = 0; k < 1 << lgc; k++) t += bins[(i << lgc) + k];
+    part[(int64_t)blockIdx.x * NS * g.nrbins + i] = t;
+  }
 }
 
 // Binning of stored spectra [d][d][hz] (no FFT): one wave per (kx, ky) row,
@@ -366,9 +398,9 @@ __global__ void __launch_bounds__(BIN_THREADS) k_bin_stored(const typename Cx<T>
       const C vb = NF == 2 ? fb[row * hz + kz] : va;
       double c[3];
       mode_terms<C, NF>(va, vb, h, dc, c);
-      run_add<NS>(r, b, c, bins, g.nrbins);
+      run_add<NS>(r, b, c, bins, g.nrbins, 0);
     }
-    run_flush<NS>(r, bins, g.nrbins);
+    run_flush<NS>(r, bins, g.nrbins, 0);
   }
   __syncthreads();
   for (int i = threadIdx.x; i < NS * g.nrbins; i += BIN_THREADS) part[(int64_t)blockIdx.x * NS * g.nrbins + i] = bins[i];
@@ -548,7 +580,7 @@ static int fused_block(int prec, int64_t d, int64_t hz, int nf, int ns, int nrbi
   int B = col_block(prec, d, hz);
   while (B >= 1) {
     const int64_t lds = ((int64_t)nf * B + 1) * d * csize + (int64_t)((ns * nrbins + 1) & ~1) * 8 + d * 4 +
-                        nrbins * 4;
+                        bin_lds_slots(nrbins) * 4;
     if (lds <= LDS_LIMIT && d * B <= elems && BIN_THREADS % B == 0) return B;
     B /= 2;
   }
@@ -556,47 +588,45 @@ static int fused_block(int prec, int64_t d, int64_t hz, int nf, int ns, int nrbi
 }
 
 template <typename T, int NF>
-static size_t fused_lds(const Plan &a, int B, int nrbins, bool pp) {
+static size_t fused_lds(const Plan &a, int B, int nrbins, bool pp, int lgc = 0) {
   using C = typename Cx<T>::C;
   constexpr int NS = NF == 1 ? 1 : 3;
-  return ((size_t)NF * B + (pp ? B : 0) + 1) * a.d * sizeof(C) + (size_t)((NS * nrbins + 1) & ~1) * 8 +
-         (size_t)a.d * 4 + (size_t)nrbins * 4;
+  return ((size_t)NF * B + (pp ? B : 0) + 1) * a.d * sizeof(C) + (size_t)(((NS * nrbins << lgc) + 1) & ~1) * 8 +
+         (size_t)a.d * 4 + (size_t)bin_lds_slots(nrbins) * 4;
 }
 
-// Whether the REG1 instance applies to plan rp (one field with ping-pong
-// buffers): every thread holds one first-stage butterfly, or (some_idle)
-// at most one.
+// Whether every thread holds at most one butterfly of plan rp's first stage
+// (exactly: one each), as the REG1 instances need.
 template <typename T>
-static bool fused_reg1(const Plan &a, int B, bool pp, const RadixPlan &rp, bool some_idle = false) {
+static bool fused_reg1(const Plan &a, int B, const RadixPlan &rp, bool exactly) {
   const int64_t tot = a.d * B, cap = (int64_t)BIN_THREADS * BinCfg<T>::MAXE;
-  return pp && rp.st[0].R == BinCfg<T>::MAXE && (some_idle ? tot <= cap : tot == cap) && rp.nst % 2 == 0;
+  return rp.st[0].R == BinCfg<T>::MAXE && (exactly ? tot == cap : tot <= cap);
 }
 
 // Persistent grid of the fused kernel: as many workgroups as stay resident
 // (occupancy of this instance x CUs), at most one per column block.
 template <typename T, int NF, bool REG1, bool R2L = false, int CT = 0>
-static int fused_grid(const Plan &a, int B, int nrbins, bool pp) {
+static int fused_grid(const Plan &a, int B, int nrbins, bool pp, int lgc) {
   int per_cu = 0;
   GENPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu,
                                                           reinterpret_cast<const void *>(&k_xpass_bin<T, NF, REG1, R2L, CT>),
-                                                          BIN_THREADS, fused_lds<T, NF>(a, B, nrbins, pp)));
+                                                          BIN_THREADS, fused_lds<T, NF>(a, B, nrbins, pp, lgc)));
   const int64_t nblk = col_map(a.d, a.hz, B).nblk;
   return (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), nblk));
 }
 
 template <typename T, int NF, bool REG1, bool R2L = false, int CT = 0>
 static void launch_fused(Plan &a, Plan *b, const BinTables &bt, const RadixPlan &rp, int B, bool keep, bool pp,
-                         double *part, int G) {
+                         int lgc, double *part, int G) {
   using C = typename Cx<T>::C;
-  constexpr int NS = NF == 1 ? 1 : 3;
   // the R2L instance finishes the transform only in registers for the binning
   GENPK_REQUIRE(!(R2L && keep), "the fused pass cannot keep the spectrum with the last stage in the binning");
   const C *tw = (a.prec == 4) ? (const C *)a.fft.tw_d_f32.ptr : (const C *)a.fft.tw_d_f64.ptr;
   BinGeom g{a.d, a.hz, bt.nrbins, bt.q2bin.as<int>(), bt.thr.as<int64_t>(), a.wtab.as<float>(), bt.lq};
-  const size_t lds = fused_lds<T, NF>(a, B, bt.nrbins, pp);
+  const size_t lds = fused_lds<T, NF>(a, B, bt.nrbins, pp, lgc);
   Stage st(a, "xpass_bin");
   hipLaunchKernelGGL((k_xpass_bin<T, NF, REG1, R2L, CT>), dim3(G), dim3(BIN_THREADS), lds, a.stream, a.field.as<C>(),
-                     b ? b->field.as<C>() : (C *)nullptr, g, col_map(a.d, a.hz, B), rp, tw, keep ? 1 : 0, pp ? 1 : 0, part);
+                     b ? b->field.as<C>() : (C *)nullptr, g, col_map(a.d, a.hz, B), rp, tw, keep ? 1 : 0, pp ? 1 : 0, lgc, part);
   GENPK_LAUNCH_CHECK();
 }
 
@@ -619,25 +649,28 @@ struct FusedShape {
   RadixPlan rp;
   int B = 0;
   bool pp = false, reg1 = false, r2l = false, ct = false;
+  int lgc = 0;
   int G = 0;
 };
 
 template <typename T>
 static int fused_grid_of(const Plan &a, bool cross, const FusedShape &s, int nrbins) {
-  if (cross) return fused_grid<T, 2, false>(a, s.B, nrbins, false);
-  if (s.r2l && s.ct) return fused_grid<T, 1, true, true, 1024>(a, s.B, nrbins, s.pp);
-  if (s.r2l) return fused_grid<T, 1, true, true>(a, s.B, nrbins, s.pp);
-  if (s.reg1) return fused_grid<T, 1, true>(a, s.B, nrbins, s.pp);
-  return fused_grid<T, 1, false>(a, s.B, nrbins, s.pp);
+  if (cross && s.reg1) return fused_grid<T, 2, true>(a, s.B, nrbins, false, s.lgc);
+  if (cross) return fused_grid<T, 2, false>(a, s.B, nrbins, false, s.lgc);
+  if (s.r2l && s.ct) return fused_grid<T, 1, true, true, 1024>(a, s.B, nrbins, s.pp, s.lgc);
+  if (s.r2l) return fused_grid<T, 1, true, true>(a, s.B, nrbins, s.pp, s.lgc);
+  if (s.reg1) return fused_grid<T, 1, true>(a, s.B, nrbins, s.pp, s.lgc);
+  return fused_grid<T, 1, false>(a, s.B, nrbins, s.pp, s.lgc);
 }
 
 template <typename T>
 static void launch_fused_of(Plan &a, Plan *b, const BinTables &bt, const FusedShape &s, double *part) {
-  if (b) launch_fused<T, 2, false>(a, b, bt, s.rp, s.B, false, false, part, s.G);
-  else if (s.r2l && s.ct) launch_fused<T, 1, true, true, 1024>(a, b, bt, s.rp, s.B, false, s.pp, part, s.G);
-  else if (s.r2l) launch_fused<T, 1, true, true>(a, b, bt, s.rp, s.B, false, s.pp, part, s.G);
-  else if (s.reg1) launch_fused<T, 1, true>(a, b, bt, s.rp, s.B, false, s.pp, part, s.G);
-  else launch_fused<T, 1, false>(a, b, bt, s.rp, s.B, false, s.pp, part, s.G);
+  if (b && s.reg1) launch_fused<T, 2, true>(a, b, bt, s.rp, s.B, false, false, s.lgc, part, s.G);
+  else if (b) launch_fused<T, 2, false>(a, b, bt, s.rp, s.B, false, false, s.lgc, part, s.G);
+  else if (s.r2l && s.ct) launch_fused<T, 1, true, true, 1024>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
+  else if (s.r2l) launch_fused<T, 1, true, true>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
+  else if (s.reg1) launch_fused<T, 1, true>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
+  else launch_fused<T, 1, false>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
 }
 
 static FusedShape fused_shape(const Plan &a, const Plan *b, int nrbins) {
@@ -650,17 +683,20 @@ static FusedShape fused_shape(const Plan &a, const Plan *b, int nrbins) {
   s.pp = !b && (a.prec == 4 ? fused_lds<float, 1>(a, B, nrbins, true)
                             : fused_lds<double, 1>(a, B, nrbins, true)) <= (size_t)LDS_LIMIT;
   s.rp = a.rp_d;
-  s.reg1 = !b && (a.prec == 4 ? fused_reg1<float>(a, B, s.pp, s.rp) : fused_reg1<double>(a, B, s.pp, s.rp));
-  // FP32 with a last stage of radix 2: that stage runs in the binning
-  s.r2l = s.reg1 && a.prec == 4 && s.rp.st[s.rp.nst - 1].R == 2;
-  if (!b && a.prec == 4 && !s.r2l) {
+  auto reg1 = [&](const RadixPlan &rp, bool exactly) {
+    return (b || s.pp) && (a.prec == 4 ? fused_reg1<float>(a, B, rp, exactly) : fused_reg1<double>(a, B, rp, exactly));
+  };
+  s.reg1 = reg1(s.rp, false);
+  if (!b && a.prec == 4) {
+    // FP32 with a last stage of radix 2: that stage runs in the binning
+    s.r2l = s.rp.nst % 2 == 0 && s.rp.st[s.rp.nst - 1].R == 2 && reg1(s.rp, true);
     // the plan's own ordering (the column passes') does not start with a
     // radix 8 and end with a radix 2 in an even number of stages, or its
     // columns leave threads idle: the x pass takes a plan of its length that
     // does, where the register first stage applies (512 = 8 8 8 -> 8 8 4 2:
     // 0.40 -> 0.30 ms at 512^3)
-    const RadixPlan xp = radix_plan_8_to_2((int)a.d);
-    if (xp.nst > 0 && fused_reg1<float>(a, B, s.pp, xp, true)) {
+    const RadixPlan xp = s.r2l ? RadixPlan{} : radix_plan_8_to_2((int)a.d);
+    if (!s.r2l && xp.nst > 0 && reg1(xp, false)) {
       s.rp = xp;
       s.reg1 = s.r2l = true;
     }
@@ -669,6 +705,11 @@ static FusedShape fused_shape(const Plan &a, const Plan *b, int nrbins) {
   // n = 1024 (the others would spill registers)
   s.ct = s.r2l && is_plan_8882(s.rp);
   const bool cross = b != nullptr;
+  auto lds_of = [&](int lgc) {
+    return cross ? (a.prec == 4 ? fused_lds<float, 2>(a, B, nrbins, false, lgc) : fused_lds<double, 2>(a, B, nrbins, false, lgc))
+                 : (a.prec == 4 ? fused_lds<float, 1>(a, B, nrbins, s.pp, lgc) : fused_lds<double, 1>(a, B, nrbins, s.pp, lgc));
+  };
+  while (s.lgc < LGC_MAX && lds_of(s.lgc + 1) <= (size_t)LDS_LIMIT) s.lgc++;
   s.G = a.prec == 4 ? fused_grid_of<float>(a, cross, s, nrbins) : fused_grid_of<double>(a, cross, s, nrbins);
   return s;
 }
