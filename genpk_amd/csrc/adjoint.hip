@@ -232,8 +232,6 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
       constexpr int HB = MAXE / 2;
       const int half = n / 2;
       const int jb = (threadIdx.x >> lgb) * HB;
-      // modes jj (kx = jj) and jj + n/2 (kx = jj - n/2, kx = n/2 at jj = 0)
-      // each keep a bin tracker along their run
       const int kz = (int)c.kz0 + b, ky = (int)kv(y, d);
       const int a = ky * ky + kz * kz;
       const float wy = lw.swt[y], wz = lw.swt[min(kz, (int)d - 1)];

@@ -44,3 +44,23 @@ def test_fused_binning_equals_stored_binning(gpu, prec, d, nrbins):
     rel = scount.double() * 2.0 ** -52 + (6e-6 if prec == "f32" and d % 16 == 0 else 0.0)
     for got, ref, size in ((fp, sp, sp), (fcross[0], saa, saa), (fcross[1], sbb, sbb), (fcross[2], sab, (saa * sbb).sqrt())):
         assert bool(((got - ref).abs() <= rel * size).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,d", [("f64", 34), ("f32", 90)])
+def test_stored_binning_without_lds_tables(gpu, prec, d):
+    """Two fields with 6700 bins leave no LDS for the window factors and the
+    thresholds; one field's bins do.  The bound is the first test's."""
+    import torch
+    print("CASE", prec, d, flush=True)
+    nrbins = 6700
+    g = torch.Generator(device="cuda").manual_seed(d)
+    a, b = (genpk_amd.Plan(d, prec) for _ in range(2))
+    for p in (a, b):
+        p.import_density(torch.randn(p.grid.shape, device="cuda", dtype=p.real_dtype, generator=g))
+        p.r2c()
+    (paa, pbb, _), count, _ = a.bin(nrbins, other=b)
+    for p, got in ((a, paa), (b, pbb)):
+        ref, c1, _ = p.bin(nrbins)
+        assert torch.equal(count, c1)
+        assert bool(((got - ref).abs() <= count.double() * 2.0 ** -52 * ref).all())
