@@ -47,7 +47,7 @@ def test_fused_binning_equals_stored_binning(gpu, prec, d, nrbins):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("prec,d", [("f64", 34), ("f32", 90)])
+@pytest.mark.parametrize("prec,d", [("f64", 36), ("f32", 90)])
 def test_stored_binning_without_lds_tables(gpu, prec, d):
     """Two fields with 6700 bins leave no LDS for the window factors and the
     thresholds; one field's bins do.  The bound is the first test's."""
