@@ -77,10 +77,12 @@ struct DepParams {
 template <typename Real, int NM, int RW, bool STD>
 __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict__ rec,
                                                          const uint32_t *__restrict__ item_tile,
-                                                         const uint32_t *__restrict__ item_start,
+                                                         const uint32_t *__restrict__ part_start,
                                                          const uint32_t *__restrict__ start,
                                                          const uint32_t *__restrict__ blist,
-                                                         const uint32_t *__restrict__ part_start, DepParams P,
+                                                         const uint32_t *__restrict__ counts,
+                                                         const uint32_t *__restrict__ cost,
+                                                         const uint32_t *__restrict__ share, DepParams P,
                                                          Real *__restrict__ tiles, double *__restrict__ partials) {
   using Acc = unsigned long long;
   constexpr int UNR = 4;
@@ -121,22 +123,58 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   // most 256 slots divide the 1024 threads)
   const int lg = T.lg;
   const uint32_t in = threadIdx.x & ((1u << lg) - 1), te = threadIdx.x >> lg, eu = (uint32_t)DEP_THREADS >> lg;
-  auto range_of = [&](uint32_t it, ItemRange &o) { return item_range(item_tile, item_start, start, T.ks, T.max_items, it, o); };
+  // this workgroup's items (k_dir's schedule): w, w + grid, ... of split
+  // tiles, then [one0, one1); NONE after the last
+  constexpr uint32_t NONE = 0xffffffffu;
+  const uint32_t nsplit = counts[1], none1 = counts[2];
+  uint32_t one0, one1;
+  if (nsplit + none1 <= gridDim.x) {
+    one0 = max((uint32_t)blockIdx.x, nsplit);
+    one1 = blockIdx.x < nsplit ? one0 : min(one0 + 1, nsplit + none1);
+  } else {
+    // the first item of one tile whose middle is at or past the share's
+    // bound: 64 samples a step
+    auto first_from = [&](uint32_t at) {
+      uint32_t lo = 0, len = none1;
+      while (len > 0) {
+        const uint32_t step = (len + 63) / 64, s = (threadIdx.x & 63) * step;
+        const uint32_t below = (uint32_t)__popcll(__ballot(s < len && cost[lo + s] < at));
+        if (below == 0) break;
+        const uint32_t end = min(len, below * step);
+        lo += (below - 1) * step + 1;
+        len = end - ((below - 1) * step + 1);
+      }
+      return lo;
+    };
+    one0 = nsplit + (blockIdx.x == 0 ? 0u : first_from(share[blockIdx.x]));
+    one1 = nsplit + (blockIdx.x + 1 == gridDim.x ? none1 : first_from(share[blockIdx.x + 1]));
+  }
+  auto first_one = [&]() { return one0 < one1 ? one0 : NONE; };
+  auto next_of = [&](uint32_t it) -> uint32_t {
+    if (it < nsplit) return it + gridDim.x < nsplit ? it + gridDim.x : first_one();
+    return it < NONE && it + 1 < one1 ? it + 1 : NONE;
+  };
+  auto range_of = [&](uint32_t it, ItemRange &o) {
+    if (it == NONE) return false;
+    item_range(item_tile, part_start, start, nsplit, T.max_parts, it, o);
+    return true;
+  };
   struct {
-    uint32_t item, lb, ents, rel;  // the batch: entries [rel, rel + UNR * eu) of the item's `ents`
+    uint32_t lb, ents, rel;  // the batch: entries [rel, rel + UNR * eu) of the item's `ents`
   } ld;
-  ItemRange ahead;  // the item after ld's
+  uint32_t ahead_item;  // the item after ld's
+  ItemRange ahead;
   bool ahead_ok;
   auto load_step = [&]() {  // to the next batch (past the last item: ents = 0)
     ld.rel += UNR * eu;
     while (ld.rel >= ld.ents) {
-      ld.item += gridDim.x;
       ld.rel = 0;
       ld.ents = 0;
       if (!ahead_ok) break;
       ld.lb = ahead.lb;
       ld.ents = ahead.le - ahead.lb;
-      ahead_ok = range_of(ld.item + gridDim.x, ahead);
+      ahead_item = next_of(ahead_item);
+      ahead_ok = range_of(ahead_item, ahead);
     }
   };
   auto load_entries = [&]() {
@@ -169,16 +207,16 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
 #pragma unroll
       for (int q = 0; q < RW; q++) r[u][q] = nx[u][q];
   };
-  // Persistent over the items (item, item + gridDim.x, ...).  Every load
+  // Persistent over the workgroup's items.  Every load
   // issued before an item's flush has arrived before it too: the flush's
   // stores then drain while the next item accumulates (a wait for loads
   // issued before them, the counter being in order and the stores' count not
   // known, would wait for the stores as well).
-  uint32_t item = blockIdx.x;
+  uint32_t item = blockIdx.x < nsplit ? blockIdx.x : first_one();
   ItemRange ir;
   bool have = range_of(item, ir);
-  ahead_ok = have && range_of(item + gridDim.x, ahead);
-  ld.item = item;
+  ahead_item = have ? next_of(item) : NONE;
+  ahead_ok = range_of(ahead_item, ahead);
   ld.lb = have ? ir.lb : 0u;
   ld.ents = have ? ir.le - ir.lb : 0u;
   ld.rel = 0;
@@ -193,7 +231,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   __syncthreads();
   while (have) {
     const int64_t k = ir.k;
-    const uint32_t m = ir.m, j = ir.j, ents = ir.le - ir.lb;
+    const uint32_t m = ir.m, ents = ir.le - ir.lb;
     const int ntz = P.kg.ntz, nty = P.kg.nty;
     // 32-bit multiply-high, not 64-bit divisions (~130 scalar instructions each)
     const uint32_t kxy = P.fntz.div((uint32_t)k), kx = P.fnty.div(kxy);
@@ -203,7 +241,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
     const int ox = tx * TX, oy = ty * TY, oz = tz * TZ;
     const int wx = min(TX, P.kg.d - ox), wy = min(TY, P.kg.d - oy), wz = min(TZ, P.kg.d - oz);  // the tile's own cells
     // the next item (uniform over the workgroup)
-    const uint32_t nitem = item + gridDim.x;
+    const uint32_t nitem = next_of(item);
     ItemRange nir;
     const bool next = range_of(nitem, nir);
     for (uint32_t e0 = 0; e0 < ents; e0 += UNR * eu) {
@@ -307,7 +345,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
     } else {
       // a split tile: this item's raw accumulators (fixed-point integers, or
       // the FP64 sums), which k_reduce_partials adds up
-      Acc *out = reinterpret_cast<Acc *>(partials) + (int64_t)(part_start[k] + j) * P.cells;
+      Acc *out = reinterpret_cast<Acc *>(partials) + (int64_t)item * P.cells;
       for (int64_t c = threadIdx.x; c < P.cells; c += DEP_THREADS) {
         out[c] = acc[c];
         acc[c] = 0;
@@ -326,7 +364,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
 // order of the records within a tile is not fixed); FP64 partials (masses
 // beyond the fixed-point range) add in item order.
 template <typename Real, int NM>
-__global__ void __launch_bounds__(256) k_reduce_partials(const uint32_t *__restrict__ nheavy,
+__global__ void __launch_bounds__(256) k_reduce_partials(const uint32_t *__restrict__ counts,
                                                          const uint32_t *__restrict__ heavy,
                                                          const uint32_t *__restrict__ part_start,
                                                          const double *__restrict__ partials, DepParams P,
@@ -341,14 +379,14 @@ __global__ void __launch_bounds__(256) k_reduce_partials(const uint32_t *__restr
   const uint64_t *raw = reinterpret_cast<const uint64_t *>(partials);
   const int64_t cells = P.cells;
   const int64_t nblk = ceil_div(cells, 256);
-  const int64_t units = (int64_t)(*nheavy) * nblk;
+  const int64_t units = (int64_t)counts[0] * nblk;
   for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
     // units < 2^31 (heavy tiles < 2^22, blocks per tile < 2^8): 32-bit multiply-high
     const uint32_t h = P.fnblk.div((uint32_t)u);
     const uint32_t k = heavy[h];
     const int64_t c = (int64_t)((uint32_t)u - h * (uint32_t)nblk) * 256 + threadIdx.x;
     if (c >= cells) continue;
-    const uint32_t m = P.list.item_start[k + 1] - P.list.item_start[k];
+    const uint32_t m = part_start[k + 1] - part_start[k];
     const int64_t at = (int64_t)part_start[k] * cells + c;
     double s;
     if (fixed) {
@@ -484,24 +522,17 @@ __global__ void __launch_bounds__(FOLD_THREADS) k_fold(const Real *__restrict__ 
   }
 }
 
-// Persistent grid of the deposit: the workgroups that stay resident (one
-// per CU with a 147 KB tile), at most one per item.
-template <typename Real, int NM, int RW, bool STD>
-int64_t deposit_grid_of(size_t lds, int64_t max_items) {
+// Deposit workgroups that stay resident on a CU (one with a 147 KB tile).
+template <typename Real, int NM, int RW>
+int deposit_per_cu(bool std_tiles, size_t lds) {
+  const void *fn = std_tiles ? reinterpret_cast<const void *>(&k_deposit<Real, NM, RW, true>)
+                             : reinterpret_cast<const void *>(&k_deposit<Real, NM, RW, false>);
   int per_cu = 0;
-  GENPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &per_cu, reinterpret_cast<const void *>(&k_deposit<Real, NM, RW, STD>), DEP_THREADS, lds));
-  return std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), max_items));
+  GENPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, DEP_THREADS, lds));
+  return std::max(per_cu, 1);
 }
 
-template <int NM, int RW>
-int64_t deposit_grid(const Plan &p, bool std_tiles, size_t lds, int64_t max_items) {
-  if (p.prec == 4)
-    return std_tiles ? deposit_grid_of<float, NM, RW, true>(lds, max_items)
-                     : deposit_grid_of<float, NM, RW, false>(lds, max_items);
-  return std_tiles ? deposit_grid_of<double, NM, RW, true>(lds, max_items)
-                   : deposit_grid_of<double, NM, RW, false>(lds, max_items);
-}
+bool std_tiles_of(const TileGeom &tg) { return tg.TX == 16 && tg.TY == 32 && tg.TZ == 32; }
 
 template <int NM, int RW>
 void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
@@ -509,9 +540,9 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
   const TileGeom &tg = p.tg;
   const int store = p.tiles_live ? 0 : 1;
   const float *sorted = o.rec;
-  const uint32_t *part_start = o.part_start, *nheavy = o.nheavy, *heavy = o.heavy;
-  const int64_t n = o.n, max_items = o.list.max_items;
-  double *partials = static_cast<double *>(p.partials.ensure((size_t)o.max_parts * tg.cells * 8 + 64));
+  const TileList &L = o.list;
+  const int64_t n = o.n;
+  double *partials = static_cast<double *>(p.partials.ensure((size_t)L.max_parts * tg.cells * 8 + 64));
 
   DepParams P;
   P.kg = kg;
@@ -532,29 +563,29 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
   const size_t lds = (size_t)tg.cells * 8;
   {
     Stage st(p, "deposit_tiles");
-    const bool std_tiles = tg.TX == 16 && tg.TY == 32 && tg.TZ == 32;
-    const dim3 grid((unsigned)deposit_grid<NM, RW>(p, std_tiles, lds, max_items)), block(DEP_THREADS);
+    const bool std_tiles = std_tiles_of(tg);
+    const dim3 grid(L.wgs), block(DEP_THREADS);
     if (p.prec == 4 && std_tiles)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, true>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
-                         o.list.start, o.list.blist, part_start, P, p.tiles.as<float>(), partials);
+      hipLaunchKernelGGL((k_deposit<float, NM, RW, true>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
+                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
     else if (p.prec == 4)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, false>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
-                         o.list.start, o.list.blist, part_start, P, p.tiles.as<float>(), partials);
+      hipLaunchKernelGGL((k_deposit<float, NM, RW, false>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
+                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
     else if (std_tiles)
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, true>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
-                         o.list.start, o.list.blist, part_start, P, p.tiles.as<double>(), partials);
+      hipLaunchKernelGGL((k_deposit<double, NM, RW, true>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
+                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
     else
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, false>), grid, block, lds, s, sorted, o.list.item_tile, o.list.item_start,
-                         o.list.start, o.list.blist, part_start, P, p.tiles.as<double>(), partials);
+      hipLaunchKernelGGL((k_deposit<double, NM, RW, false>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
+                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
     GENPK_LAUNCH_CHECK();
   }
   {
     Stage st(p, "reduce_partials");
     if (p.prec == 4)
-      hipLaunchKernelGGL((k_reduce_partials<float, NM>), dim3(1024), dim3(256), 0, s, nheavy, heavy, part_start,
+      hipLaunchKernelGGL((k_reduce_partials<float, NM>), dim3(1024), dim3(256), 0, s, L.counts, o.heavy, L.part_start,
                          partials, P, p.tiles.as<float>());
     else
-      hipLaunchKernelGGL((k_reduce_partials<double, NM>), dim3(1024), dim3(256), 0, s, nheavy, heavy, part_start,
+      hipLaunchKernelGGL((k_reduce_partials<double, NM>), dim3(1024), dim3(256), 0, s, L.counts, o.heavy, L.part_start,
                          partials, P, p.tiles.as<double>());
     GENPK_LAUNCH_CHECK();
   }
@@ -602,6 +633,14 @@ FoldGeom fold_geom(const Plan &p) {
   F.cz = tg.cz;
   F.zoff = tg.K * tg.cm;
   return F;
+}
+
+int64_t deposit_wgs(const Plan &p, int rw, int64_t max_items) {
+  const bool st = std_tiles_of(p.tg);
+  const size_t lds = (size_t)p.tg.cells * 8;
+  const int per_cu = p.prec == 4 ? (rw == 4 ? deposit_per_cu<float, 1, 4>(st, lds) : deposit_per_cu<float, 0, 3>(st, lds))
+                                 : (rw == 4 ? deposit_per_cu<double, 1, 4>(st, lds) : deposit_per_cu<double, 0, 3>(st, lds));
+  return std::min({(int64_t)per_cu * num_cus(), DEPOSIT_WGS_MAX, max_items});
 }
 
 void deposit(Plan &p, double boxsize, int64_t n, const float *pos, const float *masses, double mass, bool retain) {

@@ -86,14 +86,22 @@ enum class FieldState { None, Real, Spectrum, YDone };
 
 // The particles of a partition by tile, as the tile kernels read them: tile
 // k's records fill the listed blocks [start[k], start[k + 1]) of 2^lg record
-// slots (entry: the block in the low 32 - lg bits, its fill less one above);
-// its work items are [item_start[k], item_start[k + 1]).
+// slots (entry: the block in the low 32 - lg bits, its fill less one above).
+// Work items [0, counts[1]) are those of the split tiles, tile k's from
+// part_start[k] on (each writes a partial tile of its number), the
+// counts[2] items after them those of one tile each.
 struct TileList {
-  const uint32_t *start = nullptr, *item_start = nullptr;
-  const uint32_t *item_tile = nullptr;  // tile of each work item (max_items entries)
+  const uint32_t *start = nullptr, *part_start = nullptr;
+  // tile of each item of split tiles (max_parts entries), then of each other
+  const uint32_t *item_tile = nullptr;
+  const uint32_t *counts = nullptr;  // split tiles, their items, items of one tile
+  // the deposit's schedule over wgs workgroups (k_dir): cost of the items of
+  // one tile before the middle of each, and where each workgroup's begin
+  const uint32_t *cost = nullptr, *share = nullptr;
   const uint32_t *blist = nullptr;
   int lg = 0;
   int64_t ks = 0, max_items = 0;
+  uint32_t max_parts = 0, wgs = 1;
   __device__ __forceinline__ uint32_t slot0(uint32_t ent) const { return ent << lg; }  // first slot of the entry's block
   __device__ __forceinline__ uint32_t fill(uint32_t ent) const { return (ent >> (32 - lg)) + 1; }
 };
@@ -107,12 +115,11 @@ struct TileOrder {
   bool has_mass = false, has_perm = false;
   const uint32_t *perm1 = nullptr, *perm2 = nullptr;
   TileList list;
-  const uint32_t *part_start = nullptr;  // first partial tile of each split tile
-  const uint32_t *nheavy = nullptr, *heavy = nullptr;
+  const uint32_t *heavy = nullptr;  // the split tiles, in any order
   // with masses: [0] the bits of the largest |mass|, [1] those of the
   // smallest nonzero |mass| (0xffffffff when every mass is 0)
   const uint32_t *mrange = nullptr;
-  int64_t n = 0, max_parts = 0;  // max_parts: bound of the partial tiles
+  int64_t n = 0;
 };
 
 // Tile order kept from the last deposit made with retain = true, for the

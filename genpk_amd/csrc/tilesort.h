@@ -50,40 +50,46 @@ __device__ __forceinline__ int cell_of_x86(float p, double units, int d, double 
   return c;
 }
 
-// Work item -> tile k and its list entries [lb, le): tile k has m items that
-// split its blocks evenly; j is the item's number within the tile.
-// item_tile is read at min(item, max_items - 1) before the item count is
-// known, and used only below the count.  Returns false past the last item.
+// Work item -> tile k and its list entries [lb, le).  Items below nsplit are
+// those of split tiles, m > 1 of tile k from item part_start[k] on, which
+// split its blocks evenly; the others are one per tile (m = 1).
 struct ItemRange {
   int64_t k;
-  uint32_t m, j, lb, le;
+  uint32_t m, lb, le;
 };
 // The tables come as restrict kernel arguments (not inside a struct), so that
 // these uniform reads are scalar loads also after the kernel has stored.
-__device__ __forceinline__ bool item_range(const uint32_t *__restrict__ item_tile,
-                                           const uint32_t *__restrict__ item_start,
-                                           const uint32_t *__restrict__ start, int64_t ks, int64_t max_items,
+__device__ __forceinline__ void item_range(const uint32_t *__restrict__ item_tile,
+                                           const uint32_t *__restrict__ part_start,
+                                           const uint32_t *__restrict__ start, uint32_t nsplit, uint32_t max_parts,
                                            uint32_t item, ItemRange &r) {
-  const uint32_t total = item_start[ks];
-  const uint32_t k = item_tile[min((int64_t)item, max_items - 1)];
-  if (item >= total) return false;
+  const bool split = item < nsplit;
+  const uint32_t k = item_tile[split ? item : item - nsplit + max_parts];
   r.k = k;
-  const uint32_t i0 = item_start[k], i1 = item_start[k + 1];
-  const uint32_t t0 = start[k], t1 = start[k + 1];
-  r.m = i1 - i0;
-  r.j = item - i0;
-  const uint32_t per = r.m == 1 ? t1 - t0 : (t1 - t0 + r.m - 1) / r.m;  // most tiles are one item
-  r.lb = min(t1, t0 + r.j * per);
-  r.le = min(t1, r.lb + per);
-  return true;
+  r.m = 1;
+  r.lb = start[k];
+  r.le = start[k + 1];
+  if (split) {
+    const uint32_t p0 = part_start[k];
+    r.m = part_start[k + 1] - p0;
+    const uint32_t per = (r.le - r.lb + r.m - 1) / r.m;
+    r.lb = min(r.le, r.lb + (item - p0) * per);
+    r.le = min(r.le, r.lb + per);
+  }
 }
 
 // Records per work item at most for n particles over `tiles` tiles:
 // DEPOSIT_ITEM_MAX, halved (down to DEPOSIT_ITEM_MIN) while the items would
-// number fewer than four per CU or one full item would hold more than half
-// of a CU's share of the particles, so that a few heavy tiles still spread
-// over the CUs (their items' partial tiles are summed afterwards).
+// number fewer than four per CU or one full item would hold more than half of
+// a CU's share of the particles (a quarter, where that leaves tiles of twice
+// the mean in one item), so that heavy tiles spread evenly over the CUs (their
+// items' partial tiles are summed afterwards).
 uint32_t deposit_item_max(int64_t n, int64_t tiles);
+
+// Workgroups of the deposit over records of rw floats: those that stay
+// resident, at most DEPOSIT_WGS_MAX and one per item.
+constexpr int64_t DEPOSIT_WGS_MAX = 1024;
+int64_t deposit_wgs(const Plan &p, int rw, int64_t max_items);
 
 // Partition the n particles of one call (n <= 2^31) by tile into plan
 // scratch and build the work items (at most deposit_item_max records each).

@@ -41,6 +41,25 @@ def _positions(torch, n, kind):
 
 
 @pytest.mark.gpu
+def test_many_split_tiles(gpu):
+    """More than 1024 split tiles (1280 tiles of 4^3 cells with about 34000
+    particles each, items of at most 32768): the same sums as with the default
+    tiles, exact integers as above."""
+    import torch
+    n = 44000000
+    g = torch.Generator(device="cuda").manual_seed(2)
+    pos = torch.rand((n, 3), device="cuda", generator=g) * BOX
+    pos[:, 0] *= 5 / 16
+    got = []
+    for shape in ((4, 4, 4), (16, 32, 32)):
+        p = genpk_amd.Plan(64, "f64").set_options(shape)
+        p.clear()
+        p.deposit(pos, BOX)
+        got.append(p.export_density().clone())
+    assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,d", CASES)
 @pytest.mark.parametrize("kind", ["spread", "cell"])
 @pytest.mark.parametrize("masses", [False, True])
