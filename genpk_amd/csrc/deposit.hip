@@ -124,11 +124,15 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   const int lg = T.lg;
   const uint32_t in = threadIdx.x & ((1u << lg) - 1), te = threadIdx.x >> lg, eu = (uint32_t)DEP_THREADS >> lg;
   // this workgroup's items (k_dir's schedule): w, w + grid, ... of split
-  // tiles, then [one0, one1); NONE after the last
+  // tiles, then one0, one0 + ostep, ... below one1; NONE after the last
   constexpr uint32_t NONE = 0xffffffffu;
   const uint32_t nsplit = counts[1], none1 = counts[2];
-  uint32_t one0, one1;
-  if (nsplit + none1 <= gridDim.x) {
+  uint32_t one0, one1, ostep = 1;
+  if (nsplit == 0) {
+    one0 = blockIdx.x;
+    one1 = none1;
+    ostep = gridDim.x;
+  } else if (nsplit + none1 <= gridDim.x) {
     one0 = max((uint32_t)blockIdx.x, nsplit);
     one1 = blockIdx.x < nsplit ? one0 : min(one0 + 1, nsplit + none1);
   } else {
@@ -152,7 +156,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   auto first_one = [&]() { return one0 < one1 ? one0 : NONE; };
   auto next_of = [&](uint32_t it) -> uint32_t {
     if (it < nsplit) return it + gridDim.x < nsplit ? it + gridDim.x : first_one();
-    return it < NONE && it + 1 < one1 ? it + 1 : NONE;
+    return it < NONE && it + ostep < one1 ? it + ostep : NONE;
   };
   auto range_of = [&](uint32_t it, ItemRange &o) {
     if (it == NONE) return false;

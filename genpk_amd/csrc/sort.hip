@@ -229,14 +229,26 @@ __device__ __forceinline__ uint32_t wave_offsets(uint32_t *whist, int nbt, int h
   return tot;
 }
 
+// Inclusive scan of a whole wave by DPP moves, with no LDS round trip: within
+// the rows of 16 lanes, then row 0's and 2's sums into the rows after them and
+// the first half's into the second.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t t = __shfl_up(v, off, 64);
-    if (lane >= off) v += t;
-  }
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
   return v;
+}
+
+// Of the waves' totals in LDS: the sum of those before this wave's, and of
+// all (one read per lane and a scan, not a read and an add per wave).
+__device__ __forceinline__ uint32_t waves_before(const uint32_t *wtot, uint32_t &all) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t t = wtot[lane & (SORT_WAVES - 1)], incl = wave_incl_scan(lane < SORT_WAVES ? t : 0u);
+  all = __builtin_amdgcn_readlane(incl, SORT_WAVES - 1);
+  return __builtin_amdgcn_readlane(incl, wave) - __builtin_amdgcn_readlane(t, wave);
 }
 
 // One round of a block-wide exclusive scan (one value per thread), added to
@@ -248,13 +260,8 @@ __device__ __forceinline__ uint32_t block_scan_round(uint32_t v, uint32_t (*wtot
   const uint32_t incl = wave_incl_scan(v);
   if (lane == 63) wtot[rd & 1][wave] = incl;
   __syncthreads();
-  uint32_t run = carry + incl - v, all = 0;
-#pragma unroll
-  for (int w = 0; w < SORT_WAVES; w++) {
-    const uint32_t t = wtot[rd & 1][w];
-    if (w < wave) run += t;
-    all += t;
-  }
+  uint32_t all;
+  const uint32_t run = carry + incl - v + waves_before(wtot[rd & 1], all);
   carry += all;
   return run;
 }
@@ -531,7 +538,10 @@ __global__ void k_seg_tot(const uint32_t *__restrict__ t1scan, int64_t g1, int n
 //
 // Schedule: the deposit's workgroup w takes the items w, w + wgs, ... of split
 // tiles, then a run of the items of one tile, whose bounds share every
-// workgroup the same cost in all (an item costs its records and icost).  With
+// workgroup the same cost in all (an item costs its record slots and icost).
+// Without split tiles no tile is heavy and the items are strided over the
+// workgroups (shared by cost they took 5 us more here and gained nothing:
+// 13.8e6 lattice particles at 360^3).  With
 // all items strided over the workgroups the one with the most heavy tiles held
 // 1.5 to 2 times the mean of clumped particles: deposit 0.221 -> 0.173 ms for
 // 2e7 at 384^3, 0.83 -> 0.55 for 1e8 at 512^3, 5.70 -> 5.12 for 2^30 at 1024^3.
@@ -607,7 +617,9 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
       v[0][i] = ents;
       v[1][i] = m == 1 ? 1u : 0u;
       v[2][i] = m > 1 ? m : 0u;
-      v[3][i] = (m > 1 ? recs / m + D.icost : m == 1 ? recs + D.icost : 0u) >> D.cshift;  // an item's
+      const uint32_t slots = (ents << D.lg) >> D.cshift;
+      v[3][i] = m == 0 ? 0u : slots + D.icost;
+      if (m > 1) v[3][i] = slots / m + D.icost;  // an item's
       if (k < D.nb) D.tot[k] = 0ull;
 #pragma unroll
       for (int j = 0; j < NV; j++) sum[j] += j == 3 && m > 1 ? 0u : v[j][i];
@@ -622,12 +634,11 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < NV; j++)
-      for (int w = 0; w < SORT_WAVES; w++) {
-        const uint32_t x = wt[rd][j][w];
-        if (w < wave) run[j] += x;
-        carry[j] += x;
-      }
+    for (int j = 0; j < NV; j++) {
+      uint32_t all;
+      run[j] += waves_before(wt[rd][j], all);
+      carry[j] += all;
+    }
 #pragma unroll
     for (int i = 0; i < DIR_PER; i++) {
       const int64_t k = k0 + i;
@@ -669,7 +680,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
       for (uint32_t q = lane; q < t.z; q += 64) split_item(t.x, t.y + q, t.w);
     }
   }
-  if (!D.unit && carry[1] + carry[2] > D.wgs) {
+  if (!D.unit && carry[2] && carry[1] + carry[2] > D.wgs) {
     // what each workgroup has left to the mean of all, in proportion of the
     // cost of the items of one tile (fewer items: one each, k_deposit)
     __syncthreads();
@@ -1040,10 +1051,12 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   D.max_parts = (uint32_t)max_parts;
   D.wgs = (uint32_t)deposit_wgs(p, RW, max_items);
   D.fwgs = FastDiv(D.wgs);
-  // the flush of a tile takes about as long as the records of an eighth of
-  // its cells
-  D.icost = (uint32_t)(tg.cells / 8);
-  while (((n + ks * (int64_t)D.icost) >> D.cshift) >= (int64_t)1 << 31) D.cshift++;
+  // the flush of a tile and the waits around it take about as long as the
+  // records of an eighth of its cells (a quarter and a half measured the same
+  // within 3%)
+  const int64_t icost = tg.cells / 8;
+  while (((slots + max_items * icost) >> D.cshift) >= (int64_t)1 << 31) D.cshift++;
+  D.icost = (uint32_t)(icost >> D.cshift);
   D.nonfinite = static_cast<uint32_t *>(p.nonfinite.ensure(64));
   D.mrange = mrange;
   D.mrange_w = mrange_w;
