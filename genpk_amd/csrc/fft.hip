@@ -52,7 +52,7 @@ template <> struct FftCfg<double> { static constexpr int ELEMS = 4096; static co
 template <typename T, bool FROM_TILES, bool BFLY = false, int CT = 0, bool STD = false>
 __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) k_r2c_z(T *__restrict__ field, const T *__restrict__ tiles,
                                                       FoldGeom fg, FastDiv fdd, int64_t rowlen, int64_t nrows, int L,
-                                                      FastDiv fdM, FastDiv fdM1, RadixPlan rp,
+                                                      FastDiv fdM, FastDiv fdK, RadixPlan rp,
                                                       const typename Cx<T>::C *__restrict__ twM,
                                                       const typename Cx<T>::C *__restrict__ twd) {
   using C = typename Cx<T>::C;
@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
   const int tot = L * M;
   // twiddles of the M-point FFT and of the even/odd split, staged in LDS
   C *stw = buf + lds_len<true>((int64_t)L * M);  // [M]
-  C *sxw = stw + M;               // [M+1]
+  C *sxw = stw + M;               // [NK]
   if constexpr (BFLY) {
     // butterfly u = threadIdx.x + FFT_THREADS * i: row u / NQ, inputs
     // u % NQ + NQ * r (NQ = M / 8)
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
       }
     }
     for (int i = threadIdx.x; i < M; i += FFT_THREADS) stw[i] = twM[i];
-    for (int i = threadIdx.x; i <= M; i += FFT_THREADS) sxw[i] = twd[i];
+    for (int i = threadIdx.x; i < (M + 1) / 2; i += FFT_THREADS) sxw[i] = twd[i];
     __syncthreads();
     if constexpr (CT == 512)
       lds_fft_ct<512, 8, -1, false, MAXE, false, C, true, 8, 8>(buf, buf, L, 0, stw);
@@ -245,56 +245,41 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
     if (i < tot) buf[lds_ix<true>(i)] = v[q];
   }
   for (int i = threadIdx.x; i < M; i += FFT_THREADS) stw[i] = twM[i];
-  for (int i = threadIdx.x; i <= M; i += FFT_THREADS) sxw[i] = twd[i];
+  for (int i = threadIdx.x; i < (M + 1) / 2; i += FFT_THREADS) sxw[i] = twd[i];
   __syncthreads();
   if constexpr (CT == 512)
     lds_fft_ct<512, 1, -1, false, MAXE, false, C, true, 8, 8, 8>(buf, buf, L, 0, stw);
   else
     lds_fft<-1, false, MAXE, C, true>(buf, rp, L, 0, 1, M, stw);
   }
-  // X_k = (Z_k + conj Z_{M-k})/2 - i/2 * w^k (Z_k - conj Z_{M-k}),  w = exp(-2 pi i / d)
-  auto split = [&](C zk, C zc, C w) {
-    const C e = C{(zk.x + zc.x) * (T)0.5, (zk.y + zc.y) * (T)0.5};
-    const C o = C{(zk.y - zc.y) * (T)0.5, -(zk.x - zc.x) * (T)0.5};  // (zk - zc) / (2i)
-    return cadd(e, cmul(o, w));
+  // X_k = E + w^k O and X_{M-k} = conj(E - w^k O) with E = (Z_k + conj Z_{M-k}) / 2,
+  // O = (Z_k - conj Z_{M-k}) / 2i, w = exp(-2 pi i / d) and Z_M = Z_0: one thread
+  // forms both (each by its own thread took twice the LDS reads and index
+  // arithmetic, in a pass that fills the SIMDs (0.9 to 1.0 VALU instructions a
+  // cycle in FP32): 0.258 -> 0.244 ms at 360^3 FP64, 0.570 -> 0.550 at 512^3,
+  // 0.99 -> 0.91 at 720^3 FP32, but 2.17 -> 2.20 at 1024^3)
+  auto split = [&](int l, int k, C w) {
+    const C zk = buf[lds_ix<true>(l * M + k)], zc = buf[lds_ix<true>(l * M + (k == 0 ? 0 : M - k))];
+    const C e = C{(zk.x + zc.x) * (T)0.5, (zk.y - zc.y) * (T)0.5};
+    const C o = cmul(C{(zk.y + zc.y) * (T)0.5, (zc.x - zk.x) * (T)0.5}, w);
+    C *row = reinterpret_cast<C *>(field + (row0 + l) * rowlen);
+    row[k] = cadd(e, o);
+    row[M - k] = C{e.x - o.x, o.y - e.y};
+    // k = M / 2 is its own partner, with w^(M/2) = -i
+    if (k == 0 && M % 2 == 0) row[M / 2] = cconj(buf[lds_ix<true>(l * M + M / 2)]);
   };
-  if (M == FFT_THREADS) {
-    // output k = threadIdx.x of every row (L <= MAXE rows), and k = M by thread 0
-    const int k = threadIdx.x;
-    const C w = sxw[k], wm = sxw[M];
-#pragma unroll
-    for (int l = 0; l < MAXE; l++) {
-      if (l < nl) {
-        const C zk = buf[lds_ix<true>(l * M + k)];
-        const C zc = cconj(buf[lds_ix<true>(l * M + (k == 0 ? 0 : M - k))]);
-        C *row = reinterpret_cast<C *>(field + (row0 + l) * rowlen);
-        row[k] = split(zk, zc, w);
-        if (k == 0) row[M] = split(zk, zc, wm);
-      }
-    }
-    return;
-  }
-  if (FFT_THREADS % M == 0) {
-    // M a smaller power of two: output k = threadIdx.x % M of rows
-    // threadIdx.x / M + FFT_THREADS / M * i, and k = M by the threads of k = 0
-    const int k = threadIdx.x & (M - 1), rpi = FFT_THREADS / M;
-    const C w = sxw[k], wm = sxw[M];
+  const int NK = (M + 1) / 2;
+  if ((NK & (NK - 1)) == 0 && NK <= FFT_THREADS) {
+    // a power of two: a thread keeps its k
+    const int k = threadIdx.x & (NK - 1), rpi = FFT_THREADS / NK;
+    const C w = sxw[k];
 #pragma unroll 4
-    for (int l = threadIdx.x / M; l < nl; l += rpi) {
-      const C zk = buf[lds_ix<true>(l * M + k)];
-      const C zc = cconj(buf[lds_ix<true>(l * M + (k == 0 ? 0 : M - k))]);
-      C *row = reinterpret_cast<C *>(field + (row0 + l) * rowlen);
-      row[k] = split(zk, zc, w);
-      if (k == 0) row[M] = split(zk, zc, wm);
-    }
+    for (int l = threadIdx.x / NK; l < nl; l += rpi) split(l, k, w);
     return;
   }
-  const int nout = M + 1;
-  for (int i = threadIdx.x; i < nl * nout; i += FFT_THREADS) {
-    const int l = (int)fdM1.div((uint32_t)i), k = i - l * nout;
-    const C zk = buf[lds_ix<true>(l * M + (k == M ? 0 : k))];
-    const C zc = cconj(buf[lds_ix<true>(l * M + (k == 0 ? 0 : M - k))]);
-    reinterpret_cast<C *>(field + (row0 + l) * rowlen)[k] = split(zk, zc, sxw[k]);
+  for (int i = threadIdx.x; i < nl * NK; i += FFT_THREADS) {
+    const int l = (int)fdK.div((uint32_t)i), k = i - l * NK;
+    split(l, k, sxw[k]);
   }
 }
 
@@ -533,7 +518,7 @@ static void r2c_z_impl(Plan &p, bool from_tiles) {
   const C *twd = (p.prec == 4) ? (const C *)p.fft.tw_d_f32.ptr : (const C *)p.fft.tw_d_f64.ptr;
   const FoldGeom fg = fold_geom(p);
   const dim3 grid((unsigned)ceil_div(nrows, L));
-  const size_t lds = ((size_t)lds_len<true>((int64_t)L * M) + 2 * M + 1) * sizeof(C);
+  const size_t lds = ((size_t)lds_len<true>((int64_t)L * M) + M + (M + 1) / 2) * sizeof(C);
   // the d = 1024 plan of radices 8, 8, 8 runs compile-time stages
   const bool ct512 = M == 512 && rp.nst == 3 && rp.st[0].R == 8 && rp.st[1].R == 8 && rp.st[2].R == 8;
   // FP64 at d = 1024 (seven rows a workgroup) reads the rows element-wise:
@@ -545,37 +530,37 @@ static void r2c_z_impl(Plan &p, bool from_tiles) {
     Stage st(p, "fold_fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, true, true, 512, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
-                       FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                       FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && bfly && ct512) {
     Stage st(p, "fold_fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, true, true, 512>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
-                       FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                       FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && bfly) {
     Stage st(p, "fold_fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, true, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
-                       FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                       FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && ct512 && std_tiles) {
     Stage st(p, "fold_fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, true, false, 512, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
-                       FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                       FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && ct512) {
     Stage st(p, "fold_fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, true, false, 512>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
-                       FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                       FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles) {
     Stage st(p, "fold_fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
-                       FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                       FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else {
     Stage st(p, "fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, false>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        (const T *)nullptr, fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
-                       FastDiv((uint32_t)(M + 1)), rp, twM, twd);
+                       FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   }
   GENPK_LAUNCH_CHECK();
 }

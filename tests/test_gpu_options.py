@@ -188,3 +188,24 @@ def test_options_errors(gpu):
     q = genpk_amd.Plan(16, "f64")
     q.set_options((16, 32, 32), 0)         # clamped to the grid
     assert q.options()["tiles"] == (16, 16, 16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("d", [2, 4, 6, 8, 10, 18, 30, 64, 72, 150, 162])
+def test_spectrum_pairs_edges(gpu, d, prec):
+    """The even/odd split forms the modes k and d/2 - k together: half lengths
+    that are odd, even, one, and with a power of two of pairs or not.  A
+    transform's errors are about eps sqrt(log2 N) of its rms, sqrt(N) here;
+    the bound is 8 eps log2 N of it."""
+    import numpy as np
+    import torch
+    print("CASE", d, prec, flush=True)
+    p = genpk_amd.Plan(d, prec)
+    g = torch.Generator(device="cuda").manual_seed(d)
+    x = torch.randn(p.grid.shape, device="cuda", dtype=p.real_dtype, generator=g)
+    p.import_density(x)
+    got = p.r2c().cpu().numpy().reshape(d, d, d // 2 + 1).astype(np.complex128)
+    ref = np.fft.rfftn(x.cpu().numpy().reshape(d, d, -1)[:, :, :d].astype(np.float64))
+    eps = 2.0 ** -53 if prec == "f64" else 2.0 ** -24
+    assert np.abs(got - ref).max() <= 8 * eps * np.log2(d ** 3) * np.sqrt(d ** 3)
