@@ -93,6 +93,19 @@ __device__ __forceinline__ void run_add(RunAcc &r, int b, const double *c, doubl
   for (int s = 0; s < NS; s++) r.v[s] += c[s];
 }
 
+// Terms of a pair of modes of one weight, kx and -kx: their products add before
+// the weight (the second pair of values 0 for a mode alone).
+template <typename C, int NF>
+__device__ __forceinline__ void pair_terms(const C &fa, const C &ga, const C &fb, const C &gb, double h, double dc,
+                                           double *c) {
+  auto dot = [](const C &u, const C &v) { return (double)u.x * (double)v.x + (double)u.y * (double)v.y; };
+  c[0] = h * (dot(fa, fa) + dot(ga, ga)) * dc;
+  if (NF == 2) {
+    c[1] = h * (dot(fb, fb) + dot(gb, gb)) * dc;
+    c[2] = h * (dot(fa, fb) + dot(ga, gb)) * dc;
+  }
+}
+
 template <typename C, int NF>
 __device__ __forceinline__ void mode_terms(const C &fa, const C &fb, double h, double dc, double *c) {
   const double ax = (double)fa.x, ay = (double)fa.y;
@@ -132,6 +145,11 @@ struct BinGeom {
 // binning, each thread pairing stage inputs j and j + n/2 into modes j and
 // j + n/2 in registers.
 //
+// Binning: a thread takes the modes kx and -kx of a column together, which
+// share |k|^2, so that a pair takes one bin lookup, one weight and one step of
+// the run: x pass + bin 1.87 -> 1.61 ms at 1024^3 FP32, 0.113 -> 0.098 at
+// 360^3; FP64 3.82 -> 3.60 at 1024^3, 0.036 -> 0.033 at 200^3.
+//
 // The registers hold the next block's loads while a block is binned: a
 // spilled value read back there waits for all of them (one spilled register
 // made the binning of a block 4.9 us instead of 2.7 at 1024^3 FP32), so each
@@ -163,10 +181,10 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
   const int64_t d = g.d, hz = g.hz;
   const int64_t estride = d * hz;
   const int64_t nblk = cm.nblk;
-  // bin-phase mapping: thread -> column b, contiguous run of e
+  // bin-phase mapping: thread -> column b, contiguous run of kx >= 0
   const int tpc = BIN_THREADS >> lgb;            // threads per column (B divides BIN_THREADS)
   const int my_b = threadIdx.x & (B - 1);
-  const int per = (n + tpc - 1) / tpc;
+  const int half = n / 2, per = (half + tpc - 1) / tpc;
   const int e0 = (int)(threadIdx.x >> lgb) * per;
   // register-staged loads of column block v: all its global reads in flight
   // together; with REG1 at a stride of the first stage's butterfly count
@@ -249,82 +267,103 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
       const int a = ky * ky + kz * kz;
       const float wy = wt[y], wz = wt[kz];
       RunAcc r;
-      // this thread's run of at most MAXE modes along x (per <= MAXE as
-      // n * B <= BIN_THREADS * MAXE); with one field all its LDS reads are
-      // issued first (two fields would not fit the registers)
+      // the modes kx and -kx of a column share |k|^2, so bin and weight: they
+      // are binned as one (see the kernel's comment)
+      auto weight = [&](int kx) {
+        const float gw = (wt[kx] * wy) * wz;  // the reference's ((wx*wy)*wz) in float
+        double dc = (double)gw * (double)gw;
+        return dc * dc;
+      };
+      auto bin_of = [&](int kx) { return bin_lds(max(a + kx * kx, 1), thr32, g.nrbins, g.lq); };
+      const C zero = C{0, 0};
       if constexpr (R2L) {
         // the last stage: butterfly jj pairs stage inputs jj and jj + n/2
-        // (the latter times w^jj) into modes jj and jj + n/2
-        constexpr int HB = MAXE / 2;
-        const int half = n / 2;
-        const int jb = (int)(threadIdx.x >> lgb) * HB;  // below half exactly for the loaders
-        C mo[MAXE];
+        // (the latter times w^jj) into modes jj and jj + n/2; with butterfly
+        // n/2 - jj, whose modes are -jj - n/2 and -jj, a thread holds two
+        // pairs.  Butterfly 0 (modes 0 and n/2, alone) goes with butterfly
+        // n/4 (modes n/4 and -n/4).
+        constexpr int HB = MAXE / 4;
+        const int jb = (int)(threadIdx.x >> lgb) * HB;  // below n/4 exactly for the loaders
+        C lo[HB], hi[HB], lo2[HB], hi2[HB];
         if (loader) {
-#pragma unroll
-        for (int q = 0; q < HB; q++) {
-          const int jj = jb + q;
-          const C a0 = res[(jj << lgb) + my_b];
-          const C v1 = cmul(res[((jj + half) << lgb) + my_b], stw[jj]);
-          mo[q] = cadd(a0, v1);
-          mo[q + HB] = csub(a0, v1);
-        }
-        // half the modes at a time: their bins, then their terms (all eight
-        // bins at once spill registers with the compile-time stages)
-#pragma unroll
-        for (int m = 0; m < MAXE; m += HB) {
-          const int eb = m ? jb + half : jb, kb = m ? jb - half : jb;  // d / 2 counts as -d / 2
-          int bq[HB];
-#pragma unroll
-          for (int q = 0; q < HB; q++) bq[q] = bin_lds(max(a + (kb + q) * (kb + q), 1), thr32, g.nrbins, g.lq);
+          auto last_stage = [&](int jj, C &l, C &u) {
+            const C a0 = res[(jj << lgb) + my_b];
+            const C v1 = cmul(res[((jj + half) << lgb) + my_b], stw[jj]);
+            l = cadd(a0, v1);
+            u = csub(a0, v1);
+          };
 #pragma unroll
           for (int q = 0; q < HB; q++) {
-            if (a != 0 || eb + q != 0) {
-              const float gw = (wt[eb + q] * wy) * wz;  // the reference's ((wx*wy)*wz) in float
-              double dc = (double)gw * (double)gw;
-              dc *= dc;
-              double t[3];
-              mode_terms<C, NF>(mo[m + q], mo[m + q], h, dc, t);
+            const int jj = jb + q;
+            last_stage(jj, lo[q], hi[q]);
+            last_stage(jj == 0 ? half / 2 : half - jj, lo2[q], hi2[q]);
+          }
+          int bq[2 * HB];
+#pragma unroll
+          for (int q = 0; q < HB; q++) {
+            bq[q] = bin_of(jb + q);
+            bq[q + HB] = bin_of(half - jb - q);
+          }
+          double t[3];
+#pragma unroll
+          for (int q = 0; q < HB; q++) {
+            const int kx = jb + q;
+            if (a != 0 || kx != 0) {
+              pair_terms<C, NF>(lo[q], kx == 0 ? zero : hi2[q], zero, zero, h, weight(kx), t);
               run_add<NS>(r, bq[q], t, my_bins, g.nrbins, lgc);
             }
           }
-        }
-        }
-        run_flush<NS>(r, my_bins, g.nrbins, lgc);
-      } else {
-      constexpr bool BATCH = NF == 1;
-      C ma[BATCH ? MAXE : 1];
-      float wx[BATCH ? MAXE : 1];
-      if (BATCH) {
 #pragma unroll
-        for (int j = 0; j < MAXE; j++) {
-          const int e = e0 + j;
-          if (j < per && e < n) {
-            ma[BATCH ? j : 0] = res[(e << lgb) + my_b];
-            if (!REG1) wx[BATCH ? j : 0] = wt[e];
+          for (int q = 0; q < HB; q++) {
+            const int kx = half - jb - q;
+            pair_terms<C, NF>(hi[q], kx == half ? zero : lo2[q], zero, zero, h, weight(kx), t);
+            run_add<NS>(r, bq[q + HB], t, my_bins, g.nrbins, lgc);
+          }
+          if (jb == 0) {
+            pair_terms<C, NF>(lo2[0], hi2[0], zero, zero, h, weight(half / 2), t);
+            run_add<NS>(r, bin_of(half / 2), t, my_bins, g.nrbins, lgc);
           }
         }
-      }
+      } else {
+        // this thread's run of at most MAXP pairs kx, -kx along x (per <= MAXP as
+        // n * B <= BIN_THREADS * MAXE); kx = 0 goes with kx = n/2, both alone.
+        // With one field all its LDS reads are issued first (two fields would
+        // not fit the registers)
+        constexpr int MAXP = MAXE / 2;
+        constexpr bool BATCH = NF == 1;
+        C ma[BATCH ? MAXP : 1], mb[BATCH ? MAXP : 1];
+        auto at = [&](int e) { return (e << lgb) + my_b; };
+        auto partner = [&](int e) { return e == 0 ? half : n - e; };
+        if (BATCH) {
 #pragma unroll
-      for (int j = 0; j < MAXE; j++) {
-        const int e = e0 + j;
-        if (j < per && e < n) {
-          const int kx = e <= d / 2 ? e : e - (int)d;
-          const int q = a + kx * kx;
-          if (q != 0) {
-            const int b = bin_lds(q, thr32, g.nrbins, g.lq);
-            const float gw = ((BATCH && !REG1 ? wx[BATCH ? j : 0] : wt[e]) * wy) * wz;  // the reference's ((wx*wy)*wz) in float
-            double dc = (double)gw * (double)gw;
-            dc *= dc;
-            const C fa_m = BATCH ? ma[BATCH ? j : 0] : res[(e << lgb) + my_b];
-            const C fb_m = NF == 2 ? res[tot + (e << lgb) + my_b] : fa_m;
+          for (int j = 0; j < MAXP; j++) {
+            const int e = e0 + j;
+            if (j < per && e < half) {
+              ma[BATCH ? j : 0] = res[at(e)];
+              mb[BATCH ? j : 0] = res[at(partner(e))];
+            }
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < MAXP; j++) {
+          const int e = e0 + j;
+          if (j < per && e < half) {
+            const C f = BATCH ? ma[BATCH ? j : 0] : res[at(e)];
+            const C fm = BATCH ? mb[BATCH ? j : 0] : res[at(partner(e))];
+            const C u = NF == 2 ? res[tot + at(e)] : zero, um = NF == 2 ? res[tot + at(partner(e))] : zero;
             double t[3];
-            mode_terms<C, NF>(fa_m, fb_m, h, dc, t);
-            run_add<NS>(r, b, t, my_bins, g.nrbins, lgc);
+            if (a + e != 0) {
+              pair_terms<C, NF>(f, e == 0 ? zero : fm, u, e == 0 ? zero : um, h, weight(e), t);
+              run_add<NS>(r, bin_of(e), t, my_bins, g.nrbins, lgc);
+            }
+            if (e == 0) {
+              pair_terms<C, NF>(fm, zero, um, zero, h, weight(half), t);
+              run_add<NS>(r, bin_of(half), t, my_bins, g.nrbins, lgc);
+            }
           }
         }
       }
       run_flush<NS>(r, my_bins, g.nrbins, lgc);
-      }
     }
     if constexpr (REG1 && NF == 1) {
       // the next first stage writes the buffer the binning did not read
