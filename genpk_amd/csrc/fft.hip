@@ -36,10 +36,14 @@ template <> struct FftCfg<double> { static constexpr int ELEMS = 4096; static co
 // register budget of two waves per SIMD is available.  The rows sit in LDS
 // with one element of padding per 32 (lds_ix), which spreads the strided
 // writes of the FFT stages over the banks.
-// BFLY (from the tile store, a first stage of radix 8, L * M / 8 <= 2 *
-// FFT_THREADS): each thread loads the eight inputs of up to two butterflies
-// of the first stage straight from the tile store and runs that stage from
-// registers.  CT = 512: the plan is M = 512 = 8 * 8 * 8 (d = 1024), run with
+// BFLY (from the tile store; the first stage's radix, 0: element by element):
+// each thread loads the inputs of whole butterflies of the first stage
+// straight from the tile store, one row's place for all of a butterfly's, and
+// runs that stage from registers.  The pass fills the SIMDs where each
+// element looks up its own place: 0.173 -> 0.138 ms at 360^3 FP32 (first radix
+// 4), 0.037 -> 0.029 at 200^3, 0.106 -> 0.088 at 300^3 (first radix 2); FP64
+// 0.243 -> 0.206 at 360^3, 1.00 -> 0.84 at 600^3.
+// CT = 512: the plan is M = 512 = 8 * 8 * 8 (d = 1024), run with
 // compile-time stages (fft_stage_ct); 0: any plan.  STD (with CT = 512):
 // the default 16 x 32 x 32 tiles, whose store offsets (below 2^31 at d =
 // 1024) are computed in 32 bits from compile-time strides, in the butterfly
@@ -49,7 +53,7 @@ template <> struct FftCfg<double> { static constexpr int ELEMS = 4096; static co
 // CU (waves_per_eu: four waves per SIMD): fold and z pass together 2.28 ->
 // 2.06 ms at 1024^3 FP32 and 0.069 -> 0.061 at 256^3 against two in-place
 // fold launches before the pass.
-template <typename T, bool FROM_TILES, bool BFLY = false, int CT = 0, bool STD = false>
+template <typename T, bool FROM_TILES, int BFLY = 0, int CT = 0, bool STD = false>
 __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) k_r2c_z(T *__restrict__ field, const T *__restrict__ tiles,
                                                       FoldGeom fg, FastDiv fdd, int64_t rowlen, int64_t nrows, int L,
                                                       FastDiv fdM, FastDiv fdK, RadixPlan rp,
@@ -66,16 +70,17 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
   // twiddles of the M-point FFT and of the even/odd split, staged in LDS
   C *stw = buf + lds_len<true>((int64_t)L * M);  // [M]
   C *sxw = stw + M;               // [NK]
-  if constexpr (BFLY) {
+  if constexpr (BFLY != 0) {
+    constexpr int R0 = BFLY, NB = R0 == 8 ? 2 : (MAXE + R0 - 1) / R0;
     // butterfly u = threadIdx.x + FFT_THREADS * i: row u / NQ, inputs
-    // u % NQ + NQ * r (NQ = M / 8)
-    const int NQ = M / 8;
+    // u % NQ + NQ * r (NQ = M / R0)
+    const int NQ = M / R0;
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < NB; i++) {
       const int u = threadIdx.x + FFT_THREADS * i;
-      const int b = CT ? u / (CT / 8) : (int)fdM.div((uint32_t)(8 * u)), j = u - b * NQ;
+      const int b = CT ? u / (CT / 8) : (int)fdM.div((uint32_t)(R0 * u)), j = u - b * NQ;
       if (b < L) {
-        C w[8];
+        C w[R0];
         if (STD && b < nl) {
           static_assert(!STD || CT == 512, "standard tiles with the d = 1024 loaders");
           // d = 1024, tiles 16 x 32 x 32 (17 x 33 halo'd rows of 32 per tile):
@@ -87,9 +92,9 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
           const uint32_t jz = (uint32_t)j >> 4, lz = 2u * ((uint32_t)j & 15u);
           const uint32_t base = (txy * 32u + jz) * CM + rr * 32u + lz;
           const T *tb = tiles + base;
-          T zh8[8];
+          T zh8[R0];
 #pragma unroll
-          for (int r = 0; r < 8; r++) {
+          for (int r = 0; r < R0; r++) {
             w[r] = C{tb[r * 4 * CM], tb[r * 4 * CM + 1]};
             // the previous tile along z's z-halo cell: tile column 4 r + jz - 1
             // (for r = jz = 0 the last column, 31, periodically)
@@ -97,20 +102,20 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
             zh8[r] = lz == 0 ? tiles[(uint32_t)fg.zoff + (txy * 32u + tzp) * CZ + rr] : (T)0;
           }
           if ((x & 15u) == 0 || (y & 31u) == 0)
-            add_halo_rows<T, 8, sizeof(T) == 4 ? 4 : 2>(tiles, fg, row_fold(fg, (int)x, (int)y), [&](int r) { return 2 * (j + 64 * r); }, w,
+            add_halo_rows<T, R0, R0 % 4 ? R0 : sizeof(T) == 4 ? 4 : 2>(tiles, fg, row_fold(fg, (int)x, (int)y), [&](int r) { return 2 * (j + 64 * r); }, w,
                                 zh8);
           if (lz == 0) {
 #pragma unroll
-            for (int r = 0; r < 8; r++) w[r].x = w[r].x + zh8[r];  // one rounding, as below
+            for (int r = 0; r < R0; r++) w[r].x = w[r].x + zh8[r];  // one rounding, as below
           }
         } else if (b < nl) {
           const int64_t row = row0 + b;
           const int x = (int)fdd.div((uint32_t)row), y = (int)(row - (int64_t)x * fg.d);
           const RowFold rf = row_fold(fg, x, y);
           const int64_t txy = rf.t, rr = rf.r;
-          T zh8[8];
+          T zh8[R0];
 #pragma unroll
-          for (int r = 0; r < 8; r++) {
+          for (int r = 0; r < R0; r++) {
             const int z = 2 * (j + NQ * r);
             const int tz = z >> fg.sz, lz = z & (fg.TZ - 1);
             const int64_t at = txy * fg.ntz * fg.cm + (int64_t)tz * fg.cm + rr * fg.TZ + lz;
@@ -126,16 +131,16 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
             }
           }
           if (rf.fx || rf.fy)
-            add_halo_rows<T, 8, sizeof(T) == 4 ? 4 : 2>(tiles, fg, rf, [&](int r) { return 2 * (j + NQ * r); }, w, zh8);
+            add_halo_rows<T, R0, R0 % 4 ? R0 : sizeof(T) == 4 ? 4 : 2>(tiles, fg, rf, [&](int r) { return 2 * (j + NQ * r); }, w, zh8);
 #pragma unroll
-          for (int r = 0; r < 8; r++) w[r].x = w[r].x + zh8[r];  // as the element-wise load: one rounding
+          for (int r = 0; r < R0; r++) w[r].x = w[r].x + zh8[r];  // as the element-wise load: one rounding
         } else {
 #pragma unroll
-          for (int r = 0; r < 8; r++) w[r] = C{0, 0};
+          for (int r = 0; r < R0; r++) w[r] = C{0, 0};
         }
-        Dft<8, -1, C>::run(w);
+        Dft<R0, -1, C>::run(w);
 #pragma unroll
-        for (int r = 0; r < 8; r++) buf[lds_ix<true>(b * M + 8 * j + r)] = w[r];
+        for (int r = 0; r < R0; r++) buf[lds_ix<true>(b * M + R0 * j + r)] = w[r];
       }
     }
     for (int i = threadIdx.x; i < M; i += FFT_THREADS) stw[i] = twM[i];
@@ -523,34 +528,47 @@ static void r2c_z_impl(Plan &p, bool from_tiles) {
   const bool ct512 = M == 512 && rp.nst == 3 && rp.st[0].R == 8 && rp.st[1].R == 8 && rp.st[2].R == 8;
   // FP64 at d = 1024 (seven rows a workgroup) reads the rows element-wise:
   // the butterfly loader measured 3.50 -> 3.73 ms there (0.52 -> 0.47 ms at 512)
-  const bool bfly = rp.st[0].R == 8 && rp.nst >= 2 && (int64_t)L * (M / 8) <= 2 * FFT_THREADS &&
-                    (sizeof(T) == 4 || !ct512);
+  // the first stage from registers, for every radix it can have (one stage alone,
+  // d <= 16, runs element by element)
+  const int r0 = rp.nst >= 2 ? rp.st[0].R : 0;
+  const bool bfly = r0 == 8 && (int64_t)L * (M / 8) <= 2 * FFT_THREADS && (sizeof(T) == 4 || !ct512);
   const bool std_tiles = p.d == 1024 && fg.TX == 16 && fg.TY == 32 && fg.TZ == 32;
   if (from_tiles && bfly && ct512 && std_tiles) {
     Stage st(p, "fold_fft_z");
-    hipLaunchKernelGGL((k_r2c_z<T, true, true, 512, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
+    hipLaunchKernelGGL((k_r2c_z<T, true, 8, 512, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
                        FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && bfly && ct512) {
     Stage st(p, "fold_fft_z");
-    hipLaunchKernelGGL((k_r2c_z<T, true, true, 512>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
+    hipLaunchKernelGGL((k_r2c_z<T, true, 8, 512>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
                        FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && bfly) {
     Stage st(p, "fold_fft_z");
-    hipLaunchKernelGGL((k_r2c_z<T, true, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
+    hipLaunchKernelGGL((k_r2c_z<T, true, 8>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
                        FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && ct512 && std_tiles) {
     Stage st(p, "fold_fft_z");
-    hipLaunchKernelGGL((k_r2c_z<T, true, false, 512, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
+    hipLaunchKernelGGL((k_r2c_z<T, true, 0, 512, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
                        FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
   } else if (from_tiles && ct512) {
     Stage st(p, "fold_fft_z");
-    hipLaunchKernelGGL((k_r2c_z<T, true, false, 512>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
+    hipLaunchKernelGGL((k_r2c_z<T, true, 0, 512>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
                        p.tiles.as<const T>(), fg, FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M),
                        FastDiv((uint32_t)((M + 1) / 2)), rp, twM, twd);
+  } else if (from_tiles && r0 >= 2 && r0 <= 5) {
+    Stage st(p, "fold_fft_z");
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(), p.tiles.as<const T>(), fg,
+                         FastDiv((uint32_t)p.d), p.rowlen, nrows, L, FastDiv((uint32_t)M), FastDiv((uint32_t)((M + 1) / 2)),
+                         rp, twM, twd);
+    };
+    if (r0 == 2) go(k_r2c_z<T, true, 2>);
+    else if (r0 == 3) go(k_r2c_z<T, true, 3>);
+    else if (r0 == 4) go(k_r2c_z<T, true, 4>);
+    else go(k_r2c_z<T, true, 5>);
   } else if (from_tiles) {
     Stage st(p, "fold_fft_z");
     hipLaunchKernelGGL((k_r2c_z<T, true>), grid, dim3(FFT_THREADS), lds, p.stream, p.field.as<T>(),
