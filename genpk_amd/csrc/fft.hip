@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_c2r_z(T *__restrict__ field, in
 // any plan.  R0 (a first radix below COLE): each thread loads the inputs of
 // COLE / R0 whole butterflies of the first stage and runs it from registers
 // (y pass FP32 0.060 -> 0.052 ms at 300^3, 0.261 -> 0.214 at 486^3, 1.54 -> 1.35
-// at 900^3, where the x pass alone takes 1.80 instead of 1.70).
+// at 900^3; cols_impl says where not).
 template <typename T, int SIGN, int CT = 0, int R0 = 0>
 __global__ void __launch_bounds__(COL_THREADS) k_cols(typename Cx<T>::C *__restrict__ f, ColMap cm, int axis,
                                                      RadixPlan rp, const typename Cx<T>::C *__restrict__ tw) {
@@ -638,7 +638,18 @@ static void cols_impl(Plan &p, int axis) {
   // the compile-time instances fill every thread (n * B = COL_THREADS * COLE)
   const bool full = p.d * B == (int64_t)COL_THREADS * FftCfg<T>::COLE;
   const bool ct1024 = is_plan_8882(rp) && full;
-  if (rp.st[0].R == FftCfg<T>::COLE && p.d * B <= (int64_t)COL_THREADS * FftCfg<T>::COLE) {
+  // FP32 blocks of less than a line (8 columns of 8 bytes from d = 514 on): the
+  // x pass is faster element by element than with a partly filled workgroup's
+  // first stage, or one of a smaller radix, from registers, by 2 to 16% (1.62
+  // against 1.84 ms at 900^3, 1.90 against 2.10 at 960^3; even from 1200 on), and the y
+  // pass by up to 8% with a first radix of 8 (0.416 against 0.451 ms at 600^3,
+  // 5.02 against 5.18 at 1280^3; 2% slower at 720^3).  With whole lines, in FP64
+  // and along y with a smaller radix the register stage is the faster one, or even
+  constexpr int COLE = FftCfg<T>::COLE;
+  const bool by_elements = sizeof(T) == 4 && p.d > 512 && (rp.st[0].R == COLE ? !full : axis == 0);
+  if (by_elements) {
+    hipLaunchKernelGGL((k_cols<T, SIGN>), grid, block, lds, p.stream, p.field.as<C>(), cm, axis, rp, tw);
+  } else if (rp.st[0].R == FftCfg<T>::COLE && p.d * B <= (int64_t)COL_THREADS * FftCfg<T>::COLE) {
     const bool l2 = rp.nst > 1 && rp.st[rp.nst - 1].R == 2;
     constexpr int CT4 = FftCfg<T>::COLE == 4 ? 1024 : 0;
     auto go = [&](auto kernel) {
