@@ -262,7 +262,8 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
   // forms both (each by its own thread took twice the LDS reads and index
   // arithmetic, in a pass that fills the SIMDs (0.9 to 1.0 VALU instructions a
   // cycle in FP32): 0.258 -> 0.244 ms at 360^3 FP64, 0.570 -> 0.550 at 512^3,
-  // 0.99 -> 0.91 at 720^3 FP32, but 2.17 -> 2.20 at 1024^3)
+  // 0.99 -> 0.91 at 720^3 FP32; even at 1024^3, 2.00 to 2.19 ms either way from
+  // one process to the next)
   auto split = [&](int l, int k, C w) {
     const C zk = buf[lds_ix<true>(l * M + k)], zc = buf[lds_ix<true>(l * M + (k == 0 ? 0 : M - k))];
     const C e = C{(zk.x + zc.x) * (T)0.5, (zk.y - zc.y) * (T)0.5};
