@@ -531,10 +531,16 @@ __global__ void k_seg_tot(const uint32_t *__restrict__ t1scan, int64_t g1, int n
 // Directory of the buckets of a pass, from their totals (list entries << 32
 // | records): every bucket's first list entry; of the segments of a second
 // pass, the bucket of each workgroup's first slot; of tiles, the work items,
-// the item -> tile table and the deposit's schedule.  One workgroup: a bucket
-// count of 65 536 is 16 rounds, and the scans, tables and flags that it
-// replaces were a dozen launches of 2 to 5 us each.  The totals are cleared
+// the item -> tile table and the deposit's schedule.  The totals are cleared
 // for the next sort.
+//
+// Up to DIR_ONE buckets one workgroup does it all (k_dir; the scans, tables and
+// flags that it replaces were a dozen launches of 2 to 5 us each).  It takes
+// 6.5 us per round of 4096 buckets, so more of them are cut into sections, a
+// workgroup each: k_dir_sums (a section's sums), k_dir (each section from the
+// sums of those before it) and k_dir_end (split items, shares).  With the
+// lists 105 -> 23 us at 65 536 tiles, 359 -> 27 at 2^18, 2990 -> 47 at 2^21
+// (2^20 particles or fewer); 16384 buckets 30 -> 21.
 //
 // Schedule: the deposit's workgroup w takes the items w, w + wgs, ... of split
 // tiles, then a run of the items of one tile, whose bounds share every
@@ -558,7 +564,8 @@ struct DirArgs {
   // tiles: items of at most 2^limax records and 2^17 record slots; store: every
   // real tile gets at least one item (so untouched tiles are written as zeros)
   int store, lg, limax;
-  uint32_t *pstart, *heavy, *counts, *cost, *share;  // [nb + 1], split tiles; TileList
+  // [nb + 1]; split tiles; TileList (counts[3]: cost of the items of one tile)
+  uint32_t *pstart, *heavy, *counts, *cost, *share;
   uint32_t max_parts, wgs, icost;
   FastDiv fwgs;
   int cshift;  // costs are in units of 2^cshift records, so that their sum stays below 2^31
@@ -566,65 +573,180 @@ struct DirArgs {
   uint32_t *mrange;       // with masses: reduced from mrange_w[2 * nw]
   const uint32_t *mrange_w;
   int64_t nw;
+  int64_t sec;            // buckets of a workgroup's section (whole rounds)
+  uint4 *secsum;          // [sections] (one section: none)
 };
 constexpr int DIR_PER = 4;  // buckets per thread and round
-constexpr uint32_t DIR_HEAVY = 1024;  // split tiles whose items are written at the end (further ones: by their thread)
+constexpr int64_t DIR_ROUND = (int64_t)SORT_THREADS * DIR_PER;
+constexpr int64_t DIR_ONE = 2 * DIR_ROUND;
+constexpr uint32_t DIR_HEAVY = 1024;  // split tiles that one workgroup keeps in LDS
+constexpr int DIR_NV = 4;  // prefix sums: list entries, items of one tile, items of split tiles, cost of the former
 
-__global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
-  constexpr int NV = 4;  // prefix sums: list entries, items of one tile, items of split tiles, cost of the former
-  __shared__ uint32_t wt[2][NV][SORT_WAVES], wtot[2][SORT_WAVES];
-  __shared__ uint32_t load_of[DEPOSIT_WGS_MAX];  // cost of each workgroup's items of split tiles
-  __shared__ uint4 split_tiles[DIR_HEAVY];  // tile, first item, items, cost of one
-  __shared__ uint32_t hcount, smr[2];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  auto split_item = [&](uint32_t k, uint32_t q, uint32_t c) {
-    D.utile[q] = k;
-    atomicAdd(&load_of[q - D.fwgs.div(q) * D.wgs], c);
-  };
-  if (threadIdx.x == 0) {
-    hcount = 0;
-    smr[0] = 0u;
-    smr[1] = 0xffffffffu;
-    if (D.nonfinite) *D.nonfinite = 0u;
+// Entries and items of bucket k with totals t: v as in DIR_NV, but for v[3],
+// the cost of an item (also of a split tile).
+__device__ __forceinline__ void dir_values(const DirArgs &D, int64_t k, unsigned long long t, uint32_t (&v)[DIR_NV]) {
+  const uint32_t eslots = 1u << (LG_ITEM_MAX - D.lg);  // list entries of 2^17 record slots
+  const uint32_t ents = (uint32_t)(t >> 32), recs = (uint32_t)t;
+  uint32_t m = 0;
+  if (D.unit == 0 && k < D.kreal) {
+    if (recs == 0) m = D.store ? 1u : 0u;
+    else m = max((recs + (1u << D.limax) - 1) >> D.limax, (ents + (eslots - 1)) >> (LG_ITEM_MAX - D.lg));
   }
+  v[0] = ents;
+  v[1] = m == 1 ? 1u : 0u;
+  v[2] = m > 1 ? m : 0u;
+  const uint32_t slots = (ents << D.lg) >> D.cshift;
+  v[3] = m == 0 ? 0u : (m > 1 ? slots / m : slots) + D.icost;
+}
+
+__global__ void __launch_bounds__(SORT_THREADS) k_dir_sums(DirArgs D) {
+  __shared__ uint32_t wt[DIR_NV][SORT_WAVES];
+  const int64_t b0 = blockIdx.x * D.sec, b1 = min(D.nb, b0 + D.sec);
+  uint32_t sum[DIR_NV] = {};
+  for (int64_t k = b0 + threadIdx.x; k < b1; k += SORT_THREADS) {
+    uint32_t v[DIR_NV];
+    dir_values(D, k, D.tot[k], v);
+#pragma unroll
+    for (int j = 0; j < DIR_NV; j++) sum[j] += j == 3 && v[2] ? 0u : v[j];
+  }
+#pragma unroll
+  for (int j = 0; j < DIR_NV; j++) {
+    const uint32_t incl = wave_incl_scan(sum[j]);
+    if ((threadIdx.x & 63) == 63) wt[j][threadIdx.x >> 6] = incl;
+  }
+  __syncthreads();
+  uint32_t all[DIR_NV];
+#pragma unroll
+  for (int j = 0; j < DIR_NV; j++) waves_before(wt[j], all[j]);
+  if (threadIdx.x == 0) {
+    D.secsum[blockIdx.x] = make_uint4(all[0], all[1], all[2], all[3]);
+    if (blockIdx.x == 0) D.counts[0] = 0;
+  }
+}
+
+// The split tiles' items, numbered from pstart on, the deposit's shares and the
+// masses' range, by one workgroup, once every bucket's start and the nheavy
+// split tiles are written; the first nknown of them also stand in known (tile,
+// first item, items, cost of one), which saves two round trips to memory.
+// carry: the sums of all buckets.
+__device__ __forceinline__ void dir_end(const DirArgs &D, uint32_t nheavy, const uint4 *known, uint32_t nknown,
+                                        const uint32_t (&carry)[DIR_NV]) {
+  __shared__ uint32_t wtot[2][SORT_WAVES];
+  __shared__ uint32_t load_of[DEPOSIT_WGS_MAX];  // cost of each workgroup's items of split tiles
+  __shared__ uint32_t smr[2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   load_of[threadIdx.x] = 0;
   static_assert(DEPOSIT_WGS_MAX == SORT_THREADS, "one thread per workgroup of the deposit");
-  const uint32_t eslots = 1u << (LG_ITEM_MAX - D.lg);  // list entries of 2^17 record slots
-  uint32_t carry[NV] = {};
+  if (threadIdx.x == 0) {
+    smr[0] = 0u;
+    smr[1] = 0xffffffffu;
+  }
+  __syncthreads();
+  // every wave reads up to 64 split tiles at once (each wave's SORT_WAVES
+  // apart, so that few tiles spread over the waves), then writes the items of
+  // one after another (one thread per tile was a chain of up to hundreds of stores)
+  for (uint32_t h0 = wave; h0 < nheavy; h0 += SORT_THREADS) {
+    const uint32_t h = h0 + lane * SORT_WAVES;
+    uint4 t = make_uint4(0u, 0u, 0u, 0u);
+    if (h < nknown) {
+      t = known[h];
+    } else if (h < nheavy) {
+      t.x = D.heavy[h];
+      t.y = D.pstart[t.x];
+      t.z = D.pstart[t.x + 1] - t.y;
+      t.w = (((D.start[t.x + 1] - D.start[t.x]) << D.lg) >> D.cshift) / t.z + D.icost;
+    }
+    for (int i = 0; i < 64 && h0 + i * SORT_WAVES < nheavy; i++) {
+      const uint32_t k = __builtin_amdgcn_readlane(t.x, i), p0 = __builtin_amdgcn_readlane(t.y, i);
+      const uint32_t m = __builtin_amdgcn_readlane(t.z, i), c = __builtin_amdgcn_readlane(t.w, i);
+      for (uint32_t q = p0 + lane; q < p0 + m; q += 64) {
+        D.utile[q] = k;
+        atomicAdd(&load_of[q - D.fwgs.div(q) * D.wgs], c);
+      }
+    }
+  }
+  if (carry[2] && carry[1] + carry[2] > D.wgs) {
+    // what each workgroup has left to the mean of all, in proportion of the
+    // cost of the items of one tile (fewer items: one each, k_deposit)
+    __syncthreads();
+    const uint32_t own = threadIdx.x < D.wgs ? load_of[threadIdx.x] : 0u;
+    uint32_t all = 0, rest = 0;
+    block_scan_round(own, wtot, 0, all);
+    const uint32_t mean = (uint32_t)(((unsigned long long)all + carry[3] + D.wgs - 1) / D.wgs);
+    const uint32_t before = block_scan_round(threadIdx.x < D.wgs && mean > own ? mean - own : 0u, wtot, 1, rest);
+    if (threadIdx.x < D.wgs) D.share[threadIdx.x] = (uint32_t)((double)carry[3] * before / max(rest, 1u));
+  }
+  if (D.mrange) {
+    uint32_t mx = 0u, mn = 0xffffffffu;
+    for (int64_t i = threadIdx.x; i < D.nw; i += SORT_THREADS) {
+      mx = max(mx, D.mrange_w[2 * i]);
+      mn = min(mn, D.mrange_w[2 * i + 1]);
+    }
+    atomicMax(&smr[0], mx);
+    atomicMin(&smr[1], mn);
+    __syncthreads();
+    if (threadIdx.x < 2) D.mrange[threadIdx.x] = smr[threadIdx.x];
+  }
+}
+
+__global__ void __launch_bounds__(SORT_THREADS) k_dir_end(DirArgs D) {
+  const uint32_t carry[DIR_NV] = {0u, D.counts[2], D.counts[1], D.counts[3]};
+  dir_end(D, D.counts[0], nullptr, 0u, carry);
+}
+
+template <bool ONE>
+__global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
+  constexpr int NV = DIR_NV;
+  __shared__ uint32_t wt[2][NV][SORT_WAVES];
+  __shared__ uint4 split_tiles[ONE ? DIR_HEAVY : 1];  // as dir_end's known
+  __shared__ uint32_t hcount;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t b0 = ONE ? 0 : blockIdx.x * D.sec, b1 = ONE ? D.nb : min(D.nb, b0 + D.sec);
+  if (threadIdx.x == 0) {
+    hcount = 0;
+    if (D.nonfinite && blockIdx.x == 0) *D.nonfinite = 0u;
+  }
   unsigned long long t[DIR_PER];
-  auto div_up = [&](uint32_t x) { return x == 0 ? 0u : D.funit.div(x - 1) + 1; };  // entries < 2^31
   auto load = [&](int64_t r0) {
 #pragma unroll
     for (int i = 0; i < DIR_PER; i++) {
       const int64_t k = r0 + threadIdx.x * DIR_PER + i;
-      t[i] = k < D.nb ? D.tot[k] : 0ull;
+      t[i] = k < b1 ? D.tot[k] : 0ull;
     }
   };
-  load(0);
+  load(b0);
+  uint32_t carry[NV] = {};
+  if constexpr (!ONE) {
+    uint32_t sum[NV] = {};
+    for (uint32_t w = threadIdx.x; w < blockIdx.x; w += SORT_THREADS) {
+      const uint4 s = D.secsum[w];
+      sum[0] += s.x;
+      sum[1] += s.y;
+      sum[2] += s.z;
+      sum[3] += s.w;
+    }
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+      const uint32_t incl = wave_incl_scan(sum[j]);
+      if (lane == 63) wt[1][j][wave] = incl;  // (the first round writes wt[0])
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NV; j++) waves_before(wt[1][j], carry[j]);
+  }
+  auto div_up = [&](uint32_t x) { return x == 0 ? 0u : D.funit.div(x - 1) + 1; };  // entries < 2^31
   int rd = 0;
-  for (int64_t r0 = 0; r0 < D.nb; r0 += SORT_THREADS * DIR_PER, rd ^= 1) {
+  for (int64_t r0 = b0; r0 < b1; r0 += DIR_ROUND, rd ^= 1) {
     const int64_t k0 = r0 + threadIdx.x * DIR_PER;
-    uint32_t v[NV][DIR_PER], sum[NV] = {};
+    uint32_t v[DIR_PER][NV], sum[NV] = {};
 #pragma unroll
     for (int i = 0; i < DIR_PER; i++) {
-      const int64_t k = k0 + i;
-      const uint32_t ents = (uint32_t)(t[i] >> 32), recs = (uint32_t)t[i];
-      uint32_t m = 0;
-      if (D.unit == 0 && k < D.kreal) {
-        if (recs == 0) m = D.store ? 1u : 0u;
-        else m = max((recs + (1u << D.limax) - 1) >> D.limax, (ents + (eslots - 1)) >> (LG_ITEM_MAX - D.lg));
-      }
-      v[0][i] = ents;
-      v[1][i] = m == 1 ? 1u : 0u;
-      v[2][i] = m > 1 ? m : 0u;
-      const uint32_t slots = (ents << D.lg) >> D.cshift;
-      v[3][i] = m == 0 ? 0u : slots + D.icost;
-      if (m > 1) v[3][i] = slots / m + D.icost;  // an item's
-      if (k < D.nb) D.tot[k] = 0ull;
+      dir_values(D, k0 + i, t[i], v[i]);
+      if (k0 + i < b1) D.tot[k0 + i] = 0ull;
 #pragma unroll
-      for (int j = 0; j < NV; j++) sum[j] += j == 3 && m > 1 ? 0u : v[j][i];
+      for (int j = 0; j < NV; j++) sum[j] += j == 3 && v[i][2] ? 0u : v[i][j];
     }
-    load(r0 + SORT_THREADS * DIR_PER);
+    load(r0 + DIR_ROUND);
     uint32_t run[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) {
@@ -642,76 +764,47 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
 #pragma unroll
     for (int i = 0; i < DIR_PER; i++) {
       const int64_t k = k0 + i;
-      if (k < D.nb) {
+      if (k < b1) {
         D.start[k] = run[0];
         if (D.unit) {
           // the workgroups whose first entry lies in this bucket
-          const uint32_t w1 = div_up(run[0] + v[0][i]);
+          const uint32_t w1 = div_up(run[0] + v[i][0]);
           for (uint32_t w = div_up(run[0]); w < w1; w++) D.utile[w] = (uint32_t)k;
         } else {
           D.pstart[k] = run[2];
-          if (v[1][i]) {
+          if (v[i][1]) {
             D.utile[D.max_parts + run[1]] = (uint32_t)k;
-            D.cost[run[1]] = run[3] + v[3][i] / 2;
-          } else if (v[2][i]) {
-            const uint32_t h = atomicAdd(&hcount, 1u);
+            D.cost[run[1]] = run[3] + v[i][3] / 2;
+          } else if (v[i][2]) {
+            const uint32_t h = atomicAdd(ONE ? &hcount : &D.counts[0], 1u);
             D.heavy[h] = (uint32_t)k;
-            if (h < DIR_HEAVY)
-              split_tiles[h] = make_uint4((uint32_t)k, run[2], v[2][i], v[3][i]);
-            else
-              for (uint32_t q = 0; q < v[2][i]; q++) split_item((uint32_t)k, run[2] + q, v[3][i]);
+            if (ONE && h < DIR_HEAVY) split_tiles[h] = make_uint4((uint32_t)k, run[2], v[i][2], v[i][3]);
           }
         }
       }
 #pragma unroll
-      for (int j = 0; j < NV; j++) run[j] += j == 3 && v[2][i] ? 0u : v[j][i];
+      for (int j = 0; j < NV; j++) run[j] += j == 3 && v[i][2] ? 0u : v[i][j];
     }
-  }
-  if (threadIdx.x == 0) {
-    D.start[D.nb] = carry[0];
-    if (!D.unit) D.pstart[D.nb] = carry[2];
-  }
-  if (!D.unit && carry[2]) {
-    // the items of split tiles, a wave per tile (one thread per tile was a
-    // chain of up to hundreds of stores)
-    __syncthreads();
-    for (uint32_t h = wave; h < min(hcount, DIR_HEAVY); h += SORT_WAVES) {
-      const uint4 t = split_tiles[h];
-      for (uint32_t q = lane; q < t.z; q += 64) split_item(t.x, t.y + q, t.w);
-    }
-  }
-  if (!D.unit && carry[2] && carry[1] + carry[2] > D.wgs) {
-    // what each workgroup has left to the mean of all, in proportion of the
-    // cost of the items of one tile (fewer items: one each, k_deposit)
-    __syncthreads();
-    const uint32_t own = threadIdx.x < D.wgs ? load_of[threadIdx.x] : 0u;
-    uint32_t all = 0, rest = 0;
-    block_scan_round(own, wtot, 0, all);
-    const uint32_t mean = (uint32_t)(((unsigned long long)all + carry[3] + D.wgs - 1) / D.wgs);
-    const uint32_t before = block_scan_round(threadIdx.x < D.wgs && mean > own ? mean - own : 0u, wtot, 1, rest);
-    if (threadIdx.x < D.wgs) D.share[threadIdx.x] = (uint32_t)((double)carry[3] * before / max(rest, 1u));
   }
   for (int64_t i = threadIdx.x; i < D.npiece; i += SORT_THREADS) D.piece[i] = make_uint4(0u, 0u, 0u, 0u);
-  if (D.mrange) {
-    uint32_t mx = 0u, mn = 0xffffffffu;
-    for (int64_t i = threadIdx.x; i < D.nw; i += SORT_THREADS) {
-      mx = max(mx, D.mrange_w[2 * i]);
-      mn = min(mn, D.mrange_w[2 * i + 1]);
-    }
-    atomicMax(&smr[0], mx);
-    atomicMin(&smr[1], mn);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
+  if (b1 == D.nb && threadIdx.x == 0) {
+    D.start[D.nb] = carry[0];
     if (!D.unit) {
-      D.counts[0] = hcount;
+      D.pstart[D.nb] = carry[2];
       D.counts[1] = carry[2];
       D.counts[2] = carry[1];
+      D.counts[3] = carry[3];
     }
-    if (D.mrange) {
-      D.mrange[0] = smr[0];
-      D.mrange[1] = smr[1];
+  }
+  if (ONE && !D.unit) {
+    if (carry[2] || D.mrange) {
+      // beyond split_tiles, dir_end reads what other waves of this workgroup
+      // have written (a fence among workgroups would write the L2 back: 4 us)
+      __threadfence_block();
+      __syncthreads();
+      dir_end(D, hcount, split_tiles, min(hcount, (uint32_t)DIR_HEAVY), carry);
     }
+    if (threadIdx.x == 0) D.counts[0] = carry[2] ? hcount : 0u;
   }
 }
 
@@ -879,8 +972,26 @@ uint32_t *pg_buffers(DevBuf &buf, const PgLayout &L, int nb, PgOut &pg, unsigned
   return blist;
 }
 
-void launch_dir(const DirArgs &D, hipStream_t s) {
-  hipLaunchKernelGGL(k_dir, dim3(1), dim3(SORT_THREADS), 0, s, D);
+// Sections of a directory of nb buckets (k_dir): a workgroup each, at most 1024.
+int64_t dir_section(int64_t nb) {
+  if (nb <= DIR_ONE) return ceil_div(nb, DIR_ROUND) * DIR_ROUND;
+  return ceil_div(ceil_div(nb, DIR_ROUND), SORT_THREADS) * DIR_ROUND;
+}
+
+void launch_dir(DirArgs &D, hipStream_t s) {
+  D.sec = dir_section(D.nb);
+  const dim3 grid((unsigned)ceil_div(D.nb, D.sec)), block(SORT_THREADS);
+  GENPK_REQUIRE(grid.x == 1 || (!D.unit && D.secsum), "directory of segments in sections");
+  if (grid.x == 1) {
+    hipLaunchKernelGGL(k_dir<true>, grid, block, 0, s, D);
+    GENPK_LAUNCH_CHECK();
+    return;
+  }
+  hipLaunchKernelGGL(k_dir_sums, grid, block, 0, s, D);
+  GENPK_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_dir<false>, grid, block, 0, s, D);
+  GENPK_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_dir_end, dim3(1), block, 0, s, D);
   GENPK_LAUNCH_CHECK();
 }
 
@@ -1032,7 +1143,8 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
                                  ceil_div(slots, (int64_t)DEPOSIT_ITEM_MAX));
   const int64_t max_items = tg.K + max_parts;
   const int64_t ts = (ks + 4) / 4 * 4;
-  uint32_t *ib = static_cast<uint32_t *>(p.item_start.ensure((size_t)ts * 4 * 4 + 64));
+  const int64_t nsec = ceil_div(ks, dir_section(ks));
+  uint32_t *ib = static_cast<uint32_t *>(p.item_start.ensure((size_t)(ts + nsec) * 4 * 4 + 64));
   uint32_t *item_tile = static_cast<uint32_t *>(p.item_tile.ensure((size_t)max_items * 4));
   DirArgs D{};
   D.tot = tot;
@@ -1046,6 +1158,7 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   D.limax = ilog2(imax);
   D.pstart = ib + 2 * ts;
   D.heavy = ib + 3 * ts;
+  D.secsum = reinterpret_cast<uint4 *>(ib + 4 * ts);
   D.counts = static_cast<uint32_t *>(p.heavy.ensure(64 + DEPOSIT_WGS_MAX * 4));
   D.share = D.counts + 16;
   D.max_parts = (uint32_t)max_parts;
