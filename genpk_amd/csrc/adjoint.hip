@@ -292,9 +292,7 @@ struct GatherParams {
 // coalesced.
 template <typename T, int NM, int GM>
 __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__restrict__ G, const float *__restrict__ rec,
-                                                                 const uint32_t *__restrict__ item_tile,
-                                                                 const uint32_t *__restrict__ part_start,
-                                                                 const uint32_t *__restrict__ start,
+                                                                 const uint4 *__restrict__ items,
                                                                  const uint32_t *__restrict__ blist,
                                                                  const uint32_t *__restrict__ counts,
                                                                  GatherParams P, float *__restrict__ out) {
@@ -311,7 +309,7 @@ __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__rest
   const uint32_t nsplit = counts[1];
   if (item >= nsplit + counts[2]) return;
   ItemRange ir;
-  item_range(item_tile, part_start, start, nsplit, P.list.max_parts, item, ir);
+  item_range(items, nsplit, P.list.max_parts, item, ir);
   if (ir.lb >= ir.le) return;
   const int64_t k = ir.k;
   const int ntz = P.kg.ntz, nty = P.kg.nty, d = P.kg.d;
@@ -537,8 +535,8 @@ void gather_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass, fl
   P.fnty = FastDiv((uint32_t)tg.nty);
   const int64_t grid = ceil_div(o.list.max_items, 8 * GATHER_RUN) * 8 * GATHER_RUN;
   hipLaunchKernelGGL((k_gather_tiles<T, NM, GM>), dim3((unsigned)grid), dim3(GATHER_THREADS),
-                     (size_t)tg.cells * sizeof(T), p.stream, p.field.as<const T>(), o.rec, o.list.item_tile, o.list.part_start,
-                     o.list.start, o.list.blist, o.list.counts, P, out);
+                     (size_t)tg.cells * sizeof(T), p.stream, p.field.as<const T>(), o.rec, o.list.items, o.list.blist,
+                     o.list.counts, P, out);
   GENPK_LAUNCH_CHECK();
 }
 

@@ -76,9 +76,7 @@ struct DepParams {
 // offsets fold into the LDS instructions' immediate offsets.
 template <typename Real, int NM, int RW, bool STD>
 __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict__ rec,
-                                                         const uint32_t *__restrict__ item_tile,
-                                                         const uint32_t *__restrict__ part_start,
-                                                         const uint32_t *__restrict__ start,
+                                                         const uint4 *__restrict__ items,
                                                          const uint32_t *__restrict__ blist,
                                                          const uint32_t *__restrict__ counts,
                                                          const uint32_t *__restrict__ cost,
@@ -160,7 +158,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   };
   auto range_of = [&](uint32_t it, ItemRange &o) {
     if (it == NONE) return false;
-    item_range(item_tile, part_start, start, nsplit, T.max_parts, it, o);
+    item_range(items, nsplit, T.max_parts, it, o);
     return true;
   };
   struct {
@@ -235,7 +233,8 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   __syncthreads();
   while (have) {
     const int64_t k = ir.k;
-    const uint32_t m = ir.m, ents = ir.le - ir.lb;
+    const uint32_t ents = ir.le - ir.lb;
+    const bool split = item < nsplit;
     const int ntz = P.kg.ntz, nty = P.kg.nty;
     // 32-bit multiply-high, not 64-bit divisions (~130 scalar instructions each)
     const uint32_t kxy = P.fntz.div((uint32_t)k), kx = P.fnty.div(kxy);
@@ -313,7 +312,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
 #pragma unroll
     for (int u = 0; u < UNR; u++) asm volatile("" : "+v"(ent[u]));
     __syncthreads();
-    if (m == 1) {
+    if (!split) {
       // rows of TZ values (aligned), then the z-halo plane
       // (32-bit cell indices: a tile's accumulator holds fewer than 2^24 cells)
       Real *rows = tiles + k * P.cm;
@@ -570,17 +569,17 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
     const bool std_tiles = std_tiles_of(tg);
     const dim3 grid(L.wgs), block(DEP_THREADS);
     if (p.prec == 4 && std_tiles)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, true>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
-                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
+      hipLaunchKernelGGL((k_deposit<float, NM, RW, true>), grid, block, lds, s, sorted, L.items, L.blist,
+                         L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
     else if (p.prec == 4)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, false>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
-                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
+      hipLaunchKernelGGL((k_deposit<float, NM, RW, false>), grid, block, lds, s, sorted, L.items, L.blist,
+                         L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
     else if (std_tiles)
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, true>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
-                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
+      hipLaunchKernelGGL((k_deposit<double, NM, RW, true>), grid, block, lds, s, sorted, L.items, L.blist,
+                         L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
     else
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, false>), grid, block, lds, s, sorted, L.item_tile, L.part_start,
-                         L.start, L.blist, L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
+      hipLaunchKernelGGL((k_deposit<double, NM, RW, false>), grid, block, lds, s, sorted, L.items, L.blist,
+                         L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
     GENPK_LAUNCH_CHECK();
   }
   {

@@ -92,8 +92,9 @@ enum class FieldState { None, Real, Spectrum, YDone };
 // counts[2] items after them those of one tile each.
 struct TileList {
   const uint32_t *start = nullptr, *part_start = nullptr;
-  // tile of each item of split tiles (max_parts entries), then of each other
-  const uint32_t *item_tile = nullptr;
+  // each item of split tiles (max_parts entries), then each other: tile, first
+  // list entry, the entry after its last
+  const uint4 *items = nullptr;
   const uint32_t *counts = nullptr;  // split tiles, their items, items of one tile
   // the deposit's schedule over wgs workgroups (k_dir): cost of the items of
   // one tile before the middle of each, and where each workgroup's begin
@@ -180,7 +181,7 @@ struct Plan {
   bool tiles_live = false;  // tiles hold deposits not yet folded
 
   // sort / deposit scratch
-  DevBuf recA, recB, table1, seginfo, item_start, heavy, partials, item_tile;
+  DevBuf recA, recB, table1, seginfo, item_start, heavy, partials, items;
   DevBuf permA, permB;      // sort permutations kept for the adjoint gather
   DevBuf pages1, pages;     // block headers, counts and lists of a paged first and of the last sort pass
   DevBuf sort_tot;          // bucket totals of the sort passes

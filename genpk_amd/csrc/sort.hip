@@ -531,7 +531,7 @@ __global__ void k_seg_tot(const uint32_t *__restrict__ t1scan, int64_t g1, int n
 // Directory of the buckets of a pass, from their totals (list entries << 32
 // | records): every bucket's first list entry; of the segments of a second
 // pass, the bucket of each workgroup's first slot; of tiles, the work items,
-// the item -> tile table and the deposit's schedule.  The totals are cleared
+// the table of the items and the deposit's schedule.  The totals are cleared
 // for the next sort.
 //
 // Up to DIR_ONE buckets one workgroup does it all (k_dir; the scans, tables and
@@ -556,7 +556,9 @@ __global__ void k_seg_tot(const uint32_t *__restrict__ t1scan, int64_t g1, int n
 struct DirArgs {
   unsigned long long *tot;
   int64_t nb, kreal;      // buckets; those below kreal are real tiles
-  uint32_t *start, *utile;  // [nb + 1]; tile of each item (TileList::item_tile) or first_seg
+  uint32_t *start;        // [nb + 1]
+  uint32_t *first_seg;    // segments: the bucket of each workgroup's first slot
+  uint4 *items;           // tiles: TileList::items
   uint32_t unit;          // segments: list entries per workgroup (0: tiles)
   FastDiv funit;
   uint4 *piece;           // segments: the second pass's pieces, cleared
@@ -627,10 +629,11 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir_sums(DirArgs D) {
 // The split tiles' items, numbered from pstart on, the deposit's shares and the
 // masses' range, by one workgroup, once every bucket's start and the nheavy
 // split tiles are written; the first nknown of them also stand in known (tile,
-// first item, items, cost of one), which saves two round trips to memory.
+// first item, items, cost of one) and known_at (list entries), which saves two
+// round trips to memory.
 // carry: the sums of all buckets.
-__device__ __forceinline__ void dir_end(const DirArgs &D, uint32_t nheavy, const uint4 *known, uint32_t nknown,
-                                        const uint32_t (&carry)[DIR_NV]) {
+__device__ __forceinline__ void dir_end(const DirArgs &D, uint32_t nheavy, const uint4 *known, const uint2 *known_at,
+                                        uint32_t nknown, const uint32_t (&carry)[DIR_NV]) {
   __shared__ uint32_t wtot[2][SORT_WAVES];
   __shared__ uint32_t load_of[DEPOSIT_WGS_MAX];  // cost of each workgroup's items of split tiles
   __shared__ uint32_t smr[2];
@@ -648,19 +651,26 @@ __device__ __forceinline__ void dir_end(const DirArgs &D, uint32_t nheavy, const
   for (uint32_t h0 = wave; h0 < nheavy; h0 += SORT_THREADS) {
     const uint32_t h = h0 + lane * SORT_WAVES;
     uint4 t = make_uint4(0u, 0u, 0u, 0u);
+    uint2 at = make_uint2(0u, 0u);
     if (h < nknown) {
       t = known[h];
+      at = known_at[h];
     } else if (h < nheavy) {
       t.x = D.heavy[h];
       t.y = D.pstart[t.x];
       t.z = D.pstart[t.x + 1] - t.y;
-      t.w = (((D.start[t.x + 1] - D.start[t.x]) << D.lg) >> D.cshift) / t.z + D.icost;
+      at = make_uint2(D.start[t.x], D.start[t.x + 1]);
+      t.w = (((at.y - at.x) << D.lg) >> D.cshift) / t.z + D.icost;
     }
+    const uint32_t entries = t.z ? (at.y - at.x + t.z - 1) / t.z : 0u;  // of an item
     for (int i = 0; i < 64 && h0 + i * SORT_WAVES < nheavy; i++) {
       const uint32_t k = __builtin_amdgcn_readlane(t.x, i), p0 = __builtin_amdgcn_readlane(t.y, i);
       const uint32_t m = __builtin_amdgcn_readlane(t.z, i), c = __builtin_amdgcn_readlane(t.w, i);
-      for (uint32_t q = p0 + lane; q < p0 + m; q += 64) {
-        D.utile[q] = k;
+      const uint32_t lb = __builtin_amdgcn_readlane(at.x, i), le = __builtin_amdgcn_readlane(at.y, i);
+      const uint32_t per = __builtin_amdgcn_readlane(entries, i);
+      for (uint32_t j = lane; j < m; j += 64) {
+        const uint32_t q = p0 + j, b = min(le, lb + j * per);
+        D.items[q] = make_uint4(k, b, min(le, b + per), 0u);
         atomicAdd(&load_of[q - D.fwgs.div(q) * D.wgs], c);
       }
     }
@@ -691,14 +701,15 @@ __device__ __forceinline__ void dir_end(const DirArgs &D, uint32_t nheavy, const
 
 __global__ void __launch_bounds__(SORT_THREADS) k_dir_end(DirArgs D) {
   const uint32_t carry[DIR_NV] = {0u, D.counts[2], D.counts[1], D.counts[3]};
-  dir_end(D, D.counts[0], nullptr, 0u, carry);
+  dir_end(D, D.counts[0], nullptr, nullptr, 0u, carry);
 }
 
 template <bool ONE>
 __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
   constexpr int NV = DIR_NV;
   __shared__ uint32_t wt[2][NV][SORT_WAVES];
-  __shared__ uint4 split_tiles[ONE ? DIR_HEAVY : 1];  // as dir_end's known
+  __shared__ uint4 split_tiles[ONE ? DIR_HEAVY : 1];  // as dir_end's known and known_at
+  __shared__ uint2 split_at[ONE ? DIR_HEAVY : 1];
   __shared__ uint32_t hcount;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t b0 = ONE ? 0 : blockIdx.x * D.sec, b1 = ONE ? D.nb : min(D.nb, b0 + D.sec);
@@ -769,16 +780,19 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
         if (D.unit) {
           // the workgroups whose first entry lies in this bucket
           const uint32_t w1 = div_up(run[0] + v[i][0]);
-          for (uint32_t w = div_up(run[0]); w < w1; w++) D.utile[w] = (uint32_t)k;
+          for (uint32_t w = div_up(run[0]); w < w1; w++) D.first_seg[w] = (uint32_t)k;
         } else {
           D.pstart[k] = run[2];
           if (v[i][1]) {
-            D.utile[D.max_parts + run[1]] = (uint32_t)k;
+            D.items[D.max_parts + run[1]] = make_uint4((uint32_t)k, run[0], run[0] + v[i][0], 0u);
             D.cost[run[1]] = run[3] + v[i][3] / 2;
           } else if (v[i][2]) {
             const uint32_t h = atomicAdd(ONE ? &hcount : &D.counts[0], 1u);
             D.heavy[h] = (uint32_t)k;
-            if (ONE && h < DIR_HEAVY) split_tiles[h] = make_uint4((uint32_t)k, run[2], v[i][2], v[i][3]);
+            if (ONE && h < DIR_HEAVY) {
+              split_tiles[h] = make_uint4((uint32_t)k, run[2], v[i][2], v[i][3]);
+              split_at[h] = make_uint2(run[0], run[0] + v[i][0]);
+            }
           }
         }
       }
@@ -802,7 +816,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
       // have written (a fence among workgroups would write the L2 back: 4 us)
       __threadfence_block();
       __syncthreads();
-      dir_end(D, hcount, split_tiles, min(hcount, (uint32_t)DIR_HEAVY), carry);
+      dir_end(D, hcount, split_tiles, split_at, min(hcount, (uint32_t)DIR_HEAVY), carry);
     }
     if (threadIdx.x == 0) D.counts[0] = carry[2] ? hcount : 0u;
   }
@@ -1086,7 +1100,7 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
     D.tot = tot + ks;
     D.nb = D.kreal = nhi;
     D.start = sb;
-    D.utile = sb + ss;
+    D.first_seg = sb + ss;
     D.piece = pg2.piece;
     D.npiece = S.L2.pieces;
     if (S.paged1) {
@@ -1145,14 +1159,13 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   const int64_t ts = (ks + 4) / 4 * 4;
   const int64_t nsec = ceil_div(ks, dir_section(ks));
   uint32_t *ib = static_cast<uint32_t *>(p.item_start.ensure((size_t)(ts + nsec) * 4 * 4 + 64));
-  uint32_t *item_tile = static_cast<uint32_t *>(p.item_tile.ensure((size_t)max_items * 4));
   DirArgs D{};
   D.tot = tot;
   D.nb = ks;
   D.kreal = tg.K;
   D.start = ib;
   D.cost = ib + ts;
-  D.utile = item_tile;
+  D.items = static_cast<uint4 *>(p.items.ensure((size_t)max_items * 16));
   D.store = every_tile ? 1 : 0;
   D.lg = S.L2.lg;
   D.limax = ilog2(imax);
@@ -1189,7 +1202,7 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   o.has_perm = with_perm;
   o.perm1 = perm1;
   o.perm2 = perm2;
-  o.list = {D.start, D.pstart, item_tile, D.counts, D.cost, D.share, blist, S.L2.lg, ks, max_items, D.max_parts, D.wgs};
+  o.list = {D.start, D.pstart, D.items, D.counts, D.cost, D.share, blist, S.L2.lg, ks, max_items, D.max_parts, D.wgs};
   o.heavy = D.heavy;
   o.mrange = mrange;
   o.n = n;
