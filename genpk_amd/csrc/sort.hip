@@ -931,22 +931,27 @@ struct PgLayout {
   int64_t slots() const { return blocks << lg; }
 };
 
-// A paged pass over at most `slots` input slots in nseg buckets.  Every
-// workgroup takes the same number of slots: one round of one workgroup per
-// CU, or more rounds as long as each workgroup keeps minsub sub-chunks and
-// the partly filled blocks (one per piece and digit at most) stay below a
-// sixth of the slots (or 2^26: about 1 GB).  Shorter ranges run beside each other in time on
-// neighbouring parts of the pools, and finish evenly: with two rounds instead
-// of eight the first pass takes 0.80 instead of 0.74 ms (2^27 records, 64
-// digits), with two instead of 16 the second 7.2 instead of 6.5 ms (2^30
-// records).
-PgLayout paged_layout(int64_t slots, int64_t nseg, int nb, int rw, int lo, int hi, int minsub) {
+// A paged pass over at most `slots` input slots (in blocks of 2^inlg) in nseg
+// buckets.  Every workgroup takes the same number of slots: one round of one
+// workgroup per CU, or more rounds as long as each workgroup keeps minsub
+// sub-chunks and the partly filled blocks (one per piece and digit at most)
+// stay below a sixth of the slots (or 2^26: about 1 GB).  Shorter ranges run
+// beside each other in time on neighbouring parts of the pools, and finish
+// evenly: with two rounds instead of eight the first pass takes 0.80 instead
+// of 0.74 ms (2^27 records, 64 digits), with two instead of 16 the second 7.2
+// instead of 6.5 ms (2^30 records).  Few slots in many buckets are cut below a
+// sub-chunk, down to a workgroup per bucket: a piece takes 2.5 us whatever it
+// holds, and one workgroup that walked all of them 624 us (1000
+// records in 256 buckets; 13 spread out).
+PgLayout paged_layout(int64_t slots, int64_t nseg, int nb, int rw, int lo, int hi, int minsub, int inlg = 0) {
   PgLayout L;
   L.h = partition_shape(nb, rw, true, partition_plmax(slots));
   const int64_t subn = (int64_t)SORT_THREADS * L.h.pl, cus = num_cus();
   for (int64_t rounds = 1; rounds <= 16; rounds *= 2) {
     PgLayout M = L;
     M.chunk = std::max(subn, ceil_div(ceil_div(slots, rounds * cus), subn) * subn);
+    if (nseg > 1 && M.chunk == subn)
+      M.chunk = std::min(subn, std::max((int64_t)1, ceil_div(slots >> inlg, std::min(nseg, cus))) << inlg);
     M.G = ceil_div(slots, M.chunk);
     M.pieces = nseg > 1 ? M.G + nseg : M.G;
     M.lg = pick_lg(slots / M.pieces, nb, lo, hi);
@@ -1038,7 +1043,7 @@ SortLayout sort_layout(const Plan &p, int64_t n, int rw) {
     S.paged1 = S.slots1 <= ((int64_t)1 << 32);
   }
   if (!S.paged1) S.slots1 = n;
-  S.L2 = paged_layout(S.slots1, nhi, nlo, rw, 3, 8, 2);
+  S.L2 = paged_layout(S.slots1, nhi, nlo, rw, 3, 8, 2, S.paged1 ? S.L1.lg : 0);
   return S;
 }
 

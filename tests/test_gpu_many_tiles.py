@@ -63,3 +63,26 @@ def test_many_tiles(gpu, d, tiles, n, kind, masses):
         p.import_density(G)
         grads.append(p.adjoint_gather(pos, BOX, m))
     assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
+
+
+# few records in many buckets: the second pass's workgroups take fewer records
+# than a sub-chunk, down to one (n <= 256 buckets)
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 1000, 40000, 300000])
+@pytest.mark.parametrize("d,tiles", [(256, (4, 8, 16)), (320, (16, 32, 32)), (512, (16, 32, 32))])
+def test_few_records_in_many_buckets(gpu, d, tiles, n):
+    import torch
+    print("CASE", d, tiles, n, flush=True)
+    pos = _positions(torch, n, "spread")
+    a, b = genpk_amd.Plan(d, "f64").set_options(tiles), genpk_amd.Plan(d, "f64").set_options((32, 16, 16))
+    got = []
+    for p in (a, b):
+        p.clear()
+        p.deposit(pos, BOX, retain=True)
+        got.append(p.export_density().clone())
+    assert torch.equal(got[0], got[1])
+    grads = []
+    for p in (a, b):
+        p.import_density(got[0])
+        grads.append(p.adjoint_gather(pos, BOX))
+    assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
