@@ -64,7 +64,9 @@ struct Src {
 //   block-list entries (2^lg each), of a first pass's buckets, bucket s from
 //   record or entry start[s] on; first_seg[g] is the bucket of g's first slot.
 //   A workgroup handles the part of each bucket in its range as a piece of
-//   its own (a bucket's digits are not another's).
+//   its own (a bucket's digits are not another's); piece w + s is workgroup
+//   w's of bucket s, and IN_LIST lacks[w + s] the slots of its blocks that
+//   hold no record.
 enum { IN_RAW = 0, IN_SEG = 1, IN_LIST = 2 };
 struct InMap {
   int64_t n = 0, chunk = 0;
@@ -73,9 +75,8 @@ struct InMap {
 };
 
 // Output of a paged pass: a pool of blocks of 2^lg record slots, in which
-// every piece (a workgroup's slots of one bucket) has a range large enough for
-// its full blocks and one partly filled block per digit.  Piece w + s is
-// workgroup w's of bucket s; its range starts at block (first slot >> lg) +
+// every piece has a range large enough for its full blocks and one partly
+// filled block per digit: it starts at block (records before the piece >> lg) +
 // (w + s) (nb + 1).
 struct PgOut {
   uint16_t *hdr = nullptr;    // digit of each taken block, written with the block's first record
@@ -295,6 +296,7 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__re
                                                                const uint32_t *__restrict__ blist,
                                                                const uint32_t *__restrict__ start,
                                                                const uint32_t *__restrict__ first_seg,
+                                                               const uint32_t *__restrict__ lacks,
                                                                float *__restrict__ dst, InMap im, KeyGeom kg,
                                                                DigitSel ds, int nb, int hw,
                                                                const uint32_t *__restrict__ offsets,
@@ -325,7 +327,16 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__re
   int64_t pe = IN == IN_RAW ? ce : min(ce, (int64_t)start[seg + 1] << sh);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint32_t pb = 1u << pg.lg;
-  uint32_t blk0 = PAGED ? (uint32_t)(cb >> pg.lg) + (blockIdx.x + seg) * (uint32_t)(nb + 1) : 0u;  // the piece's blocks
+  // slots before the piece that hold no record
+  uint32_t lack = 0;
+  if constexpr (IN == IN_LIST) {
+    uint32_t t = 0;
+    for (uint32_t p = threadIdx.x; p < blockIdx.x + seg; p += SORT_THREADS) t += lacks[p];
+    block_scan_round(t, wtot, 0, lack);
+    __syncthreads();  // wtot is written again
+  }
+  // the piece's blocks
+  uint32_t blk0 = PAGED ? (uint32_t)((cb - lack) >> pg.lg) + (blockIdx.x + seg) * (uint32_t)(nb + 1) : 0u;
   uint32_t taken = 0;                                                                      // blocks taken so far
   for (int i = threadIdx.x; i < nb; i += SORT_THREADS) {
     if constexpr (PAGED) dcnt[i] = 0;
@@ -499,7 +510,8 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__re
         pg.base[at] = (uint32_t)(atomicAdd(&pg.tot[(int64_t)seg * nb + dg], add) >> 32);
       }
       if (threadIdx.x == 0) pg.piece[p] = make_uint4(blk0, taken, seg, 0u);
-      blk0 = (uint32_t)(s1 >> pg.lg) + (blockIdx.x + nseg) * (uint32_t)(nb + 1);
+      if constexpr (IN == IN_LIST) lack += lacks[p];
+      blk0 = (uint32_t)((s1 - lack) >> pg.lg) + (blockIdx.x + nseg) * (uint32_t)(nb + 1);
       taken = 0;
     }
     s0 = s1;
@@ -561,7 +573,8 @@ struct DirArgs {
   uint4 *items;           // tiles: TileList::items
   uint32_t unit;          // segments: list entries per workgroup (0: tiles)
   FastDiv funit;
-  uint4 *piece;           // segments: the second pass's pieces, cleared
+  uint4 *piece;           // segments: the second pass's pieces and their lacks, cleared
+  uint32_t *lacks;
   int64_t npiece;
   // tiles: items of at most 2^limax records and 2^17 record slots; store: every
   // real tile gets at least one item (so untouched tiles are written as zeros)
@@ -800,7 +813,10 @@ __global__ void __launch_bounds__(SORT_THREADS) k_dir(DirArgs D) {
       for (int j = 0; j < NV; j++) run[j] += j == 3 && v[i][2] ? 0u : v[i][j];
     }
   }
-  for (int64_t i = threadIdx.x; i < D.npiece; i += SORT_THREADS) D.piece[i] = make_uint4(0u, 0u, 0u, 0u);
+  for (int64_t i = threadIdx.x; i < D.npiece; i += SORT_THREADS) {
+    D.piece[i] = make_uint4(0u, 0u, 0u, 0u);
+    D.lacks[i] = 0u;
+  }
   if (b1 == D.nb && threadIdx.x == 0) {
     D.start[D.nb] = carry[0];
     if (!D.unit) {
@@ -842,6 +858,32 @@ __global__ void __launch_bounds__(SORT_THREADS) k_list(PgOut pg, int nb, const u
   }
 }
 
+// lacks[w + s]: the empty slots of the listed blocks of piece w + s of a second
+// pass, whose workgroup w takes entries [w * unit, (w + 1) * unit).  One
+// workgroup each.  (Added up with global atomics where the list is written it
+// took 13 us at 2^27 records instead of 2.5.)
+constexpr int LACK_THREADS = 256;
+__global__ void __launch_bounds__(LACK_THREADS) k_lacks(const uint32_t *__restrict__ blist,
+                                                        const uint32_t *__restrict__ start,
+                                                        const uint32_t *__restrict__ first_seg, int nseg, int lg,
+                                                        uint32_t unit, uint32_t *__restrict__ lacks) {
+  __shared__ uint32_t part[2][LACK_THREADS / 64];
+  const uint32_t e0 = blockIdx.x * unit, e1 = min(start[nseg], e0 + unit);
+  if (e0 >= e1) return;
+  uint32_t s = first_seg[blockIdx.x];
+  for (uint32_t lo = e0, rd = 0; lo < e1; rd ^= 1) {
+    const uint32_t hi = min(e1, start[s + 1]);
+    uint32_t t = 0;
+    for (uint32_t e = lo + threadIdx.x; e < hi; e += LACK_THREADS) t += (1u << lg) - ((blist[e] >> (32 - lg)) + 1);
+    t = wave_incl_scan(t);
+    if ((threadIdx.x & 63) == 63) part[rd][threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x == 0 && lo < hi) lacks[blockIdx.x + s] = part[rd][0] + part[rd][1] + part[rd][2] + part[rd][3];
+    lo = hi;
+    s++;
+  }
+}
+
 struct PtShape {
   int pl;
   bool db;
@@ -877,39 +919,44 @@ int partition_plmax(int64_t n) {
   return per <= 2 * SORT_THREADS ? 2 : per <= 4 * SORT_THREADS ? 4 : 8;
 }
 
+// Arguments of a partition pass: what it reads (the caller's arrays, or a first
+// pass's records with their bucket starts and, paged, their block list), what
+// it writes, and of a counted pass the scanned offsets, of a paged one the pool.
+struct PtArgs {
+  const float *pos = nullptr, *masses = nullptr;
+  const uint32_t *blist = nullptr, *start = nullptr, *first_seg = nullptr, *lacks = nullptr;
+  InMap im;
+  int64_t grid = 0;
+  DigitSel ds;
+  int nb = 0;
+  PtShape h;
+  float *dst = nullptr;
+  uint32_t *perm = nullptr, *mrange_w = nullptr;
+  const uint32_t *offsets = nullptr;
+  PgOut pg;
+};
+
 template <int NM, int IN, bool PAGED, bool PERM>
-void launch_partition_perm(int64_t grid, hipStream_t s, const float *pos, const float *masses, const uint32_t *blist,
-                           const uint32_t *start, const uint32_t *first_seg, float *dst, const InMap &im, const KeyGeom &kg, const DigitSel &ds, int nb,
-                           const PtShape &h, const uint32_t *offsets, uint32_t *perm, uint32_t *mrange_w,
-                           const PgOut &pg) {
-  GENPK_REQUIRE(nb <= 2048, "sort digit too wide");
-  const size_t lds = partition_lds(nb, Src<NM>::RW, h, PAGED);
+void launch_partition_perm(const PtArgs &A, const KeyGeom &kg, hipStream_t s) {
+  GENPK_REQUIRE(A.nb <= 2048, "sort digit too wide");
+  const size_t lds = partition_lds(A.nb, Src<NM>::RW, A.h, PAGED);
   GENPK_REQUIRE(lds <= 160 * 1024 - 512, "sort pass does not fit in LDS");
-  const dim3 g((unsigned)grid), b(SORT_THREADS);
-#define GENPK_PART(PL, DB)                                                                                       \
-  hipLaunchKernelGGL((k_partition<NM, PL, DB, IN, PAGED, PERM>), g, b, lds, s, pos, masses, blist, start, first_seg, \
-                     dst, im, kg, ds, nb, h.hw, offsets, perm, mrange_w, pg)
-  if (h.pl == 8 && h.db) GENPK_PART(8, true);
-  else if (h.pl == 8) GENPK_PART(8, false);
-  else if (h.pl == 4 && h.db) GENPK_PART(4, true);
-  else if (h.pl == 4) GENPK_PART(4, false);
-  else GENPK_PART(2, false);
-#undef GENPK_PART
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)A.grid), dim3(SORT_THREADS), lds, s, A.pos, A.masses, A.blist, A.start,
+                       A.first_seg, A.lacks, A.dst, A.im, kg, A.ds, A.nb, A.h.hw, A.offsets, A.perm, A.mrange_w, A.pg);
+  };
+  if (A.h.pl == 8 && A.h.db) go(k_partition<NM, 8, true, IN, PAGED, PERM>);
+  else if (A.h.pl == 8) go(k_partition<NM, 8, false, IN, PAGED, PERM>);
+  else if (A.h.pl == 4 && A.h.db) go(k_partition<NM, 4, true, IN, PAGED, PERM>);
+  else if (A.h.pl == 4) go(k_partition<NM, 4, false, IN, PAGED, PERM>);
+  else go(k_partition<NM, 2, false, IN, PAGED, PERM>);
   GENPK_LAUNCH_CHECK();
 }
 
 template <int NM, int IN, bool PAGED>
-void launch_partition(int64_t grid, hipStream_t s, const float *pos, const float *masses, const uint32_t *blist,
-                      const uint32_t *start, const uint32_t *first_seg, float *dst, const InMap &im, const KeyGeom &kg, const DigitSel &ds, int nb, const PtShape &h,
-                      const uint32_t *offsets, uint32_t *perm, uint32_t *mrange_w, const PgOut &pg) {
-  if (perm)
-    launch_partition_perm<NM, IN, PAGED, true>(grid, s, pos, masses, blist, start, first_seg, dst, im, kg, ds, nb, h,
-                                               offsets, perm,
-                                               mrange_w, pg);
-  else
-    launch_partition_perm<NM, IN, PAGED, false>(grid, s, pos, masses, blist, start, first_seg, dst, im, kg, ds, nb, h,
-                                               offsets, perm,
-                                                mrange_w, pg);
+void launch_partition(const PtArgs &A, const KeyGeom &kg, hipStream_t s) {
+  if (A.perm) launch_partition_perm<NM, IN, PAGED, true>(A, kg, s);
+  else launch_partition_perm<NM, IN, PAGED, false>(A, kg, s);
 }
 
 // log2 of a paged pass's block: a quarter to a half of the records that a
@@ -931,11 +978,11 @@ struct PgLayout {
   int64_t slots() const { return blocks << lg; }
 };
 
-// A paged pass over at most `slots` input slots (in blocks of 2^inlg) in nseg
-// buckets.  Every workgroup takes the same number of slots: one round of one
+// A paged pass of n records in at most `slots` input slots (in blocks of
+// 2^inlg) of nseg buckets.  Every workgroup takes the same number of slots: one round of one
 // workgroup per CU, or more rounds as long as each workgroup keeps minsub
 // sub-chunks and the partly filled blocks (one per piece and digit at most)
-// stay below a sixth of the slots (or 2^26: about 1 GB).  Shorter ranges run
+// stay below a sixth of the records (or 2^26: about 1 GB).  Shorter ranges run
 // beside each other in time on neighbouring parts of the pools, and finish
 // evenly: with two rounds instead of eight the first pass takes 0.80 instead
 // of 0.74 ms (2^27 records, 64 digits), with two instead of 16 the second 7.2
@@ -943,7 +990,8 @@ struct PgLayout {
 // sub-chunk, down to a workgroup per bucket: a piece takes 2.5 us whatever it
 // holds, and one workgroup that walked all of them 624 us (1000
 // records in 256 buckets; 13 spread out).
-PgLayout paged_layout(int64_t slots, int64_t nseg, int nb, int rw, int lo, int hi, int minsub, int inlg = 0) {
+PgLayout paged_layout(int64_t n, int64_t slots, int64_t nseg, int nb, int rw, int lo, int hi, int minsub,
+                      int inlg = 0) {
   PgLayout L;
   L.h = partition_shape(nb, rw, true, partition_plmax(slots));
   const int64_t subn = (int64_t)SORT_THREADS * L.h.pl, cus = num_cus();
@@ -956,8 +1004,8 @@ PgLayout paged_layout(int64_t slots, int64_t nseg, int nb, int rw, int lo, int h
     M.pieces = nseg > 1 ? M.G + nseg : M.G;
     M.lg = pick_lg(slots / M.pieces, nb, lo, hi);
     const int64_t partial = M.pieces * (nb + 1);
-    M.blocks = (slots >> M.lg) + partial + 1;
-    if (rounds > 1 && (M.chunk < minsub * subn || (partial << M.lg) > std::max(slots / 6, (int64_t)1 << 26))) break;
+    M.blocks = (n >> M.lg) + partial + 1;
+    if (rounds > 1 && (M.chunk < minsub * subn || (partial << M.lg) > std::max(n / 6, (int64_t)1 << 26))) break;
     L = M;
   }
   return L;
@@ -975,13 +1023,15 @@ bool first_paged(const Plan &p, int64_t n) {
 }
 
 // Workspace of a paged pass in one buffer: pieces, per-piece counts, last
-// blocks and bases, the block list and the blocks' digits.
-uint32_t *pg_buffers(DevBuf &buf, const PgLayout &L, int nb, PgOut &pg, unsigned long long *tot) {
+// blocks and bases, the block list, the blocks' digits and the
+// pieces' lacks.
+uint32_t *pg_buffers(DevBuf &buf, const PgLayout &L, int nb, PgOut &pg, unsigned long long *tot, uint32_t **lacks) {
   const size_t blocks = (size_t)L.blocks, wd = (size_t)L.pieces * nb;
   GENPK_REQUIRE((uint64_t)L.slots() <= ((uint64_t)1 << 32), "sort pool too large");
-  uint32_t *b = static_cast<uint32_t *>(buf.ensure((4 * (size_t)L.pieces + 3 * wd + blocks + (blocks + 1) / 2) * 4));
+  uint32_t *b = static_cast<uint32_t *>(buf.ensure((5 * (size_t)L.pieces + 3 * wd + blocks + (blocks + 1) / 2) * 4));
   pg.piece = reinterpret_cast<uint4 *>(b);
-  pg.cnt = b + 4 * L.pieces;
+  *lacks = b + 4 * L.pieces;
+  pg.cnt = b + 5 * L.pieces;
   pg.last = pg.cnt + wd;
   pg.base = pg.last + wd;
   uint32_t *blist = pg.base + wd;
@@ -1033,17 +1083,17 @@ SortLayout sort_layout(const Plan &p, int64_t n, int rw) {
   const int nhi = 1 << tg.hi_bits, nlo = 1 << tg.lo_bits;
   S.two = tg.passes == 2;
   if (!S.two) {
-    S.L2 = paged_layout(n, 1, nhi, rw, 3, 8, 8);
+    S.L2 = paged_layout(n, n, 1, nhi, rw, 3, 8, 8);
     return S;
   }
   S.paged1 = first_paged(p, n);
   if (S.paged1) {
-    S.L1 = paged_layout(n, 1, nhi, rw, 6, 8, 8);
+    S.L1 = paged_layout(n, n, 1, nhi, rw, 6, 8, 8);
     S.slots1 = S.L1.slots();
     S.paged1 = S.slots1 <= ((int64_t)1 << 32);
   }
   if (!S.paged1) S.slots1 = n;
-  S.L2 = paged_layout(S.slots1, nhi, nlo, rw, 3, 8, 2, S.paged1 ? S.L1.lg : 0);
+  S.L2 = paged_layout(n, S.slots1, nhi, nlo, rw, 3, 8, 2, S.paged1 ? S.L1.lg : 0);
   return S;
 }
 
@@ -1077,68 +1127,91 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
     mrange_w = mrange + 2;
   }
 
-  PgOut pg2;
-  uint32_t *blist = pg_buffers(p.pages, S.L2, S.two ? nlo : nhi, pg2, tot);
-  const DigitSel dlo = digit_sel(kg, 0, S.two ? tg.lo_bits : tg.hi_bits);
-  float *out;
+  // the last pass, and before it the first of two
+  PtArgs P2;
+  uint32_t *lacks;
+  uint32_t *blist = pg_buffers(p.pages, S.L2, S.two ? nlo : nhi, P2.pg, tot, &lacks);
+  const PgOut &pg2 = P2.pg;
+  P2.grid = S.L2.G;
+  P2.im.n = n;
+  P2.im.chunk = S.L2.chunk;
+  P2.ds = digit_sel(kg, 0, S.two ? tg.lo_bits : tg.hi_bits);
+  P2.nb = S.two ? nlo : nhi;
+  P2.h = S.L2.h;
+  P2.dst = S.two ? B : A;
   if (!S.two) {
-    out = A;
+    P2.pos = pos;
+    P2.masses = masses;
+    P2.perm = perm1;
+    P2.mrange_w = mrange_w;
     Stage st(p, "sort_downsweep1");
-    InMap im;
-    im.n = n;
-    im.chunk = S.L2.chunk;
-    launch_partition<NM, IN_RAW, true>(S.L2.G, s, pos, masses, nullptr, nullptr, nullptr, out, im, kg, dlo, nhi, S.L2.h, nullptr, perm1, mrange_w, pg2);
+    launch_partition<NM, IN_RAW, true>(P2, kg, s);
   } else {
-    out = B;
-    const DigitSel dhi = digit_sel(kg, tg.lo_bits, tg.hi_bits);
+    PtArgs P1;
+    P1.pos = pos;
+    P1.masses = masses;
+    P1.im.n = n;
+    P1.im.chunk = S.paged1 ? S.L1.chunk : chunk1;
+    P1.grid = g1;
+    P1.ds = digit_sel(kg, tg.lo_bits, tg.hi_bits);
+    P1.nb = nhi;
+    P1.dst = A;
+    P1.perm = perm1;
+    P1.mrange_w = mrange_w;
     // segments of pass 2: first list entry (or record), and the segment of
     // each workgroup's first
     const int64_t ss = nhi + 4;
     uint32_t *sb = static_cast<uint32_t *>(p.seginfo.ensure((size_t)(ss + S.L2.G) * 4));
-    InMap im1, im2;
-    const uint32_t *list1 = nullptr;
-    im1.n = n;
-    im1.chunk = S.paged1 ? S.L1.chunk : chunk1;
-    im2.nseg = nhi;
-    im2.chunk = S.L2.chunk;
     DirArgs D{};
     D.tot = tot + ks;
     D.nb = D.kreal = nhi;
     D.start = sb;
     D.first_seg = sb + ss;
     D.piece = pg2.piece;
+    D.lacks = lacks;
     D.npiece = S.L2.pieces;
+    P2.pos = A;
+    P2.start = sb;
+    P2.first_seg = sb + ss;
+    P2.lacks = lacks;
+    P2.im.nseg = nhi;
+    P2.perm = perm2;
     if (S.paged1) {
       // pass 1, paged: the positions are read once
-      PgOut pg1;
-      uint32_t *blist1 = pg_buffers(p.pages1, S.L1, nhi, pg1, tot + ks);
+      uint32_t *lacks1;
+      uint32_t *blist1 = pg_buffers(p.pages1, S.L1, nhi, P1.pg, tot + ks, &lacks1);
+      P1.h = S.L1.h;
       {
         Stage st(p, "sort_downsweep1");
-        launch_partition<NM, IN_RAW, true>(S.L1.G, s, pos, masses, nullptr, nullptr, nullptr, A, im1, kg, dhi, nhi, S.L1.h, nullptr, perm1, mrange_w,
-                                           pg1);
+        launch_partition<NM, IN_RAW, true>(P1, kg, s);
       }
       Stage st(p, "sort_pages");
       D.unit = (uint32_t)(S.L2.chunk >> S.L1.lg);
       D.funit = FastDiv(D.unit);
       launch_dir(D, s);
-      hipLaunchKernelGGL(k_list, dim3((unsigned)S.L1.pieces), dim3(SORT_THREADS), nhi * 4, s, pg1, nhi, D.start, blist1);
+      hipLaunchKernelGGL(k_list, dim3((unsigned)S.L1.pieces), dim3(SORT_THREADS), nhi * 4, s, P1.pg, nhi, D.start,
+                         blist1);
       GENPK_LAUNCH_CHECK();
-      list1 = blist1;
-      im2.lg = S.L1.lg;
+      hipLaunchKernelGGL(k_lacks, dim3((unsigned)S.L2.G), dim3(LACK_THREADS), 0, s, blist1, sb, sb + ss, nhi, S.L1.lg,
+                         D.unit, lacks);
+      GENPK_LAUNCH_CHECK();
+      P2.blist = blist1;
+      P2.im.lg = S.L1.lg;
     } else {
       // pass 1, counted
       uint32_t *t1 = static_cast<uint32_t *>(p.table1.ensure((size_t)nhi * g1 * 4));
+      P1.h = partition_shape(nhi, RW, false, 8);
+      P1.offsets = t1;
       {
         Stage st(p, "sort_upsweep1");
-        hipLaunchKernelGGL((k_upsweep<NM>), dim3((unsigned)g1), dim3(SORT_THREADS), nhi * 4, s, raw, im1, kg, dhi,
+        hipLaunchKernelGGL((k_upsweep<NM>), dim3((unsigned)g1), dim3(SORT_THREADS), nhi * 4, s, raw, P1.im, kg, P1.ds,
                            nhi, t1);
         GENPK_LAUNCH_CHECK();
       }
       exclusive_scan_u32(t1, t1, (int64_t)nhi * g1, p.scan_tmp, s);
       {
         Stage st(p, "sort_downsweep1");
-        launch_partition<NM, IN_RAW, false>(g1, s, pos, masses, nullptr, nullptr, nullptr, A, im1, kg, dhi, nhi, partition_shape(nhi, RW, false, 8), t1,
-                                            perm1, mrange_w, PgOut{});
+        launch_partition<NM, IN_RAW, false>(P1, kg, s);
       }
       hipLaunchKernelGGL(k_seg_tot, dim3((unsigned)ceil_div(nhi, 256)), dim3(256), 0, s, t1, g1, nhi, n, tot + ks);
       GENPK_LAUNCH_CHECK();
@@ -1148,9 +1221,9 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
     }
     Stage st(p, "sort_downsweep2");
     if (S.paged1)
-      launch_partition<NM, IN_LIST, true>(S.L2.G, s, A, nullptr, list1, sb, sb + ss, out, im2, kg, dlo, nlo, S.L2.h, nullptr, perm2, nullptr, pg2);
+      launch_partition<NM, IN_LIST, true>(P2, kg, s);
     else
-      launch_partition<NM, IN_SEG, true>(S.L2.G, s, A, nullptr, list1, sb, sb + ss, out, im2, kg, dlo, nlo, S.L2.h, nullptr, perm2, nullptr, pg2);
+      launch_partition<NM, IN_SEG, true>(P2, kg, s);
   }
 
   // the tiles' block lists and work items
@@ -1195,19 +1268,20 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   {
     Stage st(p, "sort_tiles");
     launch_dir(D, s);
-    hipLaunchKernelGGL(k_list, dim3((unsigned)S.L2.pieces), dim3(SORT_THREADS), (S.two ? nlo : nhi) * 4, s, pg2, S.two ? nlo : nhi,
-                       D.start, blist);
+    hipLaunchKernelGGL(k_list, dim3((unsigned)S.L2.pieces), dim3(SORT_THREADS), P2.nb * 4, s, pg2, P2.nb, D.start,
+                       blist);
     GENPK_LAUNCH_CHECK();
   }
   p.sort_tot_zero = ntot;
 
-  o.rec = out;
+  o.rec = P2.dst;
   o.rw = RW;
   o.has_mass = NM != 0;
   o.has_perm = with_perm;
   o.perm1 = perm1;
   o.perm2 = perm2;
-  o.list = {D.start, D.pstart, D.items, D.counts, D.cost, D.share, blist, S.L2.lg, ks, max_items, D.max_parts, D.wgs};
+  o.list = {D.start, D.pstart, D.items, D.counts, D.cost,      D.share,
+            blist,   S.L2.lg,  ks,      max_items, D.max_parts, D.wgs};
   o.heavy = D.heavy;
   o.mrange = mrange;
   o.n = n;
