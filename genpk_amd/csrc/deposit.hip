@@ -545,7 +545,7 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
   const float *sorted = o.rec;
   const TileList &L = o.list;
   const int64_t n = o.n;
-  double *partials = static_cast<double *>(p.partials.ensure((size_t)L.max_parts * tg.cells * 8 + 64));
+  double *partials = o.partials;
 
   DepParams P;
   P.kg = kg;

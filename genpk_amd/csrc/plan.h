@@ -117,6 +117,7 @@ struct TileOrder {
   const uint32_t *perm1 = nullptr, *perm2 = nullptr;
   TileList list;
   const uint32_t *heavy = nullptr;  // the split tiles, in any order
+  double *partials = nullptr;       // room for the partial tiles of their items
   // with masses: [0] the bits of the largest |mass|, [1] those of the
   // smallest nonzero |mass| (0xffffffff when every mass is 0)
   const uint32_t *mrange = nullptr;

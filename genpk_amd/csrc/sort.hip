@@ -1075,7 +1075,18 @@ struct SortLayout {
   bool two = false, paged1 = false;
   PgLayout L1, L2;  // paged first pass (of two), last pass
   int64_t slots1 = 0;  // slots that a first pass of two writes
+  uint32_t imax = 0;   // records of a work item at most
+  int64_t max_parts = 0;  // items of split tiles at most
 };
+
+// Items of split tiles at most: a tile of r records in r + w slots has m =
+// max(ceil(r / imax), ceil((r + w) / 2^17)) items, and where m > 1 the first is at
+// most 2 r / imax, the second at most 2 r / 2^17 + 2 w / 2^17 (imax <= 2^17), so m
+// is at most 2 r / imax + 2 w / 2^17.
+void set_max_parts(SortLayout &S, const Plan &p, int64_t n) {
+  S.imax = deposit_item_max(n, p.tg.K);
+  S.max_parts = 2 * (ceil_div(n, (int64_t)S.imax) + ceil_div(S.L2.slots() - n, (int64_t)DEPOSIT_ITEM_MAX));
+}
 
 SortLayout sort_layout(const Plan &p, int64_t n, int rw) {
   SortLayout S;
@@ -1084,6 +1095,7 @@ SortLayout sort_layout(const Plan &p, int64_t n, int rw) {
   S.two = tg.passes == 2;
   if (!S.two) {
     S.L2 = paged_layout(n, n, 1, nhi, rw, 3, 8, 8);
+    set_max_parts(S, p, n);
     return S;
   }
   S.paged1 = first_paged(p, n);
@@ -1094,6 +1106,7 @@ SortLayout sort_layout(const Plan &p, int64_t n, int rw) {
   }
   if (!S.paged1) S.slots1 = n;
   S.L2 = paged_layout(n, S.slots1, nhi, nlo, rw, 3, 8, 2, S.paged1 ? S.L1.lg : 0);
+  set_max_parts(S, p, n);
   return S;
 }
 
@@ -1228,12 +1241,8 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
 
   // the tiles' block lists and work items
   TileOrder o;
-  const uint32_t imax = deposit_item_max(n, tg.K);
   const int64_t slots = S.L2.slots();
-  // split tiles have m > 1 items, at most twice the item sizes that fill them
-  const int64_t max_parts = 2 * ((imax < (uint32_t)DEPOSIT_ITEM_MAX ? ceil_div(n, (int64_t)imax) : 0) +
-                                 ceil_div(slots, (int64_t)DEPOSIT_ITEM_MAX));
-  const int64_t max_items = tg.K + max_parts;
+  const int64_t max_items = tg.K + S.max_parts;
   const int64_t ts = (ks + 4) / 4 * 4;
   const int64_t nsec = ceil_div(ks, dir_section(ks));
   uint32_t *ib = static_cast<uint32_t *>(p.item_start.ensure((size_t)(ts + nsec) * 4 * 4 + 64));
@@ -1246,13 +1255,13 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   D.items = static_cast<uint4 *>(p.items.ensure((size_t)max_items * 16));
   D.store = every_tile ? 1 : 0;
   D.lg = S.L2.lg;
-  D.limax = ilog2(imax);
+  D.limax = ilog2(S.imax);
   D.pstart = ib + 2 * ts;
   D.heavy = ib + 3 * ts;
   D.secsum = reinterpret_cast<uint4 *>(ib + 4 * ts);
   D.counts = static_cast<uint32_t *>(p.heavy.ensure(64 + DEPOSIT_WGS_MAX * 4));
   D.share = D.counts + 16;
-  D.max_parts = (uint32_t)max_parts;
+  D.max_parts = (uint32_t)S.max_parts;
   D.wgs = (uint32_t)deposit_wgs(p, RW, max_items);
   D.fwgs = FastDiv(D.wgs);
   // the flush of a tile and the waits around it take about as long as the
@@ -1283,6 +1292,7 @@ TileOrder sort_impl(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, con
   o.list = {D.start, D.pstart, D.items, D.counts, D.cost,      D.share,
             blist,   S.L2.lg,  ks,      max_items, D.max_parts, D.wgs};
   o.heavy = D.heavy;
+  o.partials = (S.two ? p.recA : p.partials).as<double>();
   o.mrange = mrange;
   o.n = n;
   return o;
@@ -1317,13 +1327,17 @@ TileOrder sort_by_tile(Plan &p, const KeyGeom &kg, int64_t n, const float *pos, 
   // recA); with the permutations the other one also takes the adjoint
   // gather's output records (up to 4 floats per slot of the sorted pool).
   // perm2 is indexed by pass-1 slots.
+  // The partial tiles too lie in the pool that the last pass has read (2.8 GB
+  // of their own at 2^30 records).
   const size_t last = (size_t)S.L2.slots(), gather = with_perm ? last * 16 : 0;
+  const size_t parts = (size_t)S.max_parts * p.tg.cells * 8 + 64;
   if (S.two) {
-    p.recA.ensure(std::max((size_t)S.slots1 * rw * 4, gather));
+    p.recA.ensure(std::max({(size_t)S.slots1 * rw * 4, gather, parts}));
     p.recB.ensure(last * rw * 4);
   } else {
     p.recA.ensure(last * rw * 4);
     if (with_perm) p.recB.ensure(gather);
+    p.partials.ensure(parts);
   }
   if (with_perm) {
     p.permA.ensure((size_t)n * 4);

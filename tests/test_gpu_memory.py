@@ -40,3 +40,35 @@ def test_first_forward_memory(gpu, d, n, masses):
     bound = tiles * cells * 4 + 2 * pool * (16 if masses else 12) + 2 * (pool // (1 << 17) + 1) * cells * 8 + n // 4 + (64 << 20)
     print(f"taken {taken / 1e9:.3f} GB, bound {bound / 1e9:.3f} GB", flush=True)
     assert taken <= bound
+
+
+@pytest.mark.gpu
+def test_partial_tiles_share_the_first_pool(gpu):
+    """Where the partition takes two passes the partial tiles of split tiles lie
+    in the first pass's pool, which the second pass has read: the bound above
+    without them.  A second deposit of clumped particles (split tiles) and one
+    from the kept order are equal to the first."""
+    import torch
+    d, n = 1024, 1 << 30
+    print("CASE", d, n, flush=True)
+    pos = torch.rand((n, 3), device="cuda") * BOX
+    p = genpk_amd.Plan(d, "f32")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    p.deposit(pos, BOX)
+    torch.cuda.synchronize()
+    taken = before - torch.cuda.mem_get_info()[0]
+    bound = 65536 * 17 * 33 * 33 * 4 + 2 * (n + n // 6) * 12 + n // 4 + (64 << 20)
+    print(f"taken {taken / 1e9:.3f} GB, bound {bound / 1e9:.3f} GB", flush=True)
+    assert taken <= bound
+    del p, pos
+    d, n = 512, 20000000
+    pos = (torch.randn((n, 3), device="cuda") * 3.0 + 50.0).contiguous()
+    p = genpk_amd.Plan(d, "f64")
+    got = []
+    for again in (False, False, True):
+        p.clear()
+        p.redeposit() if again else p.deposit(pos, BOX, retain=True)
+        got.append(p.export_density().clone())
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    assert abs(float(got[0].sum()) - n) <= 1e-6 * n
