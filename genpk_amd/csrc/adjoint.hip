@@ -66,14 +66,18 @@ struct AdjWeight {
 
 // The adjoint weight from LDS: the per-bin factors 2 lambda_b / (M^2 C_b), the
 // window factors and the bin thresholds, so that a mode's weight costs no
-// global read and no division.
+// global read and no division.  Only the thresholds that bin_lds reads: at
+// 1024^3 in FP64 the tables of 1024 bins then fit to the byte (adjoint x pass
+// 8.83 -> 6.97 ms).
 struct LdsWeight {
   double *sfb;  // [nrbins]
   float *swt;   // [d]
-  int *sthr;    // [nrbins + 1]
+  int *sthr;    // [bin_lds_slots(nrbins)]
   int nrbins;
   float lq;
-  static size_t bytes(int64_t d, int nrbins) { return (size_t)nrbins * 8 + (size_t)d * 4 + (size_t)(nrbins + 1) * 4; }
+  static size_t bytes(int64_t d, int nrbins) {
+    return (size_t)nrbins * 8 + (size_t)d * 4 + (size_t)bin_lds_slots(nrbins) * 4;
+  }
   // fill the tables (16-byte aligned at) with the whole workgroup; no barrier
   __device__ __forceinline__ void init(void *at, const AdjWeight &w, int64_t d) {
     sfb = static_cast<double *>(at);
@@ -86,7 +90,7 @@ struct LdsWeight {
       sfb[i] = c ? 2.0 * w.lambda[i] * w.inv_m2 / (double)c : 0.0;
     }
     for (int i = threadIdx.x; i < d; i += blockDim.x) swt[i] = w.wtab[i];
-    for (int i = threadIdx.x; i <= w.nrbins; i += blockDim.x) sthr[i] = (int)w.thr[i];
+    for (int i = threadIdx.x; i < bin_lds_slots(w.nrbins); i += blockDim.x) sthr[i] = (int)w.thr[i];
   }
   // weight of array index xi along x of a column with a = ky^2 + kz^2 and
   // window factors wy, wz
@@ -179,10 +183,10 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
 // stage runs from the loaded registers, the stages alternate between two
 // LDS buffers (one barrier each), and the next block's loads are in flight
 // during this block's inverse transform and stores.
-// LW: the weight from LDS tables.  LT (with LW, a last radix 2): the last forward stage runs in registers with the
-// weight (LdsWeight), and each thread's modes find their bin by tracking the
-// thresholds along kx.  (Compile-time stages for n = 1024 spill
-// registers here: 5.2 -> 7.3 ms at 1024^3, against 4.3 ms without.)
+// LW: the weight from LDS tables (LdsWeight).  LT (with LW, a last radix 2):
+// the last forward stage runs in registers, each mode weighted before it is
+// written.  (Compile-time stages for n = 1024 spill registers here: 5.2 -> 7.3
+// ms at 1024^3, against 4.3 ms without.)
 template <typename T, bool LT, bool LW>
 __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C *__restrict__ f, ColMap cm,
                                                              RadixPlan rp, const typename Cx<T>::C *__restrict__ tw, AdjWeight w) {
@@ -253,7 +257,7 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C 
     } else {
       res = lds_fft_pp<-1, true, MAXE>(buf2, buf, rp, B, lgb, B, 1, stw, 1);
       const int kz = (int)c.kz0 + b, ky = (int)kv(y, d);
-        for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
+      for (int i = threadIdx.x; i < tot; i += ADJ_THREADS) {
         const int e = i >> lgb;
         if (b < c.nb) {
           const double s = LW ? lw.at(e, n, ky * ky + kz * kz, lw.swt[y], lw.swt[kz]) : w.at(e, y, kz, d);
