@@ -158,8 +158,8 @@ template <typename T, int NF, bool REG1, bool R2L = false, int CT = 0>
 __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__restrict__ fa,
                                                             typename Cx<T>::C *__restrict__ fb, BinGeom g, ColMap cm,
                                                             RadixPlan rp,
-                                                            const typename Cx<T>::C *__restrict__ tw, int keep,
-                                                            int pp, int lgc, double *__restrict__ part) {
+                                                            const typename Cx<T>::C *__restrict__ tw, int pp,
+                                                            int lgc, double *__restrict__ part) {
   using C = typename Cx<T>::C;
   constexpr int NS = NF == 1 ? 1 : 3;
   static_assert(!R2L || REG1, "the radix-2 last stage in the binning needs the register first stage");
@@ -213,7 +213,6 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
   for (int64_t v = blockIdx.x; v < nblk; v += gridDim.x) {
     const ColMap::Block c = cm.at(xcd_block((uint32_t)v, (uint32_t)nblk));
     const int64_t y = c.outer;
-    const int64_t off = y * hz + c.kz0;
     C *res = buf;
     if constexpr (REG1 && NF == 2) {
       __syncthreads();  // the previous block's binning is done with buf
@@ -248,15 +247,6 @@ __global__ void __launch_bounds__(BIN_THREADS) k_xpass_bin(typename Cx<T>::C *__
       } else {
         lds_fft<-1, true, MAXE>(buf, rp, B, lgb, B, 1, stw);
         if (NF == 2) lds_fft<-1, true, MAXE>(buf + n * B, rp, B, lgb, B, 1, stw);
-      }
-    }
-    if (keep) {
-      for (int i = threadIdx.x; i < n * B; i += BIN_THREADS) {
-        const int e = i >> lgb;  // of column my_b
-        if (my_b < c.nb) {
-          fa[off + e * estride + my_b] = res[i];
-          if (NF == 2) fb[off + e * estride + my_b] = res[n * B + i];
-        }
       }
     }
     if (v + gridDim.x < nblk) load(v + gridDim.x);
@@ -682,17 +672,15 @@ static int fused_grid(const Plan &a, int B, int nrbins, bool pp, int lgc) {
 }
 
 template <typename T, int NF, bool REG1, bool R2L = false, int CT = 0>
-static void launch_fused(Plan &a, Plan *b, const BinTables &bt, const RadixPlan &rp, int B, bool keep, bool pp,
+static void launch_fused(Plan &a, Plan *b, const BinTables &bt, const RadixPlan &rp, int B, bool pp,
                          int lgc, double *part, int G) {
   using C = typename Cx<T>::C;
-  // the R2L instance finishes the transform only in registers for the binning
-  GENPK_REQUIRE(!(R2L && keep), "the fused pass cannot keep the spectrum with the last stage in the binning");
   const C *tw = (a.prec == 4) ? (const C *)a.fft.tw_d_f32.ptr : (const C *)a.fft.tw_d_f64.ptr;
   BinGeom g{a.d, a.hz, bt.nrbins, bt.q2bin.as<int>(), bt.thr.as<int64_t>(), a.wtab.as<float>(), bt.lq};
   const size_t lds = fused_lds<T, NF>(a, B, bt.nrbins, pp, lgc);
   Stage st(a, "xpass_bin");
   hipLaunchKernelGGL((k_xpass_bin<T, NF, REG1, R2L, CT>), dim3(G), dim3(BIN_THREADS), lds, a.stream, a.field.as<C>(),
-                     b ? b->field.as<C>() : (C *)nullptr, g, col_map(a.d, a.hz, B), rp, tw, keep ? 1 : 0, pp ? 1 : 0, lgc, part);
+                     b ? b->field.as<C>() : (C *)nullptr, g, col_map(a.d, a.hz, B), rp, tw, pp ? 1 : 0, lgc, part);
   GENPK_LAUNCH_CHECK();
 }
 
@@ -743,12 +731,12 @@ static int fused_grid_of(const Plan &a, bool cross, const FusedShape &s, int nrb
 
 template <typename T>
 static void launch_fused_of(Plan &a, Plan *b, const BinTables &bt, const FusedShape &s, double *part) {
-  if (b && s.reg1) launch_fused<T, 2, true>(a, b, bt, s.rp, s.B, false, false, s.lgc, part, s.G);
-  else if (b) launch_fused<T, 2, false>(a, b, bt, s.rp, s.B, false, false, s.lgc, part, s.G);
-  else if (s.r2l && s.ct) launch_fused<T, 1, true, true, 1024>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
-  else if (s.r2l) launch_fused<T, 1, true, true>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
-  else if (s.reg1) launch_fused<T, 1, true>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
-  else launch_fused<T, 1, false>(a, b, bt, s.rp, s.B, false, s.pp, s.lgc, part, s.G);
+  if (b && s.reg1) launch_fused<T, 2, true>(a, b, bt, s.rp, s.B, false, s.lgc, part, s.G);
+  else if (b) launch_fused<T, 2, false>(a, b, bt, s.rp, s.B, false, s.lgc, part, s.G);
+  else if (s.r2l && s.ct) launch_fused<T, 1, true, true, 1024>(a, b, bt, s.rp, s.B, s.pp, s.lgc, part, s.G);
+  else if (s.r2l) launch_fused<T, 1, true, true>(a, b, bt, s.rp, s.B, s.pp, s.lgc, part, s.G);
+  else if (s.reg1) launch_fused<T, 1, true>(a, b, bt, s.rp, s.B, s.pp, s.lgc, part, s.G);
+  else launch_fused<T, 1, false>(a, b, bt, s.rp, s.B, s.pp, s.lgc, part, s.G);
 }
 
 static FusedShape fused_shape(const Plan &a, const Plan *b, int nrbins) {
