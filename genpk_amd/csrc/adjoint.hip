@@ -189,7 +189,8 @@ __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x(typename Cx<T>::C *__
 // ms at 1024^3, against 4.3 ms without.)
 template <typename T, bool LT, bool LW>
 __global__ void __launch_bounds__(ADJ_THREADS) k_adjoint_x_pp(typename Cx<T>::C *__restrict__ f, ColMap cm,
-                                                             RadixPlan rp, const typename Cx<T>::C *__restrict__ tw, AdjWeight w) {
+                                                             RadixPlan rp, const typename Cx<T>::C *__restrict__ tw,
+                                                             AdjWeight w) {
   using C = typename Cx<T>::C;
   constexpr int MAXE = AdjCfg<T>::MAXE;
   extern __shared__ unsigned char lds_raw[];
@@ -438,10 +439,10 @@ __global__ void __launch_bounds__(GATHER_THREADS) k_gather_tiles(const T *__rest
 // perm1 and writes are coalesced; the two lookups are random reads, which
 // cost far less than scattered partial-line writes.  Each XCD (workgroup id
 // mod 8) takes runs of UNP_RUN consecutive blocks, the eight XCDs' runs side
-// by side: both partition passes are stable, so a run's particles of one
-// bucket sit together in perm2 and its lines are fetched by one L2, while
-// all XCDs stay within one window of the particles.  The grid is a multiple
-// of 8 * UNP_RUN.
+// by side: a workgroup of the first pass writes to a range of slots of its own,
+// so a run's particles of one bucket sit together in perm2 and its lines are
+// fetched by one L2, while all XCDs stay within one window of the particles.
+// The grid is a multiple of 8 * UNP_RUN.
 constexpr int UNP_RUN = 256;
 template <int RWO, int TWO>
 __global__ void k_unpermute(const float *__restrict__ rec, const uint32_t *__restrict__ perm1,
@@ -504,20 +505,21 @@ void adjoint_x_impl(Plan &p, const AdjWeight &w) {
     const size_t lds = lw ? lds_pp + lds_w : lds_pp;
     int per_cu = 0;
     GENPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, ADJ_THREADS, lds));
-    const dim3 g((unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), (int64_t)cm.nblk)));
-    if (lt)
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, true, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, rp, tw, w);
-    else if (lw)
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, true>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, rp, tw, w);
-    else
-      hipLaunchKernelGGL((k_adjoint_x_pp<T, false, false>), g, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, rp, tw, w);
+    const int64_t most = std::min<int64_t>((int64_t)std::max(per_cu, 1) * num_cus(), (int64_t)cm.nblk);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)std::max<int64_t>(1, most)), dim3(ADJ_THREADS), lds, p.stream,
+                         p.field.as<C>(), cm, rp, tw, w);
+    };
+    if (lt) go(k_adjoint_x_pp<T, true, true>);
+    else if (lw) go(k_adjoint_x_pp<T, false, true>);
+    else go(k_adjoint_x_pp<T, false, false>);
   } else {
-    const dim3 grid(cm.nblk);
     const size_t lds = (size_t)(tot + p.d) * sizeof(C);
-    if (lds + lds_w <= cap)
-      hipLaunchKernelGGL((k_adjoint_x<T, true>), grid, dim3(ADJ_THREADS), lds + lds_w, p.stream, p.field.as<C>(), cm, p.rp_d, tw, w);
-    else
-      hipLaunchKernelGGL((k_adjoint_x<T, false>), grid, dim3(ADJ_THREADS), lds, p.stream, p.field.as<C>(), cm, p.rp_d, tw, w);
+    auto go = [&](auto kernel, size_t bytes) {
+      hipLaunchKernelGGL(kernel, dim3(cm.nblk), dim3(ADJ_THREADS), bytes, p.stream, p.field.as<C>(), cm, p.rp_d, tw, w);
+    };
+    if (lds + lds_w <= cap) go(k_adjoint_x<T, true>, lds + lds_w);
+    else go(k_adjoint_x<T, false>, lds);
   }
   GENPK_LAUNCH_CHECK();
 }

@@ -9,8 +9,12 @@
 // plan buffer and builds the bin tables, so the capture allocates nothing),
 // then capture fork -> per-branch job sequences -> join on the batch stream
 // and instantiate.  Every kernel of a job rewrites what it reads later (the
-// deposit writes every tile, the binning every partial), so replays are
-// independent of earlier launches.  No counterpart in the reference.
+// deposit writes every tile, the binning every partial) but for the sort's
+// bucket totals, which have to be zero when it starts and which its directory
+// clears again (sort_impl): the build's eager run leaves them so, and every
+// replay after it, so replays do not depend on which launches came before.
+// The branches' plans are the batch's own, and nothing else sorts with them.
+// No counterpart in the reference.
 #include "fft_core.h"
 #include "plan.h"
 #include "../../include/genpk_amd.h"

@@ -384,7 +384,8 @@ constexpr int STORED_RUN = 8;
 template <typename T, int NF, bool LT>
 __global__ void __launch_bounds__(BIN_THREADS) k_bin_stored(const typename Cx<T>::C *__restrict__ fa,
                                                              const typename Cx<T>::C *__restrict__ fb, BinGeom g,
-                                                             FastDiv fhz, FastDiv fny, int lgc, double *__restrict__ part) {
+                                                             FastDiv fhz, FastDiv fny, int lgc,
+                                                             double *__restrict__ part) {
   using C = typename Cx<T>::C;
   constexpr int NS = NF == 1 ? 1 : 3, RUN = STORED_RUN;
   extern __shared__ unsigned char lds_raw[];
@@ -469,7 +470,8 @@ __global__ void __launch_bounds__(BIN_THREADS) k_bin_stored(const typename Cx<T>
 // chain of G / 8 memory round trips in one to four workgroups: 14 us for 256
 // partials, 26 for 512; this 4.)
 constexpr int FIN_BINS = 16, FIN_SLICES = 16;
-__global__ void __launch_bounds__(FIN_BINS * FIN_SLICES) k_bin_finish(int nrbins, int ns, int G, const double *__restrict__ part,
+__global__ void __launch_bounds__(FIN_BINS * FIN_SLICES)
+    k_bin_finish(int nrbins, int ns, int G, const double *__restrict__ part,
                              const int *__restrict__ count, const double *__restrict__ keffsum, double m_aa,
                              double m_bb, double m_ab, double *__restrict__ p_aa, double *__restrict__ p_bb,
                              double *__restrict__ p_ab, int *__restrict__ count_out, double *__restrict__ keffs_out) {
@@ -772,8 +774,9 @@ static FusedShape fused_shape(const Plan &a, const Plan *b, int nrbins) {
   s.ct = s.r2l && is_plan_8882(s.rp);
   const bool cross = b != nullptr;
   auto lds_of = [&](int lgc) {
-    return cross ? (a.prec == 4 ? fused_lds<float, 2>(a, B, nrbins, false, lgc) : fused_lds<double, 2>(a, B, nrbins, false, lgc))
-                 : (a.prec == 4 ? fused_lds<float, 1>(a, B, nrbins, s.pp, lgc) : fused_lds<double, 1>(a, B, nrbins, s.pp, lgc));
+    if (a.prec == 4)
+      return cross ? fused_lds<float, 2>(a, B, nrbins, false, lgc) : fused_lds<float, 1>(a, B, nrbins, s.pp, lgc);
+    return cross ? fused_lds<double, 2>(a, B, nrbins, false, lgc) : fused_lds<double, 1>(a, B, nrbins, s.pp, lgc);
   };
   while (s.lgc < LGC_MAX && lds_of(s.lgc + 1) <= (size_t)LDS_LIMIT) s.lgc++;
   s.G = a.prec == 4 ? fused_grid_of<float>(a, cross, s, nrbins) : fused_grid_of<double>(a, cross, s, nrbins);
@@ -825,7 +828,8 @@ void bin_spectra(Plan &a, Plan *b, int nrbins, bool fused_xpass, double *pow_aa,
       if (b) launch_stored<double, 2>(a, b, bt, part, G); else launch_stored<double, 1>(a, b, bt, part, G);
     }
   }
-  hipLaunchKernelGGL(k_bin_finish, dim3((unsigned)ceil_div(nrbins, FIN_BINS), (unsigned)ns), dim3(FIN_BINS * FIN_SLICES), 0, a.stream, nrbins, ns, G, part,
+  hipLaunchKernelGGL(k_bin_finish, dim3((unsigned)ceil_div(nrbins, FIN_BINS), (unsigned)ns),
+                     dim3(FIN_BINS * FIN_SLICES), 0, a.stream, nrbins, ns, G, part,
                      bt.count.as<int>(), bt.keffsum.as<double>(), b ? ma * ma : ma * mb, mb * mb, ma * mb, pow_aa,
                      b ? pow_bb : (double *)nullptr, b ? pow_ab : (double *)nullptr, count, keffs);
   GENPK_LAUNCH_CHECK();

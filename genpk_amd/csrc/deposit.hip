@@ -442,8 +442,8 @@ __global__ void __launch_bounds__(256) k_reduce_partials(const uint32_t *__restr
 // up NaN or infinite there.  Here those cells are set to NaN in the tile
 // store, at the cells cell_of_x86 gives (those of the reference on x86-64).
 // The records are scanned only when k_deposit raised the flag.  A cell's
-// own store location is written (never a halo), so the order against the
-// halo folds does not matter, and later deposits keep it NaN.
+// own store location is written (never a halo), to which the readers add the
+// halos, and later deposits keep it NaN.
 template <typename Real>
 __global__ void __launch_bounds__(256) k_poison(const float *__restrict__ rec, int rw, TileList T, KeyGeom kg,
                                                 FoldGeom fg, const uint32_t *__restrict__ nonfinite,
@@ -641,8 +641,9 @@ FoldGeom fold_geom(const Plan &p) {
 int64_t deposit_wgs(const Plan &p, int rw, int64_t max_items) {
   const bool st = std_tiles_of(p.tg);
   const size_t lds = (size_t)p.tg.cells * 8;
-  const int per_cu = p.prec == 4 ? (rw == 4 ? deposit_per_cu<float, 1, 4>(st, lds) : deposit_per_cu<float, 0, 3>(st, lds))
-                                 : (rw == 4 ? deposit_per_cu<double, 1, 4>(st, lds) : deposit_per_cu<double, 0, 3>(st, lds));
+  const int per_cu = p.prec == 4 ? rw == 4 ? deposit_per_cu<float, 1, 4>(st, lds) : deposit_per_cu<float, 0, 3>(st, lds)
+                     : rw == 4   ? deposit_per_cu<double, 1, 4>(st, lds)
+                                 : deposit_per_cu<double, 0, 3>(st, lds);
   return std::min({(int64_t)per_cu * num_cus(), DEPOSIT_WGS_MAX, max_items});
 }
 

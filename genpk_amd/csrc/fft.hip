@@ -32,8 +32,8 @@ template <> struct FftCfg<double> { static constexpr int ELEMS = 4096; static co
 // FROM_TILES: the rows are assembled from the deposit's tile store while
 // loading, halo cells folded in (the fold), so the real-space grid is never
 // written.
-// The LDS footprint (up to 64 KB) allows two workgroups per CU, so the
-// register budget of two waves per SIMD is available.  The rows sit in LDS
+// Two workgroups share a CU (up to 80 KB of LDS each, and registers for four
+// waves per SIMD: waves_per_eu).  The rows sit in LDS
 // with one element of padding per 32 (lds_ix), which spreads the strided
 // writes of the FFT stages over the banks.
 // BFLY (from the tile store; the first stage's radix, 0: element by element):
@@ -54,11 +54,10 @@ template <> struct FftCfg<double> { static constexpr int ELEMS = 4096; static co
 // 2.06 ms at 1024^3 FP32 and 0.069 -> 0.061 at 256^3 against two in-place
 // fold launches before the pass.
 template <typename T, bool FROM_TILES, int BFLY = 0, int CT = 0, bool STD = false>
-__global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) k_r2c_z(T *__restrict__ field, const T *__restrict__ tiles,
-                                                      FoldGeom fg, FastDiv fdd, int64_t rowlen, int64_t nrows, int L,
-                                                      FastDiv fdM, FastDiv fdK, RadixPlan rp,
-                                                      const typename Cx<T>::C *__restrict__ twM,
-                                                      const typename Cx<T>::C *__restrict__ twd) {
+__global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))
+k_r2c_z(T *__restrict__ field, const T *__restrict__ tiles, FoldGeom fg, FastDiv fdd, int64_t rowlen, int64_t nrows,
+        int L, FastDiv fdM, FastDiv fdK, RadixPlan rp, const typename Cx<T>::C *__restrict__ twM,
+        const typename Cx<T>::C *__restrict__ twd) {
   using C = typename Cx<T>::C;
   constexpr int MAXE = FftCfg<T>::MAXE;
   extern __shared__ unsigned char lds_raw[];
@@ -72,6 +71,7 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
   C *sxw = stw + M;               // [NK]
   if constexpr (BFLY != 0) {
     constexpr int R0 = BFLY, NB = R0 == 8 ? 2 : (MAXE + R0 - 1) / R0;
+    constexpr int HG = R0 % 4 ? R0 : sizeof(T) == 4 ? 4 : 2;  // pairs that add halos at a time
     // butterfly u = threadIdx.x + FFT_THREADS * i: row u / NQ, inputs
     // u % NQ + NQ * r (NQ = M / R0)
     const int NQ = M / R0;
@@ -102,8 +102,8 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
             zh8[r] = lz == 0 ? tiles[(uint32_t)fg.zoff + (txy * 32u + tzp) * CZ + rr] : (T)0;
           }
           if ((x & 15u) == 0 || (y & 31u) == 0)
-            add_halo_rows<T, R0, R0 % 4 ? R0 : sizeof(T) == 4 ? 4 : 2>(tiles, fg, row_fold(fg, (int)x, (int)y), [&](int r) { return 2 * (j + 64 * r); }, w,
-                                zh8);
+            add_halo_rows<T, R0, HG>(
+                tiles, fg, row_fold(fg, (int)x, (int)y), [&](int r) { return 2 * (j + 64 * r); }, w, zh8);
           if (lz == 0) {
 #pragma unroll
             for (int r = 0; r < R0; r++) w[r].x = w[r].x + zh8[r];  // one rounding, as below
@@ -131,7 +131,7 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
             }
           }
           if (rf.fx || rf.fy)
-            add_halo_rows<T, R0, R0 % 4 ? R0 : sizeof(T) == 4 ? 4 : 2>(tiles, fg, rf, [&](int r) { return 2 * (j + NQ * r); }, w, zh8);
+            add_halo_rows<T, R0, HG>(tiles, fg, rf, [&](int r) { return 2 * (j + NQ * r); }, w, zh8);
 #pragma unroll
           for (int r = 0; r < R0; r++) w[r].x = w[r].x + zh8[r];  // as the element-wise load: one rounding
         } else {
@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(FFT_THREADS) __attribute__((amdgpu_waves_per_e
 #pragma unroll
   for (int q = 0; q < MAXE; q++) {
     const int i = threadIdx.x + q * FFT_THREADS;
-    // z-halo added after all loads are in flight (a + b rounds once, as fold_value)
+    // z-halo added after all loads are in flight (a + b rounds once, as in k_fold)
     if (FROM_TILES) v[q].x = v[q].x + zh[FROM_TILES ? q : 0];
     if (i < tot) buf[lds_ix<true>(i)] = v[q];
   }

@@ -90,7 +90,9 @@ struct PgOut {
 
 // A block-list entry: the block in the low 32 - lg bits, its fill (1 to 2^lg
 // records) less one above, so that one load gives both.
-__device__ __forceinline__ uint32_t pg_entry(uint32_t blk, uint32_t fill, int lg) { return blk | (fill - 1) << (32 - lg); }
+__device__ __forceinline__ uint32_t pg_entry(uint32_t blk, uint32_t fill, int lg) {
+  return blk | (fill - 1) << (32 - lg);
+}
 
 // Tile key of a position with the cells along the axes not in `axes` (bit a:
 // axis a of x, y, z) taken as 0 and not computed: cell_of's cells, with one
@@ -468,7 +470,8 @@ __global__ void __launch_bounds__(SORT_THREADS, 4) k_partition(const float *__re
           if (mb) mn = min(mn, mb);
         }
         // where this record goes (coalesced writes, by input position or pool slot)
-        if constexpr (PERM) perm[IN == IN_LIST ? (int64_t)(wslot[IN == IN_LIST ? it : 0] + lane) : s0 + loc] = dest_of(p, dg);
+        if constexpr (PERM)
+          perm[IN == IN_LIST ? (int64_t)(wslot[IN == IN_LIST ? it : 0] + lane) : s0 + loc] = dest_of(p, dg);
       }
     }
     // the next sub-chunk loads during the barrier and the write-out
@@ -1012,9 +1015,12 @@ PgLayout paged_layout(int64_t n, int64_t slots, int64_t nseg, int nb, int rw, in
 }
 
 // Whether the first of two passes is paged (of 2^hi_bits digits): each
-// workgroup has to hold many records of a digit.  With 256 digits the counted
-// pass keeps sorts below 2^29 records, which the tests compare with paged
-// ones.
+// workgroup has to hold many records of a digit.  With 256 digits (32769 to
+// 65536 tiles) the counted pass keeps sorts below 2^29 records, against which
+// the tests check the paged one.  That costs up to 15% of the sort: at 1024^3
+// FP32 both take 0.20 ms at 2^23 records, paged and counted 0.32 and 0.33 (uniform
+// and clumped 0.32 and 0.34) at 2^24, 0.58 and 0.61 at 2^25, 1.00 and 1.13 at 2^26,
+// 3.58 and 4.19 at 2^28.
 bool first_paged(const Plan &p, int64_t n) {
   const int64_t nhi = (int64_t)1 << p.tg.hi_bits, cus = num_cus();
   if (nhi > 256) return false;
