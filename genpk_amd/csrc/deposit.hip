@@ -74,7 +74,13 @@ struct DepParams {
 // masses accumulate in FP64 LDS atomics instead.  STD: tiles of 16 x 32 x 32
 // cells (every grid of d >= 32), whose strides are constants, so the 8 corner
 // offsets fold into the LDS instructions' immediate offsets.
-template <typename Real, int NM, int RW, bool STD>
+//
+// FEW (other tile shapes, items of less than half a batch on average): what a
+// batch does not hold is skipped by the whole workgroup, not lane by lane.
+// That saves 0.16 of 1.96 ms for 2^22 records in 2^18 tiles of 4^3 cells and
+// 0.15 of 2.15 for 2^26 in 2^18 of 8^3, and costs full batches 2% (0.552 -> 0.567
+// ms for 2^27 records at 512^3).
+template <typename Real, int NM, int RW, bool STD, bool FEW = false>
 __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict__ rec,
                                                          const uint4 *__restrict__ items,
                                                          const uint32_t *__restrict__ blist,
@@ -116,6 +122,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   uint32_t ent[UNR];            // list entries of the batch whose records load next
   uint32_t em = 0;              // bit u: ent[u] is an entry
   uint32_t vm = 0, nvm = 0;     // bit u: r[u] / nx[u] holds a record
+  int ue = 0, un = 0, ur = 0;   // FEW: no entries / records of nx / of r from this u on
   const TileList &T = P.list;
   // a thread's place in the blocks is the same in every batch (blocks of at
   // most 256 slots divide the 1024 threads)
@@ -181,8 +188,11 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   };
   auto load_entries = [&]() {
     em = 0;
+    ue = 0;
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
+      if (FEW && ld.rel + u * eu >= ld.ents) break;
+      ue = u + 1;
       const uint32_t e = ld.rel + u * eu + te;
       if (e < ld.ents) {
         ent[u] = blist[ld.lb + e];
@@ -192,8 +202,10 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   };
   auto load_records = [&]() {
     nvm = 0;
+    un = ue;
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
+      if (FEW && u >= ue) break;
       if (((em >> u) & 1u) && in < T.fill(ent[u])) {
         nvm |= 1u << u;
         const float *src = rec + (int64_t)(T.slot0(ent[u]) + in) * RW;
@@ -204,6 +216,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
   };
   auto take_batch = [&]() {
     vm = nvm;
+    ur = un;
 #pragma unroll
     for (int u = 0; u < UNR; u++)
 #pragma unroll
@@ -253,6 +266,7 @@ __global__ void __launch_bounds__(DEP_THREADS) k_deposit(const float *__restrict
       load_entries();
 #pragma unroll
       for (int u = 0; u < UNR; u++) {
+        if (FEW && u >= ur) break;
         if (!((vm >> u) & 1u)) continue;
         // cell_of without its wrap: a floor cell inside the tile's own cells
         // [o, o + w) lies in [0, d), where cell_of does not wrap
@@ -568,18 +582,17 @@ void deposit_impl(Plan &p, const KeyGeom &kg, const TileOrder &o, double mass) {
     Stage st(p, "deposit_tiles");
     const bool std_tiles = std_tiles_of(tg);
     const dim3 grid(L.wgs), block(DEP_THREADS);
-    if (p.prec == 4 && std_tiles)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, true>), grid, block, lds, s, sorted, L.items, L.blist,
-                         L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
-    else if (p.prec == 4)
-      hipLaunchKernelGGL((k_deposit<float, NM, RW, false>), grid, block, lds, s, sorted, L.items, L.blist,
-                         L.counts, L.cost, L.share, P, p.tiles.as<float>(), partials);
-    else if (std_tiles)
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, true>), grid, block, lds, s, sorted, L.items, L.blist,
-                         L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
-    else
-      hipLaunchKernelGGL((k_deposit<double, NM, RW, false>), grid, block, lds, s, sorted, L.items, L.blist,
-                         L.counts, L.cost, L.share, P, p.tiles.as<double>(), partials);
+    const bool few = n < tg.K * DEP_THREADS * 2;
+    auto go = [&](auto kernel, auto *tiles) {
+      hipLaunchKernelGGL(kernel, grid, block, lds, s, sorted, L.items, L.blist, L.counts, L.cost, L.share, P, tiles,
+                         partials);
+    };
+    if (p.prec == 4 && std_tiles) go(k_deposit<float, NM, RW, true>, p.tiles.as<float>());
+    else if (p.prec == 4 && few) go(k_deposit<float, NM, RW, false, true>, p.tiles.as<float>());
+    else if (p.prec == 4) go(k_deposit<float, NM, RW, false>, p.tiles.as<float>());
+    else if (std_tiles) go(k_deposit<double, NM, RW, true>, p.tiles.as<double>());
+    else if (few) go(k_deposit<double, NM, RW, false, true>, p.tiles.as<double>());
+    else go(k_deposit<double, NM, RW, false>, p.tiles.as<double>());
     GENPK_LAUNCH_CHECK();
   }
   {
